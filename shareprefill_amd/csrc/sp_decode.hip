@@ -4,7 +4,10 @@
 // HBM-bound: K and V are read exactly once (2 * n * hkv * d * 2 bytes); everything else has to stay out of the
 // way.  The cache of one kv head is split into chunks; one workgroup streams a chunk for all query heads of the
 // group (so the group's `g` heads share every K / V byte), keeps an online softmax, and leaves an unnormalised
-// partial (o, m, l); a second tiny kernel merges the partials in chunk order.
+// partial (o, m, l); a second tiny kernel merges the partials in a fixed order.  A batch of sequences is one more grid
+// axis: per token of a small model's or short chat's step the launches and the host's way to them are what counts, and
+// one pair of launches per sequence, a workspace look-up each and a stacking copy were most of it (32 query / 8 kv heads:
+// 8 caches of 4001 tokens 137 -> 29 us = 4.5 TB/s, one of 1025 tokens 24.8 -> 15.9 us, one of 131072 100.9 -> 96.8 us).
 //
 // Both products run on the matrix core with the group's heads as a (mostly empty) 32-wide operand -- the MFMAs
 // are free here, the point is to keep the vector ALU out of the inner loop:
@@ -28,6 +31,7 @@ typedef __bf16 dc_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float dc_floatx16 __attribute__((ext_vector_type(16)));
 typedef float dc_floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 dc_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float dc_floatx4 __attribute__((ext_vector_type(4), aligned(8)));  // (partials: 8-byte aligned workspace)
 
 __device__ static __forceinline__ uint32_t dc_pack2(float a, float b) {
   dc_floatx2 f;
@@ -62,24 +66,30 @@ __device__ static __forceinline__ void dc_store(sp_bf16* tile, int t, const dc_u
   for (int i = 0; i < 8; ++i) *reinterpret_cast<dc_u32x4*>(tile + (i * 16 + (t >> 4)) * DC_PITCH + (t & 15) * 8) = r[i];
 }
 
-// grid (splits, hkv); partial layout: o [hkv][splits][g][128] fp32, ml [hkv][splits][g] float2 (m in log2 units, l)
+// grid (splits, hkv, batch); partial layout: o [batch][hkv][splits][g][128] fp32, ml [batch][hkv][splits][g] float2 (m
+// in log2 units, l).  A cache that is one chunk (splits == 1) needs no merging: the result goes straight to `out`.
 // G8 = groups of 8 heads the instance handles (g <= 8 * G8): accumulator rows r < 4 * G8 can belong to real heads
+struct DcStrides {
+  int64_t q_b, q_h, k_b, k_n, k_h, v_b, v_n, v_h;
+};
 template <int G8, bool FULL>
 __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const sp_bf16* __restrict__ v, int64_t n, int g,
-    int d, int64_t sq_h, int64_t sk_n, int64_t sk_h, int64_t sv_n, int64_t sv_h, float scale_log2,
-    int64_t keys_per_split, float* __restrict__ o_part, float2* __restrict__ ml_part) {
+    int d, DcStrides st, float scale_log2, int64_t keys_per_split, float* __restrict__ o_part,
+    float2* __restrict__ ml_part, sp_bf16* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) sp_bf16 Ks[DC_TILE * DC_PITCH];
   __shared__ __attribute__((aligned(16))) sp_bf16 Vs[DC_TILE * DC_PITCH];
   constexpr int GM = 8 * G8;
   __shared__ __attribute__((aligned(16))) sp_bf16 Ps[GM * DC_PITCH];  // probabilities [head][key]
   __shared__ float wmax[4][GM], wsum[4][GM], alpha_s[GM];
   const int split = blockIdx.x, kvh = blockIdx.y, splits = gridDim.x;
+  const int64_t bh = (int64_t)blockIdx.z * gridDim.y + kvh;  // (sequence, kv head)
+  const int64_t sk_n = st.k_n, sv_n = st.v_n;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int lh = lane & 31, hi = lane >> 5;  // operand column / row inside a 32-wide tile, lane half
   const bool head_ok = lh < g;               // this lane's S^T column is a real head
-  const sp_bf16* kh = k + (int64_t)kvh * sk_h;
-  const sp_bf16* vh = v + (int64_t)kvh * sv_h;
+  const sp_bf16* kh = k + blockIdx.z * st.k_b + kvh * st.k_h;
+  const sp_bf16* vh = v + blockIdx.z * st.v_b + kvh * st.v_h;
 
   // B operand of S^T = K . Q^T: column lh = head, k-step ks covers channels 16ks + 8hi .. +7
   dc_bf16x8 qb[8];
@@ -87,7 +97,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
   for (int ks = 0; ks < 8; ++ks) {
     dc_u32x4 raw = {0, 0, 0, 0};
     if (head_ok && (FULL || 16 * ks + 8 * hi < d))
-      raw = *reinterpret_cast<const dc_u32x4*>(q + (int64_t)(kvh * g + lh) * sq_h + 16 * ks + 8 * hi);
+      raw = *reinterpret_cast<const dc_u32x4*>(q + blockIdx.z * st.q_b + (int64_t)(kvh * g + lh) * st.q_h + 16 * ks + 8 * hi);
     qb[ks] = __builtin_bit_cast(dc_bf16x8, raw);
   }
 
@@ -187,95 +197,137 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
     }
   }
 
-  float* op = o_part + (((int64_t)kvh * splits + split) * g) * DC_D;
+  if (splits == 1) {  // (uniform)
+    __syncthreads();  // the last tile's reads of wsum are done
+    if (wave == 0 && hi == 0 && head_ok) wsum[0][lh] = l_run;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4 * G8; ++r) {
+      const int h = 8 * (r >> 2) + 4 * hi + (r & 3), c = 32 * wave + lh;
+      if (h < g && c < d) out[(bh * g + h) * d + c] = sp_f32_to_bf16(o[r] / wsum[0][h]);
+    }
+    return;
+  }
+  float* op = o_part + ((bh * splits + split) * g) * DC_D;
 #pragma unroll
   for (int r = 0; r < 4 * G8; ++r) {
     const int h = 8 * (r >> 2) + 4 * hi + (r & 3);
     if (h < g) op[h * DC_D + 32 * wave + lh] = o[r];
   }
-  if (wave == 0 && hi == 0 && head_ok) ml_part[((int64_t)kvh * splits + split) * g + lh] = make_float2(m_run, l_run);
+  if (wave == 0 && hi == 0 && head_ok) ml_part[(bh * splits + split) * g + lh] = make_float2(m_run, l_run);
 }
 
-// one workgroup of 128 threads per query head: merges the chunk partials (sums in chunk order)
+// Merges the chunk partials of one query head: eight groups of 32 threads take every eighth chunk (a thread four
+// channels, 16-byte loads), the groups meet in LDS in a fixed order.  What it costs is latency -- a launch and a chain of
+// loads as deep as a group has chunks (64 chunks at 131072 keys and 8 kv heads: eight instead of sixty-four).
 #define DC_MAX_SPLITS 512
-__global__ __launch_bounds__(DC_D) void sp_decode_combine_kernel(const float* __restrict__ o_part,
-                                                                 const float2* __restrict__ ml_part, int g, int splits,
-                                                                 int d, sp_bf16* __restrict__ out) {
+#define DC_COMBINE_GROUPS 8
+__global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kernel(
+    const float* __restrict__ o_part, const float2* __restrict__ ml_part, int g, int splits, int d,
+    sp_bf16* __restrict__ out) {
+  constexpr int THREADS = 32 * DC_COMBINE_GROUPS;
   __shared__ float w_s[DC_MAX_SPLITS];  // weight of chunk s: exp2(m_s - m), 0 for an empty chunk
-  __shared__ float red[2];
-  const int hq_idx = blockIdx.x, kvh = hq_idx / g, h = hq_idx % g, c = threadIdx.x;
-  const float2* ml = ml_part + (int64_t)kvh * splits * g + h;
+  __shared__ float red[THREADS / SP_WAVE];
+  __shared__ __attribute__((aligned(16))) float o_s[DC_COMBINE_GROUPS][DC_D];
+  const int64_t head = blockIdx.x, bh = head / g;  // (sequence, query head), (sequence, kv head)
+  const int h = (int)(head % g), t = threadIdx.x, grp = t >> 5, c4 = (t & 31) * 4;
+  const float2* ml = ml_part + bh * splits * g + h;
+  const float* op = o_part + (bh * splits * g + h) * DC_D + c4;
+  // every chunk's statistics once, kept in registers between the two passes (splits <= 2 THREADS)
+  float2 mine[DC_MAX_SPLITS / THREADS];
   float m = -INFINITY;
-  for (int s = c; s < splits; s += DC_D) m = fmaxf(m, ml[(int64_t)s * g].x);
+#pragma unroll
+  for (int j = 0; j < DC_MAX_SPLITS / THREADS; ++j) {
+    mine[j] = t + j * THREADS < splits ? ml[(int64_t)(t + j * THREADS) * g] : make_float2(-INFINITY, 0.f);
+    m = fmaxf(m, mine[j].x);
+  }
   m = sp_wave_max(m);
-  if ((c & 63) == 0) red[c >> 6] = m;
+  if ((t & 63) == 0) red[t >> 6] = m;
   __syncthreads();
-  m = fmaxf(red[0], red[1]);
-  for (int s = c; s < splits; s += DC_D) {
-    const float ms = ml[(int64_t)s * g].x;
-    w_s[s] = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - m);
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  __syncthreads();
+  float l = 0.f;
+#pragma unroll
+  for (int j = 0; j < DC_MAX_SPLITS / THREADS; ++j) {
+    const float w = mine[j].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mine[j].x - m);
+    if (t + j * THREADS < splits) w_s[t + j * THREADS] = w;
+    l += mine[j].y * w;
   }
+  l = sp_wave_sum(l);
+  if ((t & 63) == 0) red[t >> 6] = l;
   __syncthreads();
-  const float* op = o_part + ((int64_t)kvh * splits * g + h) * DC_D + c;
-  float l = 0.f, o = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 8
-  for (int s = 0; s < splits; ++s) {
-    l += ml[(int64_t)s * g].y * w_s[s];
-    o += op[(int64_t)s * g * DC_D] * w_s[s];
+  for (int s = grp; s < splits; s += DC_COMBINE_GROUPS) {
+    const dc_floatx4 x = *reinterpret_cast<const dc_floatx4*>(op + (int64_t)s * g * DC_D);
+    const float w = w_s[s];
+    o.x += x[0] * w, o.y += x[1] * w, o.z += x[2] * w, o.w += x[3] * w;
   }
-  if (c < d) out[(int64_t)hq_idx * d + c] = sp_f32_to_bf16(o / l);
+  *reinterpret_cast<float4*>(&o_s[grp][c4]) = o;
+  __syncthreads();
+  if (t < d) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < DC_COMBINE_GROUPS; ++j) acc += o_s[j][t];
+    out[head * d + t] = sp_f32_to_bf16(acc / ((red[0] + red[1]) + (red[2] + red[3])));
+  }
 }
 
 // ---- host -------------------------------------------------------------------------------------------------
-static int dc_splits(int64_t n, int32_t hkv) {
+// Chunks per (sequence, kv head): about two workgroups per CU over the whole batch, which is what the kernel's LDS
+// lets a CU hold, and no chunk below one tile of keys.
+static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
   const int64_t tiles = sp_ceil_div(n, DC_TILE);
-  int64_t want = sp_ceil_div(512, hkv);  // about two workgroups per CU
+  int64_t want = sp_ceil_div(512, (int64_t)hkv * batch);
   if (want > tiles) want = tiles;
   if (want < 1) want = 1;
   if (want > DC_MAX_SPLITS) want = DC_MAX_SPLITS;
   return (int)want;
 }
 
+extern "C" size_t sp_decode_batch_workspace_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
+  if (batch <= 0 || n <= 0 || hq <= 0 || hkv <= 0) return 0;
+  return (size_t)dc_splits(batch, n, hkv) * batch * hq * (DC_D * sizeof(float) + sizeof(float2));
+}
+
 extern "C" size_t sp_decode_workspace_bytes(int64_t n, int32_t hq, int32_t hkv) {
-  if (n <= 0 || hq <= 0 || hkv <= 0) return 0;
-  return (size_t)dc_splits(n, hkv) * hq * (DC_D * sizeof(float) + sizeof(float2));
+  return sp_decode_batch_workspace_bytes(1, n, hq, hkv);
 }
 
 // argument checks shared by the two entry points
-static int dc_check(const char* who, const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
-                    int32_t d, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n,
-                    int64_t v_stride_h, float softmax_scale, const void* out) {
+static int dc_check(const char* who, const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq,
+                    int32_t hkv, int32_t d, const DcStrides& st, float softmax_scale, const void* out) {
   SP_REQUIRE(q && k && v && out, SP_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
   SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT, "%s: bad shape n=%lld hq=%d hkv=%d",
              who, (long long)n, hq, hkv);
+  SP_REQUIRE(batch > 0 && batch <= 65535, SP_ERR_UNSUPPORTED, "%s: batch %d (1 to 65535)", who, batch);
   SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "%s: softmax_scale must be > 0", who);
   SP_REQUIRE(d >= 8 && d <= DC_D && d % 8 == 0, SP_ERR_UNSUPPORTED,
              "%s: head_dim %d unsupported (a multiple of 8 up to 128)", who, d);
   SP_REQUIRE(hq / hkv <= DC_GMAX, SP_ERR_UNSUPPORTED, "%s: more than %d query heads per kv head", who, DC_GMAX);
   // q, k and v are read with 16-byte loads
-  SP_REQUIRE(q_stride_h % 8 == 0 && ((uintptr_t)q % 16) == 0, SP_ERR_UNSUPPORTED,
-             "%s: q must be 16-byte aligned with a head stride multiple of 8", who);
-  SP_REQUIRE(k_stride_n % 8 == 0 && k_stride_h % 8 == 0 && v_stride_n % 8 == 0 && v_stride_h % 8 == 0 &&
-                 ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
+  SP_REQUIRE(st.q_h % 8 == 0 && st.q_b % 8 == 0 && ((uintptr_t)q % 16) == 0, SP_ERR_UNSUPPORTED,
+             "%s: q must be 16-byte aligned with strides multiple of 8", who);
+  SP_REQUIRE(st.k_n % 8 == 0 && st.k_h % 8 == 0 && st.k_b % 8 == 0 && st.v_n % 8 == 0 && st.v_h % 8 == 0 &&
+                 st.v_b % 8 == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
              SP_ERR_UNSUPPORTED, "%s: k/v must be 16-byte aligned with strides multiple of 8", who);
   return SP_OK;
 }
 
-// both kernels; `partials` holds sp_decode_workspace_bytes(n, hq, hkv) bytes, every one of which the first kernel
-// writes before the second reads it (nothing has to be cleared)
-static int dc_launch(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv, int32_t d,
-                     int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h,
-                     float softmax_scale, void* out, void* partials, hipStream_t s) {
+// both kernels; `partials` holds sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes, every one of which the first
+// kernel writes before the second reads it (nothing has to be cleared)
+static int dc_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv,
+                     int32_t d, const DcStrides& st, float softmax_scale, void* out, void* partials, hipStream_t s) {
   const int g = hq / hkv;
-  const int splits = dc_splits(n, hkv);
+  const int splits = dc_splits(batch, n, hkv);
   const int64_t keys_per_split = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE;
   float* o_part = (float*)partials;
-  float2* ml_part = (float2*)(o_part + (size_t)splits * hq * DC_D);
+  float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
 #define DC_LAUNCH_PARTIAL_(G8, FULL)                                                                                  \
-  hipLaunchKernelGGL((sp_decode_partial_kernel<G8, FULL>), dim3(splits, hkv), dim3(DC_THREADS), 0, s, (const sp_bf16*)q, \
-                     (const sp_bf16*)k, (const sp_bf16*)v, n, g, (int)d, q_stride_h, k_stride_n, k_stride_h,          \
-                     v_stride_n, v_stride_h, scale_log2, keys_per_split, o_part, ml_part)
+  hipLaunchKernelGGL((sp_decode_partial_kernel<G8, FULL>), dim3(splits, hkv, batch), dim3(DC_THREADS), 0, s,           \
+                     (const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, n, g, (int)d, st, scale_log2,            \
+                     keys_per_split, o_part, ml_part, (sp_bf16*)out)
 #define DC_LAUNCH_PARTIAL(G8)     \
   do {                            \
     if (d == DC_D)                \
@@ -293,24 +345,38 @@ static int dc_launch(const void* q, const void* k, const void* v, int64_t n, int
 #undef DC_LAUNCH_PARTIAL
 #undef DC_LAUNCH_PARTIAL_
   SP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sp_decode_combine_kernel, dim3(hq), dim3(DC_D), 0, s, o_part, ml_part, g, splits, (int)d,
-                     (sp_bf16*)out);
+  if (splits == 1) return SP_OK;
+  hipLaunchKernelGGL(sp_decode_combine_kernel, dim3((unsigned)((int64_t)batch * hq)), dim3(32 * DC_COMBINE_GROUPS), 0, s,
+                     o_part, ml_part, g, splits, (int)d, (sp_bf16*)out);
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+extern "C" int sp_decode_attn_batch_bf16(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq,
+                                         int32_t hkv, int32_t d, int64_t q_stride_b, int64_t q_stride_h,
+                                         int64_t k_stride_b, int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_b,
+                                         int64_t v_stride_n, int64_t v_stride_h, float softmax_scale, void* out,
+                                         void* workspace, size_t workspace_bytes, sp_stream_t stream) {
+  const DcStrides st = {q_stride_b, q_stride_h, k_stride_b, k_stride_n, k_stride_h, v_stride_b, v_stride_n, v_stride_h};
+  int rc = dc_check("sp_decode_attn_batch_bf16", q, k, v, batch, n, hq, hkv, d, st, softmax_scale, out);
+  if (rc) return rc;
+  SP_REQUIRE(workspace != nullptr, SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_batch_bf16: null workspace");
+  SP_REQUIRE(workspace_bytes >= sp_decode_batch_workspace_bytes(batch, n, hq, hkv) && ((uintptr_t)workspace % 8) == 0,
+             SP_ERR_WORKSPACE, "sp_decode_attn_batch_bf16: workspace too small or misaligned");
+  return dc_launch(q, k, v, batch, n, hq, hkv, d, st, softmax_scale, out, workspace, (hipStream_t)stream);
 }
 
 extern "C" int sp_decode_attn_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
                                    int32_t d, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
                                    int64_t v_stride_n, int64_t v_stride_h, float softmax_scale, void* out,
                                    void* workspace, size_t workspace_bytes, sp_stream_t stream) {
-  int rc = dc_check("sp_decode_attn_bf16", q, k, v, n, hq, hkv, d, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
-                    v_stride_h, softmax_scale, out);
+  const DcStrides st = {0, q_stride_h, 0, k_stride_n, k_stride_h, 0, v_stride_n, v_stride_h};
+  int rc = dc_check("sp_decode_attn_bf16", q, k, v, 1, n, hq, hkv, d, st, softmax_scale, out);
   if (rc) return rc;
   SP_REQUIRE(workspace != nullptr, SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_bf16: null workspace");
   SP_REQUIRE(workspace_bytes >= sp_decode_workspace_bytes(n, hq, hkv) && ((uintptr_t)workspace % 8) == 0,
              SP_ERR_WORKSPACE, "sp_decode_attn_bf16: workspace too small or misaligned");
-  return dc_launch(q, k, v, n, hq, hkv, d, q_stride_h, k_stride_n, k_stride_h, v_stride_n, v_stride_h, softmax_scale, out,
-                   workspace, (hipStream_t)stream);
+  return dc_launch(q, k, v, 1, n, hq, hkv, d, st, softmax_scale, out, workspace, (hipStream_t)stream);
 }
 
 // ---- the same step for callers that cannot allocate ---------------------------------------------------------------
@@ -343,8 +409,8 @@ extern "C" int sp_decode_attn_static_bf16(const void* q, const void* k, const vo
                                           int32_t hkv, int32_t d, int64_t q_stride_h, int64_t k_stride_n,
                                           int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h,
                                           float softmax_scale, void* out, sp_stream_t stream) {
-  int rc = dc_check("sp_decode_attn_static_bf16", q, k, v, n, hq, hkv, d, q_stride_h, k_stride_n, k_stride_h,
-                    v_stride_n, v_stride_h, softmax_scale, out);
+  const DcStrides st = {0, q_stride_h, 0, k_stride_n, k_stride_h, 0, v_stride_n, v_stride_h};
+  int rc = dc_check("sp_decode_attn_static_bf16", q, k, v, 1, n, hq, hkv, d, st, softmax_scale, out);
   if (rc) return rc;
   const size_t need = sp_decode_workspace_bytes(n, hq, hkv);
   SP_REQUIRE(need <= DC_STATIC_BYTES, SP_ERR_WORKSPACE,
@@ -354,6 +420,5 @@ extern "C" int sp_decode_attn_static_bf16(const void* q, const void* k, const vo
   void* partials = nullptr;
   rc = dc_static_scratch(&partials);
   if (rc) return rc;
-  return dc_launch(q, k, v, n, hq, hkv, d, q_stride_h, k_stride_n, k_stride_h, v_stride_n, v_stride_h, softmax_scale, out,
-                   partials, (hipStream_t)stream);
+  return dc_launch(q, k, v, 1, n, hq, hkv, d, st, softmax_scale, out, partials, (hipStream_t)stream);
 }

@@ -366,6 +366,35 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_
     return out
 
 
+def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float) -> torch.Tensor:
+    """One new token per sequence: q bf16 [B, Hq, 1, D], k / v bf16 [B, Hkv, N, D] views -> out bf16 [B, 1, Hq, D].
+
+    The whole batch runs in the launches of one sequence (decode_attention: the same kernels)."""
+    lib = _lib.load()
+    b, hq, _, d = q.shape
+    _, hkv, n, _ = k.shape
+    dev = q.device
+    for t, name in ((q, "q"), (k, "k"), (v, "v")):
+        if t.dtype != torch.bfloat16:
+            raise AssertionError(f"{name} must be bfloat16, got {t.dtype}")
+        if not t.is_cuda or t.device != dev:
+            raise ValueError(f"{name} must live on the GPU the queries are on")
+        if t.stride(3) != 1:
+            raise ValueError(f"{name} must have a contiguous head_dim axis")
+    if v.shape != k.shape or k.shape[0] != b or k.shape[3] != d:
+        raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} do not match q {tuple(q.shape)}")
+    stream = _stream_handle(dev)
+    out = torch.empty((b, 1, hq, d), dtype=torch.bfloat16, device=dev)
+    ws = _workspace("decode", lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv), dev)
+    (q_b, q_h, _, _), (k_b, k_h, k_n, _), (v_b, v_h, v_n, _) = q.stride(), k.stride(), v.stride()
+    if b == 1:
+        q_b = k_b = v_b = 0  # (the stride of an axis of one entry means nothing)
+    st = lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b, n, hq, hkv, d, q_b, q_h, k_b, k_n, k_h,
+                                       v_b, v_n, v_h, softmax_scale, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+    _lib.check(st, "sp_decode_attn_batch_bf16")
+    return out
+
+
 def rope_inplace(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> None:
     """Rotates q bf16 [Hq, N, D] and k bf16 [Hkv, N, D] (views with any token / head strides, contiguous head_dim)
     in place by the position embeddings cos / sin bf16 [N, D]:  x <- x*cos + rotate_half(x)*sin  with the roundings

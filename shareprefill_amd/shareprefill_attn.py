@@ -158,9 +158,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         # else raises from the entry point's own checks, as every other unsupported shape does.
         if query_states.dtype != torch.bfloat16:
             raise AssertionError(f"SharePrefill attention expects bfloat16 q/k/v, got {query_states.dtype}")
-        outs = [ops.decode_attention(query_states[b, :, 0], key_states[b], value_states[b], softmax_scale)
-                for b in range(bsz)]
-        return torch.stack(outs).unsqueeze(2), None
+        return ops.decode_attention_batch(query_states, key_states, value_states, softmax_scale).transpose(1, 2), None
 
     if bsz != 1:
         raise ValueError("SharePrefill prefill keeps per-cluster state for batch size 1 only")

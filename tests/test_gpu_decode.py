@@ -99,3 +99,22 @@ def test_decode_rejects_unsupported(gpu_device):
         q, k, v = _inputs(4, 2, 256, 1, d=d)
         with pytest.raises(NotImplementedError):
             ops.decode_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), 0.1)
+
+
+@pytest.mark.parametrize("b,hq,hkv,n,d", [(1, 8, 2, 1, 128), (3, 8, 2, 127, 128), (5, 28, 4, 129, 128), (2, 14, 2, 2049, 64),
+                                          (64, 8, 8, 300, 128), (65, 16, 8, 128, 64)])
+def test_decode_batch_matches_oracle(gpu_device, b, hq, hkv, n, d):
+    """Every sequence of a batch against the fp32 oracle: one key, ragged tiles, caches cut into several chunks and
+    caches that are a single chunk each (enough sequences to fill the chip: the kernel writes the result itself)."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator().manual_seed(b * n)
+    mk = lambda h, m: torch.randn(b, h, m, d, generator=gen).to(torch.bfloat16)
+    q, k, v = mk(hq, 1), mk(hkv, n), mk(hkv, n)
+    scale = d ** -0.5
+    out = ops.decode_attention_batch(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), scale).cpu().float()
+    assert out.shape == (b, 1, hq, d)
+    for i in sorted({0, b // 2, b - 1}):
+        ref = O.decode_attention(q[i, :, 0], k[i], v[i], scale)
+        assert (out[i, 0] - ref).abs().max().item() <= MAX_ABS
+        assert ((out[i, 0] - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
