@@ -224,6 +224,18 @@ int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, i
                                   float* avg_attn, void* workspace, size_t workspace_bytes, uint32_t flags,
                                   sp_stream_t stream);
 
+/* The same attention for short prompts, bs = 128, d = 64 or 128 (no padding): one kernel that reads v as it is, needs no
+ * repack and no scheduler area, and writes the pivot heads' maps itself.  Correct for any n up to 65536;
+ * sp_short_attn_max_tokens(d) is the length up to which it is the faster of the two.
+ * workspace: sp_short_attn_workspace_bytes(n, hq) bytes, needed only with decision and avg_attn (block sums). */
+int64_t sp_short_attn_max_tokens(int32_t d);
+size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq);
+int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                           int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
+                           int64_t v_stride_n, int64_t v_stride_h, float softmax_scale, const uint64_t* mask,
+                           const int32_t* decision, void* out, float* avg_attn, void* workspace,
+                           size_t workspace_bytes, sp_stream_t stream);
+
 /* ---- decode step -------------------------------------------------------------------------------
  * Replaces the flash_attn_func call of the decode branch (shareprefill_attn.py:146-155): one query token per
  * head against the whole KV cache, no mask.  q: bf16 [hq][d] (head stride in elements), k / v: bf16

@@ -1,0 +1,499 @@
+// Block-sparse causal attention for short prompts (same operation as sp_attn.hip, which takes the long ones).
+//
+// A launch over a few thousand tokens is bound by latency, not by the matrix cores: the persistent kernel's work item --
+// two rows of up to 128 keys per block step, a ticket, a block list, two barriers and an epilogue around it -- is too
+// large a part of the launch (3001 tokens, 32 heads: 384 items of up to 16 block steps on 256 CUs), and the launches that
+// prepare it (V repack, tickets, pairing) cost as much as the arithmetic of a short prompt.  This kernel needs none of
+// them and cuts the work finer:
+//   * one workgroup per (128-query block, head), 4 waves of 32 queries, two workgroups per CU (three with 64 channels): K and
+//     V tiles of 64 keys double-buffered in LDS, one barrier per tile, and a plain loop of S, softmax and P.V.  Workgroups of
+//     different rows run out of step, so one's matrix instructions fall into another's softmax; the persistent kernel's
+//     software pipeline inside the wave was built here too and measured the same (a wave alone issues an instruction about
+//     every 8 cycles, whatever it is), at twice the code;
+//   * launches that leave CUs half empty (at most two rows per CU) split a row's keys over two sets of four waves, set s taking
+//     half s of every block, and merge the two results through LDS: the chain of tiles is half as long (700 tokens, 32
+//     heads: 21.4 -> 18 us, 1500: 38.6 -> 32);
+//   * workgroups are dispatched heaviest row first, all heads of one row before the next; a CU that finishes a row takes
+//     the next one, which balances causal rows without tickets.  The query heads of a kv group share an XCD (one L2) for a
+//     row; the XCDs trade groups from row to row, or heads that keep more blocks than others would leave the other XCDs idle
+//     (8192 tokens, the bench masks: 333 us with a fixed assignment, 195 with the rotating one);
+//   * V is read as it is: the tile is row-major in LDS and the V^T operand comes from the transposing LDS read
+//     (ds_read_b64_tr_b16: the 16 lanes of a group address 4 keys x 16 channels and each receives 4 keys of its channel).
+//     S^T = K . Q^T leaves a lane with keys 4g .. 4g+3 of every 16-key tile (g = lane / 16), which is exactly what two such
+//     reads deliver, so P^T is the S^T accumulators converted to bf16 in place;
+//   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel).
+// Two rows sharing one K / V tile, as in the persistent kernel, halve the tile traffic per flop, which is why that one
+// stays for long prompts; sp_short_attn_max_tokens holds the line between the two and the figures.
+#include "sp_common.h"
+
+#include <type_traits>
+
+struct AsArgs {
+  const sp_bf16 *q, *k, *v;
+  const uint64_t* mask;      // [hq][nb][nbw]
+  const int32_t* decision;   // [hq] or null
+  sp_bf16* out;              // [n][hq][D]
+  float* avg_attn;           // [hq][nb][nb], written for pivot heads
+  float* tile_sums;          // [hq][nb (nb + 1) / 2][2][128] of pivot heads, or null: no maps wanted
+  int64_t n, sq_n, sq_h, sk_n, sk_h, sv_n, sv_h;
+  int hq, group, nb, nbw;
+  float scale_log2;
+};
+
+typedef __bf16 as_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 as_bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 as_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float as_floatx4 __attribute__((ext_vector_type(4)));
+typedef float as_floatx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t as_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
+
+#define AS_BS 128
+#define AS_TILE 64      // keys per step
+#define AS_THREADS 256  // 4 waves x 32 queries
+#define AS_WAVES 4
+#define AS_MAX_NB 512     // blocks a row's list holds
+#define AS_LDS_BYTES(D, KSPLIT) ((KSPLIT) * 4 * AS_TILE * (D) * 2)
+#define AS_HEADROOM 24.0f  // octaves the running max is set above the largest logit seen
+#define AS_NO_MAX (-1.0e30f)         // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
+#define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
+
+typedef __attribute__((address_space(3))) void* as_lds_ptr;
+typedef const __attribute__((address_space(1))) void* as_gbl_ptr;
+
+// K and V tiles are [64 keys][D] bf16 in 16-byte chunks, the chunk index XOR-swizzled by the row so that both kinds of
+// operand read are free of bank conflicts: the K read (one chunk of 16 consecutive rows) and the transposing V read (two
+// neighbouring chunks of 16 consecutive rows).  Rows of 64 channels are half a bank cycle long: two rows share a swizzle.
+template <int D>
+__device__ __forceinline__ int as_swz(int row) {
+  return D == 128 ? (row & 15) : ((row >> 1) & 7);
+}
+
+__device__ __forceinline__ uint32_t as_pack2(float a, float b) {
+  as_floatx2 f;
+  f[0] = a;
+  f[1] = b;
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, as_bf16x2));
+}
+
+// One tile by direct global -> LDS 128-bit loads: a wave-instruction fills 1 KiB (lane i writes chunk base + i and fetches
+// whichever chunk belongs there).  Row and swizzle of a lane are the same in every instruction up to a uniform step, so a
+// lane's address is a uniform base plus an offset made once; only the tile that reaches past the sequence clamps its rows
+// onto the last key (such keys lie behind every stored query).
+template <int D>
+__device__ __forceinline__ uint32_t as_lane_off(int64_t stride_n, int wave, int lane) {
+  constexpr int CHUNKS = D / 8, ROWS = 64 / CHUNKS;  // chunks per row, rows per wave-instruction
+  const int row = wave * ROWS + lane / CHUNKS;
+  return (uint32_t)(row * (int)stride_n + ((lane % CHUNKS) ^ as_swz<D>(row)) * 8) * 2u;
+}
+template <int D>
+__device__ __forceinline__ void as_issue(const sp_bf16* __restrict__ x, int64_t stride_n, int64_t key0, int64_t n,
+                                         uint32_t lane_off, char* tile, int wave, int lane) {
+  constexpr int CHUNKS = D / 8, ROWS = 64 / CHUNKS;
+  constexpr int STEP = ROWS * AS_WAVES, ITS = AS_TILE / STEP;  // rows per instruction of all waves (a multiple of the swizzle's period)
+  if (key0 + AS_TILE <= n) {
+    const char* base = reinterpret_cast<const char*>(x + key0 * stride_n);
+#pragma unroll
+    for (int it = 0; it < ITS; ++it)
+      __builtin_amdgcn_global_load_lds((as_gbl_ptr)(base + (int64_t)it * STEP * 2 * stride_n + lane_off),
+                                       (as_lds_ptr)(tile + (it * AS_WAVES + wave) * 1024), 16, 0, 0);
+  } else {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // (keeps this rare path's lane arithmetic out of the tile loop)
+#pragma unroll 1
+    for (int it = 0; it < ITS; ++it) {
+      const int seg = it * AS_WAVES + wave, row = seg * ROWS + ln / CHUNKS;
+      int64_t key = key0 + row;
+      if (key > n - 1) key = n - 1;
+      __builtin_amdgcn_global_load_lds((as_gbl_ptr)(x + key * stride_n + ((ln % CHUNKS) ^ as_swz<D>(row)) * 8),
+                                       (as_lds_ptr)(tile + seg * 1024), 16, 0, 0);
+    }
+  }
+}
+
+// Transposing LDS read the compiler does not track (valid after as_wait_v on the same registers).  Through the builtin it
+// waits for every direct-to-LDS load in flight before each of these reads -- the next tile's whole memory latency in
+// every step: 1.6 us per 64 keys where the arithmetic takes half of that.
+template <int IMM>
+__device__ __forceinline__ as_u32x2 as_read_tr(uint32_t addr) {
+  as_u32x2 r;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(IMM));
+  return r;
+}
+template <int N>
+__device__ __forceinline__ void as_wait_v(as_u32x2 (&r)[8]) {  // all but the N youngest LDS reads have landed
+  asm volatile("s_waitcnt lgkmcnt(%8)"
+               : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7])
+               : "n"(N));
+}
+template <int K, int N, typename F>
+__device__ __forceinline__ void as_static_for(F&& f) {
+  if constexpr (K < N) {
+    f(std::integral_constant<int, K>{});
+    as_static_for<K + 1, N>(f);
+  }
+}
+
+// max over the lanes l, l ^ 16, l ^ 32, l ^ 48 that share a query
+__device__ __forceinline__ float as_groupmax(float v) {
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  u = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+// KSPLIT = 2: two sets of four waves own the same queries and take the even and the odd 64-key tiles.
+template <int D, int KSPLIT>
+__global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(AsArgs a) {
+  constexpr int QT = 2;                             // 16-query tiles per wave
+  constexpr int KS = D / 32, CT = D / 16;           // channel steps of S, channel tiles of O
+  constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS * KSPLIT, WQ = 16 * QT;
+  constexpr int TILE_BYTES = AS_TILE * D * 2;
+  extern __shared__ __attribute__((aligned(1024))) char lds_all[];  // per set of waves [buffer][K | V]
+  __shared__ uint16_t list[AS_MAX_NB];
+  const int t = threadIdx.x, lane = t & 63, lq = lane & 15, g = lane >> 4;
+  const int wave8 = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wave = wave8 % WAVES, set = wave8 / WAVES;  // query band, set
+  char* const lds = lds_all + set * 4 * TILE_BYTES;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
+  int h, rr;  // head, rank of the row (0 = the last, heaviest one)
+  if ((a.hq & 7) == 0) {
+    const int per = a.hq >> 3, i = blockIdx.x >> 3;
+    rr = i / per;
+    h = ((blockIdx.x + rr) & 7) * per + i % per;
+  } else {
+    h = blockIdx.x % a.hq;
+    rr = blockIdx.x / a.hq;
+  }
+  const int r = a.nb - 1 - rr;
+  const int kvh = h / a.group;
+  const sp_bf16* kh = a.k + (int64_t)kvh * a.sk_h;
+  const sp_bf16* vh = a.v + (int64_t)kvh * a.sv_h;
+
+  const int q_off = wave * WQ + lq;  // the first of the lane's queries; the others are 16 further each
+  const int64_t qrow = (int64_t)r * AS_BS + q_off;
+  as_bf16x8 qb[QT][KS];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int64_t qr = qrow + 16 * qt < a.n ? qrow + 16 * qt : a.n - 1;
+    const sp_bf16* src = a.q + (int64_t)h * a.sq_h + qr * a.sq_n + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qb[qt][ks] = __builtin_bit_cast(as_bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
+  }
+  const uint32_t k_lane = as_lane_off<D>(a.sk_n, wave, lane), v_lane = as_lane_off<D>(a.sv_n, wave, lane);
+  auto issue = [&](int c, int half, int buf) {
+    const int64_t key0 = (int64_t)c * AS_BS + half * AS_TILE;
+    // (a last block that ends in its first half: the second half is all beyond the sequence; its one key is the last)
+    const int64_t k0 = key0 < a.n ? key0 : a.n - 1;
+    as_issue<D>(kh, a.sk_n, k0, a.n, k_lane, lds + buf * 2 * TILE_BYTES, wave, lane);
+    as_issue<D>(vh, a.sv_n, k0, a.n, v_lane, lds + buf * 2 * TILE_BYTES + TILE_BYTES, wave, lane);
+  };
+  // the row's kept blocks, ascending: every wave counts the (uniform) mask words, wave w compacts its share of them
+  int n_blk = 0, c = 0;
+  {
+    const uint64_t* row = a.mask + ((int64_t)h * a.nb + r) * a.nbw;
+    for (int wi = 0; wi <= (r >> 6); ++wi) {
+      uint64_t x = row[wi];
+      if (wi == (r >> 6) && (r & 63) != 63) x &= (2ull << (r & 63)) - 1ull;
+      if (n_blk == 0 && x != 0ull) {  // the first tile is on its way while the list is made
+        c = wi * 64 + __builtin_ctzll(x);
+        issue(c, set, 0);
+      }
+      if ((wi % (WAVES * KSPLIT)) == wave8 && ((x >> lane) & 1ull))
+        list[n_blk + __builtin_popcountll(x & ((1ull << lane) - 1ull))] = (uint16_t)(wi * 64 + lane);
+      n_blk += __builtin_popcountll(x);
+    }
+    n_blk = __builtin_amdgcn_readfirstlane(n_blk);
+  }
+  // the list is complete (a plain __syncthreads would wait for the first tile as well)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  as_floatx4 o[CT][QT], l[QT];  // l: row sums (ones . P, every row of the tile holds the sum)
+  float m[QT], l_mark[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) o[ct][qt] = (as_floatx4){0, 0, 0, 0};
+    l[qt] = (as_floatx4){0, 0, 0, 0};
+    m[qt] = AS_NO_MAX;
+    l_mark[qt] = 0.f;
+  }
+  const as_bf16x8 ones = __builtin_bit_cast(as_bf16x8, (as_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+  // pivot heads: this row's sums per 64-key tile, [column][half][128 queries]
+  float* const pu = a.tile_sums == nullptr || a.decision[h] != SP_DEC_DENSE
+                        ? nullptr
+                        : a.tile_sums + ((int64_t)h * ((int64_t)a.nb * (a.nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * (2 * AS_BS);
+
+  // LDS byte offsets of the lane's operands: K row lq, logical chunk 4 ks + g; V row 4 g + lq / 4, 8-byte piece lq % 4 of the
+  // 32 bytes of channel tile ct.  Rows 16 further have the same swizzle.
+  const int koff = lq * (D * 2), kswz = as_swz<D>(lq);
+  const int vrow = 4 * g + (lq >> 2);
+  const int voff = vrow * (D * 2) + 8 * (lq & 1), vswz = as_swz<D>(vrow), vhalf = (lq >> 1) & 1;
+
+  int c_next = 0;
+  // One step per tile of the set: KSPLIT = 1 walks both halves of every block, KSPLIT = 2 one half each.  The block list is
+  // read a block ahead of its use.
+  const int steps = KSPLIT == 1 ? 2 * n_blk : n_blk;
+  for (int st = 0; st < steps; ++st) {
+    const int i = KSPLIT == 1 ? st >> 1 : st, half = KSPLIT == 1 ? (st & 1) : set, buf = st & 1;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of the tile have landed
+    __syncthreads();                     // ... everybody's; and the other buffer's readers are done
+    if (KSPLIT == 1 && half == 0) {
+      issue(c, 1, buf ^ 1);
+      c_next = (int)list[i + 1 < n_blk ? i + 1 : i];
+    } else if (i + 1 < n_blk) {
+      if (KSPLIT == 2) c_next = (int)list[i + 1];
+      c_next = __builtin_amdgcn_readfirstlane(c_next);
+      issue(c_next, KSPLIT == 1 ? 0 : set, buf ^ 1);
+    }
+    const bool diag = c == r;
+    if (!diag || half * AS_TILE <= wave * WQ + WQ - 1) {  // (else: every key of the tile lies behind the wave's queries)
+      const char* kt_buf = lds + buf * 2 * TILE_BYTES;
+      const uint32_t vt_addr = lds_base + (uint32_t)(buf * 2 * TILE_BYTES + TILE_BYTES + voff);
+      as_floatx4 s[4][QT];
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) s[kt][qt] = (as_floatx4){0, 0, 0, 0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const as_u32x4 raw = *reinterpret_cast<const as_u32x4*>(kt_buf + kt * 16 * (D * 2) + koff + (((4 * ks + g) ^ kswz) << 4));
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt)
+            s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), qb[qt][ks], s[kt][qt], 0, 0, 0);
+        }
+      }
+      if (diag) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (half * AS_TILE + 16 * kt + 4 * g + j > q_off + 16 * qt) s[kt][qt][j] = -INFINITY;
+      }
+      uint32_t pk[QT][8];
+      auto softmax = [&](int qt) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          float e[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][qt][j], a.scale_log2, -m[qt]));
+          pk[qt][2 * kt] = as_pack2(e[0], e[1]);
+          pk[qt][2 * kt + 1] = as_pack2(e[2], e[3]);
+        }
+      };
+      uint32_t det = 0u;
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        softmax(qt);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) det |= pk[qt][i] | pk[qt][i + 1];
+      }
+      // The running max is lazy, as in the persistent kernel: it moves only when some probability came out at 2 or more
+      // (or is inf: a row's first keys), and then this tile's probabilities are formed again before they are used.
+      if (__ballot((det & AS_P_TOO_LARGE) != 0u) != 0ull) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          float mx = -INFINITY;
+#pragma unroll
+          for (int kt = 0; kt < 4; ++kt)
+            mx = fmaxf(mx, fmaxf(fmaxf(s[kt][qt][0], s[kt][qt][1]), fmaxf(s[kt][qt][2], s[kt][qt][3])));
+          const float m_new = fmaxf(m[qt], as_groupmax(mx) * a.scale_log2 + AS_HEADROOM);
+          const float alpha = __builtin_amdgcn_exp2f(m[qt] - m_new);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) o[ct][qt] *= alpha;
+          l[qt] *= alpha;
+          l_mark[qt] *= alpha;
+          m[qt] = m_new;
+          softmax(qt);
+        }
+      }
+      // O += V^T . P: groups of four channel tiles of one 32-key half, the next group's operands on their way
+      constexpr int GR = CT / 2;  // groups
+      as_u32x2 vr[2][8];
+      auto fetch = [&](auto gc) {
+        constexpr int gi = decltype(gc)::value, hh = gi / (GR / 2), c0 = (gi % (GR / 2)) * 4;
+        as_static_for<0, 4>([&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          const uint32_t ad = vt_addr + (uint32_t)(((2 * (c0 + u) + vhalf) ^ vswz) << 4);
+          vr[gi & 1][2 * u] = as_read_tr<hh * 32 * (D * 2)>(ad);
+          vr[gi & 1][2 * u + 1] = as_read_tr<hh * 32 * (D * 2) + 16 * (D * 2)>(ad);
+        });
+      };
+      fetch(std::integral_constant<int, 0>{});
+      as_static_for<0, GR>([&](auto gc) {
+        constexpr int gi = decltype(gc)::value, hh = gi / (GR / 2), c0 = (gi % (GR / 2)) * 4;
+        if constexpr (gi + 1 < GR) {
+          fetch(std::integral_constant<int, gi + 1>{});
+          as_wait_v<8>(vr[gi & 1]);
+        } else {
+          as_wait_v<0>(vr[gi & 1]);
+        }
+        as_bf16x8 p[QT];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+          p[qt] = __builtin_bit_cast(as_bf16x8, (as_u32x4){pk[qt][4 * hh], pk[qt][4 * hh + 1], pk[qt][4 * hh + 2], pk[qt][4 * hh + 3]});
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const as_u32x4 raw = __builtin_shufflevector(vr[gi & 1][2 * u], vr[gi & 1][2 * u + 1], 0, 1, 2, 3);
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt)
+            o[c0 + u][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), p[qt], o[c0 + u][qt], 0, 0, 0);
+        }
+        if constexpr (c0 == 0) {
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) l[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[qt], l[qt], 0, 0, 0);
+        }
+      });
+    }
+    if (pu != nullptr) {  // pivot head: the tile's softmax mass, log2 units (-inf where the wave skipped the tile)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const float u = __builtin_amdgcn_logf(l[qt][0] - l_mark[qt]) + m[qt];
+        l_mark[qt] = l[qt][0];
+        if (g == 0) pu[(int64_t)(2 * c + half) * AS_BS + q_off + 16 * qt] = u;
+      }
+    }
+    if (KSPLIT == 2 || half == 1) c = c_next;
+  }
+
+  if constexpr (KSPLIT == 2) {  // the second set hands its O, max and sums over through LDS (its own tile buffers' space)
+    as_floatx4* const xo = reinterpret_cast<as_floatx4*>(lds_all) + wave * (CT * QT) * 64 + lane;  // [wave][ct, qt][lane]
+    float2* const xs = reinterpret_cast<float2*>(lds_all + AS_BS * D * 4) + (wave * QT) * 64 + lane;  // [set][wave][qt][lane]
+    __syncthreads();  // the tiles are consumed
+    if (set == 1) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) xo[(ct * QT + qt) * 64] = o[ct][qt];
+    }
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) xs[(set * WAVES * QT + qt) * 64] = make_float2(m[qt], l[qt][0]);
+    __syncthreads();
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const float2 x = xs[((set ^ 1) * WAVES * QT + qt) * 64];
+      const float m_new = fmaxf(m[qt], x.x);
+      const float mine = __builtin_amdgcn_exp2f(m[qt] - m_new), other = __builtin_amdgcn_exp2f(x.x - m_new);
+      m[qt] = m_new;
+      // (one expression for both sets, so that both hold the same sum)
+      l[qt][0] = set == 0 ? l[qt][0] * mine + x.y * other : x.y * other + l[qt][0] * mine;
+      if (set == 0) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) o[ct][qt] = o[ct][qt] * mine + xo[(ct * QT + qt) * 64] * other;
+      }
+    }
+  }
+  float inv_l[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    inv_l[qt] = 1.0f / l[qt][0];
+    if (set == 0 && qrow + 16 * qt < a.n) {
+      sp_bf16* dst = a.out + ((qrow + 16 * qt) * a.hq + h) * D + 4 * g;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        *reinterpret_cast<uint2*>(dst + ct * 16) = make_uint2(as_pack2(o[ct][qt][0] * inv_l[qt], o[ct][qt][1] * inv_l[qt]),
+                                                              as_pack2(o[ct][qt][2] * inv_l[qt], o[ct][qt][3] * inv_l[qt]));
+    }
+  }
+  if (pu == nullptr) return;  // (uniform)
+  // pivot head: avg[r][c] = mean over the block's valid queries of (sum of the two halves' exp2(u - m[q])) / l[q].  A wave
+  // reads back its own sums (its own stores), folds its queries, and the waves meet in LDS.
+  float* const part = reinterpret_cast<float*>(lds_all);  // [block][wave]
+  __syncthreads();                                        // LDS is free, the stores of pu have left
+  for (int i = 0; i < n_blk; ++i) {
+    const int c = (int)list[i];
+    float x = 0.f;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+      if (qrow + 16 * qt < a.n) {
+        const float* u = pu + (int64_t)(2 * c) * AS_BS + q_off + 16 * qt;
+#pragma unroll
+        for (int hf = 0; hf < 2; hf += KSPLIT)
+          x += __builtin_amdgcn_exp2f(u[(hf + set) * AS_BS] - m[qt]) * inv_l[qt];
+      }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, SP_WAVE);
+    if (lane == 0) part[i * (WAVES * KSPLIT) + wave8] = x;
+  }
+  __syncthreads();
+  const int64_t rem = a.n - (int64_t)r * AS_BS;
+  const float inv_q = 1.0f / (float)(rem < AS_BS ? (int)rem : AS_BS);
+  for (int i = t; i < n_blk; i += THREADS) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES * KSPLIT; ++w) x += part[i * (WAVES * KSPLIT) + w];
+    a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = x * inv_q;
+  }
+}
+
+// ---- host ---------------------------------------------------------------------------------------------
+// The line between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs on a dense
+// mask (32 query / 8 kv heads, whole call with everything it launches, one box, us here / there): 128 channels, dense mask
+// 4096 tokens 146 / 172, 6177 321 / 313, 8192 551 / 477; the bench masks at coverage 0.95 4096 58 / 87, 6177 96 / 121, 8192
+// 176 / 190, 16384 738 / 637.  64 channels, where the persistent kernel computes on zero-padded tiles: dense 8192 310 / 324,
+// 24576 2671 / 2629, the bench masks 8192 115 / 150, 32768 1886 / 1761, plus there the padding itself.
+extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
+  return d == 64 ? 32768 : 6656;
+}
+
+extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {
+  if (n <= 0 || hq <= 0) return 0;
+  const size_t nb = (size_t)sp_ceil_div(n, AS_BS);
+  return (size_t)hq * (nb * (nb + 1) / 2) * 2 * AS_BS * sizeof(float);
+}
+
+extern "C" int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
+                                      int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                      int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,
+                                      const uint64_t* mask, const int32_t* decision, void* out, float* avg_attn,
+                                      void* workspace, size_t workspace_bytes, sp_stream_t stream) {
+  SP_REQUIRE(q && k && v && mask && out, SP_ERR_INVALID_ARGUMENT, "sp_short_attn_fwd_bf16: null pointer");
+  SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT,
+             "sp_short_attn_fwd_bf16: bad shape n=%lld hq=%d hkv=%d", (long long)n, hq, hkv);
+  SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "sp_short_attn_fwd_bf16: softmax_scale must be > 0");
+  SP_REQUIRE(d == 128 || d == 64, SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: head_dim %d unsupported (64 or 128)", d);
+  SP_REQUIRE((q_stride_n | q_stride_h | k_stride_n | k_stride_h | v_stride_n | v_stride_h) % 8 == 0 &&
+                 ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0,
+             SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: tensors must be 16-byte aligned, strides multiple of 8");
+  SP_REQUIRE(k_stride_n >= 0 && v_stride_n >= 0 && AS_BS * k_stride_n < (1ll << 31) && AS_BS * v_stride_n < (1ll << 31),
+             SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: token strides %lld / %lld unsupported", (long long)k_stride_n,
+             (long long)v_stride_n);
+  const int64_t nb = sp_ceil_div(n, AS_BS);
+  SP_REQUIRE(nb <= AS_MAX_NB && nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: n=%lld hq=%d too large",
+             (long long)n, hq);
+  const bool maps = decision != nullptr && avg_attn != nullptr;
+  SP_REQUIRE(!maps || (workspace && workspace_bytes >= sp_short_attn_workspace_bytes(n, hq) && ((uintptr_t)workspace % 4) == 0),
+             SP_ERR_WORKSPACE, "sp_short_attn_fwd_bf16: workspace missing, misaligned or too small");
+  const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
+                    maps ? (float*)workspace : nullptr, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
+                    v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), softmax_scale * 1.4426950408889634f};
+  const dim3 grid((unsigned)(nb * hq));
+  // Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
+  // 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).
+  const bool split = nb * hq <= 512;
+  static bool attr_set[64] = {false};  // per device, once (idempotent)
+  int dev = 0;
+  SP_HIP(hipGetDevice(&dev));
+  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: device index %d", dev);
+  if (!attr_set[dev]) {
+    const void* kernels[4] = {(const void*)sp_attn_short_kernel<64, 1>, (const void*)sp_attn_short_kernel<128, 1>,
+                              (const void*)sp_attn_short_kernel<64, 2>, (const void*)sp_attn_short_kernel<128, 2>};
+    for (const void* f : kernels)
+      SP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AS_LDS_BYTES(128, 2)));
+    attr_set[dev] = true;
+  }
+  auto launch = [&](auto kernel, int ksplit) {
+    hipLaunchKernelGGL(kernel, grid, dim3(AS_THREADS * ksplit), AS_LDS_BYTES(d, ksplit), (hipStream_t)stream, a);
+  };
+  if (d == 64)
+    split ? launch(sp_attn_short_kernel<64, 2>, 2) : launch(sp_attn_short_kernel<64, 1>, 1);
+  else
+    split ? launch(sp_attn_short_kernel<128, 2>, 2) : launch(sp_attn_short_kernel<128, 1>, 1);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}

@@ -334,6 +334,36 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     return out
 
 
+def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None) -> torch.Tensor:
+    """block_sparse_attention for short prompts (block size 128, head_dim 64 or 128): q [Hq,N,D], k/v [Hkv,N,D] views,
+    mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D].  One launch, whatever decision says: v is read as it is and the maps of
+    DENSE heads are written by the same kernel."""
+    lib = _lib.load()
+    _check_hnd(q, "q")
+    _check_hnd(k, "k")
+    _check_hnd(v, "v")
+    hq, n, d = q.shape
+    assert n == k.shape[1] == v.shape[1], "q_len must equal k_len"
+    assert mask.is_contiguous() and mask.dtype == torch.int64
+    dev = q.device
+    stream = _stream_handle(dev)
+    out = torch.empty(n, hq, d, dtype=torch.bfloat16, device=dev)
+    ws, ws_bytes = None, 0
+    if decision is not None and avg_attn is not None:
+        ws_bytes = lib.sp_short_attn_workspace_bytes(n, hq)
+        ws = _workspace("attn_short", ws_bytes, dev)
+    timer = kernel_timer
+    if timer is not None:
+        timer.start("attn")
+    st = lib.sp_short_attn_fwd_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), n, hq, k.shape[0], d, q.stride(1), q.stride(0),
+                                    k.stride(1), k.stride(0), v.stride(1), v.stride(0), softmax_scale, mask.data_ptr(),
+                                    _ptr(decision), out.data_ptr(), _ptr(avg_attn), _ptr(ws), ws_bytes, stream)
+    if timer is not None:
+        timer.stop("attn")
+    _lib.check(st, "sp_short_attn_fwd_bf16")
+    return out
+
+
 def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float,
                      out: Optional[torch.Tensor] = None, static_scratch: bool = False) -> torch.Tensor:
     """q bf16 [Hq, D] (one token), k / v bf16 [Hkv, N, D] views -> out bf16 [Hq, D].

@@ -174,6 +174,9 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
     nb = -(-q_len // block_size)
     sharing = module.attention_sharing
     minb, maxb = budget_blocks(config.min_budget, config.max_budget, block_size)
+    # a short prompt's attention is one launch that reads v as it is (ops.short_attention); longer ones repack v and run
+    # the persistent kernel
+    short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
     if q_len < block_size or (nb <= minb and nb <= maxb and getattr(config, "dense_short_prompts", True)):
         # (a) Shorter than one block: a single diagonal block, nothing to select (the reference cannot run here).
         # (b) The prompt has no more blocks than the minimum budget, nor than the maximum.  Every head's budgets are
@@ -188,26 +191,33 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         # full path instead.
         avg_attn = torch.zeros(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
         mask = _dense_causal_mask(num_heads, nb, q.device)
-        out = ops.block_sparse_attention(q, k, v, mask, block_size, softmax_scale, pair_rows=True,
-                                         half_channels=model_dim != head_dim)
+        if short:
+            out = ops.short_attention(q, k, v, mask, softmax_scale)
+        else:
+            out = ops.block_sparse_attention(q, k, v, mask, block_size, softmax_scale, pair_rows=True,
+                                             half_channels=model_dim != head_dim)
         if q_len >= block_size:
             sharing.note_dense_layer(module.layer_idx, num_heads, nb)
         return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
 
     # Room for the block sums of this layer's possible pivots (at most 16 GiB of it; pivots beyond that take the
     # recomputing pass).  How many heads can become pivots is known from the table alone.
-    slab = _lib.load().sp_attn_pivot_scratch_bytes(q_len, block_size)
-    max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
-    ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
     avg_attn = torch.empty(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
-    ops.repack_v(v, block_size, ws[0])
+    if not short:
+        slab = _lib.load().sp_attn_pivot_scratch_bytes(q_len, block_size)
+        max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
+        ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
+        ops.repack_v(v, block_size, ws[0])
     avg_attn.zero_()
     plan = sharing.plan_layer(q, k, module.layer_idx, block_size, minb, maxb, config.pattern_threshold,
                               config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold,
                               scale_dim=model_dim)
-    out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
-                                     avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,
-                                     half_channels=model_dim != head_dim)
+    if short:
+        out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0])
+    else:
+        out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
+                                         avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,
+                                         half_channels=model_dim != head_dim)
     sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
     return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
 
