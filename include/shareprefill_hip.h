@@ -111,7 +111,8 @@ int sp_pool_bf16(const void* x, void* y, int64_t n, int32_t h, int32_t d, int64_
  * torch_bhn_sumpool (attn/utils.py:33-44): softmax over all keys of the last bs queries
  * (scaled by 1/sqrt(d), causal inside the last bs columns), column mean -> vert_tok[hq][n],
  * anti-diagonal mean -> slash_tok[hq][n], and their block sums vert_blk / slash_blk [hq][nb].
- * bs: 16, 32, 64 or 128 (attention_sharing.py:127 takes any; shareprefill_attn.py:509-516 allows these); d 128;
+ * bs: 16, 32, 64 or 128 (attention_sharing.py:127 takes any; shareprefill_attn.py:509-516 allows these); d 128, or 64
+ * with the model's head_dim named in flags (SP_FLAG_SCALE_DIM);
  * n >= bs (the kernels work on the last 128 token positions' queries and drop the rows a smaller block, or a
  * shorter prompt, lacks).
  * workspace: sp_lastq_scores_workspace_bytes(...) bytes of device scratch. */

@@ -193,7 +193,7 @@ class AttentionSharing:
         state = self._ensure_state(nb, dev)
         hc = self._head_cluster_tensor(layer_idx, hq, dev)
 
-        flags = self.flags | (_lib.SP_FLAG_SCALE_DIM(scale_dim) if scale_dim and scale_dim != d else 0)
+        flags = self.flags | (_lib.SP_FLAG_SCALE_DIM(scale_dim) if scale_dim and (scale_dim != d or d == 64) else 0)
         vert_tok, slash_tok, vert_blk, slash_blk = ops.lastq_scores(q, k, block_size, flags)
         nv, ns = ops.cover_budgets(vert_tok, slash_tok, block_size, pattern_threshold, minb, maxb)
         kbar = ops.pool_avg(k, block_size)
@@ -209,7 +209,8 @@ class AttentionSharing:
         plan.max_pivots = self.max_pivots(layer_idx, hq)
         if self.keep_debug:
             plan.vert_tok, plan.slash_tok, plan.vert_blk, plan.slash_blk = vert_tok, slash_tok, vert_blk, slash_blk
-            plan.kbar, plan.avg_qk, plan.js_qa, plan.js_v, plan.js_s = kbar, avg_qk, js_qa, js_v, js_s
+            plan.kbar = torch.nn.functional.pad(kbar, (0, 128 - d))  # [nb, Hkv, 128], zero beyond the model's channels
+            plan.avg_qk, plan.js_qa, plan.js_v, plan.js_s = avg_qk, js_qa, js_v, js_s
             plan.qa_probs = qa_probs.clone()
         if self.plans and not (self.keep_plans or self.keep_debug):
             self.plans[-1].mask = None

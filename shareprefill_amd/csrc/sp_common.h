@@ -42,9 +42,9 @@ static inline float sp_inv_sqrt_dim(uint32_t flags, int d) {
 }
 
 // ---- kernels of one source file launched from another ----
-// pooled block probabilities of query-aware heads on the matrix core (sp_scores.hip), head_dim 128
+// pooled block probabilities of query-aware heads on the matrix core (sp_scores.hip), head_dim 64 or 128
 int sp_block_probs_mfma_launch(const void* qbar, const void* kbar, const int32_t* decision, int32_t hq, int32_t hkv,
-                               int32_t nb, uint32_t flags, float* probs, hipStream_t stream);
+                               int32_t d, int32_t nb, uint32_t flags, float* probs, hipStream_t stream);
 
 // ---- bf16 <-> fp32 -------------------------------------------------------------------------------
 typedef uint16_t sp_bf16;

@@ -20,7 +20,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 #define LQ_ROWS 128          // query rows (= block size)
 #define LQ_TILE 128          // keys per tile
-#define LQ_D 128             // head dim
+                             // D, the head dim, is 64 or 128: a template parameter of every kernel here
 #define LQ_THREADS 256       // 4 waves per head, wave w owns 32 query rows of the last block
 #define LQ_MIN_TILES 1       // key tiles per workgroup of the statistics kernel: a power of two, at most 32 -- as many as
 #define LQ_MAX_TILES 32      // still leave one round of workgroups at long sequences, as few as give one at short ones
@@ -30,11 +30,11 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #define LQ_LOG2E 1.4426950408889634f
 #define LQ_NO_MAX (-1.0e30f)
 
-// lane's operand: scaled last-block queries, 8 k-steps x 8 bf16; MFMA row m = lane % 32 of wave w is query 32 w + m of
+// lane's operand: scaled last-block queries, D / 16 k-steps x 8 bf16; MFMA row m = lane % 32 of wave w is query 32 w + m of
 // the last block, or query 127 - (32 w + m) with REVERSED
-template <bool REVERSED>
+template <bool REVERSED, int KS>
 __device__ static __forceinline__ void lq_load_q(const sp_bf16* __restrict__ q, int64_t n, int64_t sq_n, int wave, int lane,
-                                        float inv_sqrt_d, bf16x8 (&qa)[8]) {
+                                        float inv_sqrt_d, bf16x8 (&qa)[KS]) {
   const int row = REVERSED ? LQ_ROWS - 1 - (wave * 32 + (lane & 31)) : wave * 32 + (lane & 31);
   // (a prompt shorter than 128 tokens, possible with a block size below 128: the rows in front of its first token
   // read token 0 and are dropped by the probabilities kernel like every row in front of the last block)
@@ -42,7 +42,7 @@ __device__ static __forceinline__ void lq_load_q(const sp_bf16* __restrict__ q, 
   if (tok < 0) tok = 0;
   const sp_bf16* src = q + tok * sq_n + 8 * (lane >> 5);
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
+  for (int ks = 0; ks < KS; ++ks) {
     uint4 raw = *reinterpret_cast<const uint4*>(src + 16 * ks);
     uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -73,7 +73,9 @@ typedef __bf16 lq_bf16x2 __attribute__((ext_vector_type(2)));
 //   * the product is taken transposed, S^T = K . Q^T: in the 32x32 accumulators a lane then owns ONE query (column
 //     lane % 32) and 16 of the tile's keys per 32-key group, so the running max and sum are two registers, not 32,
 //     and the fold at the end is one exchange between the two lane halves.
-#define LQ_KSW_BYTES (LQ_TILE * LQ_D * 2)  // 32 KiB: [128 keys][16 chunks of 16 bytes], chunk c of row r at c ^ ((r >> SWZ) & 15)
+// 32 KiB (D = 128) or 16 KiB: 256-byte lines of 16 chunks of 16 bytes, position p of line l holding chunk p ^ ((l >> SWZ) & 15)
+// of the line.  A line is a key's 128 channels, or the 64 channels of keys 2 l and 2 l + 1.
+#define LQ_KSW_BYTES(D) (LQ_TILE * (D) * 2)
 
 typedef __attribute__((address_space(3))) void* lq_lds_ptr;
 typedef const __attribute__((address_space(1))) void* lq_gbl_ptr;
@@ -94,52 +96,67 @@ static inline __host__ __device__ int lq_pairs(int group) { return (group + LQ_W
 // change from tile to tile -- row (4 w + lane / 16) * stride + swizzled chunk, computed once: with SWZ = 0 the
 // chunk is the same for all four instructions, with SWZ = 2 it takes two values (it % 2).  Only the one tile that
 // reaches past the end of the sequence clamps its rows onto the last key (masked later), lane by lane.
-template <int SWZ>
+// With D = 64 a line holds two keys, the swizzles shift by one bit less (lines instead of keys), and two instructions fill
+// the tile; the lane offset is the same for all of them.
+template <int D, int SWZ>
 struct LqKLane {
-  uint32_t off[SWZ == 0 ? 1 : 2];
+  uint32_t off[D == 128 && SWZ != 0 ? 2 : 1];
 };
 
-template <int SWZ>
-__device__ static __forceinline__ LqKLane<SWZ> lq_k_lane(int64_t sk_n, int wave8, int lane) {
-  LqKLane<SWZ> kl;
-  const int row0 = wave8 * 4 + (lane >> 4);  // instruction `it` adds 32 rows
+// byte offset in LDS of 16-byte chunk c of key r, for a lane whose line swizzle ((line >> SWZ) & 15) is known
+template <int D>
+__device__ static __forceinline__ int lq_line(int r) { return D == 128 ? r : r >> 1; }
+template <int D>
+__device__ static __forceinline__ int lq_chunk(int r, int c) { return D == 128 ? c : (r & 1) * 8 + c; }
+
+template <int D, int SWZ>
+__device__ static __forceinline__ LqKLane<D, SWZ> lq_k_lane(int64_t sk_n, int wave8, int lane) {
+  LqKLane<D, SWZ> kl;
+  const int line0 = wave8 * 4 + (lane >> 4);  // instruction `it` adds 32 lines
 #pragma unroll
-  for (int v = 0; v < (SWZ == 0 ? 1 : 2); ++v) {
-    const int cl = (lane & 15) ^ (((32 * v + row0) >> SWZ) & 15);
-    kl.off[v] = (uint32_t)(row0 * (int)sk_n * 2 + cl * 16);
+  for (int v = 0; v < (int)(sizeof(kl.off) / sizeof(kl.off[0])); ++v) {
+    const int cl = (lane & 15) ^ (((32 * v + line0) >> SWZ) & 15);
+    if (D == 128)
+      kl.off[v] = (uint32_t)(line0 * (int)sk_n * 2 + cl * 16);
+    else
+      kl.off[v] = (uint32_t)((2 * line0 + (cl >> 3)) * (int)sk_n * 2 + (cl & 7) * 16);
   }
   return kl;
 }
 
-template <int SWZ>
+template <int D, int SWZ>
 __device__ static __forceinline__ void lq_issue_k_direct(const sp_bf16* __restrict__ k, int64_t n, int64_t sk_n, int64_t kb,
-                                                         char* ks, int wave8, int lane, const LqKLane<SWZ>& kl) {
+                                                         char* ks, int wave8, int lane, const LqKLane<D, SWZ>& kl) {
+  constexpr int ITS = D / 32, KEYS = 4096 / D;  // instructions per wave, keys per instruction of all waves
+  constexpr int OFFS = sizeof(kl.off) / sizeof(kl.off[0]);
   if (kb + LQ_TILE <= n) {
     const char* base = reinterpret_cast<const char*>(k + kb * sk_n);
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const char* src = base + (int64_t)it * 32 * sk_n * 2;  // uniform
-      __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(src + kl.off[SWZ == 0 ? 0 : it & 1]),
+    for (int it = 0; it < ITS; ++it) {
+      const char* src = base + (int64_t)it * KEYS * sk_n * 2;  // uniform
+      __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(src + kl.off[it % OFFS]),
                                        (lq_lds_ptr)(ks + (it * 8 + wave8) * 1024), 16, 0, 0);
     }
   } else {
 #pragma unroll 1
-    for (int it = 0; it < 4; ++it) {
+    for (int it = 0; it < ITS; ++it) {
       const int seg = it * 8 + wave8;
-      const int row = seg * 4 + (lane >> 4);
-      const int cl = (lane & 15) ^ ((row >> SWZ) & 15);
-      int64_t key = kb + row;
+      const int line = seg * 4 + (lane >> 4);
+      const int cl = (lane & 15) ^ ((line >> SWZ) & 15);
+      int64_t key = kb + (D == 128 ? line : 2 * line + (cl >> 3));
       if (key > n - 1) key = n - 1;
-      __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(k + key * sk_n + cl * 8), (lq_lds_ptr)(ks + seg * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(k + key * sk_n + (D == 128 ? cl : cl & 7) * 8), (lq_lds_ptr)(ks + seg * 1024),
+                                       16, 0, 0);
     }
   }
 }
 
+template <int D>
 __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, int64_t n, int hkv, int group, int64_t sq_n,
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, int n_chunks, int tiles_per_wg,
     float2* __restrict__ partial /* [hq][n_chunks][128] */) {
-  __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES];
+  __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES(D)];
   const int pairs = lq_pairs(group);
   const int kvh = blockIdx.y / pairs;
   const int chunk = blockIdx.x;
@@ -151,20 +168,20 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
   const int lq = lane & 31, hi = lane >> 5;
   const sp_bf16* qh = q + (int64_t)h * sq_h;
   const sp_bf16* kh = k + (int64_t)kvh * sk_h;
-  bf16x8 qa[8];  // the lane's query (row 32 wave + lq of the last block), channels 16 ks + 8 hi .. + 7
-  lq_load_q<false>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
+  bf16x8 qa[D / 16];  // the lane's query (row 32 wave + lq of the last block), channels 16 ks + 8 hi .. + 7
+  lq_load_q<false, D / 16>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
   float m = LQ_NO_MAX, l = 0.f;
   const int64_t n_tiles = sp_ceil_div(n, LQ_TILE);
   const int64_t tile0 = (int64_t)chunk * tiles_per_wg;
   // byte offset of the lane's operand chunk inside a 32-key group: row lq, logical chunk 2 ks + hi
-  const int row_off = lq * 256;
-  const LqKLane<0> kl = lq_k_lane<0>(sk_n, wave8, lane);
+  const int row_off = lq_line<D>(lq) * 256, swz = lq_line<D>(lq) & 15;
+  const LqKLane<D, 0> kl = lq_k_lane<D, 0>(sk_n, wave8, lane);
   for (int t = 0; t < tiles_per_wg; ++t) {
     const int64_t tile = tile0 + t;
     if (tile >= n_tiles) break;
     const int64_t kb = tile * LQ_TILE;
     __syncthreads();  // the previous tile's operand reads are done
-    lq_issue_k_direct<0>(kh, n, sk_n, kb, Ksw, wave8, lane, kl);
+    lq_issue_k_direct<D, 0>(kh, n, sk_n, kb, Ksw, wave8, lane, kl);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct loads have landed
     __syncthreads();
     if (!has_head) continue;
@@ -179,11 +196,11 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
       floatx16 acc[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const char* src = Ksw + (2 * half + j) * 32 * 256 + row_off;
+        const char* src = Ksw + (2 * half + j) * 32 * D * 2 + row_off;
         floatx16 c = {0};
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-          const uint4 raw = *reinterpret_cast<const uint4*>(src + (((2 * ks + hi) ^ (lq & 15)) << 4));
+        for (int ks = 0; ks < D / 16; ++ks) {
+          const uint4 raw = *reinterpret_cast<const uint4*>(src + ((lq_chunk<D>(lq, 2 * ks + hi) ^ swz) << 4));
           c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, raw), qa[ks], c, 0, 0, 0);
         }
         acc[j] = c;
@@ -317,15 +334,16 @@ struct LqpHeadLds {
   float bpart[2][2][4];     // [tile parity][slash, vertical][wave] block-sum parts
   float zero16[4];
 };
-#define LQP_LDS_BYTES (2 * LQ_KSW_BYTES + LQ_WG_HEADS * sizeof(LqpHeadLds))
+#define LQP_LDS_BYTES(D) (2 * LQ_KSW_BYTES(D) + LQ_WG_HEADS * sizeof(LqpHeadLds))
 
+template <int D>
 __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, int64_t n, int hkv, int group, int64_t sq_n,
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, const float2* __restrict__ rowstat,
     float* __restrict__ vert_tok, float* __restrict__ slash_tok, float* __restrict__ vert_blk,
     float* __restrict__ slash_blk, int64_t nb, int tiles_per_wg, int bs) {
   extern __shared__ __attribute__((aligned(1024))) char lqp_lds[];
-  char* R2 = lqp_lds;  // [2][LQ_KSW_BYTES]
+  char* R2 = lqp_lds;  // [2][LQ_KSW_BYTES(D)]
   const int pairs = lq_pairs(group);
   const int kvh = blockIdx.y / pairs;
   const int wave8 = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -333,13 +351,13 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   const int hg = (blockIdx.y % pairs) * LQ_WG_HEADS + (wave8 >> 2);
   const bool has_head = hg < group;  // (wave-uniform)
   const int h = kvh * group + (has_head ? hg : 0);
-  LqpHeadLds& L = reinterpret_cast<LqpHeadLds*>(lqp_lds + 2 * LQ_KSW_BYTES)[wave8 >> 2];
+  LqpHeadLds& L = reinterpret_cast<LqpHeadLds*>(lqp_lds + 2 * LQ_KSW_BYTES(D))[wave8 >> 2];
   const int tid = threadIdx.x & (LQ_THREADS - 1);  // thread within the head's four waves
   const int lq = lane & 31, hi = lane >> 5;
   const sp_bf16* qh = q + (int64_t)h * sq_h;
   const sp_bf16* kh = k + (int64_t)kvh * sk_h;
-  bf16x8 qa[8];
-  lq_load_q<true>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
+  bf16x8 qa[D / 16];
+  lq_load_q<true, D / 16>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
   // per row: max + log2(sum), so that a probability is exp2(logit * log2 e - rm): the normalisation rides in the
   // exponent instead of costing a multiplication per element
   // A block size below 128 has its last block's queries in the tail of the 128 rows: the rows in front of them get
@@ -362,19 +380,20 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   if (tid < LQ_TILE) L.carry[(t_begin & 1) ^ 1][tid] = 0.f;  // nothing is carried into the first tile
   if (tid < 4) L.zero16[tid] = 0.f;
   // B operand of key sub-tile nt, k-step ks: K row 4 lq + nt, logical 16-byte chunk 2 ks + hi (swizzled by row / 4)
-  const int b_off = lq * 1024;
+  const int b_off = lq * 4 * D * 2;
   const int b_swz = lq & 15;
 
-  const LqKLane<2> kl = lq_k_lane<2>(sk_n, wave8, lane);
-  lq_issue_k_direct<2>(kh, n, sk_n, t_begin * LQ_TILE, R2 + (t_begin & 1) * LQ_KSW_BYTES, wave8, lane, kl);
+  constexpr int SWZ = D == 128 ? 2 : 1;  // lines / 4 rows
+  const LqKLane<D, SWZ> kl = lq_k_lane<D, SWZ>(sk_n, wave8, lane);
+  lq_issue_k_direct<D, SWZ>(kh, n, sk_n, t_begin * LQ_TILE, R2 + (t_begin & 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
   for (int64_t tile = t_begin; tile < t_end; ++tile) {
     const int64_t kb = tile * LQ_TILE;
     const int par = (int)(tile & 1);
-    const char* R = R2 + par * LQ_KSW_BYTES;
+    const char* R = R2 + par * LQ_KSW_BYTES(D);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's direct loads of this tile have landed
     __syncthreads();  // ... and everyone's; the previous tile's K reads and digest reads are done
     if (tile + 1 < t_end)  // the next K tile, into the buffer the previous tile has left
-      lq_issue_k_direct<2>(kh, n, sk_n, kb + LQ_TILE, R2 + (par ^ 1) * LQ_KSW_BYTES, wave8, lane, kl);
+      lq_issue_k_direct<D, SWZ>(kh, n, sk_n, kb + LQ_TILE, R2 + (par ^ 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
     if (tid == 0 && tile > first && has_head && write_blk) {  // the previous tile's block sums: its parts were complete one barrier ago
       const float* bp = &L.bpart[par ^ 1][0][0];
       slash_blk[(int64_t)h * nb + tile - 1] = bp[0] + bp[1];
@@ -385,11 +404,11 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
       floatx16 acc[4];
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt) {
-        const char* src = R + b_off + nt * 256;
+        const char* src = R + b_off + lq_line<D>(nt) * 256;
         floatx16 c = {0};
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-          const uint4 raw = *reinterpret_cast<const uint4*>(src + (((2 * ks + hi) ^ b_swz) << 4));
+        for (int ks = 0; ks < D / 16; ++ks) {
+          const uint4 raw = *reinterpret_cast<const uint4*>(src + ((lq_chunk<D>(nt, 2 * ks + hi) ^ b_swz) << 4));
           c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], __builtin_bit_cast(bf16x8, raw), c, 0, 0, 0);
         }
         acc[nt] = c;
@@ -550,17 +569,19 @@ __global__ __launch_bounds__(256) void sp_lastq_block_sums_kernel(const float* _
 // leave at once.
 #define BPM_THREADS 256
 
-// 32 segments of 1 KiB (4 pooled-key rows each): instruction `it` of wave w (0..3) fills segment 4 it + w
+// 32 segments of 1 KiB (4 lines of pooled keys each; 16 segments for D = 64): instruction `it` of wave w (0..3) fills
+// segment 4 it + w
+template <int D>
 __device__ static __forceinline__ void bpm_issue_k(const sp_bf16* __restrict__ kb_head, int64_t row_stride, int nb,
                                                    int c_tile, char* ks, int wave, int lane) {
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
+  for (int it = 0; it < D / 16; ++it) {
     const int seg = it * 4 + wave;
-    const int row = seg * 4 + (lane >> 4);
-    const int cl = (lane & 15) ^ (row & 15);
-    int key = c_tile * LQ_TILE + row;
+    const int line = seg * 4 + (lane >> 4);
+    const int cl = (lane & 15) ^ (line & 15);
+    int key = c_tile * LQ_TILE + (D == 128 ? line : 2 * line + (cl >> 3));
     if (key > nb - 1) key = nb - 1;  // rows past the end are clamped onto the last pooled key (masked later)
-    __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(kb_head + (int64_t)key * row_stride + cl * 8),
+    __builtin_amdgcn_global_load_lds((lq_gbl_ptr)(kb_head + (int64_t)key * row_stride + (D == 128 ? cl : cl & 7) * 8),
                                      (lq_lds_ptr)(ks + seg * 1024), 16, 0, 0);
   }
 }
@@ -575,28 +596,29 @@ __device__ static __forceinline__ void bpm_round_pair(floatx16& v, int r) {
   v[r + 1] = __uint_as_float(pk & 0xffff0000u);
 }
 
+template <int D>
 __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
-    const sp_bf16* __restrict__ qbar /* [nb][hq][128] */, const sp_bf16* __restrict__ kbar /* [nb][hkv][128] */,
+    const sp_bf16* __restrict__ qbar /* [nb][hq][D] */, const sp_bf16* __restrict__ kbar /* [nb][hkv][D] */,
     const int32_t* __restrict__ decision, int hq, int hkv, int nb, uint32_t flags, float inv_sqrt_d,
     float* __restrict__ probs /* [hq][nb][nb] */) {
-  __shared__ __attribute__((aligned(1024))) char Ks[LQ_KSW_BYTES];
+  __shared__ __attribute__((aligned(1024))) char Ks[LQ_KSW_BYTES(D)];
   __shared__ float2 rstat[LQ_ROWS];
   const int rt = blockIdx.x, h = blockIdx.y;
   if (decision[h] != SP_DEC_QA) return;
   const int kvh = h / (hq / hkv);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int lq = lane & 31, hi = lane >> 5;
-  const sp_bf16* kb_head = kbar + (int64_t)kvh * LQ_D;
-  const int64_t k_stride = (int64_t)hkv * LQ_D;
+  const sp_bf16* kb_head = kbar + (int64_t)kvh * D;
+  const int64_t k_stride = (int64_t)hkv * D;
   // the lane's operand row: pooled query rt * 128 + 32 wave + lq (clamped), scaled and rounded as the reference's
   // avg_q / sqrt(d) in bf16
-  bf16x8 qa[8];
+  bf16x8 qa[D / 16];
   {
     int row = rt * LQ_ROWS + wave * 32 + lq;
     if (row > nb - 1) row = nb - 1;
-    const sp_bf16* src = qbar + ((int64_t)row * hq + h) * LQ_D + 8 * hi;
+    const sp_bf16* src = qbar + ((int64_t)row * hq + h) * D + 8 * hi;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
+    for (int ks = 0; ks < D / 16; ++ks) {
       uint4 raw = *reinterpret_cast<const uint4*>(src + 16 * ks);
       uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -609,7 +631,7 @@ __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
       qa[ks] = __builtin_bit_cast(bf16x8, raw);
     }
   }
-  const int row_off = lq * 256;
+  const int row_off = lq_line<D>(lq) * 256, swz = lq_line<D>(lq) & 15;
 
   // ---- pass 1: row maximum (base-2 units) and sum, transposed product: the lane's query is row 32 wave + lq ----
   {
@@ -617,7 +639,7 @@ __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
     const int my_row = rt * LQ_ROWS + wave * 32 + lq;
     for (int ct = 0; ct <= rt; ++ct) {
       __syncthreads();
-      bpm_issue_k(kb_head, k_stride, nb, ct, Ks, wave, lane);
+      bpm_issue_k<D>(kb_head, k_stride, nb, ct, Ks, wave, lane);
       __builtin_amdgcn_s_waitcnt(0x0F70);
       __syncthreads();
 #pragma unroll 1
@@ -625,11 +647,11 @@ __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
         floatx16 acc[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const char* src = Ks + (2 * half + j) * 32 * 256 + row_off;
+          const char* src = Ks + (2 * half + j) * 32 * D * 2 + row_off;
           floatx16 c = {0};
 #pragma unroll
-          for (int ks = 0; ks < 8; ++ks) {
-            const uint4 raw = *reinterpret_cast<const uint4*>(src + (((2 * ks + hi) ^ (lq & 15)) << 4));
+          for (int ks = 0; ks < D / 16; ++ks) {
+            const uint4 raw = *reinterpret_cast<const uint4*>(src + ((lq_chunk<D>(lq, 2 * ks + hi) ^ swz) << 4));
             c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, raw), qa[ks], c, 0, 0, 0);
           }
           acc[j] = c;
@@ -679,16 +701,16 @@ __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
   // ---- pass 2: probabilities; acc[nt][r] = S[row 32 wave + 8 (r / 4) + 4 hi + r % 4][key 32 nt + lq] ----
   for (int ct = 0; ct <= rt; ++ct) {
     __syncthreads();
-    bpm_issue_k(kb_head, k_stride, nb, ct, Ks, wave, lane);
+    bpm_issue_k<D>(kb_head, k_stride, nb, ct, Ks, wave, lane);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
 #pragma unroll 1
     for (int nt = 0; nt < 4; ++nt) {
-      const char* src = Ks + nt * 32 * 256 + row_off;
+      const char* src = Ks + nt * 32 * D * 2 + row_off;
       floatx16 c = {0};
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(src + (((2 * ks + hi) ^ (lq & 15)) << 4));
+      for (int ks = 0; ks < D / 16; ++ks) {
+        const uint4 raw = *reinterpret_cast<const uint4*>(src + ((lq_chunk<D>(lq, 2 * ks + hi) ^ swz) << 4));
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[ks], __builtin_bit_cast(bf16x8, raw), c, 0, 0, 0);
       }
       if (flags & SP_FLAG_LOGITS_BF16) {
@@ -717,12 +739,15 @@ __global__ __launch_bounds__(BPM_THREADS, 2) void sp_block_probs_mfma_kernel(
   }
 }
 
-// launcher for sp_queryaware_select_bf16 (head_dim 128)
+// launcher for sp_queryaware_select_bf16 (head_dim 64 or 128)
 int sp_block_probs_mfma_launch(const void* qbar, const void* kbar, const int32_t* decision, int32_t hq, int32_t hkv,
-                               int32_t nb, uint32_t flags, float* probs, hipStream_t stream) {
-  hipLaunchKernelGGL(sp_block_probs_mfma_kernel, dim3((unsigned)sp_ceil_div(nb, LQ_ROWS), hq), dim3(BPM_THREADS), 0, stream,
-                     (const sp_bf16*)qbar, (const sp_bf16*)kbar, decision, (int)hq, (int)hkv, (int)nb, flags,
-                     sp_inv_sqrt_dim(flags, LQ_D), probs);
+                               int32_t d, int32_t nb, uint32_t flags, float* probs, hipStream_t stream) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)sp_ceil_div(nb, LQ_ROWS), hq), dim3(BPM_THREADS), 0, stream,
+                       (const sp_bf16*)qbar, (const sp_bf16*)kbar, decision, (int)hq, (int)hkv, (int)nb, flags,
+                       sp_inv_sqrt_dim(flags, d), probs);
+  };
+  d == 64 ? launch(sp_block_probs_mfma_kernel<64>) : launch(sp_block_probs_mfma_kernel<128>);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -774,7 +799,8 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
              "sp_lastq_scores_bf16: hq=%d must be a positive multiple of hkv=%d", hq, hkv);
   SP_REQUIRE(bs == 128 || bs == 64 || bs == 32 || bs == 16, SP_ERR_UNSUPPORTED,
              "sp_lastq_scores_bf16: block size %d unsupported (16, 32, 64 or 128)", bs);
-  SP_REQUIRE(d == LQ_D, SP_ERR_UNSUPPORTED, "sp_lastq_scores_bf16: head_dim %d unsupported (only 128)", d);
+  SP_REQUIRE(d == 128 || (d == 64 && ((flags >> 8) & 0xffu) != 0u), SP_ERR_UNSUPPORTED,
+             "sp_lastq_scores_bf16: head_dim %d unsupported (128, or 64 with SP_FLAG_SCALE_DIM in flags)", d);
   SP_REQUIRE(n >= bs, SP_ERR_INVALID_ARGUMENT, "sp_lastq_scores_bf16: seq_len %lld is shorter than one block",
              (long long)n);
   SP_REQUIRE(q_stride_n % 8 == 0 && q_stride_h % 8 == 0 && k_stride_n % 8 == 0 && k_stride_h % 8 == 0 &&
@@ -792,9 +818,12 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
   const int group = hq / hkv;
   hipStream_t s = (hipStream_t)stream;
   const int wg_rows = hkv * lq_pairs(group);  // workgroups per key chunk: LQ_WG_HEADS heads of one kv group each
-  hipLaunchKernelGGL(sp_lastq_stats_kernel, dim3(n_chunks, wg_rows), dim3(LQ_WG_THREADS), 0, s, (const sp_bf16*)q,
-                     (const sp_bf16*)k, n, hkv, group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d,
-                     flags, n_chunks, tiles_per_wg, partial);
+  auto launch_stats = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n_chunks, wg_rows), dim3(LQ_WG_THREADS), 0, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
+                       group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, n_chunks, tiles_per_wg,
+                       partial);
+  };
+  d == 64 ? launch_stats(sp_lastq_stats_kernel<64>) : launch_stats(sp_lastq_stats_kernel<128>);
   SP_LAUNCH_CHECK();
   hipLaunchKernelGGL(sp_lastq_combine_kernel, dim3(hq), dim3(LQ_ROWS * LQ_COMBINE_GROUPS), 0, s, partial, n_chunks,
                      rowstat);
@@ -804,15 +833,20 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
   SP_HIP(hipGetDevice(&dev));
   SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "sp_lastq_scores_bf16: device index %d", dev);
   if (!attr_set[dev]) {
-    SP_HIP(hipFuncSetAttribute((const void*)sp_lastq_probs_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)LQP_LDS_BYTES));
+    SP_HIP(hipFuncSetAttribute((const void*)sp_lastq_probs_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)LQP_LDS_BYTES(64)));
+    SP_HIP(hipFuncSetAttribute((const void*)sp_lastq_probs_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)LQP_LDS_BYTES(128)));
     attr_set[dev] = true;
   }
   const int tiles_probs = lq_probs_tiles_per_wg(nb_tiles, wg_rows);
   const int grid_x = (int)sp_ceil_div(nb_tiles, tiles_probs);
-  hipLaunchKernelGGL(sp_lastq_probs_kernel, dim3(grid_x, wg_rows), dim3(LQ_WG_THREADS), LQP_LDS_BYTES, s, (const sp_bf16*)q,
-                     (const sp_bf16*)k, n, hkv, group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d,
-                     flags, rowstat, vert_tok, slash_tok, vert_blk, slash_blk, nb_tiles, tiles_probs, (int)bs);
+  auto launch_probs = [&](auto kernel, size_t lds) {
+    hipLaunchKernelGGL(kernel, dim3(grid_x, wg_rows), dim3(LQ_WG_THREADS), lds, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
+                       group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, rowstat, vert_tok, slash_tok,
+                       vert_blk, slash_blk, nb_tiles, tiles_probs, (int)bs);
+  };
+  d == 64 ? launch_probs(sp_lastq_probs_kernel<64>, LQP_LDS_BYTES(64)) : launch_probs(sp_lastq_probs_kernel<128>, LQP_LDS_BYTES(128));
   SP_LAUNCH_CHECK();
   if (bs != LQ_ROWS) {
     const int64_t total = (int64_t)hq * nb;

@@ -28,15 +28,21 @@ KERNEL_HEAD_DIM = 128
 PADDED_HEAD_DIMS = (16, 32, 64)  # the reference's other head sizes (shareprefill_attn.py:503-508)
 
 
-def pad_head_dim(*tensors: torch.Tensor):
-    """The kernels are built for head_dim 128.  The reference's smaller head sizes run on them with the head_dim axis
-    zero-padded: no dot product changes (q.k gains exact zeros, the extra output channels are P.0 = 0 and are cut
-    off again), the softmax scale and the selection's 1/sqrt(head_dim) keep the model's head_dim.  Costs a copy of
-    q / k / v; the attention kernel is told that channels 64.. are zero and skips their products (SP_ATTN_HALF_CHANNELS),
-    so its arithmetic is that of head_dim 64."""
+def pad_head_dim(*tensors: torch.Tensor, width: int = KERNEL_HEAD_DIM):
+    """The persistent kernel is built for head_dim 128, the selection and the short-prompt kernel for 128 and 64.  Smaller
+    head sizes run on them with the head_dim axis zero-padded: no dot product changes (q.k gains exact zeros, the extra
+    output channels are P.0 = 0 and are cut off again), the softmax scale and the selection's 1/sqrt(head_dim) keep the
+    model's head_dim.  Costs a copy of q / k / v; the persistent kernel is told that channels 64.. are zero and skips their
+    products (SP_ATTN_HALF_CHANNELS), so its arithmetic is that of head_dim 64."""
     d = tensors[0].shape[-1]
-    return tuple(torch.nn.functional.pad(t, (0, KERNEL_HEAD_DIM - d)) for t in tensors)
+    return tuple(torch.nn.functional.pad(t, (0, width - d)) for t in tensors)
 
+
+
+def _rows_16_byte_aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy of it if its rows cannot be read with 16-byte loads."""
+    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[1:-1])
+    return t if ok else t.contiguous()
 
 
 def _dense_causal_mask(hq: int, nb: int, device) -> torch.Tensor:
@@ -162,21 +168,26 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
 
     if bsz != 1:
         raise ValueError("SharePrefill prefill keeps per-cluster state for batch size 1 only")
-    if model_dim in PADDED_HEAD_DIMS:
-        query_states, key_states, value_states = pad_head_dim(query_states, key_states, value_states)
-    head_dim = query_states.shape[-1]
     assert query_states.dtype == torch.bfloat16, "SharePrefill attention expects bfloat16 q/k/v"
     assert key_states.shape[2] == q_len, "prefill expects q_len == k_len (no cached prefix)"
-    _lib.load()
+    block_size = config.block_size
+    # a short prompt's attention is one launch that reads v as it is (ops.short_attention) and takes 64 channels as they
+    # are; longer ones repack v and run the persistent kernel on 128
+    head_dim = 64 if model_dim in PADDED_HEAD_DIMS else model_dim
+    short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
+    if model_dim in PADDED_HEAD_DIMS:
+        if not short:
+            head_dim = KERNEL_HEAD_DIM
+        if model_dim != head_dim:
+            query_states, key_states, value_states = pad_head_dim(query_states, key_states, value_states, width=head_dim)
+        else:
+            query_states, key_states, value_states = (_rows_16_byte_aligned(t) for t in
+                                                      (query_states, key_states, value_states))
 
     q, k, v = query_states[0], key_states[0], value_states[0]
-    block_size = config.block_size
     nb = -(-q_len // block_size)
     sharing = module.attention_sharing
     minb, maxb = budget_blocks(config.min_budget, config.max_budget, block_size)
-    # a short prompt's attention is one launch that reads v as it is (ops.short_attention); longer ones repack v and run
-    # the persistent kernel
-    short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
     if q_len < block_size or (nb <= minb and nb <= maxb and getattr(config, "dense_short_prompts", True)):
         # (a) Shorter than one block: a single diagonal block, nothing to select (the reference cannot run here).
         # (b) The prompt has no more blocks than the minimum budget, nor than the maximum.  Every head's budgets are

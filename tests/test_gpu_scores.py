@@ -108,3 +108,25 @@ def test_lastq_scores_rejects_unsupported(gpu_device):
     q = torch.zeros(2, 64, 128, dtype=torch.bfloat16, device=gpu_device)
     with pytest.raises(ValueError):
         ops.lastq_scores(q, q, 128)
+
+
+@pytest.mark.parametrize("hq,hkv,n", [(3, 1, 128), (4, 2, 129), (14, 2, 1000), (8, 8, 2304), (7, 1, 4095)])
+def test_64_channel_scores_equal_the_zero_padded_ones_bit_for_bit(gpu_device, hq, hkv, n):
+    """head_dim 64 as it is against the same heads zero-padded to 128 channels (whose products and sums it shares): the
+    token vectors and block sums, and the pooled block probabilities of query-aware heads."""
+    from shareprefill_amd import _lib, ops
+
+    q, k, _ = synthetic.planted_qkv(hq, hkv, n, 64, 5 + n, q_head_gain=1.0)
+    q, k = q[0].to(gpu_device), k[0].to(gpu_device)
+    wide = [torch.nn.functional.pad(t, (0, 64)) for t in (q, k)]
+    flags = _lib.SP_FLAG_LOGITS_BF16 | _lib.SP_FLAG_SCALE_DIM(64)
+    for a, b in zip(ops.lastq_scores(q, k, 128, flags), ops.lastq_scores(*wide, 128, flags)):
+        assert torch.equal(a, b)
+    nb = -(-n // 128)
+    decision = torch.full((hq,), _lib.SP_DEC_QA, dtype=torch.int32, device=gpu_device)
+    got = []
+    for qx, kx in ((q, k), wide):
+        mask = torch.zeros(hq, nb, (nb + 63) // 64, dtype=torch.int64, device=gpu_device)
+        probs = ops.queryaware_select(ops.pool_avg(qx, 128), ops.pool_avg(kx, 128), decision, mask, 0.9, flags)
+        got.append((probs, mask))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
