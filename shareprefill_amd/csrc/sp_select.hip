@@ -235,10 +235,29 @@ __global__ __launch_bounds__(SEL_THREADS) void sp_gsel_pick_kernel(GselState* __
 }
 
 // ---- the same descent by ONE workgroup per vector, histograms in LDS only -------------------------------------------
-// For short vectors (a few thousand to 16 K entries) the multi-workgroup descent is nothing but launch latency: ten
-// launches whose kernels run a few microseconds each.  Here one workgroup of SEL_THREADS threads makes the three
-// passes over its vector itself; the arithmetic (keys, fixed-point masses, pick rule, tie rule) is the very same
-// code, so both paths select the same entries.
+// The multi-workgroup descent is ten launches, most of them a few microseconds of launch latency.  Here one workgroup of
+// CS_THREADS threads makes the passes over its vector itself; keys, fixed-point masses, pick rule and tie rule are the
+// same integers, so both paths select the same entries.
+// What bounds it: LDS atomics on equal addresses (the values of a probability vector share few exponents, so the lanes of
+// a wave meet in a handful of bins) and the barriers of the workgroup.  Hence four levels of 8, 8, 8 and 7 key bits
+// with CS_COPIES histograms side by side, lane % CS_COPIES choosing one (at most four lanes of a wave on an address),
+// two barriers per level, and a pick that every wave makes for itself from the 256 folded bins, without another barrier.
+// Vectors of at most CS_ITEMS entries per thread stay in registers for all levels; longer ones are read again.
+// 64 vectors, one launch against three levels of 2048 bins (one workgroup up to 16384 values, ten launches above): 3001
+// values 16.7 -> 11.0 us, 16384 25.9 -> 14.5, 32768 58 -> 25, 131072 80 -> 75; at 262144 the ten launches take 106 us and
+// one would take 109, hence GSEL_ONE_LEN.  32 maps of 64 x 64 blocks 20.6 -> 13.8 us, 256 x 256 67 -> 68.5 and, what most
+// layers meet, no map enabled 30.6 -> 6.7; at 512 x 512 the ten launches are ahead (96 us against 227), hence GSEL_ONE_NB.
+#define CS_THREADS 1024
+#define CS_BINS 256
+#define CS_COPIES 16
+#define CS_ITEMS 16
+struct CoverShared {
+  unsigned long long sum[CS_BINS * CS_COPIES];
+  uint32_t cnt[CS_BINS * CS_COPIES];
+  unsigned long long bin_sum[CS_BINS];
+  uint32_t bin_cnt[CS_BINS];
+};
+
 __device__ static inline GselState sel_fresh_state(long long t_le, bool enabled) {
   GselState s;
   s.rem = t_le < 0 ? 0ull : (unsigned long long)t_le;
@@ -252,99 +271,257 @@ __device__ static inline GselState sel_fresh_state(long long t_le, bool enabled)
   return s;
 }
 
-template <int LEVEL>
-__device__ static inline void sel_hist_add(SelShared& sh, const GselState& s, float val) {
-  constexpr int shift = LEVEL == 0 ? 21 : (LEVEL == 1 ? 10 : 0);
-  constexpr int width = LEVEL == 2 ? 10 : 11;
-  constexpr int pshift = LEVEL == 0 ? 32 : (LEVEL == 1 ? 21 : 10);
-  const uint32_t key = sp_sort_key(val);
-  if (pshift < 32 && (key >> (pshift & 31)) != s.prefix) return;
-  const uint32_t b = (key >> shift) & ((1u << width) - 1u);
-  atomicAdd(&sh.cnt[b], 1u);
-  const unsigned long long fx = sp_to_fixed(val);
-  if (fx) atomicAdd(&sh.sum[b], fx);
+// Lane exchanges of the fold and the pick go through DPP moves: as LDS permutes (30 per level, times 16 waves) they cost
+// more than everything else in a level.
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ static __forceinline__ uint32_t cs_dpp(uint32_t v) {  // lanes without a source (or outside ROW_MASK) get 0
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, false);
+}
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ static __forceinline__ unsigned long long cs_dpp64(unsigned long long v) {
+  return ((unsigned long long)cs_dpp<CTRL, ROW_MASK>((uint32_t)(v >> 32)) << 32) | cs_dpp<CTRL, ROW_MASK>((uint32_t)v);
+}
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ static __forceinline__ void cs_scan_step(uint32_t& c, unsigned long long& m) {
+  c += cs_dpp<CTRL, ROW_MASK>(c);
+  m += cs_dpp64<CTRL, ROW_MASK>(m);
+}
+__device__ static __forceinline__ uint32_t cs_lane(uint32_t v, int src) {  // src uniform
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, src);
 }
 
-__device__ static inline void sel_hist_clear(SelShared& sh) {
-  sh.sum[threadIdx.x] = 0;
-  sh.sum[threadIdx.x + SEL_THREADS] = 0;
-  sh.cnt[threadIdx.x] = 0;
-  sh.cnt[threadIdx.x + SEL_THREADS] = 0;
+// sp_to_fixed of a value whose key is normal or infinite (no sign, no NaN, no zero): one 64-bit shift
+__device__ static __forceinline__ unsigned long long cs_fixed(uint32_t key) {
+  const int right = 140 - (int)(key >> 23);  // floor(m 2^(e - 102)) = (m << 38) >> (140 - e), m < 2^24
+  const unsigned long long m = (unsigned long long)((key & 0x7fffffu) | 0x800000u) << 38;
+  return right < 0 ? SP_FX_SAT : m >> (right < 63 ? right : 63);
+}
+
+// histograms zero; ends with a barrier
+__device__ static inline void cover_begin(CoverShared& sh) {
+  for (int i = threadIdx.x; i < CS_BINS * CS_COPIES; i += CS_THREADS) {
+    sh.sum[i] = 0;
+    sh.cnt[i] = 0;
+  }
   __syncthreads();
+}
+
+// One level: for_each(f) calls f(value) for each of this thread's values.  Called by all CS_THREADS threads with the same
+// `s` and zero histograms; returns the same updated `s` to every thread and leaves the histograms zero again.
+template <typename ForEach>
+__device__ static inline void cover_level(CoverShared& sh, GselState& s, int level, ForEach&& for_each) {
+  const int width = level == 3 ? 7 : 8;
+  const int shift = level == 3 ? 0 : 23 - 8 * level;  // (the sign bit of a key is never set)
+  const int t = threadIdx.x, lane = t & 63;
+  const int copy = t & (CS_COPIES - 1);
+  const uint32_t prefix = s.prefix;
+  for_each([&](float val) {
+    const uint32_t key = sp_sort_key(val);
+    if ((key >> (shift + width)) != prefix || key < 0x00800000u) return;  // (zeros carry no mass: never the cut)
+    const uint32_t at = ((key >> shift) & ((1u << width) - 1u)) * CS_COPIES + copy;
+    atomicAdd(&sh.cnt[at], 1u);
+    atomicAdd(&sh.sum[at], cs_fixed(key));
+  });
+  __syncthreads();
+  {  // four threads fold a bin's copies and leave them zero; the masses of empty bins are not read
+    const int bin = t >> 2, part = t & 3;
+    uint4* pc = reinterpret_cast<uint4*>(sh.cnt + bin * CS_COPIES + part * 4);
+    ulonglong2* ps = reinterpret_cast<ulonglong2*>(sh.sum + bin * CS_COPIES + part * 4);
+    const uint4 c4 = *pc;
+    uint32_t c = (c4.x + c4.y) + (c4.z + c4.w);
+    unsigned long long m = 0;
+    if (c) {
+      const ulonglong2 s0 = ps[0], s1 = ps[1];
+      m = (s0.x + s0.y) + (s1.x + s1.y);
+      *pc = make_uint4(0, 0, 0, 0);
+      ps[0] = ps[1] = make_ulonglong2(0, 0);
+    }
+    cs_scan_step<0xB1>(c, m);  // quad_perm [1, 0, 3, 2]
+    cs_scan_step<0x4E>(c, m);  // quad_perm [2, 3, 0, 1]
+    if (part == 0) {
+      sh.bin_cnt[bin] = c;
+      sh.bin_sum[bin] = m;
+    }
+  }
+  __syncthreads();
+  // every wave by itself: lane l owns bins 255 - 4 l .. 252 - 4 l, the running mass comes from the top.  (The next level's
+  // fold overwrites the bins only behind that level's first barrier, which this wave reaches after its pick.)
+  uint32_t c[4];
+  unsigned long long m[4];
+  {
+    const uint4 c4 = *reinterpret_cast<const uint4*>(sh.bin_cnt + (CS_BINS - 4 - 4 * lane));
+    const ulonglong2 lo = *reinterpret_cast<const ulonglong2*>(sh.bin_sum + (CS_BINS - 4 - 4 * lane));
+    const ulonglong2 hi = *reinterpret_cast<const ulonglong2*>(sh.bin_sum + (CS_BINS - 2 - 4 * lane));
+    c[0] = c4.w, c[1] = c4.z, c[2] = c4.y, c[3] = c4.x;
+    m[0] = hi.y, m[1] = hi.x, m[2] = lo.y, m[3] = lo.x;
+  }
+  uint32_t c_incl = (c[0] + c[1]) + (c[2] + c[3]);
+  unsigned long long m_incl = (m[0] + m[1]) + (m[2] + m[3]);
+  const uint32_t c_own = c_incl;
+  const unsigned long long m_own = m_incl;
+  cs_scan_step<0x111>(c_incl, m_incl);       // row_shr 1, 2, 4, 8: inclusive scan of each row of 16 lanes
+  cs_scan_step<0x112>(c_incl, m_incl);
+  cs_scan_step<0x114>(c_incl, m_incl);
+  cs_scan_step<0x118>(c_incl, m_incl);
+  cs_scan_step<0x142, 0xa>(c_incl, m_incl);  // row_bcast15 into rows 1 and 3
+  cs_scan_step<0x143, 0xc>(c_incl, m_incl);  // row_bcast31 into rows 2 and 3
+  uint32_t c_above = c_incl - c_own, found = 0, f_above = 0, f_cnt = 0;
+  unsigned long long m_above = m_incl - m_own, f_mass = 0;
+  int f_bin = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {  // the first bin behind which the running mass exceeds what is left
+    if (!found && m_above <= s.rem && m_above + m[u] > s.rem) {
+      found = 1;
+      f_bin = CS_BINS - 1 - 4 * lane - u;
+      f_above = c_above;
+      f_mass = m_above;
+      f_cnt = c[u];
+    }
+    c_above += c[u];
+    m_above += m[u];
+  }
+  const unsigned long long who = __ballot(found != 0);
+  if (who == 0ull) {  // the running mass never exceeds the budget (top level only): keep everything
+    s.all = 1;
+    return;
+  }
+  const int src = __ffsll((long long)who) - 1;
+  f_bin = (int)cs_lane((uint32_t)f_bin, src);
+  f_above = cs_lane(f_above, src);
+  f_cnt = cs_lane(f_cnt, src);
+  f_mass = ((unsigned long long)cs_lane((uint32_t)(f_mass >> 32), src) << 32) | cs_lane((uint32_t)f_mass, src);
+  s.prefix = (prefix << width) | (uint32_t)f_bin;
+  s.above += f_above;
+  s.rem -= f_mass;
+  if (level == 3) {  // the bin is one value: as many of its entries as the budget left holds
+    s.n_equal = f_cnt;
+    const unsigned long long each = sp_to_fixed(__uint_as_float(s.prefix));
+    unsigned long long take = each ? s.rem / each : (unsigned long long)f_cnt;
+    if (take > f_cnt) take = f_cnt;
+    s.n_take = (uint32_t)take;
+  }
+}
+
+template <typename ForEach>
+__device__ static inline void cover_descent(CoverShared& sh, GselState& s, ForEach&& for_each) {
+  cover_begin(sh);
+  // (a loop, not four instances: code that runs once per launch is paid for in instruction fetches)
+#pragma unroll 1
+  for (int level = 0; level < 4 && !s.all; ++level) cover_level(sh, s, level, for_each);  // (uniform)
 }
 
 // flat vectors (score_cover_topk, the budgets): vectors 0..n0-1 are rows of x0, the others rows of x1
-#define GSEL_SMALL_LEN 16384
-template <int LEVEL>
-__device__ static inline void sel_flat_level(SelShared& sh, GselState& s, const float* __restrict__ xv, int len) {
-  sel_hist_clear(sh);
-  for (int i = threadIdx.x; i < len; i += SEL_THREADS) sel_hist_add<LEVEL>(sh, s, xv[i]);
-  __syncthreads();
-  sel_pick_level<LEVEL>(sh, s);
-}
+struct CoverCountArgs {
+  const float *x0, *x1;
+  int n0, len;
+  long long t_le;
+  int32_t *out0, *out1;
+  int bs, minb, maxb;
+};
 
-__global__ __launch_bounds__(SEL_THREADS) void sp_gsel_count_small_kernel(
-    const float* __restrict__ x0, const float* __restrict__ x1, int n0, int len, long long t_le,
-    int32_t* __restrict__ out0, int32_t* __restrict__ out1, int bs, int minb, int maxb) {
-  __shared__ SelShared sh;
-  const int v = blockIdx.x;
-  const float* xv = v < n0 ? x0 + (int64_t)v * len : x1 + (int64_t)(v - n0) * len;
-  GselState s = sel_fresh_state(t_le, true);
+__device__ static void cover_count_vector(CoverShared& sh, const CoverCountArgs& a, int v) {
+  const float* xv = v < a.n0 ? a.x0 + (int64_t)v * a.len : a.x1 + (int64_t)(v - a.n0) * a.len;
+  GselState s = sel_fresh_state(a.t_le, true);
+  const int t = threadIdx.x, len = a.len;
   if (s.enabled) {
-    sel_flat_level<0>(sh, s, xv, len);
-    if (!s.all) sel_flat_level<1>(sh, s, xv, len);
-    if (!s.all) sel_flat_level<2>(sh, s, xv, len);
-  }
-  if (threadIdx.x == 0) {  // as sp_gsel_count_kernel
-    long long m = 0;
-    if (t_le >= 0) m = s.all ? (long long)len : (long long)s.above + s.n_take;
-    long long r = m + 1;
-    if (bs > 0) {
-      r = r / bs + 1;
-      if (r < minb) r = minb;
-      if (r > maxb) r = maxb;
+    float val[CS_ITEMS];
+    auto load = [&](int i0) {  // CS_ITEMS loads in flight
+#pragma unroll
+      for (int i = 0; i < CS_ITEMS; ++i) {
+        const int at = i0 + i * CS_THREADS + t;
+        val[i] = at < len ? xv[at] : 0.f;
+      }
+    };
+    auto each = [&](int i0, auto&& f) {
+#pragma unroll
+      for (int i = 0; i < CS_ITEMS; ++i) {
+        if (i0 + i * CS_THREADS >= len) break;  // (uniform)
+        f(val[i]);  // (past the end: zeros, which are left out of the histograms)
+      }
+    };
+    if (len <= CS_ITEMS * CS_THREADS) {
+      load(0);
+      cover_descent(sh, s, [&](auto&& f) { each(0, f); });
+    } else {
+      cover_descent(sh, s, [&](auto&& f) {
+        for (int i0 = 0; i0 < len; i0 += CS_ITEMS * CS_THREADS) {
+          load(i0);
+          each(i0, f);
+        }
+      });
     }
-    if (v < n0)
-      out0[v] = (int32_t)r;
+  }
+  if (t == 0) {  // as sp_gsel_count_kernel
+    long long m = 0;
+    if (a.t_le >= 0) m = s.all ? (long long)len : (long long)s.above + s.n_take;
+    long long r = m + 1;
+    if (a.bs > 0) {
+      r = r / a.bs + 1;
+      if (r < a.minb) r = a.minb;
+      if (r > a.maxb) r = a.maxb;
+    }
+    if (v < a.n0)
+      a.out0[v] = (int32_t)r;
     else
-      out1[v - n0] = (int32_t)r;
+      a.out1[v - a.n0] = (int32_t)r;
   }
 }
 
-// lower triangle of an [nb][nb] map (score_cover_idx), nb <= GSEL_SMALL_NB: wave w of the 16 owns rows w, w+16, ...
-#define GSEL_SMALL_NB 128
-template <int LEVEL>
-__device__ static inline void sel_tri_level(SelShared& sh, GselState& s, const float* __restrict__ xv, int nb) {
-  sel_hist_clear(sh);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int r = wave; r < nb; r += SEL_THREADS / SP_WAVE)
-    for (int c = lane; c <= r; c += SP_WAVE) sel_hist_add<LEVEL>(sh, s, xv[(int64_t)r * nb + c]);
-  __syncthreads();
-  sel_pick_level<LEVEL>(sh, s);
+#define GSEL_ONE_LEN 131072
+__global__ __launch_bounds__(CS_THREADS) void sp_cover_count_kernel(CoverCountArgs a) {
+  __shared__ __attribute__((aligned(16))) CoverShared sh;
+  cover_count_vector(sh, a, blockIdx.x);
 }
 
-__global__ __launch_bounds__(SEL_THREADS) void sp_gsel_small_kernel(const float* __restrict__ x,
-                                                                    const int32_t* __restrict__ enable,
-                                                                    int enable_match, int nb, int nbw, long long t_le,
-                                                                    uint64_t* __restrict__ mask) {
-  __shared__ SelShared sh;
-  __shared__ uint32_t row_ties[GSEL_SMALL_NB];
-  const int v = blockIdx.x;
-  if (!gsel_enabled(enable, enable_match, v)) return;
-  const float* xv = x + (int64_t)v * nb * nb;
-  uint64_t* mv = mask + (int64_t)v * nb * nbw;
+// lower triangle of an [nb][nb] map (score_cover_idx), nb <= GSEL_ONE_NB
+#define GSEL_ONE_NB 256
+__device__ static void cover_select_map(CoverShared& sh, uint32_t* row_ties /* LDS [GSEL_ONE_NB] */, const float* __restrict__ xv,
+                                        int nb, int nbw, long long t_le, uint64_t* __restrict__ mv) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int WAVES = CS_THREADS / SP_WAVE;
   GselState s = sel_fresh_state(t_le, true);
   if (s.enabled) {
-    sel_tri_level<0>(sh, s, xv, nb);
-    if (!s.all) sel_tri_level<1>(sh, s, xv, nb);
-    if (!s.all) sel_tri_level<2>(sh, s, xv, nb);
+    // Rows p and nb - 1 - p of the triangle together have nb + 1 entries: entry j of pair p.  A wave takes pairs wave,
+    // wave + 16, ..., 64 entries at a time, so that hardly any lane idles above the diagonal.
+    const int pairs = (nb + 1) / 2;
+    auto at = [&](int p, int j) -> const float* {
+      const int r = nb - 1 - p;
+      return j <= p ? xv + (int64_t)p * nb + j : j <= nb && r != p ? xv + (int64_t)r * nb + (j - p - 1) : nullptr;
+    };
+    float val[12];
+    if (nb <= 2 * SP_WAVE) {  // in registers: four pairs of up to 129 entries
+#pragma unroll
+      for (int i = 0; i < 12; ++i) {
+        const int p = wave + WAVES * (i / 3), j = SP_WAVE * (i % 3) + lane;
+        const float* src = p < pairs ? at(p, j) : nullptr;
+        val[i] = src ? *src : 0.f;  // (zeros are left out of the histograms)
+      }
+      cover_descent(sh, s, [&](auto&& f) {
+#pragma unroll
+        for (int i = 0; i < 12; ++i)
+          if (wave + WAVES * (i / 3) < pairs && SP_WAVE * (i % 3) <= nb) f(val[i]);  // (uniform)
+      });
+    } else {
+      cover_descent(sh, s, [&](auto&& f) {
+        for (int p = wave; p < pairs; p += WAVES)
+          for (int j0 = 0; j0 <= nb; j0 += 8 * SP_WAVE) {  // eight loads in flight
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const float* src = at(p, j0 + SP_WAVE * i + lane);
+              val[i] = src ? *src : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if (j0 + SP_WAVE * i <= nb) f(val[i]);  // (uniform)
+          }
+      });
+    }
   }
   // the boundary group of equal values is taken partially: its n_take lowest indices (row-major) win
   const bool ranked = s.enabled && !s.all && s.n_take != 0 && s.n_take < s.n_equal;
   const bool take_all_equal = s.all || s.n_take >= s.n_equal;
   if (ranked) {
-    for (int r = wave; r < nb; r += SEL_THREADS / SP_WAVE) {
+    for (int r = wave; r < nb; r += WAVES) {
       uint32_t cnt = 0;
       for (int c0 = 0; c0 <= r; c0 += SP_WAVE) {
         const int c = c0 + lane;
@@ -354,10 +531,12 @@ __global__ __launch_bounds__(SEL_THREADS) void sp_gsel_small_kernel(const float*
     }
     __syncthreads();
   }
-  for (int r = wave; r < nb; r += SEL_THREADS / SP_WAVE) {
-    uint32_t before = 0;  // members of the boundary group in rows above this one (uniform per wave)
+  uint32_t before_rows = 0;  // members of the boundary group in the rows in front of row `counted` (uniform per wave)
+  int counted = 0;
+  for (int r = wave; r < nb; r += WAVES) {
     if (ranked)
-      for (int i = 0; i < r; ++i) before += row_ties[i];
+      for (; counted < r; ++counted) before_rows += row_ties[counted];
+    uint32_t before = before_rows;
     for (int c0 = 0; c0 <= r; c0 += SP_WAVE) {
       const int c = c0 + lane;
       bool sel = false, eq = false;
@@ -377,6 +556,17 @@ __global__ __launch_bounds__(SEL_THREADS) void sp_gsel_small_kernel(const float*
       if (lane == 0 && bal) mv[(int64_t)r * nbw + (c0 >> 6)] |= bal;
     }
   }
+}
+
+__global__ __launch_bounds__(CS_THREADS) void sp_cover_select_kernel(const float* __restrict__ x,
+                                                                      const int32_t* __restrict__ enable,
+                                                                      int enable_match, int nb, int nbw, long long t_le,
+                                                                      uint64_t* __restrict__ mask) {
+  __shared__ __attribute__((aligned(16))) CoverShared sh;
+  __shared__ uint32_t row_ties[GSEL_ONE_NB];
+  const int v = blockIdx.x;
+  if (!gsel_enabled(enable, enable_match, v)) return;
+  cover_select_map(sh, row_ties, x + (int64_t)v * nb * nb, nb, nbw, t_le, mask + (int64_t)v * nb * nbw);
 }
 
 __global__ __launch_bounds__(GSEL_THREADS) void sp_gsel_emit_kernel(const float* __restrict__ x, int nb, int nbw,
@@ -560,8 +750,8 @@ static int gsel_run(const float* x, const int32_t* enable, int enable_match, int
   SP_REQUIRE(workspace && workspace_bytes >= sp_cover_select_workspace_bytes(n_vec) && ((uintptr_t)workspace % 8) == 0,
              SP_ERR_WORKSPACE, "%s: workspace missing, misaligned or too small", who);
   const int nbw = (nb + 63) / 64;
-  if (nb <= GSEL_SMALL_NB) {  // one workgroup per map does the whole descent and writes the bits
-    hipLaunchKernelGGL(sp_gsel_small_kernel, dim3(n_vec), dim3(SEL_THREADS), 0, s, x, enable, enable_match, nb, nbw,
+  if (nb <= GSEL_ONE_NB) {  // one workgroup per map does the whole descent and writes the bits
+    hipLaunchKernelGGL(sp_cover_select_kernel, dim3(n_vec), dim3(CS_THREADS), 0, s, x, enable, enable_match, nb, nbw,
                        (long long)sp_thr_le(score), mask);
     SP_LAUNCH_CHECK();
     return SP_OK;
@@ -598,9 +788,9 @@ static int gsel_count_run(const float* x0, const float* x1, int n0, int n_vec, i
   unsigned long long* gsum = reinterpret_cast<unsigned long long*>(st + n_vec);
   uint32_t* gcnt = reinterpret_cast<uint32_t*>(gsum + (size_t)n_vec * SEL_BINS);
   const long long t_le = (long long)sp_thr_le(thr);
-  if (len <= GSEL_SMALL_LEN) {  // one workgroup per vector, one launch
-    hipLaunchKernelGGL(sp_gsel_count_small_kernel, dim3(n_vec), dim3(SEL_THREADS), 0, s, x0, x1, n0, (int)len, t_le, out0,
-                       out1, bs, minb, maxb);
+  if (len <= GSEL_ONE_LEN) {  // one workgroup per vector, one launch
+    const CoverCountArgs a = {x0, x1, n0, (int)len, t_le, out0, out1, bs, minb, maxb};
+    hipLaunchKernelGGL(sp_cover_count_kernel, dim3(n_vec), dim3(CS_THREADS), 0, s, a);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }

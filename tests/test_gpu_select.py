@@ -87,6 +87,43 @@ def test_cover_select_global_skips_disabled(gpu_device):
     assert int(mask[0].abs().sum()) == 0 and int(mask[1].abs().sum()) != 0
 
 
+@pytest.mark.parametrize("n", [1, 63, 1025, 16384, 16385, 40000, 131072, 131073])
+def test_cover_count_at_path_boundaries(gpu_device, n):
+    """Register-resident vectors end at 16384 entries, one workgroup per vector at 131072."""
+    from shareprefill_amd import ops
+
+    x = _probs(4, n, n + 1, sharp=4.0)
+    x[1] = 1.0 / n
+    x[2, n // 2:] = 0.0
+    x[3] *= 1e-9  # the budget is never reached
+    for thr in (0.3, 0.95):
+        got = ops.cover_count(x.to(gpu_device).contiguous(), thr).cpu().tolist()
+        assert got == [O.cover_count(x[i].numpy(), thr) for i in range(4)]
+
+
+@pytest.mark.parametrize("nb", [1, 2, 63, 65, 127, 128, 129, 255, 256, 257])
+def test_cover_select_global_at_path_boundaries(gpu_device, nb):
+    """Register-resident maps end at 128 blocks, one workgroup per map at 256; random maps, uniform rows (the boundary
+    group of equal values spans rows), a map whose mass stays below the budget."""
+    from shareprefill_amd import ops
+
+    g = torch.Generator().manual_seed(nb)
+    tri = torch.tril(torch.ones(nb, nb, dtype=torch.bool))
+    a = torch.softmax((torch.randn(3, nb, nb, generator=g) * 2).masked_fill(~tri, float("-inf")), dim=-1)
+    a[1] = torch.where(tri, torch.tensor(1.0 / nb), torch.tensor(0.0))
+    a[2] *= 0.25
+    score = float(np.float32(0.37 * nb))
+    mask = torch.zeros(3, nb, (nb + 63) // 64, dtype=torch.int64, device=gpu_device)
+    ops.cover_select_global(a.to(gpu_device).contiguous(), score, mask, torch.ones(3, dtype=torch.int32, device=gpu_device))
+    got = ops.mask_to_bool(mask, nb).cpu().numpy()
+    for v in range(3):
+        want = np.zeros(nb * nb, dtype=bool)
+        want[O.cover_keep_le(a[v].numpy().reshape(-1), score)] = True
+        want = want.reshape(nb, nb) & tri.numpy()
+        want[0, 0] = True
+        assert np.array_equal(got[v], want), f"map {v}"
+
+
 @pytest.mark.parametrize("nb", [8, 64, 100, 1024])
 def test_cover_select_rows_bit_exact(gpu_device, nb):
     from shareprefill_amd import ops
