@@ -188,6 +188,22 @@ size_t sp_cover_select_workspace_bytes(int32_t n_vec);
 int sp_cover_select_global(const float* x, const int32_t* enable, int32_t n_vec, int32_t nb, float score,
                            uint64_t* mask, void* workspace, size_t workspace_bytes, sp_stream_t stream);
 
+/* ---- the whole selection of one layer (attention_sharing.py:105-366) ------------------------------
+ * sp_lastq_scores_bf16 .. sp_queryaware_select_bf16 above in one call and fewer launches, with the same results.
+ * per_head: int32 [5][hq] = decision, vertical / slash budgets, final vertical / slash budgets.  mask: [hq][nb][nbw].
+ * qa_probs: fp32 [hq][nb][nb] scratch.  avg_attn: fp32 [hq][nb][nb], 16-byte aligned, cleared, or null.  pattern_threshold
+ * is taken to fp32 where sp_cover_budgets takes a float.  scratch: 256-byte aligned, sp_select_layer_scratch_bytes(...) bytes; offsets, if
+ * not null, receives the byte offsets in it of vert_tok, slash_tok, vert_blk, slash_blk, avg_qk, js_qa, js_v, js_s,
+ * use_qa and kbar (10 values), for a caller that wants to look at them. */
+size_t sp_select_layer_scratch_bytes(int64_t n, int32_t hq, int32_t hkv, int32_t d, int32_t bs, int64_t* offsets);
+int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                         int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
+                         uint32_t flags, const sp_cluster_state* state /* host */, const int32_t* head_cluster,
+                         int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
+                         float similarity_threshold, double fallback_threshold, float queryaware_threshold,
+                         void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
+                         float* avg_attn, sp_stream_t stream);
+
 /* ---- GQA causal block-sparse flash attention ------------------------------------------------
  * Replaces triton_block_wise_prefill_attention / block_wise_prefill_attention_kernel /
  * count_kernel (shareprefill_attn.py:187-620).  out: bf16 [n][hq][d] contiguous.  Only blocks set in

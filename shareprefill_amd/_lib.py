@@ -64,6 +64,9 @@ SIGNATURES = {
     "sp_build_mask": (_I32, [_ST, _P, _P, _P, _P, _P, _P, _I32, _I32, _P, _P]),
     "sp_queryaware_select_score": (_F, [_D, _I32]),
     "sp_queryaware_select_bf16": (_I32, [_P, _P, _P, _I32, _I32, _I32, _I32, _U32, _D, _P, _P, _P, _SZ, _P]),
+    "sp_select_layer_scratch_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32, _P]),
+    "sp_select_layer_bf16": (_I32, [_P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I32, _U32, _ST, _P, _I32, _I32,
+                                    _I32, _D, _F, _D, _F, _P, _SZ, _P, _P, _P, _P, _P]),
     "sp_cover_select_workspace_bytes": (_SZ, [_I32]),
     "sp_cover_select_global": (_I32, [_P, _P, _I32, _I32, _F, _P, _P, _SZ, _P]),
     "sp_attn_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32]),

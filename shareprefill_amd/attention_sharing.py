@@ -181,8 +181,9 @@ class AttentionSharing:
     def plan_layer(self, q: torch.Tensor, k: torch.Tensor, layer_idx: int, block_size: int, min_budget: int,
                    max_budget: int, pattern_threshold: float = 0.9, similarity_threshold: float = 0.5,
                    fallback_threshold: float = 0.9, queryaware_threshold: float = 0.1,
-                   scale_dim: Optional[int] = None) -> LayerPlan:
+                   scale_dim: Optional[int] = None, avg_attn: Optional[torch.Tensor] = None) -> LayerPlan:
         """q [Hq, N, D], k [Hkv, N, D] bf16 views; budgets in blocks.  Enqueues the whole selection.
+        avg_attn: contiguous fp32 [Hq, nb, nb] that is cleared on the way.
         scale_dim: the model's head_dim when q / k have been zero-padded to D (the scores then scale by
         1/sqrt(scale_dim), attention_sharing.py:127 of the reference)."""
         hq, n, d = q.shape
@@ -194,23 +195,16 @@ class AttentionSharing:
         hc = self._head_cluster_tensor(layer_idx, hq, dev)
 
         flags = self.flags | (_lib.SP_FLAG_SCALE_DIM(scale_dim) if scale_dim and (scale_dim != d or d == 64) else 0)
-        vert_tok, slash_tok, vert_blk, slash_blk = ops.lastq_scores(q, k, block_size, flags)
-        nv, ns = ops.cover_budgets(vert_tok, slash_tok, block_size, pattern_threshold, minb, maxb)
-        kbar = ops.pool_avg(k, block_size)
-        avg_qk, js_qa, use_qa = ops.queryaware_test(q, kbar, vert_blk, block_size, queryaware_threshold, flags)
-        decision, js_v, js_s, nv_f, ns_f = ops.share_decide(state, hc, layer_idx, vert_blk, slash_blk, use_qa, nv, ns,
-                                                            minb, similarity_threshold, fallback_threshold)
-        mask = ops.build_mask(state, hc, decision, vert_blk, slash_blk, nv_f, ns_f)
-        # query-aware heads: pooled Q only for them (head_enable), selection skipped on device for the others
-        qbar = ops.pool_avg(q, block_size, tail_mode=_lib.SP_POOL_TAIL_RESCALE, head_enable=use_qa)
-        qa_probs = ops.queryaware_select(qbar, kbar, decision, mask, pattern_threshold, flags,
-                                         probs=self._qa_scratch(hq, nb, dev))
+        qa_probs = self._qa_scratch(hq, nb, dev)
+        mask, (decision, nv, ns, nv_f, ns_f), floats = ops.select_layer(
+            state, hc, layer_idx, q, k, block_size, flags, minb, maxb, pattern_threshold, similarity_threshold,
+            fallback_threshold, queryaware_threshold, qa_probs, avg_attn=avg_attn, keep_floats=self.keep_debug)
         plan = LayerPlan(layer_idx, nb, mask, decision, nv, ns, nv_f, ns_f)
         plan.max_pivots = self.max_pivots(layer_idx, hq)
         if self.keep_debug:
-            plan.vert_tok, plan.slash_tok, plan.vert_blk, plan.slash_blk = vert_tok, slash_tok, vert_blk, slash_blk
-            plan.kbar = torch.nn.functional.pad(kbar, (0, 128 - d))  # [nb, Hkv, 128], zero beyond the model's channels
-            plan.avg_qk, plan.js_qa, plan.js_v, plan.js_s = avg_qk, js_qa, js_v, js_s
+            for name, value in floats.items():
+                setattr(plan, name, value)
+            plan.kbar = torch.nn.functional.pad(plan.kbar, (0, 128 - d))  # [nb, Hkv, 128], zero beyond the model's channels
             plan.qa_probs = qa_probs.clone()
         if self.plans and not (self.keep_plans or self.keep_debug):
             self.plans[-1].mask = None

@@ -42,6 +42,11 @@ static inline float sp_inv_sqrt_dim(uint32_t flags, int d) {
 }
 
 // ---- kernels of one source file launched from another ----
+// last-query scores, and the block averages of K in the same launches when kbar is not null (sp_scores.hip)
+int sp_lastq_scores_run(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d, int64_t q_stride_n,
+                        int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs, uint32_t flags,
+                        void* workspace, size_t workspace_bytes, float* vert_tok, float* slash_tok, float* vert_blk,
+                        float* slash_blk, void* kbar, hipStream_t stream);
 // pooled block probabilities of query-aware heads on the matrix core (sp_scores.hip), head_dim 64 or 128
 int sp_block_probs_mfma_launch(const void* qbar, const void* kbar, const int32_t* decision, int32_t hq, int32_t hkv,
                                int32_t d, int32_t nb, uint32_t flags, float* probs, hipStream_t stream);

@@ -6,14 +6,15 @@
 //
 // Three kernels:
 //   stats   : per (head, key chunk) the running row max / row sum of the logits (bf16 MFMA);
-//   combine : folds the chunk partials into one (max, 1/sum) per query row, in chunk order;
+//   combine : folds the chunk partials into one (max, 1/sum) per query row, in a fixed order; up to LQ_FOLD_CHUNKS chunks
+//             the third kernel does that itself;
 //   probs   : recomputes the logits tile by tile; the column sums (vertical) and, through a permutation of keys and
 //             query rows, the anti-diagonal sums (slash) both start in registers, and only a 32 KiB digest of the
 //             128x128 probability tile goes through LDS.  A slash bin receives its upper part from the previous key
 //             tile; that part is carried through LDS, and each workgroup recomputes one leading tile so that no
 //             cross-workgroup accumulation (and no float atomic) is needed.
 // Every sum runs in a fixed order, so results are reproducible run to run.
-#include "sp_common.h"
+#include "sp_pool.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -155,9 +156,19 @@ template <int D>
 __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, int64_t n, int hkv, int group, int64_t sq_n,
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, int n_chunks, int tiles_per_wg,
-    float2* __restrict__ partial /* [hq][n_chunks][128] */) {
+    float2* __restrict__ partial /* [hq][n_chunks][128] */, PoolArgs pool) {
   __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES(D)];
   const int pairs = lq_pairs(group);
+  // The rows of the grid behind the scores' own pool K beside them (dispatched last, two units per workgroup): a launch of
+  // its own takes 5 us whatever it does, and the keys are on their way through the caches anyway.
+  if ((int)blockIdx.y >= hkv * pairs) {
+    static_assert(LQ_WG_THREADS == 2 * POOL_THREADS && LQ_KSW_BYTES(64) >= 2 * POOL_SPLIT * POOL_CHUNKS * 8 * 4, "");
+    const int half = threadIdx.x / POOL_THREADS;
+    const int64_t unit = 2 * ((int64_t)(blockIdx.y - hkv * pairs) * gridDim.x + blockIdx.x) + half;
+    pool_unit<SP_POOL_AVG>(pool, unit, threadIdx.x % POOL_THREADS,
+                           reinterpret_cast<float(*)[POOL_CHUNKS][8]>(Ksw) + half * POOL_SPLIT);
+    return;
+  }
   const int kvh = blockIdx.y / pairs;
   const int chunk = blockIdx.x;
   const int wave8 = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -258,6 +269,7 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
 // One workgroup per head: 8 groups of 128 threads; group j folds chunks j, j+8, ... of every row, then the eight
 // group results are merged in a fixed order.
 #define LQ_COMBINE_GROUPS 8
+#define LQ_FOLD_CHUNKS 32  // chunks up to which the probabilities kernel folds them in its prologue instead: 16 loads per lane
 __global__ __launch_bounds__(LQ_ROWS * LQ_COMBINE_GROUPS) void sp_lastq_combine_kernel(
     const float2* __restrict__ partial, int n_chunks, float2* __restrict__ rowstat /* [hq][128] */) {
   __shared__ float gm[LQ_COMBINE_GROUPS][LQ_ROWS], gl[LQ_COMBINE_GROUPS][LQ_ROWS];
@@ -340,6 +352,7 @@ template <int D>
 __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, int64_t n, int hkv, int group, int64_t sq_n,
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, const float2* __restrict__ rowstat,
+    const float2* __restrict__ partial, int n_chunks /* 0: rowstat holds the folded statistics */,
     float* __restrict__ vert_tok, float* __restrict__ slash_tok, float* __restrict__ vert_blk,
     float* __restrict__ slash_blk, int64_t nb, int tiles_per_wg, int bs) {
   extern __shared__ __attribute__((aligned(1024))) char lqp_lds[];
@@ -356,8 +369,48 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   const int lq = lane & 31, hi = lane >> 5;
   const sp_bf16* qh = q + (int64_t)h * sq_h;
   const sp_bf16* kh = k + (int64_t)kvh * sk_h;
+  const int64_t n_tiles = sp_ceil_div(n, LQ_TILE);
+  const int64_t first = (int64_t)blockIdx.x * tiles_per_wg;
+  const int64_t t_begin = first > 0 ? first - 1 : 0;
+  const int64_t t_end = first + tiles_per_wg < n_tiles ? first + tiles_per_wg : n_tiles;
+  constexpr int SWZ = D == 128 ? 2 : 1;  // lines / 4 rows
+  const LqKLane<D, SWZ> kl = lq_k_lane<D, SWZ>(sk_n, wave8, lane);
+  lq_issue_k_direct<D, SWZ>(kh, n, sk_n, t_begin * LQ_TILE, R2 + (t_begin & 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
   bf16x8 qa[D / 16];
   lq_load_q<true, D / 16>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
+  float2* const fold = reinterpret_cast<float2*>(L.D);  // [128] (max, 1 / sum) per query row
+  if (n_chunks > 0) {
+    // two lanes per row: lane u takes chunk groups 4 u .. 4 u + 3 of the combine kernel's eight (chunk mod 8), and the
+    // sums meet in that kernel's order
+    static_assert(LQ_THREADS == 2 * LQ_ROWS && LQ_COMBINE_GROUPS == 8 && LQ_FOLD_CHUNKS == 32, "");
+    const int row = tid >> 1, u = tid & 1;
+    const float2* p = partial + (int64_t)h * n_chunks * LQ_ROWS + row;
+    float2 v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = 8 * i + 4 * u + j;
+        v[j][i] = c < n_chunks ? p[(int64_t)c * LQ_ROWS] : make_float2(LQ_NO_MAX, 0.f);
+      }
+    float m = LQ_NO_MAX;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, v[j][i].x);
+    m = fmaxf(m, __shfl_xor(m, 1, SP_WAVE));
+    float g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      g[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) g[j] += v[j][i].y * __builtin_amdgcn_exp2f(v[j][i].x - m);
+    }
+    const float l = (g[0] + g[1]) + (g[2] + g[3]);
+    const float l2 = __shfl_xor(l, 1, SP_WAVE);
+    if (u == 0) fold[row] = make_float2(m, 1.0f / (l + l2));
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the first K tile stays in flight)
+  }
   // per row: max + log2(sum), so that a probability is exp2(logit * log2 e - rm): the normalisation rides in the
   // exponent instead of costing a multiplication per element
   // A block size below 128 has its last block's queries in the tail of the 128 rows: the rows in front of them get
@@ -366,15 +419,11 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int qi = LQ_ROWS - 1 - lq_row_of(wave, lane, r);  // query index inside the last 128 tokens
-    const float2 st = rowstat[h * LQ_ROWS + qi];
+    const float2 st = n_chunks > 0 ? fold[qi] : rowstat[h * LQ_ROWS + qi];
     rm[r] = qi >= LQ_ROWS - bs ? st.x - __builtin_amdgcn_logf(st.y) : INFINITY;  // st.y = 1 / sum; v_log_f32 is log2
   }
-  const int64_t n_tiles = sp_ceil_div(n, LQ_TILE);
-  const int64_t first = (int64_t)blockIdx.x * tiles_per_wg;
   const float inv_rows = 1.0f / (float)bs;
   const bool write_blk = bs == LQ_ROWS;  // the block sums of smaller blocks come from sp_lastq_block_sums_kernel
-  const int64_t t_begin = first > 0 ? first - 1 : 0;
-  const int64_t t_end = first + tiles_per_wg < n_tiles ? first + tiles_per_wg : n_tiles;
   float* Dm = L.D;
   float* Dh = Dm + 32 * LQ_TILE;
   if (tid < LQ_TILE) L.carry[(t_begin & 1) ^ 1][tid] = 0.f;  // nothing is carried into the first tile
@@ -383,9 +432,6 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   const int b_off = lq * 4 * D * 2;
   const int b_swz = lq & 15;
 
-  constexpr int SWZ = D == 128 ? 2 : 1;  // lines / 4 rows
-  const LqKLane<D, SWZ> kl = lq_k_lane<D, SWZ>(sk_n, wave8, lane);
-  lq_issue_k_direct<D, SWZ>(kh, n, sk_n, t_begin * LQ_TILE, R2 + (t_begin & 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
   for (int64_t tile = t_begin; tile < t_end; ++tile) {
     const int64_t kb = tile * LQ_TILE;
     const int par = (int)(tile & 1);
@@ -788,11 +834,11 @@ extern "C" size_t sp_lastq_scores_workspace_bytes(int64_t n, int32_t hq, int32_t
   return partial + rowstat;
 }
 
-extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
-                                    int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
-                                    int32_t bs, uint32_t flags, void* workspace, size_t workspace_bytes,
-                                    float* vert_tok, float* slash_tok, float* vert_blk, float* slash_blk,
-                                    sp_stream_t stream) {
+// kbar: where the averages of K's blocks go ([nb][hkv][d] bf16), or null when they are not wanted
+int sp_lastq_scores_run(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d, int64_t q_stride_n,
+                        int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs, uint32_t flags,
+                        void* workspace, size_t workspace_bytes, float* vert_tok, float* slash_tok, float* vert_blk,
+                        float* slash_blk, void* kbar, hipStream_t s) {
   SP_REQUIRE(q && k && vert_tok && slash_tok && vert_blk && slash_blk && workspace, SP_ERR_INVALID_ARGUMENT,
              "sp_lastq_scores_bf16: null pointer");
   SP_REQUIRE(hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT,
@@ -816,18 +862,24 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
   float2* rowstat = partial + (size_t)hq * lq_chunks(n, hq) * LQ_ROWS;
   const float inv_sqrt_d = sp_inv_sqrt_dim(flags, d);
   const int group = hq / hkv;
-  hipStream_t s = (hipStream_t)stream;
   const int wg_rows = hkv * lq_pairs(group);  // workgroups per key chunk: LQ_WG_HEADS heads of one kv group each
+  PoolArgs pool = {};
+  if (kbar != nullptr) pool = pool_args(k, kbar, n, hkv, d, k_stride_n, k_stride_h, bs, SP_POOL_TAIL_TRUE_LENGTH, nullptr);
+  const int64_t pool_rows = sp_ceil_div(sp_ceil_div(pool.units, 2), n_chunks);
+  SP_REQUIRE(wg_rows + pool_rows <= 65535, SP_ERR_UNSUPPORTED, "sp_lastq_scores_bf16: grid too large");
   auto launch_stats = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(n_chunks, wg_rows), dim3(LQ_WG_THREADS), 0, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
+    hipLaunchKernelGGL(kernel, dim3(n_chunks, wg_rows + pool_rows), dim3(LQ_WG_THREADS), 0, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
                        group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, n_chunks, tiles_per_wg,
-                       partial);
+                       partial, pool);
   };
   d == 64 ? launch_stats(sp_lastq_stats_kernel<64>) : launch_stats(sp_lastq_stats_kernel<128>);
   SP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sp_lastq_combine_kernel, dim3(hq), dim3(LQ_ROWS * LQ_COMBINE_GROUPS), 0, s, partial, n_chunks,
-                     rowstat);
-  SP_LAUNCH_CHECK();
+  const bool fold = n_chunks <= LQ_FOLD_CHUNKS;
+  if (!fold) {
+    hipLaunchKernelGGL(sp_lastq_combine_kernel, dim3(hq), dim3(LQ_ROWS * LQ_COMBINE_GROUPS), 0, s, partial, n_chunks,
+                       rowstat);
+    SP_LAUNCH_CHECK();
+  }
   static bool attr_set[64] = {false};  // per device, once (idempotent)
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));
@@ -843,8 +895,8 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
   const int grid_x = (int)sp_ceil_div(nb_tiles, tiles_probs);
   auto launch_probs = [&](auto kernel, size_t lds) {
     hipLaunchKernelGGL(kernel, dim3(grid_x, wg_rows), dim3(LQ_WG_THREADS), lds, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
-                       group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, rowstat, vert_tok, slash_tok,
-                       vert_blk, slash_blk, nb_tiles, tiles_probs, (int)bs);
+                       group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, rowstat,
+                       (const float2*)partial, fold ? n_chunks : 0, vert_tok, slash_tok, vert_blk, slash_blk, nb_tiles, tiles_probs, (int)bs);
   };
   d == 64 ? launch_probs(sp_lastq_probs_kernel<64>, LQP_LDS_BYTES(64)) : launch_probs(sp_lastq_probs_kernel<128>, LQP_LDS_BYTES(128));
   SP_LAUNCH_CHECK();
@@ -855,4 +907,13 @@ extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int
     SP_LAUNCH_CHECK();
   }
   return SP_OK;
+}
+
+extern "C" int sp_lastq_scores_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                                    int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
+                                    int32_t bs, uint32_t flags, void* workspace, size_t workspace_bytes,
+                                    float* vert_tok, float* slash_tok, float* vert_blk, float* slash_blk,
+                                    sp_stream_t stream) {
+  return sp_lastq_scores_run(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, workspace,
+                             workspace_bytes, vert_tok, slash_tok, vert_blk, slash_blk, nullptr, (hipStream_t)stream);
 }

@@ -14,7 +14,7 @@
 //     sorted order, integer prefix scan -- a literal sort / cumsum / threshold.
 #include <cstring>
 
-#include "sp_common.h"
+#include "sp_pool.h"
 
 #define SEL_THREADS 1024
 #define SEL_BINS 2048
@@ -981,16 +981,32 @@ __device__ static float wave_sqrt_js(const float* __restrict__ p, const float* _
 // query-aware test (attention_sharing.py:193-202)
 // ------------------------------------------------------------------------------------------------
 #define QA_THREADS 1024
-__global__ __launch_bounds__(QA_THREADS) void sp_queryaware_test_kernel(
-    const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ kbar, const float* __restrict__ vert_blk, int64_t n,
-    int hq, int hkv, int d, int64_t sq_n, int64_t sq_h, int bs, int nb, uint32_t flags, float inv_sqrt_d, float thr,
-    float* __restrict__ avg_qk, float* __restrict__ js_qa, int32_t* __restrict__ use_qa) {
-  extern __shared__ float qa_lds[];
+struct QaArgs {
+  const sp_bf16 *q, *kbar;
+  const float* vert_blk;
+  int64_t n, sq_n, sq_h;
+  int hq, hkv, d, bs, nb;
+  uint32_t flags;
+  float inv_sqrt_d, thr;
+  float* avg_qk;
+  float* js_qa;
+  int32_t* use_qa;
+};
+static inline size_t qa_lds_bytes(int d, int nb) { return (size_t)(d + (nb > 16 * d ? nb : 16 * d)) * sizeof(float); }
+
+// Head h, by all QA_THREADS threads.  wave_extra(w): what waves 1.. do while wave 0 forms the divergence (no barrier in it).
+template <typename Extra>
+__device__ static __forceinline__ void queryaware_head(const QaArgs& a, int h, float* qa_lds, Extra&& wave_extra) {
+  const sp_bf16 *__restrict__ q = a.q, *__restrict__ kbar = a.kbar;
+  const float* __restrict__ vert_blk = a.vert_blk;
+  const int64_t n = a.n, sq_n = a.sq_n, sq_h = a.sq_h;
+  const int hq = a.hq, hkv = a.hkv, d = a.d, bs = a.bs, nb = a.nb;
+  const uint32_t flags = a.flags;
+  const float inv_sqrt_d = a.inv_sqrt_d;
   float* qmean = qa_lds;       // [d]
   float* logit = qa_lds + d;   // [nb]
   __shared__ float red[QA_THREADS / SP_WAVE];
   __shared__ float bcast;
-  const int h = blockIdx.x;
   const int kvh = h / (hq / hkv);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // mean over the last bs queries of bf16(q / sqrt(d)), rounded to bf16 (last_q.mean(1), :197-199): thread
@@ -1078,22 +1094,28 @@ __global__ __launch_bounds__(QA_THREADS) void sp_queryaware_test_kernel(
   for (int b = threadIdx.x; b < nb; b += QA_THREADS) {
     const float p = logit[b] / gsum;
     logit[b] = p;
-    avg_qk[(int64_t)h * nb + b] = p;
+    a.avg_qk[(int64_t)h * nb + b] = p;
   }
   __syncthreads();
   if (wave == 0) {
     const float js = wave_sqrt_js(logit, vert_blk + (int64_t)h * nb, nb, lane);
     if (lane == 0) {
-      js_qa[h] = js;
-      use_qa[h] = (js < thr) ? 1 : 0;  // NaN compares false
+      a.js_qa[h] = js;
+      a.use_qa[h] = (js < a.thr) ? 1 : 0;  // NaN compares false
     }
+  } else {
+    wave_extra(wave);
   }
 }
 
-extern "C" int sp_queryaware_test_bf16(const void* q, const void* kbar, const float* vert_blk, int64_t n, int32_t hq,
-                                       int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h, int32_t bs,
-                                       uint32_t flags, float queryaware_threshold, float* avg_qk, float* js_qa,
-                                       int32_t* use_qa, sp_stream_t stream) {
+__global__ __launch_bounds__(QA_THREADS) void sp_queryaware_test_kernel(QaArgs a) {
+  extern __shared__ float qa_lds[];
+  queryaware_head(a, blockIdx.x, qa_lds, [](int) {});
+}
+
+static int queryaware_args(QaArgs* a, const void* q, const void* kbar, const float* vert_blk, int64_t n, int32_t hq,
+                           int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h, int32_t bs, uint32_t flags,
+                           float queryaware_threshold, float* avg_qk, float* js_qa, int32_t* use_qa) {
   SP_REQUIRE(q && kbar && vert_blk && avg_qk && js_qa && use_qa, SP_ERR_INVALID_ARGUMENT,
              "sp_queryaware_test_bf16: null pointer");
   SP_REQUIRE(hq > 0 && hkv > 0 && hq % hkv == 0 && d % 8 == 0 && n >= bs && bs > 0, SP_ERR_INVALID_ARGUMENT,
@@ -1102,11 +1124,21 @@ extern "C" int sp_queryaware_test_bf16(const void* q, const void* kbar, const fl
   SP_REQUIRE(d <= 256, SP_ERR_UNSUPPORTED, "sp_queryaware_test_bf16: head_dim %d too large", d);
   SP_REQUIRE(q_stride_n % 8 == 0 && q_stride_h % 8 == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)kbar % 16) == 0,
              SP_ERR_UNSUPPORTED, "sp_queryaware_test_bf16: q / kbar must be 16-byte aligned with strides multiple of 8");
-  const size_t lds = (size_t)(d + (nb > 16 * d ? nb : 16 * d)) * sizeof(float);
-  SP_REQUIRE(lds <= 60000, SP_ERR_UNSUPPORTED, "sp_queryaware_test_bf16: nb=%d too large", nb);
-  hipLaunchKernelGGL(sp_queryaware_test_kernel, dim3(hq), dim3(QA_THREADS), lds, (hipStream_t)stream,
-                     (const sp_bf16*)q, (const sp_bf16*)kbar, vert_blk, n, hq, hkv, d, q_stride_n, q_stride_h, bs, nb,
-                     flags, sp_inv_sqrt_dim(flags, d), queryaware_threshold, avg_qk, js_qa, use_qa);
+  SP_REQUIRE(qa_lds_bytes(d, nb) <= 60000, SP_ERR_UNSUPPORTED, "sp_queryaware_test_bf16: nb=%d too large", nb);
+  *a = QaArgs{(const sp_bf16*)q, (const sp_bf16*)kbar, vert_blk, n, q_stride_n, q_stride_h, hq, hkv, d, bs, nb, flags,
+              sp_inv_sqrt_dim(flags, d), queryaware_threshold, avg_qk, js_qa, use_qa};
+  return SP_OK;
+}
+
+extern "C" int sp_queryaware_test_bf16(const void* q, const void* kbar, const float* vert_blk, int64_t n, int32_t hq,
+                                       int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h, int32_t bs,
+                                       uint32_t flags, float queryaware_threshold, float* avg_qk, float* js_qa,
+                                       int32_t* use_qa, sp_stream_t stream) {
+  QaArgs a;
+  const int rc = queryaware_args(&a, q, kbar, vert_blk, n, hq, hkv, d, q_stride_n, q_stride_h, bs, flags,
+                                 queryaware_threshold, avg_qk, js_qa, use_qa);
+  if (rc != SP_OK) return rc;
+  hipLaunchKernelGGL(sp_queryaware_test_kernel, dim3(hq), dim3(QA_THREADS), qa_lds_bytes(d, a.nb), (hipStream_t)stream, a);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -1220,27 +1252,28 @@ __device__ static void vs_sets(const float* __restrict__ vert, const float* __re
 // head_cluster[h] names a slot of the state only inside [0, n_clusters); -1 (no shared cluster) and anything a
 // caller got wrong must never be used as an index into the slabs
 __device__ __forceinline__ bool sp_slot_ok(const sp_cluster_state& st, int c) { return c >= 0 && c < st.n_clusters; }
-// similarity of every candidate head against its cluster's stored pivot (pivots of EARLIER layers only: this
-// launch precedes the layer's election)
+// sqrt-JS of head h's pooled vector (0: vertical, 1: slash) against its cluster's stored pivot (pivots of EARLIER layers
+// only: the launch precedes the layer's election); NaN where there is none.  One wave.
+__device__ static __forceinline__ float share_similarity(const sp_cluster_state& st, int c, int h, int which,
+                                                         const float* __restrict__ blk, int lane) {
+  if (!sp_slot_ok(st, c) || st.info[c * 8 + 0] < 0 || st.info[c * 8 + 1] == 0) return NAN;
+  return wave_sqrt_js((which == 0 ? st.vert : st.slash) + (int64_t)c * st.nb, blk + (int64_t)h * st.nb, st.nb, lane);
+}
 __global__ __launch_bounds__(2 * SP_WAVE) void sp_share_similarity_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, const float* __restrict__ vert_blk,
     const float* __restrict__ slash_blk, const int32_t* __restrict__ use_qa, float* __restrict__ js_v,
     float* __restrict__ js_s) {
-  const int nb = st.nb;
   const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = head_cluster[h];
   float js = NAN;
-  if (sp_slot_ok(st, c) && !use_qa[h] && st.info[c * 8 + 0] >= 0 && st.info[c * 8 + 1] != 0)
-    js = wave == 0 ? wave_sqrt_js(st.vert + (int64_t)c * nb, vert_blk + (int64_t)h * nb, nb, lane)
-                   : wave_sqrt_js(st.slash + (int64_t)c * nb, slash_blk + (int64_t)h * nb, nb, lane);
+  if (!use_qa[h]) js = share_similarity(st, head_cluster[h], h, wave, wave == 0 ? vert_blk : slash_blk, lane);
   if (lane == 0) (wave == 0 ? js_v : js_s)[h] = js;
 }
 
 __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, int layer_idx, int hq,
     const int32_t* __restrict__ use_qa, const int32_t* __restrict__ nv, const int32_t* __restrict__ ns, int minb,
-    float sim_thr, double fb_thr, int32_t* __restrict__ decision, const float* __restrict__ js_v,
-    const float* __restrict__ js_s, int32_t* __restrict__ nv_f, int32_t* __restrict__ ns_f) {
+    float sim_thr, double fb_thr, int32_t* __restrict__ decision, float* __restrict__ js_v,
+    float* __restrict__ js_s, int32_t* __restrict__ nv_f, int32_t* __restrict__ ns_f) {
   // The reference walks the heads in ascending order (attention_sharing.py:209-295): the first head of a shared
   // cluster that is not query-aware and finds no pivot becomes the pivot; its later siblings of the same layer find
   // a pivot without a pattern and fall back; heads of clusters with a pattern take the share test.  One thread per
@@ -1263,6 +1296,7 @@ __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
   int dec = SP_DEC_VS;
   if (qa) {
     dec = SP_DEC_QA;
+    js_v[h] = js_s[h] = NAN;  // (formed beside the query-aware test for every head)
   } else if (candidate) {
     bool first = true;
     for (int h2 = 0; h2 < h; ++h2) first = first && !(s_cand[h2] && s_slot[h2] == c);
@@ -1282,24 +1316,28 @@ __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
   ns_f[h] = reset ? minb : ns[h];
 }
 
-// newly elected pivots (the cluster's pivot is this head, elected in this layer) keep their pooled vectors and
-// their own vertical-slash sets (:223-263)
+// a newly elected pivot (the cluster's pivot is this head, elected in this layer) keeps its pooled vectors and its own
+// vertical-slash sets (:223-263); every thread of the workgroup calls it
+__device__ static __forceinline__ void share_keep(const sp_cluster_state& st, int c, int h, int layer_idx,
+                                                  const float* __restrict__ vert_blk, const float* __restrict__ slash_blk,
+                                                  int nv, int ns, uint32_t* keys, int nthreads) {
+  const int nb = st.nb;
+  if (!sp_slot_ok(st, c) || st.info[c * 8 + 0] != h || st.info[c * 8 + 4] != layer_idx) return;  // (uniform)
+  for (int i = threadIdx.x; i < nb; i += nthreads) {
+    st.vert[(int64_t)c * nb + i] = vert_blk[(int64_t)h * nb + i];
+    st.slash[(int64_t)c * nb + i] = slash_blk[(int64_t)h * nb + i];
+  }
+  vs_sets(vert_blk + (int64_t)h * nb, slash_blk + (int64_t)h * nb, nb, nv, ns, keys, st.cols + (int64_t)c * nb,
+          st.dists + (int64_t)c * nb, nthreads);
+}
 __global__ __launch_bounds__(DEC_THREADS) void sp_share_keep_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, int layer_idx,
     const float* __restrict__ vert_blk, const float* __restrict__ slash_blk, const int32_t* __restrict__ decision,
     const int32_t* __restrict__ nv, const int32_t* __restrict__ ns) {
   __shared__ __attribute__((aligned(16))) uint32_t s_keys[RS_MAX];
-  const int nb = st.nb;
   const int h = blockIdx.x;
-  const int c = head_cluster[h];
-  if (!sp_slot_ok(st, c) || decision[h] != SP_DEC_DENSE || st.info[c * 8 + 0] != h || st.info[c * 8 + 4] != layer_idx)
-    return;
-  for (int i = threadIdx.x; i < nb; i += DEC_THREADS) {
-    st.vert[(int64_t)c * nb + i] = vert_blk[(int64_t)h * nb + i];
-    st.slash[(int64_t)c * nb + i] = slash_blk[(int64_t)h * nb + i];
-  }
-  vs_sets(vert_blk + (int64_t)h * nb, slash_blk + (int64_t)h * nb, nb, nv[h], ns[h], s_keys,
-          st.cols + (int64_t)c * nb, st.dists + (int64_t)c * nb, DEC_THREADS);
+  if (decision[h] != SP_DEC_DENSE) return;
+  share_keep(st, head_cluster[h], h, layer_idx, vert_blk, slash_blk, nv[h], ns[h], s_keys, DEC_THREADS);
 }
 
 // The struct a kernel receives by value.  A caller built against the first layout of the struct (it ended with
@@ -1361,14 +1399,65 @@ extern "C" int sp_share_decide(const sp_cluster_state* state, const int32_t* hea
 // ------------------------------------------------------------------------------------------------
 #define MASK_THREADS 1024
 #define MASK_SPLIT 8  // workgroups per head: each ranks the head's vectors itself and writes a share of the rows
+// What the whole-layer selection adds to the mask launch: nothing of it depends on the mask, and each would be a launch of
+// 5 us of its own.
+struct MaskBesides {
+  int layer_idx;    // pivots elected in this layer store their vectors and sets
+  PoolArgs qpool;   // query-aware heads: the averages of Q's blocks
+  float* zero;      // [hq][nb][nb] cleared, or null
+};
+// q blocks of one query-aware head, share `part_no` of MASK_SPLIT: a chunk of 8 channels by four waves, 64 / (d / 8) blocks
+// at a time for each four waves
+__device__ static void mask_pool_q(const PoolArgs& a, int h, int nb, int part_no, char* lds) {
+  const int t = threadIdx.x % POOL_THREADS, set = threadIdx.x / POOL_THREADS;
+  const int lane = t % POOL_CHUNKS, sub = t / POOL_CHUNKS, dchunks = a.d / 8;
+  float(*part)[POOL_CHUNKS][8] = reinterpret_cast<float(*)[POOL_CHUNKS][8]>(lds) + set * POOL_SPLIT;
+  const int at_once = POOL_CHUNKS / dchunks, d0 = lane % dchunks * 8;  // (lanes beyond at_once * dchunks idle)
+  const int per = (nb + MASK_SPLIT - 1) / MASK_SPLIT, b_end = min(nb, (part_no + 1) * per);
+  for (int b0 = part_no * per; b0 < b_end; b0 += at_once * (MASK_THREADS / POOL_THREADS)) {
+    const int blk = b0 + set * at_once + lane / dchunks;
+    const bool active = lane / dchunks < at_once && blk < b_end;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (active) pool_quarter<SP_POOL_AVG>(a.x + (int64_t)h * a.sx_h + d0, a.sx_n, (int64_t)blk * a.bs, a.n, a.bs, sub, acc);
+    __syncthreads();  // the previous round's partial sums have been read
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part[sub][lane][j] = acc[j];
+    __syncthreads();
+    if (sub == 0 && active) {
+      const int64_t rem = a.n - (int64_t)blk * a.bs;
+      pool_store<SP_POOL_AVG>(part, lane, rem < a.bs ? (int)rem : a.bs, a.bs, a.tail_mode, a.y + ((int64_t)blk * a.h + h) * a.d + d0);
+    }
+  }
+}
+
+// BESIDES: grid (hq, 2 MASK_SPLIT), the second half of which pools and clears
+template <bool BESIDES>
 __global__ __launch_bounds__(MASK_THREADS) void sp_build_mask_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, const int32_t* __restrict__ decision,
     const float* __restrict__ vert_blk, const float* __restrict__ slash_blk, const int32_t* __restrict__ nv_f,
-    const int32_t* __restrict__ ns_f, int nb, int nbw, uint64_t* __restrict__ mask) {
-  __shared__ __attribute__((aligned(16))) uint32_t s_keys[RS_MAX];
+    const int32_t* __restrict__ ns_f, int nb, int nbw, uint64_t* __restrict__ mask, MaskBesides extra) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_keys[BESIDES ? MASK_THREADS * 8 : RS_MAX];
   __shared__ uint8_t s_cols[RS_MAX], s_dists[RS_MAX];
   const int h = blockIdx.x;
   const int dec = decision[h];
+  if constexpr (BESIDES) {
+    static_assert(MASK_THREADS * 8 >= RS_MAX, "");
+    if (blockIdx.y >= MASK_SPLIT) {
+      const int part_no = blockIdx.y - MASK_SPLIT;
+      if (extra.zero != nullptr) {  // (in shares of the whole array: a head's part is 4-byte aligned only)
+        const int64_t all = (int64_t)gridDim.x * nb * nb, shares = (int64_t)gridDim.x * MASK_SPLIT;
+        const int64_t per = (all / 4 + shares - 1) / shares, i0 = ((int64_t)h * MASK_SPLIT + part_no) * per;
+        const int64_t i1 = min(all / 4, i0 + per);
+        float4* z = reinterpret_cast<float4*>(extra.zero);
+        for (int64_t i = i0 + threadIdx.x; i < i1; i += MASK_THREADS) z[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (h == 0 && part_no == 0 && threadIdx.x < (all & 3)) extra.zero[(all & ~3ll) + threadIdx.x] = 0.f;
+      }
+      if (dec == SP_DEC_QA) mask_pool_q(extra.qpool, h, nb, part_no, reinterpret_cast<char*>(s_keys));
+      return;
+    }
+    if (dec == SP_DEC_DENSE && blockIdx.y == 0)  // (nothing in this launch reads what it writes)
+      share_keep(st, head_cluster[h], h, extra.layer_idx, vert_blk, slash_blk, nv_f[h], ns_f[h], s_keys, MASK_THREADS);
+  }
   if (dec != SP_DEC_DENSE)
     vs_sets(vert_blk + (int64_t)h * nb, slash_blk + (int64_t)h * nb, nb, nv_f[h], ns_f[h], s_keys, s_cols, s_dists,
             MASK_THREADS);
@@ -1428,8 +1517,9 @@ extern "C" int sp_build_mask(const sp_cluster_state* state, const int32_t* head_
              SP_ERR_INVALID_ARGUMENT, "sp_build_mask: null pointer");
   SP_REQUIRE(hq > 0 && nb > 0 && nb <= RS_MAX, SP_ERR_UNSUPPORTED, "sp_build_mask: nb=%d unsupported (max %d)", nb,
              RS_MAX);
-  hipLaunchKernelGGL(sp_build_mask_kernel, dim3(hq, MASK_SPLIT), dim3(MASK_THREADS), 0, (hipStream_t)stream,
-                     state_by_value(state), head_cluster, decision, vert_blk, slash_blk, nv_final, ns_final, nb, (nb + 63) / 64, mask);
+  hipLaunchKernelGGL(sp_build_mask_kernel<false>, dim3(hq, MASK_SPLIT), dim3(MASK_THREADS), 0, (hipStream_t)stream,
+                     state_by_value(state), head_cluster, decision, vert_blk, slash_blk, nv_final, ns_final, nb, (nb + 63) / 64, mask,
+                     MaskBesides{});
   SP_LAUNCH_CHECK();
   return SP_OK;
 }
@@ -1532,6 +1622,125 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
   const float score = sp_queryaware_select_score(pattern_threshold, nb);
   return gsel_run(probs, decision, SP_DEC_QA, hq, nb, score, mask, workspace, workspace_bytes, (hipStream_t)stream,
                   "sp_queryaware_select_bf16");
+}
+
+// ------------------------------------------------------------------------------------------------
+// the selection of one layer (attention_sharing.py:105-366) in one call
+// ------------------------------------------------------------------------------------------------
+// The stages above, with the launches folded that do not wait for each other: K's averages beside the score statistics, the
+// query-aware test and the share similarities beside the budgets, Q's averages, the pivots' own sets and the clearing of the
+// map beside the masks.  Same device code, same results.  A launch costs 5 us of the stream whatever it does; whole layer,
+// 15 launches / these 7: 3001 tokens 142 -> 120 us, 6177 (64 channels) 148 -> 127, 10007 (28 / 4 heads) 336 -> 313.
+struct HeadArgs {
+  CoverCountArgs cover;
+  int n_cover;  // workgroups 0 .. n_cover - 1: the budgets (0: made by other launches); then one per head
+  QaArgs qa;
+  sp_cluster_state st;
+  const int32_t* head_cluster;
+  const float* slash_blk;
+  float *js_v, *js_s;
+};
+#define HEAD_LDS_BYTES(d, nb) (qa_lds_bytes(d, nb) > sizeof(CoverShared) ? qa_lds_bytes(d, nb) : sizeof(CoverShared))
+__global__ __launch_bounds__(CS_THREADS) void sp_layer_heads_kernel(HeadArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char head_lds[];
+  static_assert(CS_THREADS == QA_THREADS, "");
+  if ((int)blockIdx.x < a.n_cover) {
+    cover_count_vector(*reinterpret_cast<CoverShared*>(head_lds), a.cover, blockIdx.x);
+    return;
+  }
+  const int h = (int)blockIdx.x - a.n_cover, lane = threadIdx.x & 63;
+  // (for a head that turns out query-aware too: sp_share_decide_kernel drops it)
+  queryaware_head(a.qa, h, reinterpret_cast<float*>(head_lds), [&](int wave) {
+    if (wave > 2) return;
+    const float js = share_similarity(a.st, a.head_cluster[h], h, wave - 1, wave == 1 ? a.qa.vert_blk : a.slash_blk, lane);
+    if (lane == 0) (wave == 1 ? a.js_v : a.js_s)[h] = js;
+  });
+}
+
+// scratch of the call, each part 256-byte aligned
+enum { LY_VERT_TOK, LY_SLASH_TOK, LY_VERT_BLK, LY_SLASH_BLK, LY_AVG_QK, LY_JS_QA, LY_JS_V, LY_JS_S, LY_USE_QA, LY_KBAR, LY_QBAR,
+       LY_LASTQ, LY_COVER, LY_PARTS };
+static size_t layer_scratch(int64_t n, int32_t hq, int32_t hkv, int32_t d, int32_t bs, size_t (&at)[LY_PARTS]) {
+  const size_t nb = (size_t)sp_ceil_div(n, bs), tok = (size_t)hq * n * 4, blk = (size_t)hq * nb * 4, head = (size_t)hq * 4;
+  const size_t bytes[LY_PARTS] = {tok, tok, blk, blk, blk, head, head, head, head, nb * hkv * d * 2, nb * hq * d * 2,
+                                  sp_lastq_scores_workspace_bytes(n, hq, bs), sp_cover_select_workspace_bytes(2 * hq)};
+  size_t sum = 0;
+  for (int i = 0; i < LY_PARTS; ++i) {
+    at[i] = sum;
+    sum += (bytes[i] + 255) / 256 * 256;
+  }
+  return sum;
+}
+
+extern "C" size_t sp_select_layer_scratch_bytes(int64_t n, int32_t hq, int32_t hkv, int32_t d, int32_t bs, int64_t* offsets) {
+  if (n <= 0 || hq <= 0 || hkv <= 0 || d <= 0 || bs <= 0) return 0;
+  size_t at[LY_PARTS];
+  const size_t sum = layer_scratch(n, hq, hkv, d, bs, at);
+  for (int i = 0; offsets != nullptr && i <= LY_KBAR; ++i) offsets[i] = (int64_t)at[i];
+  return sum;
+}
+
+extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                                    int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
+                                    uint32_t flags, const sp_cluster_state* state, const int32_t* head_cluster,
+                                    int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
+                                    float similarity_threshold, double fallback_threshold, float queryaware_threshold,
+                                    void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
+                                    float* avg_attn, sp_stream_t stream) {
+  SP_REQUIRE(state && head_cluster && scratch && qa_probs && per_head && mask, SP_ERR_INVALID_ARGUMENT,
+             "sp_select_layer_bf16: null pointer");
+  SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && bs > 0 && d > 0, SP_ERR_INVALID_ARGUMENT, "sp_select_layer_bf16: bad shape");
+  SP_REQUIRE(hq <= DEC_MAX_HEADS, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: hq=%d unsupported (max %d)", hq, DEC_MAX_HEADS);
+  SP_REQUIRE(sp_ceil_div(n, bs) <= RS_MAX, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: n=%lld needs more than %d blocks",
+             (long long)n, RS_MAX);
+  SP_REQUIRE(((uintptr_t)avg_attn % 16) == 0, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: avg_attn must be 16-byte aligned");
+  const int nb = (int)sp_ceil_div(n, bs);
+  int rc = check_state(state, nb, "sp_select_layer_bf16");
+  if (rc) return rc;
+  size_t at[LY_PARTS];
+  SP_REQUIRE(scratch_bytes >= layer_scratch(n, hq, hkv, d, bs, at) && ((uintptr_t)scratch % 256) == 0, SP_ERR_WORKSPACE,
+             "sp_select_layer_bf16: scratch too small or not 256-byte aligned");
+  auto part = [&](int i) { return (char*)scratch + at[i]; };
+  auto floats = [&](int i) { return (float*)part(i); };
+  float *vert_tok = floats(LY_VERT_TOK), *slash_tok = floats(LY_SLASH_TOK), *vert_blk = floats(LY_VERT_BLK),
+        *slash_blk = floats(LY_SLASH_BLK);
+  int32_t *use_qa = (int32_t*)part(LY_USE_QA), *decision = per_head, *nv = per_head + hq, *ns = nv + hq, *nv_f = ns + hq,
+          *ns_f = nv_f + hq;
+  hipStream_t s = (hipStream_t)stream;
+  HeadArgs a = {};
+  rc = queryaware_args(&a.qa, q, part(LY_KBAR), vert_blk, n, hq, hkv, d, q_stride_n, q_stride_h, bs, flags,
+                       queryaware_threshold, floats(LY_AVG_QK), floats(LY_JS_QA), use_qa);
+  if (rc != SP_OK) return rc;
+  rc = sp_lastq_scores_run(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, part(LY_LASTQ),
+                           sp_lastq_scores_workspace_bytes(n, hq, bs), vert_tok, slash_tok, vert_blk, slash_blk, part(LY_KBAR), s);
+  if (rc != SP_OK) return rc;
+  if (n <= GSEL_ONE_LEN) {
+    a.n_cover = 2 * hq;
+    a.cover = CoverCountArgs{vert_tok, slash_tok, hq, (int)n, (long long)sp_thr_le((float)pattern_threshold), nv, ns, bs,
+                             min_blocks, max_blocks};
+  } else {
+    rc = gsel_count_run(vert_tok, slash_tok, hq, 2 * hq, n, (float)pattern_threshold, nv, ns, bs, min_blocks, max_blocks,
+                        part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), s, "sp_select_layer_bf16");
+    if (rc != SP_OK) return rc;
+  }
+  a.st = state_by_value(state);
+  a.head_cluster = head_cluster;
+  a.slash_blk = slash_blk;
+  a.js_v = floats(LY_JS_V);
+  a.js_s = floats(LY_JS_S);
+  hipLaunchKernelGGL(sp_layer_heads_kernel, dim3(a.n_cover + hq), dim3(CS_THREADS), HEAD_LDS_BYTES(d, nb), s, a);
+  SP_LAUNCH_CHECK();
+  hipLaunchKernelGGL(sp_share_decide_kernel, dim3(1), dim3(DEC_MAX_HEADS), 0, s, a.st, head_cluster, layer_idx, hq, use_qa, nv,
+                     ns, min_blocks, similarity_threshold, fallback_threshold, decision, a.js_v, a.js_s, nv_f, ns_f);
+  SP_LAUNCH_CHECK();
+  const MaskBesides besides = {layer_idx,
+                               pool_args(q, part(LY_QBAR), n, hq, d, q_stride_n, q_stride_h, bs, SP_POOL_TAIL_RESCALE, use_qa),
+                               avg_attn};
+  hipLaunchKernelGGL(sp_build_mask_kernel<true>, dim3(hq, 2 * MASK_SPLIT), dim3(MASK_THREADS), 0, s, a.st, head_cluster, decision,
+                     vert_blk, slash_blk, nv_f, ns_f, nb, (nb + 63) / 64, mask, besides);
+  SP_LAUNCH_CHECK();
+  return sp_queryaware_select_bf16(part(LY_QBAR), part(LY_KBAR), decision, hq, hkv, d, nb, flags, pattern_threshold, qa_probs,
+                                   mask, part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), stream);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -8,6 +8,7 @@ head-major q/k/v given as [H, N, D] views with arbitrary token / head strides an
 from __future__ import annotations
 
 import ctypes as C
+import math
 from typing import Optional
 
 import torch
@@ -246,6 +247,45 @@ def queryaware_select(qbar, kbar, decision, mask, pattern_threshold, flags=_lib.
                                        pattern_threshold, _ptr(probs), _ptr(mask), _ptr(ws), ws.numel(), _stream(qbar.device))
     _lib.check(st, "sp_queryaware_select_bf16")
     return probs
+
+
+def select_layer(state: ClusterState, head_cluster, layer_idx, q, k, block_size, flags, min_blocks, max_blocks,
+                 pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold, qa_probs,
+                 avg_attn=None, keep_floats=False):
+    """The whole selection of one layer (attention_sharing.py:105-366) in one call: the stages above, same results.
+
+    -> (mask int64 [Hq, nb, nbw], (decision, nv, ns, nv_final, ns_final) int32 [Hq] each, floats).  qa_probs: fp32
+    [Hq, nb, nb] scratch; avg_attn, if given, is cleared.  floats: with keep_floats a dict of the float intermediates
+    (views of the call's scratch), else None."""
+    lib = _lib.load()
+    _check_hnd(q, "q")
+    _check_hnd(k, "k")
+    hq, n, d = q.shape
+    hkv = k.shape[0]
+    nb = -(-n // block_size)
+    dev = q.device
+    at = (C.c_int64 * 10)() if keep_floats else None
+    need = lib.sp_select_layer_scratch_bytes(n, hq, hkv, d, block_size, at)
+    scratch = torch.empty(need, dtype=torch.uint8, device=dev)
+    mask = torch.empty(hq, nb, (nb + 63) // 64, dtype=torch.int64, device=dev)
+    per_head = torch.empty(5, hq, dtype=torch.int32, device=dev)
+    st = lib.sp_select_layer_bf16(_ptr(q), _ptr(k), n, hq, hkv, d, q.stride(1), q.stride(0), k.stride(1), k.stride(0),
+                                  block_size, flags, state.ref(), _ptr(head_cluster), layer_idx, min_blocks, max_blocks,
+                                  pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
+                                  _ptr(scratch), need, _ptr(qa_probs), _ptr(per_head), _ptr(mask), _ptr(avg_attn),
+                                  _stream(dev))
+    _lib.check(st, "sp_select_layer_bf16")
+    floats = None
+    if keep_floats:
+        def view(i, dtype, *shape):
+            size = math.prod(shape) * torch.empty(0, dtype=dtype).element_size()
+            return scratch[at[i]:at[i] + size].view(dtype).view(*shape)
+
+        names = (("vert_tok", n), ("slash_tok", n), ("vert_blk", nb), ("slash_blk", nb), ("avg_qk", nb))
+        floats = {name: view(i, torch.float32, hq, width) for i, (name, width) in enumerate(names)}
+        floats.update({name: view(5 + i, torch.float32, hq) for i, name in enumerate(("js_qa", "js_v", "js_s"))})
+        floats["kbar"] = view(9, torch.bfloat16, nb, hkv, d)
+    return mask, per_head.unbind(0), floats
 
 
 def cover_select_global(x: torch.Tensor, score: float, mask: torch.Tensor, enable: Optional[torch.Tensor] = None):

@@ -219,10 +219,9 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
         ops.repack_v(v, block_size, ws[0])
-    avg_attn.zero_()
     plan = sharing.plan_layer(q, k, module.layer_idx, block_size, minb, maxb, config.pattern_threshold,
                               config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold,
-                              scale_dim=model_dim)
+                              scale_dim=model_dim, avg_attn=avg_attn[0])
     if short:
         out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0])
     else:
