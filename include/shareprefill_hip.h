@@ -244,6 +244,7 @@ int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, i
 /* The same attention for short prompts, bs = 128, d = 64 or 128 (no padding): one kernel that reads v as it is, needs no
  * repack and no scheduler area, and writes the pivot heads' maps itself.  Correct for any n up to 65536;
  * sp_short_attn_max_tokens(d) is the length up to which it is the faster of the two.
+ * avg_attn without decision: no head is a pivot, the maps are cleared (with decision only DENSE heads' maps are written).
  * workspace: sp_short_attn_workspace_bytes(n, hq) bytes, needed only with decision and avg_attn (block sums). */
 int64_t sp_short_attn_max_tokens(int32_t d);
 size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq);

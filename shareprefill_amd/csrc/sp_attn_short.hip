@@ -21,7 +21,9 @@
 //     (ds_read_b64_tr_b16: the 16 lanes of a group address 4 keys x 16 channels and each receives 4 keys of its channel).
 //     S^T = K . Q^T leaves a lane with keys 4g .. 4g+3 of every 16-key tile (g = lane / 16), which is exactly what two such
 //     reads deliver, so P^T is the S^T accumulators converted to bf16 in place;
-//   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel).
+//   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel); a call
+//     without decisions has its maps cleared here (a fill launch in front of the kernel costs its caller 5 us of host time:
+//     700 tokens 21.3 -> 18.7 us a layer).
 // Two rows sharing one K / V tile, as in the persistent kernel, halve the tile traffic per flop, which is why that one
 // stays for long prompts; sp_short_attn_max_tokens holds the line between the two and the figures.
 #include "sp_common.h"
@@ -37,6 +39,7 @@ struct AsArgs {
   float* tile_sums;          // [hq][nb (nb + 1) / 2][2][128] of pivot heads, or null: no maps wanted
   int64_t n, sq_n, sq_h, sk_n, sk_h, sv_n, sv_h;
   int hq, group, nb, nbw;
+  int zero_maps;             // 1: no decisions, every row of avg_attn is cleared
   float scale_log2;
 };
 
@@ -400,6 +403,8 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
                                                               as_pack2(o[ct][qt][2] * inv_l[qt], o[ct][qt][3] * inv_l[qt]));
     }
   }
+  if (a.zero_maps)
+    for (int i = t; i < a.nb; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + i] = 0.f;
   if (pu == nullptr) return;  // (uniform)
   // pivot head: avg[r][c] = mean over the block's valid queries of (sum of the two halves' exp2(u - m[q])) / l[q].  A wave
   // reads back its own sums (its own stores), folds its queries, and the waves meet in LDS.
@@ -471,7 +476,8 @@ extern "C" int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* 
              SP_ERR_WORKSPACE, "sp_short_attn_fwd_bf16: workspace missing, misaligned or too small");
   const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
                     maps ? (float*)workspace : nullptr, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
-                    v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), softmax_scale * 1.4426950408889634f};
+                    v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), decision == nullptr && avg_attn != nullptr,
+                    softmax_scale * 1.4426950408889634f};
   const dim3 grid((unsigned)(nb * hq));
   // Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
   // 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).

@@ -377,7 +377,7 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
 def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None) -> torch.Tensor:
     """block_sparse_attention for short prompts (block size 128, head_dim 64 or 128): q [Hq,N,D], k/v [Hkv,N,D] views,
     mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D].  One launch, whatever decision says: v is read as it is and the maps of
-    DENSE heads are written by the same kernel."""
+    DENSE heads are written by the same kernel (avg_attn without decision is cleared)."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")

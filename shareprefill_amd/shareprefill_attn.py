@@ -200,11 +200,12 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         # same result at a fraction of the launches.  What is not produced on this path: decisions, pivot state and
         # the pivots' block-average maps (attn_weights is all zeros).  config.dense_short_prompts = False takes the
         # full path instead.
-        avg_attn = torch.zeros(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
         mask = _dense_causal_mask(num_heads, nb, q.device)
         if short:
-            out = ops.short_attention(q, k, v, mask, softmax_scale)
+            avg_attn = torch.empty(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
+            out = ops.short_attention(q, k, v, mask, softmax_scale, avg_attn=avg_attn)  # (clears avg_attn)
         else:
+            avg_attn = torch.zeros(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
             out = ops.block_sparse_attention(q, k, v, mask, block_size, softmax_scale, pair_rows=True,
                                              half_channels=model_dim != head_dim)
         if q_len >= block_size:

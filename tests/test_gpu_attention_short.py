@@ -41,8 +41,10 @@ def test_short_attention_matches_oracle(gpu_device, hq, hkv, n, d):
     qg, kg, vg = q.to(gpu_device), k.to(gpu_device), v.to(gpu_device)
     out = ops.short_attention(qg, kg, vg, bits, d ** -0.5, decision.to(gpu_device), avg)
     assert out.shape == (n, hq, d)
-    plain = ops.short_attention(qg, kg, vg, bits, d ** -0.5)
+    cleared = torch.full_like(avg, 7.0)
+    plain = ops.short_attention(qg, kg, vg, bits, d ** -0.5, avg_attn=cleared)
     assert torch.equal(out, plain)  # (a head's output does not depend on whether its map is wanted)
+    assert not cleared.any()
     out, ref = out.transpose(0, 1).float().cpu(), ref.float()
     assert (out - ref).abs().max().item() <= MAX_ABS
     assert ((out - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
