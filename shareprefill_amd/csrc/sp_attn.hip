@@ -76,7 +76,7 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* 
 // same K / V: waves 0-3 own one, waves 4-7 the other, and both consume the same K / V^T tiles from LDS (the union
 // of the two rows' masks), which halves the L2->LDS traffic wherever the two keep the same columns -- and wherever
 // they do not, the row that does not keep a column idles while the other computes.  Two pairings exist, chosen per
-// two adjacent heads (2i, 2i+1) of a kv group by sp_attn_pairing_kernel, whichever gives the smaller unions:
+// two adjacent heads (2i, 2i+1) of a kv group by sp_attn_schedule_kernel, whichever gives the smaller unions:
 //   rows  : item (h, p) = rows 2p and 2p+1 of head h (verticals are shared, slashes shift by one block);
 //   heads : item (h, p) = row 2p + (h & 1) of heads 2i and 2i+1 (heads that share a pattern keep the same columns).
 // Items are grouped in gangs of AT_GANG consecutive pairs of ONE head (all of a head's pairs when it has fewer: a short
@@ -89,22 +89,22 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* 
 // once all eight queues are exhausted.
 // Up to 32K tokens a launch has few gangs per workgroup, the heaviest of them a large part of a workgroup's whole
 // share, and every head's K / V^T fit the memory-side cache together, so the order above (one kv head after the
-// other) only makes the last kv head's heavy rows start late: there sp_attn_order_kernel ranks the gangs by the
+// other) only makes the last kv head's heavy rows start late: there sp_attn_schedule_kernel ranks the gangs by the
 // number of blocks their items visit and the queues are dealt from that ranking, heaviest first.
 #define AT_GANG 32
 // The 1 KiB scheduler area (int indices): 0..127 eight queue tickets (one per 64 bytes), 128..191 the pivot slot of
 // every head (one byte each, AT_NO_SLOT = its block sums are not kept), 192..195 {shader cycles, 100 MHz ticks} of
 // workgroup 0, 196 the number of pivot slots in use, 200..231 the pairing of every two adjacent heads (one byte each,
-// see sp_attn_pairing_kernel), 232..239 the queue tickets of the pivot heads' launch (so that both launches of a call
-// find their tickets cleared by sp_attn_prep_kernel and nothing has to be cleared in between).
+// see sp_attn_schedule_kernel), 232..239 the queue tickets of the pivot heads' launch (so that both launches of a call
+// find their tickets cleared by sp_attn_schedule_kernel and nothing has to be cleared in between).
 #define AT_SLOT_TABLE 128
 #define AT_CLOCK_SLOT 192
 #define AT_NPIV_SLOT 196
-#define AT_ORDER_SLOT 197  // 1: the gang positions of this call go through the order table (sp_attn_order_kernel)
+#define AT_ORDER_SLOT 197  // 1: the gang positions of this call go through the order table (sp_attn_schedule_kernel)
 #define AT_PAIR_TABLE 200
 #define AT_PIVOT_TICKETS 232  // 232..239: the eight queue tickets of the pivot heads' own launch
 #define AT_NO_SLOT 255
-// Behind the 1 KiB of slots: the order table, AT_ORDER_MAX gang positions (uint16), see sp_attn_order_kernel.
+// Behind the 1 KiB of slots: the order table, AT_ORDER_MAX gang positions (uint16), see sp_attn_schedule_kernel.
 #define AT_ORDER_MAX 1024
 #define AT_SCHED_BYTES (1024 + AT_ORDER_MAX * 2)
 #define AT_MAX_HEADS 256
@@ -1111,48 +1111,30 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   }
 }
 
-// Before the forward launches: clears the queue tickets and gives the first max_pivots heads whose decision is
-// DENSE a slot for their block sums (ascending head order); every other head gets AT_NO_SLOT.
-__global__ void sp_attn_prep_kernel(int* __restrict__ sched, const int32_t* __restrict__ decision, int hq,
-                                    int max_pivots) {
-  for (int i = threadIdx.x; i < AT_SLOT_TABLE; i += blockDim.x) sched[i] = 0;
-  // pivot launch tickets; pairing table = rows 2p, 2p+1 of a head (sp_attn_pairing_kernel may choose otherwise)
-  for (int i = AT_PAIR_TABLE + threadIdx.x; i < AT_PIVOT_TICKETS + 8; i += blockDim.x) sched[i] = 0;
-  if (threadIdx.x == 0) {
-    uint8_t* slots = reinterpret_cast<uint8_t*>(sched + AT_SLOT_TABLE);
-    int cnt = 0;
-    for (int h = 0; h < hq; ++h) {
-      const bool keep = decision != nullptr && decision[h] == SP_DEC_DENSE && cnt < max_pivots;
-      slots[h] = keep ? (uint8_t)cnt++ : (uint8_t)AT_NO_SLOT;
-    }
-    sched[AT_NPIV_SLOT] = cnt;
-    sched[AT_ORDER_SLOT] = 0;
-  }
-}
+// Before the forward launches, in one launch: clears the queue tickets, hands out the pivot slots, chooses the pairing
+// and, for launches of few gangs, ranks them.
+//   slots   : the first max_pivots heads whose decision is DENSE get one for their block sums (ascending head order),
+//             every other head AT_NO_SLOT;
+//   pairing : for every two adjacent heads (2i, 2i+1), how the forward kernel pairs query blocks into work items, from
+//             the union sizes both ways over all rows,
+//               rows : |row 2p  |  row 2p+1| of each head,      heads : |row r of head 2i  |  row r of head 2i+1|:
+//             by heads when that union is strictly smaller and the two heads may share an item (same kv head, neither
+//             runs in the pivot launch);
+//   ORDER   : ranks the gangs by the work of their items -- the blocks the item's two rows visit together, plus a few
+//             blocks' worth of fixed time per item -- and writes the gang positions in descending order (ties: ascending
+//             position) into the order table.
+// Integer sums throughout, so nothing depends on the order of anything.
+// Pure latency: a launch, and chains of loads from L2.  As three launches, a thread per gang walking the gang's items one
+// after the other, it took 33 us at 10007 tokens (28 heads) and 49 at 32768 (32 heads); now one workgroup does all of it
+// for a launch that is ranked (a wave a head pair, a lane an item), and a workgroup a head pair when there is no ranking
+// (the masks of long prompts are too much for one).  Whole layer: 10007 tokens 302 -> 275 us.
+#define AT_ITEM_FIXED 6  // an item's fixed time (ticket, block list, first tiles, epilogue) in units of one block visit
+#define AT_ORDER_THREADS 1024
+#define AT_PAIRING_THREADS 256
 
-// After sp_attn_prep_kernel: chooses, for every two adjacent heads (2i, 2i+1), how the forward kernel pairs query
-// blocks into work items.  One workgroup per head pair sums the union sizes both ways over all rows,
-//   rows : |row 2p  |  row 2p+1| of each head,      heads : |row r of head 2i  |  row r of head 2i+1|,
-// and writes 1 (pair by heads) when that union is strictly smaller and the two heads may share an item: same kv
-// head, and neither runs in the pivot launch.  Integer sums: the choice does not depend on the order of anything.
-__global__ __launch_bounds__(256) void sp_attn_pairing_kernel(int* __restrict__ sched, const uint64_t* __restrict__ mask,
-                                                              int hq, int group, int nb, int nbw, int skip_slotted) {
-  __shared__ unsigned long long tot[2];
-  const int i = blockIdx.x, h0 = 2 * i, h1 = 2 * i + 1;
-  uint8_t* table = reinterpret_cast<uint8_t*>(sched + AT_PAIR_TABLE);
-  const uint8_t* slots = reinterpret_cast<const uint8_t*>(sched + AT_SLOT_TABLE);
-  const bool eligible = h1 < hq && h0 / group == h1 / group &&
-                        !(skip_slotted && (slots[h0] != AT_NO_SLOT || slots[h1] != AT_NO_SLOT));
-  if (!eligible) {  // (uniform)
-    if (threadIdx.x == 0) table[i] = 0;
-    return;
-  }
-  if (threadIdx.x < 2) tot[threadIdx.x] = 0ull;
-  __syncthreads();
-  const uint64_t* m0 = mask + (int64_t)h0 * nb * nbw;
-  const uint64_t* m1 = mask + (int64_t)h1 * nb * nbw;
-  unsigned long long by_rows = 0ull, by_heads = 0ull;
-  for (int p = threadIdx.x; 2 * p < nb; p += blockDim.x) {
+__device__ static inline void at_union_sizes(const uint64_t* __restrict__ m0, const uint64_t* __restrict__ m1, int nb,
+                                             int nbw, int p_begin, int p_step, uint32_t& by_rows, uint32_t& by_heads) {
+  for (int p = p_begin; 2 * p < nb; p += p_step) {
     const int ra = 2 * p, rb = 2 * p + 1 < nb ? 2 * p + 1 : 2 * p;
     for (int w = 0; w <= (rb >> 6); ++w) {
       const uint64_t a0 = m0[(int64_t)ra * nbw + w], b0 = m0[(int64_t)rb * nbw + w];
@@ -1161,57 +1143,123 @@ __global__ __launch_bounds__(256) void sp_attn_pairing_kernel(int* __restrict__ 
       by_heads += __builtin_popcountll(a0 | a1) + (rb != ra ? __builtin_popcountll(b0 | b1) : 0);
     }
   }
-  atomicAdd(&tot[0], by_rows);
-  atomicAdd(&tot[1], by_heads);
-  __syncthreads();
-  if (threadIdx.x == 0) table[i] = tot[1] < tot[0] ? 1 : 0;
 }
 
-// After sp_attn_pairing_kernel, for launches of at most AT_ORDER_MAX gangs: ranks the gangs by the work of their items
-// -- the blocks the item's two rows visit together, plus a few blocks' worth of fixed time per item -- and writes the
-// gang positions in descending order (ties: ascending position) into the order table.  One workgroup; integer
-// weights, so the ranking does not depend on the order of anything.
-#define AT_ITEM_FIXED 6  // an item's fixed time (ticket, block list, first tiles, epilogue) in units of one block visit
-__global__ __launch_bounds__(1024) void sp_attn_order_kernel(int* __restrict__ sched, const uint64_t* __restrict__ mask,
-                                                             int hq, int hkv, int nb, int nbw) {
-  __shared__ uint32_t weight[AT_ORDER_MAX];
+template <int LANES>
+__device__ static inline uint32_t at_lane_sum(uint32_t v) {  // over aligned groups of LANES lanes
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, SP_WAVE);
+  return v;
+}
+
+// grid: ORDER 1; otherwise a workgroup per head pair, or one with pair_rows (no pairing to choose)
+template <bool ORDER>
+__global__ __launch_bounds__(ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
+    int* __restrict__ sched, const uint64_t* __restrict__ mask, const int32_t* __restrict__ decision, int hq, int hkv,
+    int nb, int nbw, int max_pivots, int pair_rows) {
+  constexpr int THREADS = ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS, WAVES = THREADS / SP_WAVE;
+  static_assert(AT_MAX_HEADS <= AT_PAIRING_THREADS && AT_MAX_HEADS % SP_WAVE == 0, "");
+  __shared__ uint32_t dense_cnt[AT_MAX_HEADS / SP_WAVE];
+  __shared__ uint8_t slot_s[AT_MAX_HEADS];
+  __shared__ uint8_t pair_s[AT_MAX_HEADS / 2];
+  __shared__ uint32_t red[2][WAVES];
+  __shared__ uint32_t weight[ORDER ? AT_ORDER_MAX : 1];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int n_head_pairs = (hq + 1) / 2, group = hq / hkv;
+  uint8_t* const table = reinterpret_cast<uint8_t*>(sched + AT_PAIR_TABLE);
+
+  // slots (every workgroup counts for itself)
+  const bool dense = decision != nullptr && t < hq && decision[t] == SP_DEC_DENSE;
+  const uint64_t votes = __ballot(dense);
+  if (t < AT_MAX_HEADS && lane == 0) dense_cnt[wave] = (uint32_t)__builtin_popcountll(votes);
+  __syncthreads();
+  int total = 0;
+  if (t < AT_MAX_HEADS) {
+    int rank = __builtin_popcountll(votes & ((1ull << lane) - 1ull));
+#pragma unroll
+    for (int w = 0; w < AT_MAX_HEADS / SP_WAVE; ++w) {
+      if (w < wave) rank += (int)dense_cnt[w];
+      total += (int)dense_cnt[w];
+    }
+    slot_s[t] = dense && rank < max_pivots ? (uint8_t)rank : (uint8_t)AT_NO_SLOT;
+  }
+  if (blockIdx.x == 0) {
+    if (t < hq) reinterpret_cast<uint8_t*>(sched + AT_SLOT_TABLE)[t] = slot_s[t];
+    if (t < AT_SLOT_TABLE) sched[t] = 0;
+    if (t < 8) sched[AT_PIVOT_TICKETS + t] = 0;
+    if (t == 0) {
+      sched[AT_NPIV_SLOT] = total < max_pivots ? total : max_pivots;
+      sched[AT_ORDER_SLOT] = ORDER ? 1 : 0;
+    }
+  }
+  __syncthreads();
+
+  // pairing
+  auto eligible = [&](int i) {
+    const int h0 = 2 * i, h1 = 2 * i + 1;
+    return h1 < hq && h0 / group == h1 / group && slot_s[h0] == AT_NO_SLOT && slot_s[h1] == AT_NO_SLOT;
+  };
+  if (pair_rows) {
+    for (int i = t; i < n_head_pairs; i += THREADS) table[i] = 0;
+    return;
+  }
+  for (int i = ORDER ? wave : (int)blockIdx.x; i < n_head_pairs; i += ORDER ? WAVES : (int)gridDim.x) {
+    uint32_t by_rows = 0, by_heads = 0;
+    if (eligible(i)) {
+      const uint64_t* m0 = mask + (int64_t)(2 * i) * nb * nbw;
+      at_union_sizes(m0, m0 + (int64_t)nb * nbw, nb, nbw, ORDER ? lane : t, ORDER ? SP_WAVE : THREADS, by_rows, by_heads);
+      by_rows = at_lane_sum<SP_WAVE>(by_rows);
+      by_heads = at_lane_sum<SP_WAVE>(by_heads);
+      if (!ORDER) {  // (uniform: the workgroup has one head pair)
+        if (lane == 0) red[0][wave] = by_rows, red[1][wave] = by_heads;
+        __syncthreads();
+        by_rows = by_heads = 0;
+        for (int w = 0; w < WAVES; ++w) by_rows += red[0][w], by_heads += red[1][w];
+      }
+    }
+    if (ORDER ? lane == 0 : t == 0) {
+      table[i] = by_heads < by_rows ? 1 : 0;
+      pair_s[i] = by_heads < by_rows ? 1 : 0;
+    }
+  }
+  if constexpr (!ORDER) return;
+
+  __syncthreads();
   AtGeom gm;
   at_geometry(gm, hq, hkv, nb);
-  const uint8_t* pair_table = reinterpret_cast<const uint8_t*>(sched + AT_PAIR_TABLE);
-  uint16_t* order = reinterpret_cast<uint16_t*>(sched + 256);
-  for (int pos = threadIdx.x; pos < gm.n_gangs; pos += blockDim.x) {
+  static_assert(AT_GANG <= 32, "");  // a half-wave per gang, a lane per item
+  for (int pos = t >> 5; pos < gm.n_gangs; pos += THREADS / 32) {
     int h, j;
     at_gang_of(gm, pos, h, j);
-    const bool by_heads = pair_table[h >> 1] != 0;
+    const bool by_heads = pair_s[h >> 1] != 0;
     const int h_a = by_heads ? (h & ~1) : h, h_b = by_heads ? (h | 1) : h;
-    uint32_t wsum = 0;
-    for (int slot = 0; slot < gm.gang; ++slot) {
-      const int pair = gm.n_pairs - 1 - (j * gm.gang + slot);
-      if (pair < 0) break;
-      const int r_a = by_heads ? 2 * pair + (h & 1) : 2 * pair, r_b = by_heads ? r_a : r_a + 1;
-      if (r_a >= nb) continue;
+    const int slot = t & 31, pair = gm.n_pairs - 1 - (j * gm.gang + slot);
+    const int r_a = by_heads ? 2 * pair + (h & 1) : 2 * pair, r_b = by_heads ? r_a : r_a + 1;
+    uint32_t cnt = 0;
+    if (slot < gm.gang && pair >= 0 && r_a < nb) {
       const bool has_b = r_b < nb;
       const uint64_t* ma = mask + ((int64_t)h_a * nb + r_a) * nbw;
       const uint64_t* mb = mask + ((int64_t)h_b * nb + (has_b ? r_b : r_a)) * nbw;
       const int wmax = (has_b ? r_b : r_a) >> 6;
-      uint32_t cnt = AT_ITEM_FIXED;
+      cnt = AT_ITEM_FIXED;
       for (int wi = 0; wi <= wmax; ++wi)
         cnt += __builtin_popcountll(at_trim(ma[wi], wi, r_a) | (has_b ? at_trim(mb[wi], wi, r_b) : 0ull));
-      wsum += cnt;
     }
-    weight[pos] = wsum;
+    cnt = at_lane_sum<32>(cnt);
+    if (slot == 0) weight[pos] = cnt;
   }
   __syncthreads();
-  for (int pos = threadIdx.x; pos < gm.n_gangs; pos += blockDim.x) {
+  uint16_t* order = reinterpret_cast<uint16_t*>(sched + 256);
+  for (int pos = t; pos < gm.n_gangs; pos += THREADS) {
     const uint32_t wp = weight[pos];
     int rank = 0;
+#pragma unroll 8
     for (int o = 0; o < gm.n_gangs; ++o) {
       const uint32_t wo = weight[o];
       rank += (wo > wp) || (wo == wp && o < pos);
     }
     order[rank] = (uint16_t)pos;
   }
-  if (threadIdx.x == 0) sched[AT_ORDER_SLOT] = 1;
 }
 
 // ---- pivot heads with a slot: block-averaged attention map from the block sums the forward kernel kept ----
@@ -1617,23 +1665,21 @@ extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const
     max_pivots = fit > (size_t)(AT_NO_SLOT - 1) ? AT_NO_SLOT - 1 : (int)fit;
   }
   float* pivot_u = reinterpret_cast<float*>(ws + base_aligned);
-  hipLaunchKernelGGL(sp_attn_prep_kernel, dim3(1), dim3(128), 0, s, counter, decision, (int)hq, max_pivots);
-  SP_LAUNCH_CHECK();
-  if (!(flags & SP_ATTN_PAIR_ROWS)) {  // (otherwise the table stays as sp_attn_prep_kernel left it: rows paired)
-    hipLaunchKernelGGL(sp_attn_pairing_kernel, dim3((unsigned)((hq + 1) / 2)), dim3(256), 0, s, counter, mask, (int)hq,
-                       (int)(hq / hkv), (int)nb, (int)((nb + 63) / 64), max_pivots > 0 ? 1 : 0);
-    SP_LAUNCH_CHECK();
+  {
     // few gangs per workgroup and every head's K / V^T within the memory-side cache: deal the gangs heaviest first
-    // (measured on dense masks: +6 % at 16K tokens, +4 % at 32K; at 8K and below the ranking launch costs more
-    // than the better tail is worth)
+    // (measured on dense masks: +6 % at 16K tokens, +4 % at 32K; at 8K it makes no difference)
     const int64_t n_pairs = (nb + 1) / 2;
     const int64_t gang = n_pairs < AT_GANG ? n_pairs : AT_GANG;
     const int64_t n_gangs = hq * sp_ceil_div(n_pairs, gang);
-    if (nb > 64 && nb <= 256 && n_gangs <= AT_ORDER_MAX) {
-      hipLaunchKernelGGL(sp_attn_order_kernel, dim3(1), dim3(1024), 0, s, counter, mask, (int)hq, (int)hkv, (int)nb,
-                         (int)((nb + 63) / 64));
-      SP_LAUNCH_CHECK();
-    }
+    const int pair_rows = (flags & SP_ATTN_PAIR_ROWS) ? 1 : 0;
+    if (!pair_rows && nb > 64 && nb <= 256 && n_gangs <= AT_ORDER_MAX)
+      hipLaunchKernelGGL(sp_attn_schedule_kernel<true>, dim3(1), dim3(AT_ORDER_THREADS), 0, s, counter, mask, decision,
+                         (int)hq, (int)hkv, (int)nb, (int)((nb + 63) / 64), max_pivots, pair_rows);
+    else
+      hipLaunchKernelGGL(sp_attn_schedule_kernel<false>, dim3(pair_rows ? 1 : (unsigned)((hq + 1) / 2)),
+                         dim3(AT_PAIRING_THREADS), 0, s, counter, mask, decision, (int)hq, (int)hkv, (int)nb,
+                         (int)((nb + 63) / 64), max_pivots, pair_rows);
+    SP_LAUNCH_CHECK();
   }
   const size_t lds_bytes = AT_LDS_BYTES;
   // per device, once: the kernels' LDS allowance and the CU count (idempotent, so a race between two host threads
