@@ -14,6 +14,7 @@
 //     sorted order, integer prefix scan -- a literal sort / cumsum / threshold.
 #include <cstring>
 
+#include "sp_block_probs.h"
 #include "sp_pool.h"
 
 #define SEL_THREADS 1024
@@ -475,7 +476,8 @@ __global__ __launch_bounds__(CS_THREADS) void sp_cover_count_kernel(CoverCountAr
 
 // lower triangle of an [nb][nb] map (score_cover_idx), nb <= GSEL_ONE_NB
 #define GSEL_ONE_NB 256
-__device__ static void cover_select_map(CoverShared& sh, uint32_t* row_ties /* LDS [GSEL_ONE_NB] */, const float* __restrict__ xv,
+__device__ static __forceinline__ void cover_select_map(CoverShared& sh, uint32_t* row_ties /* LDS [GSEL_ONE_NB] */,
+                                                        const float* __restrict__ xv,
                                         int nb, int nbw, long long t_le, uint64_t* __restrict__ mv) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int WAVES = CS_THREADS / SP_WAVE;
@@ -1637,6 +1639,32 @@ __global__ __launch_bounds__(BP_THREADS) void sp_block_probs_kernel(
   for (int b = threadIdx.x; b < nb; b += BP_THREADS) out[b] = (b <= r) ? logit[b] / gsum : 0.f;
 }
 
+// Up to 128 blocks (16384 tokens at block size 128) a head's map is one row tile of bpm_rows, and the head's probabilities and
+// its selection are one workgroup and one launch: the map is read back by the workgroup that wrote it.  Beyond, a head's
+// row tiles are workgroups of a launch of their own.  Bound by latency (one K tile, two passes over it, the descent's
+// barriers) and, in layers without a query-aware head, by being a launch at all.  Whole layer, two launches / this one: 3001
+// tokens 110.8 -> 108.7 us, 6177 (64 channels) 122.4 -> 120.6, 10007 (28 / 4 heads) 268.9 -> 266.9; with all 32 heads
+// query-aware, 8192 tokens and the projections, 1164 -> 1161.
+template <int D>
+__global__ __launch_bounds__(CS_THREADS) void sp_queryaware_small_kernel(const sp_bf16* qbar, const sp_bf16* kbar,
+                                                                         const int32_t* __restrict__ decision, int hq, int hkv,
+                                                                         int nb, int nbw, uint32_t flags, float inv_sqrt_d,
+                                                                         float* probs, long long t_le, uint64_t* mask) {
+  __shared__ union {
+    BpmLds<D> rows;
+    struct {
+      __attribute__((aligned(16))) CoverShared cover;
+      uint32_t row_ties[GSEL_ONE_NB];
+    } sel;
+  } lds;
+  static_assert(CS_THREADS % BPM_THREADS == 0 && LQ_TILE <= GSEL_ONE_NB, "");
+  const int h = blockIdx.x;
+  if (decision[h] != SP_DEC_QA) return;
+  bpm_rows<D, CS_THREADS / BPM_THREADS>(lds.rows, qbar, kbar, 0, h, hq, hkv, nb, flags, inv_sqrt_d, probs);
+  __syncthreads();  // the map is written, the tile's LDS is free
+  cover_select_map(lds.sel.cover, lds.sel.row_ties, probs + (int64_t)h * nb * nb, nb, nbw, t_le, mask + (int64_t)h * nb * nbw);
+}
+
 // score = pattern_threshold * nb: the product of the caller's DOUBLE threshold and the block count, evaluated in
 // double as Python evaluates it (attention_sharing.py:361), then taken to fp32 as the comparison with an fp32
 // tensor takes it (utils.py:56).  A threshold that had been rounded to fp32 first would give a score one fp32 ulp
@@ -1656,6 +1684,19 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
              "sp_queryaware_select_bf16: bad shape");
   const size_t lds = (size_t)(d + nb) * sizeof(float);
   SP_REQUIRE(lds <= 60000, SP_ERR_UNSUPPORTED, "sp_queryaware_select_bf16: nb=%d too large", nb);
+  const float score = sp_queryaware_select_score(pattern_threshold, nb);
+  if ((d == 128 || d == 64) && nb <= LQ_TILE) {
+    SP_REQUIRE(workspace && workspace_bytes >= sp_cover_select_workspace_bytes(hq) && ((uintptr_t)workspace % 8) == 0,
+               SP_ERR_WORKSPACE, "sp_queryaware_select_bf16: workspace missing, misaligned or too small");  // (unused here)
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(hq), dim3(CS_THREADS), 0, (hipStream_t)stream, (const sp_bf16*)qbar, (const sp_bf16*)kbar,
+                         decision, (int)hq, (int)hkv, (int)nb, (int)((nb + 63) / 64), flags, sp_inv_sqrt_dim(flags, d), probs,
+                         (long long)sp_thr_le(score), mask);
+    };
+    d == 64 ? launch(sp_queryaware_small_kernel<64>) : launch(sp_queryaware_small_kernel<128>);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
   if (d == 128 || d == 64) {  // two passes on the matrix core, 128 rows per workgroup
     const int rc = sp_block_probs_mfma_launch(qbar, kbar, decision, hq, hkv, d, nb, flags, probs, (hipStream_t)stream);
     if (rc != SP_OK) return rc;
@@ -1665,7 +1706,6 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
                        sp_inv_sqrt_dim(flags, d), probs);
     SP_LAUNCH_CHECK();
   }
-  const float score = sp_queryaware_select_score(pattern_threshold, nb);
   return gsel_run(probs, decision, SP_DEC_QA, hq, nb, score, mask, workspace, workspace_bytes, (hipStream_t)stream,
                   "sp_queryaware_select_bf16");
 }

@@ -359,3 +359,31 @@ def test_pivot_update_with_several_dense_heads_of_one_cluster_keeps_the_highest(
         want[0, 0] = True
         assert np.array_equal(ops.mask_to_bool(many.pattern[slot], nb).cpu().numpy(), want)
         assert torch.equal(many.avg_map[slot], avg[h])
+
+
+# one workgroup per head up to 128 blocks, a workgroup per 128 rows and a selection of its own beyond
+@pytest.mark.parametrize("nb", [1, 31, 33, 64, 65, 127, 128, 129, 200])
+@pytest.mark.parametrize("hq,hkv,d", [(6, 2, 128), (5, 5, 64)])
+def test_queryaware_map_and_its_selection(gpu_device, nb, hq, hkv, d):
+    """The map against the softmax in 64 bits, the bits it selects against cover_select_global on that map; heads that
+    are not query-aware keep map and mask.  Logits in fp32 (|logit| <= 8, 128 terms): off by 8 * 128 * 2^-24 at most,
+    and the probabilities by twice that, their sums and exp2 on top: 2e-4 relative."""
+    from shareprefill_amd import _lib, ops
+
+    gen = torch.Generator().manual_seed(nb)
+    qbar, kbar = (torch.randn(nb, h, d, generator=gen).to(torch.bfloat16) for h in (hq, hkv))
+    decision = torch.tensor([3 if h % 3 != 1 else 0 for h in range(hq)], dtype=torch.int32)
+    nbw = (nb + 63) // 64
+    mask = torch.zeros(hq, nb, nbw, dtype=torch.int64, device=gpu_device)
+    probs = ops.queryaware_select(qbar.to(gpu_device), kbar.to(gpu_device), decision.to(gpu_device), mask, 0.9, 0)
+    want_mask = torch.zeros_like(mask)
+    score = _lib.load().sp_queryaware_select_score(0.9, nb)
+    for h in range(hq):
+        if decision[h] != 3:
+            continue
+        scaled = (qbar[:, h].float() * (1.0 / d ** 0.5)).to(torch.bfloat16)
+        logits = scaled.double() @ kbar[:, h // (hq // hkv)].double().T
+        logits.masked_fill_(torch.ones(nb, nb, dtype=torch.bool).triu(1), float("-inf"))
+        torch.testing.assert_close(probs[h].cpu().double(), logits.softmax(-1), rtol=2e-4, atol=1e-9)
+        ops.cover_select_global(probs[h:h + 1].contiguous(), score, want_mask[h:h + 1])
+    assert torch.equal(mask, want_mask)
