@@ -253,6 +253,14 @@ int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t 
                            int64_t v_stride_n, int64_t v_stride_h, float softmax_scale, const uint64_t* mask,
                            const int32_t* decision, void* out, float* avg_attn, void* workspace,
                            size_t workspace_bytes, sp_stream_t stream);
+/* The same with sp_pivot_update(state, head_cluster, decision, avg_attn, hq, nb, pattern_threshold) behind it, in the one
+ * launch: decision, avg_attn (cleared by the caller or sp_select_layer_bf16) and head_cluster must be given. */
+int sp_short_attn_pivot_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                           int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,
+                           int64_t v_stride_n, int64_t v_stride_h, float softmax_scale, const uint64_t* mask,
+                           const int32_t* decision, void* out, float* avg_attn, void* workspace,
+                           size_t workspace_bytes, const sp_cluster_state* state,
+                                 const int32_t* head_cluster, float pattern_threshold, sp_stream_t stream);
 
 /* ---- decode step -------------------------------------------------------------------------------
  * Replaces the flash_attn_func call of the decode branch (shareprefill_attn.py:146-155): one query token per

@@ -80,6 +80,8 @@ SIGNATURES = {
     "sp_short_attn_workspace_bytes": (_SZ, [_I64, _I32]),
     "sp_short_attn_fwd_bf16": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _P,
                                       _P, _P, _P, _SZ, _P]),
+    "sp_short_attn_pivot_fwd_bf16": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _P,
+                                      _P, _P, _P, _SZ, _ST, _P, _F, _P]),
     "sp_decode_workspace_bytes": (_SZ, [_I64, _I32, _I32]),
     "sp_decode_attn_bf16": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _F, _P, _P, _SZ,
                                    _P]),

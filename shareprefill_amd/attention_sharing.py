@@ -273,6 +273,10 @@ class AttentionSharing:
             decision = use_dense.reshape(-1)
         ops.pivot_update(self._state, hc, decision, avg_attn[0], pattern_threshold)
 
+    def pivot_slabs(self, layer_idx: int, hq: int, device, pattern_threshold: float):
+        """What ops.short_attention takes to do update_pivotal_attns itself."""
+        return self._state, self._head_cluster_tensor(layer_idx, hq, device), pattern_threshold
+
     def note_dense_layer(self, layer_idx: int, hq: int, nb: int) -> None:
         """A layer whose prompt is no longer than the minimum budget ran on the dense causal mask without any
         selection (see shareprefill_attention_core); counted for decision_histogram."""

@@ -21,12 +21,14 @@
 //     (ds_read_b64_tr_b16: the 16 lanes of a group address 4 keys x 16 channels and each receives 4 keys of its channel).
 //     S^T = K . Q^T leaves a lane with keys 4g .. 4g+3 of every 16-key tile (g = lane / 16), which is exactly what two such
 //     reads deliver, so P^T is the S^T accumulators converted to bf16 in place;
-//   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel); a call
+//   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel), and so is the
+//     row's pattern in the sharing state, which needs nothing but that row (a launch in every layer, of which all but one per
+//     cluster had nothing to do: 3001 tokens 108.6 -> 106.2 us a layer, 6177 of 64 channels 121.2 -> 119.8); a call
 //     without decisions has its maps cleared here (a fill launch in front of the kernel costs its caller 5 us of host time:
 //     700 tokens 21.3 -> 18.7 us a layer).
 // Two rows sharing one K / V tile, as in the persistent kernel, halve the tile traffic per flop, which is why that one
 // stays for long prompts; sp_short_attn_max_tokens holds the line between the two and the figures.
-#include "sp_common.h"
+#include "sp_rows.h"
 
 #include <type_traits>
 
@@ -41,6 +43,9 @@ struct AsArgs {
   int hq, group, nb, nbw;
   int zero_maps;             // 1: no decisions, every row of avg_attn is cleared
   float scale_log2;
+};
+struct AsPivotArgs : AsArgs {
+  PivotArgs pivot;
 };
 
 typedef __bf16 as_bf16x8 __attribute__((ext_vector_type(8)));
@@ -148,8 +153,10 @@ __device__ __forceinline__ float as_groupmax(float v) {
 }
 
 // KSPLIT = 2: two sets of four waves own the same queries and take the even and the odd 64-key tiles.
-template <int D, int KSPLIT>
-__global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(AsArgs a) {
+// Args = AsPivotArgs: with the pivots' patterns (an instance of its own: prompts that select nothing, whose launch is the
+// whole layer, run 1.5 % slower with that code in theirs).
+template <int D, int KSPLIT, typename Args>
+__global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(Args a) {
   constexpr int QT = 2;                             // 16-query tiles per wave
   constexpr int KS = D / 32, CT = D / 16;           // channel steps of S, channel tiles of O
   constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS * KSPLIT, WQ = 16 * QT;
@@ -434,6 +441,11 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
     for (int w = 0; w < WAVES * KSPLIT; ++w) x += part[i * (WAVES * KSPLIT) + w];
     a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = x * inv_q;
   }
+  if constexpr (std::is_same<Args, AsPivotArgs>::value) {
+    __shared__ PivotRowShared pivot_sh;
+    __syncthreads();  // the row is written, LDS is free
+    pivot_row<THREADS>(a.pivot, pivot_sh, lds_all, a.avg_attn, r, h);
+  }
 }
 
 // ---- host ---------------------------------------------------------------------------------------------
@@ -452,32 +464,33 @@ extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {
   return (size_t)hq * (nb * (nb + 1) / 2) * 2 * AS_BS * sizeof(float);
 }
 
-extern "C" int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
+static int as_launch(const char* who, const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
                                       int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
                                       int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,
                                       const uint64_t* mask, const int32_t* decision, void* out, float* avg_attn,
-                                      void* workspace, size_t workspace_bytes, sp_stream_t stream) {
-  SP_REQUIRE(q && k && v && mask && out, SP_ERR_INVALID_ARGUMENT, "sp_short_attn_fwd_bf16: null pointer");
+                                      void* workspace, size_t workspace_bytes, const PivotArgs* pivot, sp_stream_t stream) {
+  SP_REQUIRE(q && k && v && mask && out, SP_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
   SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT,
-             "sp_short_attn_fwd_bf16: bad shape n=%lld hq=%d hkv=%d", (long long)n, hq, hkv);
-  SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "sp_short_attn_fwd_bf16: softmax_scale must be > 0");
-  SP_REQUIRE(d == 128 || d == 64, SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: head_dim %d unsupported (64 or 128)", d);
+             "%s: bad shape n=%lld hq=%d hkv=%d", who, (long long)n, hq, hkv);
+  SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "%s: softmax_scale must be > 0", who);
+  SP_REQUIRE(d == 128 || d == 64, SP_ERR_UNSUPPORTED, "%s: head_dim %d unsupported (64 or 128)", who, d);
   SP_REQUIRE((q_stride_n | q_stride_h | k_stride_n | k_stride_h | v_stride_n | v_stride_h) % 8 == 0 &&
                  ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0,
-             SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: tensors must be 16-byte aligned, strides multiple of 8");
+             SP_ERR_UNSUPPORTED, "%s: tensors must be 16-byte aligned, strides multiple of 8", who);
   SP_REQUIRE(k_stride_n >= 0 && v_stride_n >= 0 && AS_BS * k_stride_n < (1ll << 31) && AS_BS * v_stride_n < (1ll << 31),
-             SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: token strides %lld / %lld unsupported", (long long)k_stride_n,
+             SP_ERR_UNSUPPORTED, "%s: token strides %lld / %lld unsupported", who, (long long)k_stride_n,
              (long long)v_stride_n);
   const int64_t nb = sp_ceil_div(n, AS_BS);
-  SP_REQUIRE(nb <= AS_MAX_NB && nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: n=%lld hq=%d too large",
+  SP_REQUIRE(nb <= AS_MAX_NB && nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "%s: n=%lld hq=%d too large", who,
              (long long)n, hq);
   const bool maps = decision != nullptr && avg_attn != nullptr;
   SP_REQUIRE(!maps || (workspace && workspace_bytes >= sp_short_attn_workspace_bytes(n, hq) && ((uintptr_t)workspace % 4) == 0),
-             SP_ERR_WORKSPACE, "sp_short_attn_fwd_bf16: workspace missing, misaligned or too small");
+             SP_ERR_WORKSPACE, "%s: workspace missing, misaligned or too small", who);
   const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
                     maps ? (float*)workspace : nullptr, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
                     v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), decision == nullptr && avg_attn != nullptr,
                     softmax_scale * 1.4426950408889634f};
+  static_assert(AS_LDS_BYTES(64, 1) >= AS_MAX_NB * 14 + AS_THREADS * 2 * 8 + 16, "");  // rs_lds_bytes(AS_MAX_NB, 2 sets)
   const dim3 grid((unsigned)(nb * hq));
   // Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
   // 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).
@@ -485,21 +498,61 @@ extern "C" int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* 
   static bool attr_set[64] = {false};  // per device, once (idempotent)
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));
-  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "sp_short_attn_fwd_bf16: device index %d", dev);
+  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "%s: device index %d", who, dev);
   if (!attr_set[dev]) {
-    const void* kernels[4] = {(const void*)sp_attn_short_kernel<64, 1>, (const void*)sp_attn_short_kernel<128, 1>,
-                              (const void*)sp_attn_short_kernel<64, 2>, (const void*)sp_attn_short_kernel<128, 2>};
+    const void* kernels[8] = {
+        (const void*)sp_attn_short_kernel<64, 1, AsArgs>,      (const void*)sp_attn_short_kernel<128, 1, AsArgs>,
+        (const void*)sp_attn_short_kernel<64, 2, AsArgs>,      (const void*)sp_attn_short_kernel<128, 2, AsArgs>,
+        (const void*)sp_attn_short_kernel<64, 1, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, 1, AsPivotArgs>,
+        (const void*)sp_attn_short_kernel<64, 2, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, 2, AsPivotArgs>};
     for (const void* f : kernels)
       SP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AS_LDS_BYTES(128, 2)));
     attr_set[dev] = true;
   }
-  auto launch = [&](auto kernel, int ksplit) {
-    hipLaunchKernelGGL(kernel, grid, dim3(AS_THREADS * ksplit), AS_LDS_BYTES(d, ksplit), (hipStream_t)stream, a);
+  auto launch = [&](auto kernel, int ksplit, const auto& args) {
+    hipLaunchKernelGGL(kernel, grid, dim3(AS_THREADS * ksplit), AS_LDS_BYTES(d, ksplit), (hipStream_t)stream, args);
   };
-  if (d == 64)
-    split ? launch(sp_attn_short_kernel<64, 2>, 2) : launch(sp_attn_short_kernel<64, 1>, 1);
-  else
-    split ? launch(sp_attn_short_kernel<128, 2>, 2) : launch(sp_attn_short_kernel<128, 1>, 1);
+  auto pick = [&](const auto& args) {
+    using Args = std::decay_t<decltype(args)>;
+    if (d == 64)
+      split ? launch(sp_attn_short_kernel<64, 2, Args>, 2, args) : launch(sp_attn_short_kernel<64, 1, Args>, 1, args);
+    else
+      split ? launch(sp_attn_short_kernel<128, 2, Args>, 2, args) : launch(sp_attn_short_kernel<128, 1, Args>, 1, args);
+  };
+  if (pivot != nullptr) {
+    AsPivotArgs with;
+    static_cast<AsArgs&>(with) = a;
+    with.pivot = *pivot;
+    pick(with);
+  } else {
+    pick(a);
+  }
   SP_LAUNCH_CHECK();
   return SP_OK;
+}
+
+extern "C" int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
+                                      int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                      int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,
+                                      const uint64_t* mask, const int32_t* decision, void* out, float* avg_attn,
+                                      void* workspace, size_t workspace_bytes, sp_stream_t stream) {
+  return as_launch("sp_short_attn_fwd_bf16", q, k, v, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
+                   v_stride_h, softmax_scale, mask, decision, out, avg_attn, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int sp_short_attn_pivot_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
+                                            int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                            int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,
+                                            const uint64_t* mask, const int32_t* decision, void* out, float* avg_attn,
+                                            void* workspace, size_t workspace_bytes, const sp_cluster_state* state,
+                                            const int32_t* head_cluster, float pattern_threshold, sp_stream_t stream) {
+  SP_REQUIRE(decision && avg_attn && head_cluster, SP_ERR_INVALID_ARGUMENT, "sp_short_attn_pivot_fwd_bf16: null pointer");
+  const int nb = (int)sp_ceil_div(n, AS_BS);
+  int rc = check_state(state, nb, "sp_short_attn_pivot_fwd_bf16");
+  if (rc) return rc;
+  SP_REQUIRE(hq <= 1024, SP_ERR_UNSUPPORTED, "sp_short_attn_pivot_fwd_bf16: hq=%d unsupported", hq);
+  const PivotArgs pivot = {state_by_value(state), head_cluster, decision, hq, nb, (nb + 63) / 64,
+                           (long long)sp_thr_lt(pattern_threshold)};
+  return as_launch("sp_short_attn_pivot_fwd_bf16", q, k, v, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
+                   v_stride_h, softmax_scale, mask, decision, out, avg_attn, workspace, workspace_bytes, state->n_clusters > 0 ? &pivot : nullptr, stream);
 }

@@ -374,10 +374,11 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     return out
 
 
-def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None) -> torch.Tensor:
+def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, pivot=None) -> torch.Tensor:
     """block_sparse_attention for short prompts (block size 128, head_dim 64 or 128): q [Hq,N,D], k/v [Hkv,N,D] views,
     mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D].  One launch, whatever decision says: v is read as it is and the maps of
-    DENSE heads are written by the same kernel (avg_attn without decision is cleared)."""
+    DENSE heads are written by the same kernel (avg_attn without decision is cleared).
+    pivot = (state, head_cluster, pattern_threshold): pivot_update with decision and avg_attn is part of the launch."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")
@@ -395,9 +396,14 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None) 
     timer = kernel_timer
     if timer is not None:
         timer.start("attn")
-    st = lib.sp_short_attn_fwd_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), n, hq, k.shape[0], d, q.stride(1), q.stride(0),
-                                    k.stride(1), k.stride(0), v.stride(1), v.stride(0), softmax_scale, mask.data_ptr(),
-                                    _ptr(decision), out.data_ptr(), _ptr(avg_attn), _ptr(ws), ws_bytes, stream)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), n, hq, k.shape[0], d, q.stride(1), q.stride(0), k.stride(1), k.stride(0),
+            v.stride(1), v.stride(0), softmax_scale, mask.data_ptr(), _ptr(decision), out.data_ptr(), _ptr(avg_attn), _ptr(ws),
+            ws_bytes)
+    if pivot is None:
+        st = lib.sp_short_attn_fwd_bf16(*args, stream)
+    else:
+        state, head_cluster, threshold = pivot
+        st = lib.sp_short_attn_pivot_fwd_bf16(*args, state.ref(), head_cluster.data_ptr(), threshold, stream)
     if timer is not None:
         timer.stop("attn")
     _lib.check(st, "sp_short_attn_fwd_bf16")

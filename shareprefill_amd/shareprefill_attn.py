@@ -224,12 +224,13 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
                               config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold,
                               scale_dim=model_dim, avg_attn=avg_attn[0])
     if short:
-        out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0])
+        out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0],
+                                  pivot=sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold))
     else:
         out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
                                          avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,
                                          half_channels=model_dim != head_dim)
-    sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
+        sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
     return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
 
 

@@ -52,3 +52,40 @@ def test_short_attention_matches_oracle(gpu_device, hq, hkv, n, d):
     assert not avg[~dense].any()
     for h in np.nonzero(dense)[0]:
         assert np.abs(avg[h] - np.asarray(maps[h])).max() <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("hq,hkv,n,d", [(6, 2, 1, 64), (6, 2, 1111, 128), (6, 6, 2177, 64), (32, 8, 2048, 128),
+                                        (32, 8, 2177, 128), (3, 1, 8300, 128)])
+def test_pivot_patterns_in_the_attention_launch(gpu_device, hq, hkv, n, d):
+    """State, maps and outputs of the launch that also updates the pivots' state equal those of two calls, to the bit,
+    with several dense heads of a cluster, a dense head without one and clusters without a dense head; counters and
+    accumulators serve a second call."""
+    from shareprefill_amd import ops
+
+    nb = -(-n // 128)
+    rng = np.random.default_rng(n + d)
+    hc = torch.tensor([(-1, 0, 1, 2, 0, 2)[h % 6] for h in range(hq)], dtype=torch.int32, device=gpu_device)
+    dense = np.array([h % 6 in (0, 1, 4) or h == 2 for h in range(hq)])
+    decision = torch.where(torch.from_numpy(dense), O.DEC_DENSE, O.DEC_VS).to(torch.int32).to(gpu_device)
+    states = [ops.ClusterState(3, nb, gpu_device, keep_maps=True) for _ in range(2)]
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    for rep in range(2):
+        mask = np.tril(rng.random((hq, nb, nb)) < 0.4)
+        mask[:, np.arange(nb), np.arange(nb)] = True
+        mask[dense] = np.tril(np.ones((nb, nb), dtype=bool))
+        bits = ops.bool_to_mask(torch.from_numpy(mask)).to(gpu_device)
+        q, k, v = (torch.randn(h, n, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h in (hq, hkv, hkv))
+        cols, dists = (torch.from_numpy(rng.random((3, nb)) < 0.3).to(gpu_device) for _ in range(2))
+        avgs = [torch.zeros(hq, nb, nb, dtype=torch.float32, device=gpu_device) for _ in range(2)]
+        for state in states:
+            state.cols.copy_(cols)
+            state.dists.copy_(dists)
+        out = ops.short_attention(q, k, v, bits, d ** -0.5, decision, avgs[0])
+        ops.pivot_update(states[0], hc, decision, avgs[0], 0.9)
+        got = ops.short_attention(q, k, v, bits, d ** -0.5, decision, avgs[1], pivot=(states[1], hc, 0.9))
+        assert torch.equal(got, out) and torch.equal(avgs[0], avgs[1])
+        for slab in ("info", "pattern", "accum", "avg_map"):  # (the third cluster's map is never written)
+            assert torch.equal(getattr(states[0], slab)[:2], getattr(states[1], slab)[:2]), slab
+        assert torch.equal(states[0].ratio.view(torch.int64), states[1].ratio.view(torch.int64))
+        assert states[1].info[:, 1].tolist() == [1, 1, 0]
+        assert not states[1].accum.any() and not states[1].info[:, 5].any()
