@@ -450,19 +450,21 @@ def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, so
     b, hq, _, d = q.shape
     _, hkv, n, _ = k.shape
     dev = q.device
-    for t, name in ((q, "q"), (k, "k"), (v, "v")):
-        if t.dtype != torch.bfloat16:
-            raise AssertionError(f"{name} must be bfloat16, got {t.dtype}")
-        if not t.is_cuda or t.device != dev:
-            raise ValueError(f"{name} must live on the GPU the queries are on")
-        if t.stride(3) != 1:
-            raise ValueError(f"{name} must have a contiguous head_dim axis")
+    (q_b, q_h, _, q_d), (k_b, k_h, k_n, k_d), (v_b, v_h, v_n, v_d) = q.stride(), k.stride(), v.stride()
+    if not (q.dtype is k.dtype is v.dtype is torch.bfloat16 and q.is_cuda and k.device == dev and v.device == dev
+            and q_d == k_d == v_d == 1):
+        for t, name in ((q, "q"), (k, "k"), (v, "v")):
+            if t.dtype != torch.bfloat16:
+                raise AssertionError(f"{name} must be bfloat16, got {t.dtype}")
+            if not t.is_cuda or t.device != dev:
+                raise ValueError(f"{name} must live on the GPU the queries are on")
+            if t.stride(3) != 1:
+                raise ValueError(f"{name} must have a contiguous head_dim axis")
     if v.shape != k.shape or k.shape[0] != b or k.shape[3] != d:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} do not match q {tuple(q.shape)}")
     stream = _stream_handle(dev)
     out = torch.empty((b, 1, hq, d), dtype=torch.bfloat16, device=dev)
     ws = _workspace("decode", lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv), dev)
-    (q_b, q_h, _, _), (k_b, k_h, k_n, _), (v_b, v_h, v_n, _) = q.stride(), k.stride(), v.stride()
     if b == 1:
         q_b = k_b = v_b = 0  # (the stride of an axis of one entry means nothing)
     st = lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b, n, hq, hkv, d, q_b, q_h, k_b, k_n, k_h,

@@ -139,6 +139,18 @@ def triton_block_wise_prefill_attention(q: torch.Tensor, k: torch.Tensor, v: tor
     return torch.stack(outs), torch.stack(avgs)
 
 
+def _decode_step(module, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor) -> torch.Tensor:
+    """One query against the whole cache (shareprefill_attn.py:146-155), nothing is selected: -> [B, 1, Hq, D] contiguous.
+
+    The HIP kernel is the only path (bf16, head_dim a multiple of 8 up to 128 -- smaller heads are padded inside the kernel,
+    the cache is read as it is -- at most 32 query heads per kv head, 16-byte aligned rows); anything else raises from the
+    entry point's own checks, as every other unsupported shape does."""
+    if query_states.dtype != torch.bfloat16:
+        raise AssertionError(f"SharePrefill attention expects bfloat16 q/k/v, got {query_states.dtype}")
+    scale = module.scaling if hasattr(module, "scaling") else 1.0 / math.sqrt(query_states.shape[3])
+    return ops.decode_attention_batch(query_states, key_states, value_states, scale)
+
+
 def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: torch.Tensor,
                                 value_states: torch.Tensor, *, gqa_interleave: bool = False
                                 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
@@ -158,13 +170,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
     del gqa_interleave
 
     if q_len == 1:
-        # decode step (shareprefill_attn.py:146-155): one query against the whole cache, nothing is selected.
-        # The HIP kernel is the only path (bf16, head_dim a multiple of 8 up to 128 -- smaller heads are padded inside
-        # the kernel, the cache is read as it is -- at most 32 query heads per kv head, 16-byte aligned rows); anything
-        # else raises from the entry point's own checks, as every other unsupported shape does.
-        if query_states.dtype != torch.bfloat16:
-            raise AssertionError(f"SharePrefill attention expects bfloat16 q/k/v, got {query_states.dtype}")
-        return ops.decode_attention_batch(query_states, key_states, value_states, softmax_scale).transpose(1, 2), None
+        return _decode_step(module, query_states, key_states, value_states).transpose(1, 2), None
 
     if bsz != 1:
         raise ValueError("SharePrefill prefill keeps per-cluster state for batch size 1 only")
@@ -245,6 +251,8 @@ def shareprefill_attention_forward(module, query_states: torch.Tensor, key_state
     if kwargs.pop("sliding_window", None) is not None:
         raise NotImplementedError("SharePrefill attention does not support sliding-window mode yet.")
     gqa_interleave = kwargs.pop("gqa_interleave", False)
+    if query_states.dim() == 4 and query_states.shape[2] == 1:
+        return _decode_step(module, query_states, key_states, value_states), None  # (in the layout wanted here)
     attn_output, attn_weights = shareprefill_attention_core(module, query_states, key_states, value_states,
                                                             gqa_interleave=gqa_interleave)
     return attn_output.transpose(1, 2).contiguous(), attn_weights
