@@ -1595,7 +1595,7 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
 // The stages above, with the launches folded that do not wait for each other: K's averages beside the score statistics, the
 // query-aware test and the share similarities beside the budgets, Q's averages, the pivots' own sets and the clearing of the
 // map beside the masks.  Same device code, same results.  A launch costs 5 us of the stream whatever it does; whole layer,
-// 15 launches / these 7: 3001 tokens 142 -> 120 us, 6177 (64 channels) 148 -> 127, 10007 (28 / 4 heads) 336 -> 313.
+// 15 launches / 7 (six up to 128 blocks since): 3001 tokens 142 -> 120 us, 6177 (64 channels) 148 -> 127, 10007 (28 / 4 heads) 336 -> 313.
 struct HeadArgs {
   CoverCountArgs cover;
   int n_cover;  // workgroups 0 .. n_cover - 1: the budgets (0: made by other launches); then one per head
