@@ -624,17 +624,15 @@ __device__ __forceinline__ float at_groupmax(float mx) {
 // accumulated in o[8] -- so numerator and denominator of the softmax see the same values and the result does not
 // depend on the largest probability being exactly 1.  No maximum per half-tile: the packed probabilities are OR-ed
 // (three instructions per step) and one test of the top exponent bit per step says whether some P(j-1) >= 2, is inf
-// or NaN (the first keys of a row, m_run = AT_NO_MAX; a logit far above the max).  Only then is the max taken from S(j-1)
+// or NaN (the first keys of a row, m_run = AT_NO_MAX; a logit more than one octave above the max).  Only then is the max taken from S(j-1)
 // -- still intact in the registers the next stage overwrites -- O and the sums are rescaled and P(j-1) is formed again;
 // P(j-1) enters O only after this test.
-// The max is set AT_HEADROOM octaves above the largest logit seen, so that only a logit that many octaves (and one) higher
-// triggers again: probabilities are then around 2^-24, which bf16 and fp32 hold as precisely as those around 1, and what
-// is 2^-102 of the largest underflows.  A rescale costs a wave 1800 cycles where a 64-key step takes 2700 -- and the
-// waves at its barrier with it --, and set at the logit itself the first tiles of most rows had several (bench masks, whole
-// layer, same box: 3001 tokens 190 -> 181 us, 32768 2.93 -> 2.85 ms, 65001 at a tenth of the blocks 2.79 -> 2.67 ms,
-// 131072 55.84 -> 55.45 ms).
+// The max is the largest logit itself, so the probabilities that weigh most are at or near 1, where bf16 loses least of them.
+// Set some octaves above it, rescales become rare (32768 tokens 2.93 -> 2.85 ms a layer, 131072 55.84 -> 55.45), but whatever
+// logit came first then fixes the fraction all later probabilities are rounded at, and the exponent's argument is coarser: at
+// 24 octaves the output was 5 to 7 % further from the attention in 64 bits (16384 tokens 1.96e-3 against 1.84e-3) and the
+// pivots' maps nearly twice as far (2.3e-5 against 1.2e-5), so it stays at 0.
 #define AT_NO_MAX (-1.0e30f)          // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
-#define AT_HEADROOM 24.0f
 #define AT_P_TOO_LARGE 0x40004000u    // bf16 pair: exponent >= 128 in either half
 
 // s_prev = S(j-1) (causal predicate applied), p = P(j-1), det = OR of its packed words.  On return p is safe to use.
@@ -649,8 +647,8 @@ __device__ __forceinline__ void at_commit(const floatx4 (&s_prev)[2][2], bf16x8 
   if (__builtin_amdgcn_ballot_w64(((det[0] | det[1]) & AT_P_TOO_LARGE) != 0u) != 0ull) {
     float mx[2];  // (S(j-1) is a whole stage old: no wait states needed before reading it)
     at_lanemax(s_prev, mx);
-    const float m_new[2] = {at_max2(m_run[0], at_groupmax(mx[0] * scale_log2) + AT_HEADROOM),
-                            at_max2(m_run[1], at_groupmax(mx[1] * scale_log2) + AT_HEADROOM)};
+    const float m_new[2] = {at_max2(m_run[0], at_groupmax(mx[0] * scale_log2)),
+                            at_max2(m_run[1], at_groupmax(mx[1] * scale_log2))};
     at_settle_o(o);
     // m_run = AT_NO_MAX on a row's first keys: alpha = 0 (O and the sums are still zero then)
     const float alpha[2] = {__builtin_amdgcn_exp2f(m_run[0] - m_new[0]), __builtin_amdgcn_exp2f(m_run[1] - m_new[1])};

@@ -62,7 +62,6 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 #define AS_WAVES 4
 #define AS_MAX_NB 512     // blocks a row's list holds
 #define AS_LDS_BYTES(D, KSPLIT) ((KSPLIT) * 4 * AS_TILE * (D) * 2)
-#define AS_HEADROOM 24.0f  // octaves the running max is set above the largest logit seen
 #define AS_NO_MAX (-1.0e30f)         // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
 #define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
 
@@ -286,9 +285,9 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
               if (half * AS_TILE + 16 * kt + 4 * g + j > q_off + 16 * qt) s[kt][qt][j] = -INFINITY;
       }
       uint32_t pk[QT][8];
-      auto softmax = [&](int qt) {
+      auto softmax = [&](int qt, int hh) {  // half hh: 32 keys
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
+        for (int kt = 2 * hh; kt < 2 * hh + 2; ++kt) {
           float e[4];
 #pragma unroll
           for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][qt][j], a.scale_log2, -m[qt]));
@@ -296,68 +295,76 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
           pk[qt][2 * kt + 1] = as_pack2(e[2], e[3]);
         }
       };
-      uint32_t det = 0u;
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
-        softmax(qt);
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) det |= pk[qt][i] | pk[qt][i + 1];
+        softmax(qt, 0);
+        softmax(qt, 1);
       }
-      // The running max is lazy, as in the persistent kernel: it moves only when some probability came out at 2 or more
-      // (or is inf: a row's first keys), and then this tile's probabilities are formed again before they are used.
-      if (__ballot((det & AS_P_TOO_LARGE) != 0u) != 0ull) {
+      as_static_for<0, 2>([&](auto hc) {
+        constexpr int hh = decltype(hc)::value;
+        // The running max is lazy, as in the persistent kernel and in its steps of 32 keys, which gives its bits: it moves
+        // only when some probability came out at 2 or more (or is inf: a row's first keys), and then the probabilities are
+        // formed again before they are used.
+        uint32_t det = 0u;
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-          float mx = -INFINITY;
+        for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-            mx = fmaxf(mx, fmaxf(fmaxf(s[kt][qt][0], s[kt][qt][1]), fmaxf(s[kt][qt][2], s[kt][qt][3])));
-          const float m_new = fmaxf(m[qt], as_groupmax(mx) * a.scale_log2 + AS_HEADROOM);
-          const float alpha = __builtin_amdgcn_exp2f(m[qt] - m_new);
+          for (int i = 4 * hh; i < 4 * hh + 4; i += 2) det |= pk[qt][i] | pk[qt][i + 1];
+        if (__ballot((det & AS_P_TOO_LARGE) != 0u) != 0ull) {
 #pragma unroll
-          for (int ct = 0; ct < CT; ++ct) o[ct][qt] *= alpha;
-          l[qt] *= alpha;
-          l_mark[qt] *= alpha;
-          m[qt] = m_new;
-          softmax(qt);
+          for (int qt = 0; qt < QT; ++qt) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kt = 2 * hh; kt < 2 * hh + 2; ++kt)
+              mx = fmaxf(mx, fmaxf(fmaxf(s[kt][qt][0], s[kt][qt][1]), fmaxf(s[kt][qt][2], s[kt][qt][3])));
+            const float m_new = fmaxf(m[qt], as_groupmax(mx * a.scale_log2));
+            const float alpha = __builtin_amdgcn_exp2f(m[qt] - m_new);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) o[ct][qt] *= alpha;
+            l[qt] *= alpha;
+            l_mark[qt] *= alpha;
+            m[qt] = m_new;
+            softmax(qt, hh);
+            if constexpr (hh == 0) softmax(qt, 1);
+          }
         }
-      }
-      // O += V^T . P: groups of four channel tiles of one 32-key half, the next group's operands on their way
-      constexpr int GR = CT / 2;  // groups
-      as_u32x2 vr[2][8];
-      auto fetch = [&](auto gc) {
-        constexpr int gi = decltype(gc)::value, hh = gi / (GR / 2), c0 = (gi % (GR / 2)) * 4;
-        as_static_for<0, 4>([&](auto uc) {
-          constexpr int u = decltype(uc)::value;
-          const uint32_t ad = vt_addr + (uint32_t)(((2 * (c0 + u) + vhalf) ^ vswz) << 4);
-          vr[gi & 1][2 * u] = as_read_tr<hh * 32 * (D * 2)>(ad);
-          vr[gi & 1][2 * u + 1] = as_read_tr<hh * 32 * (D * 2) + 16 * (D * 2)>(ad);
-        });
-      };
-      fetch(std::integral_constant<int, 0>{});
-      as_static_for<0, GR>([&](auto gc) {
-        constexpr int gi = decltype(gc)::value, hh = gi / (GR / 2), c0 = (gi % (GR / 2)) * 4;
-        if constexpr (gi + 1 < GR) {
-          fetch(std::integral_constant<int, gi + 1>{});
-          as_wait_v<8>(vr[gi & 1]);
-        } else {
-          as_wait_v<0>(vr[gi & 1]);
-        }
+        // O += V^T . P: groups of four channel tiles, the next group's operands on their way
+        constexpr int GR = CT / 4;
+        as_u32x2 vr[2][8];
+        auto fetch = [&](auto gc) {
+          constexpr int gi = decltype(gc)::value;
+          as_static_for<0, 4>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            const uint32_t ad = vt_addr + (uint32_t)(((2 * (4 * gi + u) + vhalf) ^ vswz) << 4);
+            vr[gi & 1][2 * u] = as_read_tr<hh * 32 * (D * 2)>(ad);
+            vr[gi & 1][2 * u + 1] = as_read_tr<hh * 32 * (D * 2) + 16 * (D * 2)>(ad);
+          });
+        };
         as_bf16x8 p[QT];
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
           p[qt] = __builtin_bit_cast(as_bf16x8, (as_u32x4){pk[qt][4 * hh], pk[qt][4 * hh + 1], pk[qt][4 * hh + 2], pk[qt][4 * hh + 3]});
+        fetch(std::integral_constant<int, 0>{});
+        as_static_for<0, GR>([&](auto gc) {
+          constexpr int gi = decltype(gc)::value;
+          if constexpr (gi + 1 < GR) {
+            fetch(std::integral_constant<int, gi + 1>{});
+            as_wait_v<8>(vr[gi & 1]);
+          } else {
+            as_wait_v<0>(vr[gi & 1]);
+          }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const as_u32x4 raw = __builtin_shufflevector(vr[gi & 1][2 * u], vr[gi & 1][2 * u + 1], 0, 1, 2, 3);
+          for (int u = 0; u < 4; ++u) {
+            const as_u32x4 raw = __builtin_shufflevector(vr[gi & 1][2 * u], vr[gi & 1][2 * u + 1], 0, 1, 2, 3);
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt)
-            o[c0 + u][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), p[qt], o[c0 + u][qt], 0, 0, 0);
-        }
-        if constexpr (c0 == 0) {
+            for (int qt = 0; qt < QT; ++qt)
+              o[4 * gi + u][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), p[qt], o[4 * gi + u][qt], 0, 0, 0);
+          }
+          if constexpr (gi == 0) {
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt) l[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[qt], l[qt], 0, 0, 0);
-        }
+            for (int qt = 0; qt < QT; ++qt) l[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[qt], l[qt], 0, 0, 0);
+          }
+        });
       });
     }
     if (pu != nullptr) {  // pivot head: the tile's softmax mass, log2 units (-inf where the wave skipped the tile)

@@ -20,7 +20,7 @@ MAX_ABS, MEAN_REL = 2e-2, 2.5e-3
                                       (3, 1, 8300)])   # more than one mask word per row
 def test_short_attention_matches_oracle(gpu_device, hq, hkv, n, d):
     """Random masks with dense heads among them, whose maps the kernel writes; logits that grow along the row for the last
-    head, so that the running max has to move past its headroom."""
+    head, so that the running max has to move."""
     from shareprefill_amd import ops
 
     gen = torch.Generator().manual_seed(n + d)
