@@ -118,3 +118,29 @@ def test_decode_batch_matches_oracle(gpu_device, b, hq, hkv, n, d):
         ref = O.decode_attention(q[i, :, 0], k[i], v[i], scale)
         assert (out[i, 0] - ref).abs().max().item() <= MAX_ABS
         assert ((out[i, 0] - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
+
+
+@pytest.mark.parametrize("b", [1, 128, 600])  # the four tiles of a cache: a workgroup each, two to a workgroup, all in one
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_weights_that_bf16_holds_are_not_rounded(gpu_device, b, d):
+    """The probabilities of a chunk are rounded to bf16 relative to the chunk's largest, whatever the other sequences of
+    the batch: keys whose weights in their tile are bf16 values keep them, though the tiles' largest logits lie
+    fractions of an octave apart."""
+    from shareprefill_amd import ops
+    from tests.test_gpu_attention_precision import FP32, LN2, bf16_weights, half_ulp, logit_keys
+
+    n, hq, hkv = 512, 4, 2
+    logits = torch.full((n,), -60.0)
+    for tile, top in enumerate((3.3, 2.55, 1.9, 2.87)):
+        logits[128 * tile:128 * tile + 16] = top + torch.log2(bf16_weights(16, tile))
+    k1, exact_logits = logit_keys(logits, d)
+    p = torch.softmax(exact_logits * LN2, 0)
+    q = torch.zeros(b, hq, 1, d, dtype=torch.bfloat16)
+    q[..., :3] = 1.0
+    v1 = torch.zeros(n, d, dtype=torch.bfloat16)
+    for tile in range(4):  # channel 16 tile + i: the weight of the tile's key i
+        v1[128 * tile:128 * tile + 16, 16 * tile:16 * tile + 16] = torch.eye(16)
+    k, v = (t.expand(b, hkv, n, d).contiguous().to(gpu_device) for t in (k1, v1))
+    out = ops.decode_attention_batch(q.to(gpu_device), k, v, LN2)[..., :64].double().cpu()
+    want = p.view(4, 128)[:, :16].reshape(64)
+    assert (((out - want).abs() - half_ulp(want)) / want).max().item() <= FP32
