@@ -1,4 +1,4 @@
-"""CPU-only check of the generated gfx950 code of the attention kernel.
+"""CPU-only checks of the generated gfx950 code of the attention kernels.
 
 The kernel's MFMAs are inline assembly, so the compiler knows neither their latency nor the wait states a vector
 instruction needs before it may read an MFMA result (the hardware does not interlock that read).  The source keeps
@@ -6,7 +6,12 @@ such reads far behind the MFMAs by construction, or puts the wait states into th
 (at_mfma_acc_settled in csrc/sp_attn.hip).  What the source cannot see is the register allocator: to satisfy a tied
 operand it may copy a result register with a vector move right behind the MFMA -- that happened in the pivot
 instantiation and gave wrong row sums now and then.  This test compiles the file to assembly and measures, for every
-vector / memory instruction that reads a register an MFMA wrote, how many wait states lie between the two."""
+vector / memory instruction that reads a register an MFMA wrote, how many wait states lie between the two.
+
+The short-prompt kernel (csrc/sp_attn_short.hip) reads V with transposing LDS reads in inline assembly.  The compiler
+takes their registers as written at once, so whatever it places between such a read and the wait behind it -- a register
+copy, a branch to a block with copies of its own -- may see the old contents.  The second test follows every such read to
+the s_waitcnt that covers it and lets nothing touch its registers, and no branch or label stand, in between."""
 
 import os
 import re
@@ -75,14 +80,56 @@ def test_the_scanner_sees_a_copy_placed_right_behind_an_mfma():
     assert closest_reads(chain) == []
 
 
-def test_no_vector_instruction_reads_an_mfma_result_too_early():
+def touched_in_flight(lines):
+    """-> (number of transposing LDS reads, [(read, instruction)] that touch a read's registers, branch or end a block
+    while it is in flight).  LDS operations return in order: s_waitcnt lgkmcnt(N) leaves the N youngest outstanding."""
+    count, found, queue = 0, [], []  # queue: (registers or None, text) of every LDS operation in flight, oldest first
+    for l in (line.split(";")[0].strip() for line in lines):
+        if not l or (l.startswith(".") and not l.endswith(":")):
+            continue
+        op, toks = l.split()[0], [t for t in re.split(r"[ ,]+", l)[1:] if t]
+        pending = [q for q in queue if q[0] is not None]
+        if l.endswith(":") or op.startswith(("s_branch", "s_cbranch", "s_setpc", "s_endpgm")):
+            found += [(text, l) for _, text in pending]
+            continue
+        if op == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", l)
+            if m or re.fullmatch(r"s_waitcnt 0", l):
+                left = int(m.group(1)) if m else 0
+                queue = queue[max(0, len(queue) - left):]
+            continue
+        regs = set()
+        for t in toks:
+            regs |= _regs(t)
+        found += [(text, l) for r, text in pending if r & regs]
+        if op.startswith("ds_"):
+            is_read = op.startswith("ds_read_b64_tr_b16")
+            count += is_read
+            queue.append((_regs(toks[0]) if is_read else None, l))
+    return count, found
+
+
+def test_the_scanner_sees_a_copy_of_a_read_in_flight():
+    read = ["ds_read_b64_tr_b16 v[8:9], v1 offset:64", "ds_read_b64_tr_b16 v[10:11], v1"]
+    use = ["v_mfma_f32_16x16x32_bf16 v[20:23], v[8:11], v[4:7], v[20:23]"]
+    assert touched_in_flight(read + ["s_waitcnt lgkmcnt(0)"] + use) == (2, [])
+    assert touched_in_flight(read + ["s_waitcnt lgkmcnt(1)", "v_mov_b32_e32 v3, v8"])[1] == []
+    assert len(touched_in_flight(read + ["v_mov_b32_e32 v3, v9", "s_waitcnt lgkmcnt(0)"] + use)[1]) == 1
+    assert len(touched_in_flight(read + ["s_waitcnt lgkmcnt(1)"] + use)[1]) == 1
+    assert len(touched_in_flight(read + ["s_cbranch_vccnz .LBB0_7", "s_waitcnt lgkmcnt(0)"] + use)[1]) == 2
+    assert len(touched_in_flight(read + [".LBB0_3:", "s_waitcnt lgkmcnt(0)"] + use)[1]) == 2
+    assert touched_in_flight(["s_waitcnt vmcnt(0)"] + read + ["s_waitcnt vmcnt(0)"] + use)[1] != []
+
+
+def _kernels(source, name):
+    """{mangled name: assembly lines} of the kernels called `name` in csrc/`source`, compiled as the library is."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
-    out = os.path.join(CSRC, "sp_attn.isa_check.s")
+    out = os.path.join(CSRC, source.replace(".hip", ".isa_check.s"))
     cmd = [hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
            "-packed-fp32-ops", "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-S", "--cuda-device-only",
-           os.path.join(CSRC, "sp_attn.hip"), "-o", out]
+           os.path.join(CSRC, source), "-o", out]
     try:
         subprocess.run(cmd, check=True, capture_output=True)
         text = open(out).read()
@@ -90,12 +137,26 @@ def test_no_vector_instruction_reads_an_mfma_result_too_early():
         if os.path.exists(out):
             os.remove(out)
     kernels = {}
-    for m in re.finditer(r"^(_Z\S*sp_attn_fwd_kernel\S*):.*\n", text, re.M):
+    for m in re.finditer(r"^(_Z\S*" + name + r"\S*):.*\n", text, re.M):
         start = m.end()
         kernels[m.group(1)] = text[start:text.index(".Lfunc_end", start)].split("\n")
+    return kernels
+
+
+def test_no_vector_instruction_reads_an_mfma_result_too_early():
+    kernels = _kernels("sp_attn.hip", "sp_attn_fwd_kernel")
     assert len(kernels) == 5, "the forward kernel has five instantiations (pivot x half-channel, and small blocks)"
     for name, body in kernels.items():
         assert sum("v_mfma_f32_16x16x32_bf16" in l for l in body) > 100
         reads = closest_reads(body)
         assert not reads or reads[0][0] >= MIN_WAIT_STATES, (
             f"{name}: '{reads[0][2]}' reads the result of '{reads[0][1]}' only {reads[0][0]} wait states behind it")
+
+
+def test_nothing_touches_a_transposing_read_in_flight():
+    kernels = _kernels("sp_attn_short.hip", "sp_attn_short_kernel")
+    assert len(kernels) == 8, "64 / 128 channels x one / two sets of waves x with / without the pivots' patterns"
+    for name, body in kernels.items():
+        count, found = touched_in_flight(body)
+        assert count >= 16
+        assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
