@@ -38,7 +38,8 @@ struct AsArgs {
   const int32_t* decision;   // [hq] or null
   sp_bf16* out;              // [n][hq][D]
   float* avg_attn;           // [hq][nb][nb], written for pivot heads
-  float* tile_sums;          // [hq][nb (nb + 1) / 2][2][128] of pivot heads, or null: no maps wanted
+  float* block_sums;         // [slots][nb (nb + 1) / 2][KSPLIT][128] of pivot heads
+  int slots;                 // pivot heads there is room for; -1: no maps wanted
   int64_t n, sq_n, sq_h, sk_n, sk_h, sv_n, sv_h;
   int hq, group, nb, nbw;
   int zero_maps;             // 1: no decisions, every row of avg_attn is cleared
@@ -231,10 +232,17 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
     l_mark[qt] = 0.f;
   }
   const as_bf16x8 ones = __builtin_bit_cast(as_bf16x8, (as_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-  // pivot heads: this row's sums per 64-key tile, [column][half][128 queries]
-  float* const pu = a.tile_sums == nullptr || a.decision[h] != SP_DEC_DENSE
-                        ? nullptr
-                        : a.tile_sums + ((int64_t)h * ((int64_t)a.nb * (a.nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * (2 * AS_BS);
+  // pivot heads: this row's sums per block and set of waves, [column][set][128 queries], in the slab of the head's rank among
+  // them
+  const bool pivot = a.slots >= 0 && a.decision[h] == SP_DEC_DENSE;  // (uniform)
+  float* pu = nullptr;
+  if (pivot) {
+    int slot = 0;
+    for (int i = 0; i < h; i += SP_WAVE)
+      slot += __builtin_popcountll(__ballot(i + lane < h && a.decision[i + lane < h ? i + lane : 0] == SP_DEC_DENSE));
+    if (slot < a.slots)
+      pu = a.block_sums + ((int64_t)slot * ((int64_t)a.nb * (a.nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * (KSPLIT * AS_BS);
+  }
 
   // LDS byte offsets of the lane's operands: K row lq, logical chunk 4 ks + g; V row 4 g + lq / 4, 8-byte piece lq % 4 of the
   // 32 bytes of channel tile ct.  Rows 16 further have the same swizzle.
@@ -367,12 +375,12 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
         });
       });
     }
-    if (pu != nullptr) {  // pivot head: the tile's softmax mass, log2 units (-inf where the wave skipped the tile)
+    if (pu != nullptr && (KSPLIT == 2 || half == 1)) {  // pivot head: the block's (the set's) softmax mass, log2 units
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const float u = __builtin_amdgcn_logf(l[qt][0] - l_mark[qt]) + m[qt];
         l_mark[qt] = l[qt][0];
-        if (g == 0) pu[(int64_t)(2 * c + half) * AS_BS + q_off + 16 * qt] = u;
+        if (g == 0) pu[(int64_t)(KSPLIT * c + set) * AS_BS + q_off + 16 * qt] = u;
       }
     }
     if (KSPLIT == 2 || half == 1) c = c_next;
@@ -419,8 +427,12 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
   }
   if (a.zero_maps)
     for (int i = t; i < a.nb; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + i] = 0.f;
-  if (pu == nullptr) return;  // (uniform)
-  // pivot head: avg[r][c] = mean over the block's valid queries of (sum of the two halves' exp2(u - m[q])) / l[q].  A wave
+  if (!pivot) return;  // (uniform)
+  if (pu == nullptr) {  // more pivots than the caller made room for: no map, and visibly so
+    for (int i = t; i < n_blk; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = NAN;
+    return;
+  }
+  // pivot head: avg[r][c] = mean over the block's valid queries of (sum over the sets of exp2(u - m[q])) / l[q].  A wave
   // reads back its own sums (its own stores), folds its queries, and the waves meet in LDS.
   float* const part = reinterpret_cast<float*>(lds_all);  // [block][wave]
   __syncthreads();                                        // LDS is free, the stores of pu have left
@@ -430,10 +442,7 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
       if (qrow + 16 * qt < a.n) {
-        const float* u = pu + (int64_t)(2 * c) * AS_BS + q_off + 16 * qt;
-#pragma unroll
-        for (int hf = 0; hf < 2; hf += KSPLIT)
-          x += __builtin_amdgcn_exp2f(u[(hf + set) * AS_BS] - m[qt]) * inv_l[qt];
+        x += __builtin_amdgcn_exp2f(pu[(int64_t)(KSPLIT * c + set) * AS_BS + q_off + 16 * qt] - m[qt]) * inv_l[qt];
       }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, SP_WAVE);
@@ -465,10 +474,18 @@ extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
 }
 
-extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {
+// Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
+// 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).
+static bool as_split(int64_t n, int32_t hq) { return sp_ceil_div(n, AS_BS) * hq <= 512; }
+
+extern "C" size_t sp_short_attn_pivot_scratch_bytes(int64_t n, int32_t hq) {
   if (n <= 0 || hq <= 0) return 0;
   const size_t nb = (size_t)sp_ceil_div(n, AS_BS);
-  return (size_t)hq * (nb * (nb + 1) / 2) * 2 * AS_BS * sizeof(float);
+  return nb * (nb + 1) / 2 * (as_split(n, hq) ? 2 : 1) * AS_BS * sizeof(float);
+}
+
+extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {
+  return n <= 0 || hq <= 0 ? 0 : (size_t)hq * sp_short_attn_pivot_scratch_bytes(n, hq);
 }
 
 static int as_launch(const char* who, const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
@@ -491,17 +508,17 @@ static int as_launch(const char* who, const void* q, const void* k, const void* 
   SP_REQUIRE(nb <= AS_MAX_NB && nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "%s: n=%lld hq=%d too large", who,
              (long long)n, hq);
   const bool maps = decision != nullptr && avg_attn != nullptr;
-  SP_REQUIRE(!maps || (workspace && workspace_bytes >= sp_short_attn_workspace_bytes(n, hq) && ((uintptr_t)workspace % 4) == 0),
-             SP_ERR_WORKSPACE, "%s: workspace missing, misaligned or too small", who);
+  SP_REQUIRE(!maps || workspace_bytes == 0 || (workspace && ((uintptr_t)workspace % 4) == 0), SP_ERR_WORKSPACE,
+             "%s: workspace missing or misaligned", who);
+  const size_t room = workspace_bytes / sp_short_attn_pivot_scratch_bytes(n, hq);
+  const int slots = !maps ? -1 : room < (size_t)hq ? (int)room : hq;
   const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
-                    maps ? (float*)workspace : nullptr, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
+                    (float*)workspace, slots, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
                     v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), decision == nullptr && avg_attn != nullptr,
                     softmax_scale * 1.4426950408889634f};
   static_assert(AS_LDS_BYTES(64, 1) >= AS_MAX_NB * 14 + AS_THREADS * 2 * 8 + 16, "");  // rs_lds_bytes(AS_MAX_NB, 2 sets)
   const dim3 grid((unsigned)(nb * hq));
-  // Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
-  // 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).
-  const bool split = nb * hq <= 512;
+  const bool split = as_split(n, hq);
   static bool attr_set[64] = {false};  // per device, once (idempotent)
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));

@@ -374,11 +374,13 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     return out
 
 
-def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, pivot=None) -> torch.Tensor:
+def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, pivot=None, max_pivots=None) -> torch.Tensor:
     """block_sparse_attention for short prompts (block size 128, head_dim 64 or 128): q [Hq,N,D], k/v [Hkv,N,D] views,
     mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D].  One launch, whatever decision says: v is read as it is and the maps of
     DENSE heads are written by the same kernel (avg_attn without decision is cleared).
-    pivot = (state, head_cluster, pattern_threshold): pivot_update with decision and avg_attn is part of the launch."""
+    pivot = (state, head_cluster, pattern_threshold): pivot_update with decision and avg_attn is part of the launch.
+    max_pivots: how many heads can be DENSE (an upper bound the host knows; default all of them): what is kept for their maps
+    is sized by it, and DENSE heads beyond it get NaN for a map."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")
@@ -391,8 +393,8 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, 
     out = torch.empty(n, hq, d, dtype=torch.bfloat16, device=dev)
     ws, ws_bytes = None, 0
     if decision is not None and avg_attn is not None:
-        ws_bytes = lib.sp_short_attn_workspace_bytes(n, hq)
-        ws = _workspace("attn_short", ws_bytes, dev)
+        ws_bytes = (hq if max_pivots is None else min(max_pivots, hq)) * lib.sp_short_attn_pivot_scratch_bytes(n, hq)
+        ws = _workspace("attn_short", ws_bytes, dev) if ws_bytes else None
     timer = kernel_timer
     if timer is not None:
         timer.start("attn")

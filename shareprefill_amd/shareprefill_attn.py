@@ -231,6 +231,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
                               scale_dim=model_dim, avg_attn=avg_attn[0])
     if short:
         out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0],
+                                  max_pivots=sharing.max_pivots(module.layer_idx, num_heads),
                                   pivot=sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold))
     else:
         out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,

@@ -89,3 +89,59 @@ def test_pivot_patterns_in_the_attention_launch(gpu_device, hq, hkv, n, d):
         assert torch.equal(states[0].ratio.view(torch.int64), states[1].ratio.view(torch.int64))
         assert states[1].info[:, 1].tolist() == [1, 1, 0]
         assert not states[1].accum.any() and not states[1].info[:, 5].any()
+
+
+@pytest.mark.parametrize("hq,hkv,n,d", [(6, 2, 1111, 128), (72, 8, 1111, 64), (70, 2, 1025, 128)])
+def test_block_sums_for_as_many_heads_as_can_be_pivots(gpu_device, hq, hkv, n, d):
+    """Maps, with room for exactly the dense heads, equal those with room for all heads (rows split and not, more heads than a
+    wave has lanes); a dense head there is no room for gets NaN and updates no pivot, the others are as they were."""
+    from shareprefill_amd import ops
+
+    nb = -(-n // 128)
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    q, k, v = (torch.randn(h, n, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h in (hq, hkv, hkv))
+    dense = np.arange(hq) % 5 == 1
+    decision = torch.where(torch.from_numpy(dense), O.DEC_DENSE, O.DEC_VS).to(torch.int32).to(gpu_device)
+    mask = ops.bool_to_mask(torch.ones(nb, nb, dtype=torch.bool).tril().expand(hq, nb, nb)).to(gpu_device)
+    room = int(dense.sum())
+    avgs = [torch.zeros(hq, nb, nb, dtype=torch.float32, device=gpu_device) for _ in range(3)]
+    hc = torch.arange(hq, dtype=torch.int32, device=gpu_device)
+    state = ops.ClusterState(hq, nb, gpu_device, keep_maps=False)
+    outs = [ops.short_attention(q, k, v, mask, d ** -0.5, decision, avgs[0]),
+            ops.short_attention(q, k, v, mask, d ** -0.5, decision, avgs[1], max_pivots=room),
+            ops.short_attention(q, k, v, mask, d ** -0.5, decision, avgs[2], max_pivots=room - 1, pivot=(state, hc, 0.9))]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert torch.equal(avgs[0], avgs[1]) and not avgs[0].isnan().any()
+    last = int(np.nonzero(dense)[0][-1])
+    assert avgs[2][last].isnan().any()
+    others = torch.arange(hq, device=gpu_device) != last
+    assert torch.equal(avgs[0][others], avgs[2][others])
+    want = torch.from_numpy(dense).to(gpu_device) & others
+    assert torch.equal(state.info[:, 1] != 0, want)
+    ops.short_attention(q, k, v, mask, d ** -0.5, torch.zeros_like(decision), avgs[1], max_pivots=0)
+
+
+def test_a_layer_keeps_block_sums_of_its_possible_pivots_only(gpu_device, tmp_path):
+    """32 heads of 64 channels at 32768 tokens: what stays allocated for their maps is that of the long-prompt kernel for
+    as many heads as the layer has shared clusters, and nothing in a layer without one."""
+    import json
+    import types
+
+    from shareprefill_amd import AttentionSharing, _lib, ops, shareprefill_attention_forward, synthetic
+
+    hq, hkv, n, d = 32, 8, 32768, 64
+    path = tmp_path / "table.json"  # layer 0: two shared clusters; layer 1: none
+    path.write_text(json.dumps({"clusters": {"a": [[0, h] for h in range(9)], "b": [[0, h] for h in range(9, 14)],
+                                             "c": [[1, h] for h in range(32)]}, "shared_clusters": ["a", "b"]}))
+    cfg = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=0.9, similarity_threshold=0.5,
+                                fallback_threshold=0.9, queryaware_threshold=0.0)
+    sharing = AttentionSharing(str(path))
+    qkv = synthetic.planted_qkv(hq, hkv, n, d, 1, device=gpu_device, q_head_gain=1.0)
+    held = lambda: sum(buf.numel() for key, buf in ops._workspaces.items() if key[0] == "attn_short")
+    torch.cuda.synchronize()
+    ops.release_workspaces()
+    for layer, pivots in ((1, 0), (0, 2)):
+        mod = types.SimpleNamespace(config=cfg, attention_sharing=sharing, layer_idx=layer, scaling=d ** -0.5)
+        shareprefill_attention_forward(mod, *qkv, None, scaling=d ** -0.5)
+        assert int((sharing.plans[-1].decision == _lib.SP_DEC_DENSE).sum()) == pivots
+        assert held() <= pivots * _lib.load().sp_attn_pivot_scratch_bytes(n, 128)
