@@ -38,11 +38,12 @@ def pad_head_dim(*tensors: torch.Tensor, width: int = KERNEL_HEAD_DIM):
     return tuple(torch.nn.functional.pad(t, (0, width - d)) for t in tensors)
 
 
-
 def _rows_16_byte_aligned(t: torch.Tensor) -> torch.Tensor:
-    """t, or a copy of it if its rows cannot be read with 16-byte loads."""
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[1:-1])
-    return t if ok else t.contiguous()
+    """t [1, H, N, D], or a copy of it if its rows cannot be read with 16-byte loads at 32-bit offsets inside a block."""
+    ok = (t.stride(3) == 1 and t.data_ptr() % 16 == 0 and t.stride(1) % 8 == 0 and t.stride(2) % 8 == 0
+          and t.stride(2) * 128 < 2 ** 31)
+    # (contiguous() would hand back a contiguous t as it is, whatever its address and the strides of its axes of size one)
+    return t if ok else t.clone(memory_format=torch.contiguous_format)
 
 
 def _dense_causal_mask(hq: int, nb: int, device) -> torch.Tensor:
