@@ -182,6 +182,8 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
     # are; longer ones repack v and run the persistent kernel on 128
     head_dim = 64 if model_dim in PADDED_HEAD_DIMS else model_dim
     short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
+    if model_dim == KERNEL_HEAD_DIM and value_states.stride(2) * 128 >= 2 ** 31:
+        short = False  # the short-prompt kernel's offsets inside a block of v have 32 bits, the repack's 64
     if model_dim in PADDED_HEAD_DIMS:
         if not short:
             head_dim = KERNEL_HEAD_DIM

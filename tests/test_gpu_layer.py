@@ -542,3 +542,24 @@ def test_layers_of_the_shipped_llama_table_elect_and_reuse_the_pivot_of_its_one_
     out = L["out"][0].transpose(0, 1)[20:24].float()
     assert (out - ref).abs().max().item() <= MAX_ABS
     assert ((out - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
+
+
+def test_values_a_long_way_apart(gpu_device, tmp_path):
+    """v whose tokens lie 2^24 elements apart (the short-prompt kernel has 32-bit offsets inside a block of v): the layer
+    runs, and gives what it gives on the same values side by side."""
+    from shareprefill_amd import AttentionSharing, shareprefill_attention_forward, synthetic
+
+    n, stride = 140, 2 ** 24
+    path = synthetic.write_cluster_table(synthetic.random_cluster_table(2, 1, 1, 3), str(tmp_path / "table.json"))
+    q, k, v = synthetic.planted_qkv(2, 1, n, 128, 1, device=gpu_device, q_head_gain=1.0)
+    far = torch.empty((n - 1) * stride + 128, dtype=torch.bfloat16, device=gpu_device).as_strided((1, 1, n, 128), (128, 128, stride, 1))
+    far.copy_(v)
+    outs = []
+    for values in (v, far):
+        cfg = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=0.9,
+                                    similarity_threshold=0.5, fallback_threshold=0.9, queryaware_threshold=0.1)
+        mod = types.SimpleNamespace(config=cfg, attention_sharing=AttentionSharing(path), layer_idx=0, scaling=128 ** -0.5)
+        outs.append(shareprefill_attention_forward(mod, q, k, values, None, scaling=128 ** -0.5)[0].float())
+    # both round the probabilities and the output to bf16 (bounds: test_gpu_attention.py)
+    assert (outs[0] - outs[1]).abs().max().item() <= 2e-2
+    assert ((outs[0] - outs[1]).abs().mean() / outs[0].abs().mean()).item() <= 2.5e-3
