@@ -310,6 +310,8 @@ __global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kern
 // ---- host -------------------------------------------------------------------------------------------------
 // Chunks per (sequence, kv head): about two workgroups per CU over the whole batch, which is what the kernel's LDS
 // lets a CU hold, and no chunk below one tile of keys.
+#define DC_MAX_GRID_Z 65535
+static_assert(DC_MAX_GRID_Z >= 512, "");  // (the number of chunks is 1 before a batch needs a second launch)
 static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
   const int64_t tiles = sp_ceil_div(n, DC_TILE);
   int64_t want = sp_ceil_div(512, (int64_t)hkv * batch);
@@ -334,7 +336,7 @@ static int dc_check(const char* who, const void* q, const void* k, const void* v
   SP_REQUIRE(q && k && v && out, SP_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
   SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT, "%s: bad shape n=%lld hq=%d hkv=%d",
              who, (long long)n, hq, hkv);
-  SP_REQUIRE(batch > 0 && batch <= 65535, SP_ERR_UNSUPPORTED, "%s: batch %d (1 to 65535)", who, batch);
+  SP_REQUIRE(batch > 0, SP_ERR_UNSUPPORTED, "%s: batch %d", who, batch);
   SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "%s: softmax_scale must be > 0", who);
   SP_REQUIRE(d >= 8 && d <= DC_D && d % 8 == 0, SP_ERR_UNSUPPORTED,
              "%s: head_dim %d unsupported (a multiple of 8 up to 128)", who, d);
@@ -359,10 +361,14 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
   float* o_part = (float*)partials;
   float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
-#define DC_LAUNCH_PARTIAL_(G8, FULL)                                                                                  \
-  hipLaunchKernelGGL((sp_decode_partial_kernel<G8, FULL>), dim3(splits, hkv, batch), dim3(DC_THREADS), 0, s,           \
-                     (const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, n, g, (int)d, st, scale_log2,            \
-                     keys_per_split, tiles_per_chunk, o_part, ml_part, (sp_bf16*)out)
+  // A grid's z axis ends at 65535 sequences.  (A batch that large has one workgroup per sequence and kv head: no partials.)
+#define DC_LAUNCH_PARTIAL_(G8, FULL)                                                                                   \
+  for (int64_t b0 = 0; b0 < batch; b0 += DC_MAX_GRID_Z)                                                                \
+  hipLaunchKernelGGL((sp_decode_partial_kernel<G8, FULL>),                                                             \
+                     dim3(splits, hkv, (unsigned)(batch - b0 < DC_MAX_GRID_Z ? batch - b0 : DC_MAX_GRID_Z)),           \
+                     dim3(DC_THREADS), 0, s, (const sp_bf16*)q + b0 * st.q_b, (const sp_bf16*)k + b0 * st.k_b,          \
+                     (const sp_bf16*)v + b0 * st.v_b, n, g, (int)d, st, scale_log2, keys_per_split, tiles_per_chunk,   \
+                     o_part, ml_part, (sp_bf16*)out + b0 * hq * d)
 #define DC_LAUNCH_PARTIAL(G8)     \
   do {                            \
     if (d == DC_D)                \

@@ -144,3 +144,35 @@ def test_decode_weights_that_bf16_holds_are_not_rounded(gpu_device, b, d):
     out = ops.decode_attention_batch(q.to(gpu_device), k, v, LN2)[..., :64].double().cpu()
     want = p.view(4, 128)[:, :16].reshape(64)
     assert (((out - want).abs() - half_ulp(want)) / want).max().item() <= FP32
+
+
+@pytest.mark.parametrize("b", [65535, 65536, 131075])
+def test_decode_batches_past_the_grid_limit(gpu_device, b):
+    """A grid's last axis ends at 65535: larger batches go in several launches, every sequence with its own queries and
+    cache.  With one key per sequence the output is that key's value."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator(device=gpu_device).manual_seed(b)
+    mk = lambda h: torch.randn(b, h, 1, 8, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(2), mk(1), mk(1)
+    out = ops.decode_attention_batch(q, k, v, 0.3)
+    assert torch.equal(out, v.expand(b, 2, 1, 8).transpose(1, 2))
+    # two keys: the first and the last sequence against the oracle
+    k, v = mk(2).view(b, 1, 2, 8), mk(2).view(b, 1, 2, 8)
+    out = ops.decode_attention_batch(q, k, v, 0.3)
+    for i in (0, 65534, b - 1):
+        ref = O.decode_attention(q[i, :, 0].cpu(), k[i].cpu(), v[i].cpu(), 0.3)
+        assert (out[i, 0].cpu().float() - ref).abs().max().item() <= MAX_ABS
+
+
+def test_decode_reads_a_larger_cache_up_to_the_batch(gpu_device):
+    """A cache kept for more sequences than the step has (and v for more than k)."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator(device=gpu_device).manual_seed(1)
+    mk = lambda b, h, m: torch.randn(b, h, m, 64, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(2, 4, 1), mk(3, 2, 300), mk(5, 2, 300)
+    assert torch.equal(ops.decode_attention_batch(q, k, v, 0.125), ops.decode_attention_batch(q, k[:2], v[:2], 0.125))
+    for bad in ((q, k[:1], v), (q, k, v[:1]), (q, k, v[:, :, :299])):
+        with pytest.raises(ValueError):
+            ops.decode_attention_batch(*bad, 0.125)
