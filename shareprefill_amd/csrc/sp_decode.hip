@@ -321,13 +321,19 @@ static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
   return (int)want;
 }
 
-extern "C" size_t sp_decode_batch_workspace_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
+static size_t dc_partial_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
   if (batch <= 0 || n <= 0 || hq <= 0 || hkv <= 0) return 0;
   return (size_t)dc_splits(batch, n, hkv) * batch * hq * (DC_D * sizeof(float) + sizeof(float2));
 }
 
+// a batch whose caches are one chunk each leaves no partials (at 65535 sequences of 32 heads they would be 1.1 GB)
+extern "C" size_t sp_decode_batch_workspace_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
+  if (batch <= 0 || n <= 0 || hq <= 0 || hkv <= 0 || dc_splits(batch, n, hkv) == 1) return 0;
+  return dc_partial_bytes(batch, n, hq, hkv);
+}
+
 extern "C" size_t sp_decode_workspace_bytes(int64_t n, int32_t hq, int32_t hkv) {
-  return sp_decode_batch_workspace_bytes(1, n, hq, hkv);
+  return dc_partial_bytes(1, n, hq, hkv);
 }
 
 // argument checks shared by the two entry points

@@ -469,3 +469,16 @@ def test_reference_import_paths_resolve_to_the_package():
     assert ref_utils.triton_bnhd_pool is shareprefill_amd.utils.triton_bnhd_pool
     assert triton_block_wise_prefill_attention is shareprefill_amd.shareprefill_attn.triton_block_wise_prefill_attention
     assert callable(triton_column_count_cumsum) and callable(shareprefill_attention_forward)
+
+
+def test_decode_batches_keep_partials_only_where_a_cache_is_cut():
+    """The scratch of a batched decode step is bounded by what fills the chip (1024 partials of 520 bytes per head of a
+    group), whatever the batch."""
+    from shareprefill_amd import _lib
+
+    lib = _lib.load()
+    for hq, hkv in ((32, 8), (28, 4), (8, 8), (32, 1)):
+        for n in (1, 129, 4001, 131072):
+            sizes = [lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv) for b in (1, 2, 7, 63, 64, 511, 512, 65536)]
+            assert max(sizes) <= 1024 * (hq // hkv) * 520
+            assert sizes[-1] == sizes[-2] == 0
