@@ -17,12 +17,15 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib, ops
-from .attention_sharing import budget_blocks
+from .attention_sharing import AttentionSharing, budget_blocks
 
 LOGGER = logging.getLogger(__name__)
 
 
 _dense_masks = {}
+
+# steps of AttentionSharing that a launch of this path does along with its own work
+_PLAN_LAYER, _UPDATE_PIVOTAL_ATTNS = AttentionSharing.plan_layer, AttentionSharing.update_pivotal_attns
 
 KERNEL_HEAD_DIM = 128
 PADDED_HEAD_DIMS = (16, 32, 64)  # the reference's other head sizes (shareprefill_attn.py:503-508)
@@ -229,17 +232,26 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
         ops.repack_v(v, block_size, ws[0])
+    # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
+    plan_args = {"scale_dim": model_dim}
+    plan_here = getattr(sharing.plan_layer, "__func__", None) is _PLAN_LAYER
+    if plan_here:
+        plan_args["avg_attn"] = avg_attn[0]  # (cleared on the way)
+    else:
+        avg_attn.zero_()
     plan = sharing.plan_layer(q, k, module.layer_idx, block_size, minb, maxb, config.pattern_threshold,
-                              config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold,
-                              scale_dim=model_dim, avg_attn=avg_attn[0])
+                              config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold, **plan_args)
+    update_here = short and getattr(sharing.update_pivotal_attns, "__func__", None) is _UPDATE_PIVOTAL_ATTNS
     if short:
         out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0],
-                                  max_pivots=sharing.max_pivots(module.layer_idx, num_heads),
-                                  pivot=sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold))
+                                  max_pivots=sharing.max_pivots(module.layer_idx, num_heads) if plan_here else None,
+                                  pivot=sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold)
+                                  if update_here else None)
     else:
         out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
                                          avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,
                                          half_channels=model_dim != head_dim)
+    if not update_here:
         sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
     return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
 

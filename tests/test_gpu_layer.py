@@ -563,3 +563,49 @@ def test_values_a_long_way_apart(gpu_device, tmp_path):
     # both round the probabilities and the output to bf16 (bounds: test_gpu_attention.py)
     assert (outs[0] - outs[1]).abs().max().item() <= 2e-2
     assert ((outs[0] - outs[1]).abs().mean() / outs[0].abs().mean()).item() <= 2.5e-3
+
+
+@pytest.mark.parametrize("n,d", [(1500, 128), (1500, 64), (7000, 128)])  # short prompts (one launch does both) and long ones
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_own_steps_of_a_subclass_or_wrapper_are_called(gpu_device, tmp_path, monkeypatch, n, d, how):
+    """update_pivotal_attns and plan_layer, where they are not the library's own, see every layer that selects, with the
+    arguments they had before either became part of a launch; results and state are those of the library's own."""
+    from shareprefill_amd import AttentionSharing, shareprefill_attention_forward, synthetic
+
+    path = synthetic.write_cluster_table(synthetic.random_cluster_table(8, 2, 2, 3), str(tmp_path / "table.json"))
+    cfg = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=0.9, similarity_threshold=0.5,
+                                fallback_threshold=1e9, queryaware_threshold=0.1)
+    plan_layer, update = AttentionSharing.plan_layer, AttentionSharing.update_pivotal_attns
+    seen = []
+
+    def own_plan(self, q, k, layer_idx, block_size, min_budget, max_budget, pattern_threshold=0.9, similarity_threshold=0.5,
+                 fallback_threshold=0.9, queryaware_threshold=0.1, scale_dim=None):
+        seen.append(("plan", layer_idx))
+        return plan_layer(self, q, k, layer_idx, block_size, min_budget, max_budget, pattern_threshold, similarity_threshold,
+                          fallback_threshold, queryaware_threshold, scale_dim)
+
+    def own_update(self, layer_idx, avg_attn, use_dense, pattern_threshold=0.9):
+        seen.append(("update", layer_idx))
+        return update(self, layer_idx, avg_attn, use_dense, pattern_threshold)
+
+    plain = AttentionSharing(path)
+    if how == "subclass":
+        sharing = type("Own", (AttentionSharing,), {"plan_layer": own_plan, "update_pivotal_attns": own_update})(path)
+    else:
+        sharing = AttentionSharing(path)
+    results = []
+    for s in (plain, sharing):
+        if s is sharing and how == "instance":
+            s.plan_layer, s.update_pivotal_attns = types.MethodType(own_plan, s), types.MethodType(own_update, s)
+        if s is sharing and how == "class":
+            monkeypatch.setattr(AttentionSharing, "plan_layer", own_plan)
+            monkeypatch.setattr(AttentionSharing, "update_pivotal_attns", own_update)
+        for layer in range(2):
+            qkv = synthetic.planted_qkv(8, 2, n, d, layer, device=gpu_device, q_head_gain=1.0)
+            mod = types.SimpleNamespace(config=cfg, attention_sharing=s, layer_idx=layer, scaling=d ** -0.5)
+            results.append(shareprefill_attention_forward(mod, *qkv, None, scaling=d ** -0.5))
+    assert seen == [("plan", 0), ("update", 0), ("plan", 1), ("update", 1)]
+    for want, got in zip(results[:2], results[2:]):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert plain.pivot_summary() == sharing.pivot_summary()
+    assert any(s["has_pattern"] for s in plain.pivot_summary().values())
