@@ -247,8 +247,9 @@ __global__ __launch_bounds__(SEL_THREADS) void sp_gsel_pick_kernel(GselState* __
 // Vectors of at most CS_ITEMS entries per thread stay in registers for all levels; longer ones are read again.
 // 64 vectors, one launch against three levels of 2048 bins (one workgroup up to 16384 values, ten launches above): 3001
 // values 16.7 -> 11.0 us, 16384 25.9 -> 14.5, 32768 58 -> 25, 131072 80 -> 75; at 262144 the ten launches take 106 us and
-// one would take 109, hence GSEL_ONE_LEN.  32 maps of 64 x 64 blocks 20.6 -> 13.8 us, 256 x 256 67 -> 68.5 and, what most
-// layers meet, no map enabled 30.6 -> 6.7; at 512 x 512 the ten launches are ahead (96 us against 227), hence GSEL_ONE_NB.
+// one would take 109, hence GSEL_ONE_LEN.  32 maps of 64 x 64 blocks 20.2 -> 12.8 us, 256 x 256
+// 72 -> 41 (one map 42 -> 40) and, what most layers meet, no map enabled 30.6 -> 6.7; at 512 x 512 the ten launches are ahead
+// (96 us against 227 with the entries read again in each level), hence GSEL_ONE_NB.
 #define CS_THREADS 1024
 #define CS_BINS 256
 #define CS_COPIES 16
@@ -475,50 +476,35 @@ __global__ __launch_bounds__(CS_THREADS) void sp_cover_count_kernel(CoverCountAr
   cover_count_vector(sh, a, blockIdx.x);
 }
 
-// lower triangle of an [nb][nb] map (score_cover_idx), nb <= GSEL_ONE_NB
+// lower triangle of an [nb][nb] map (score_cover_idx), nb <= NB: 128 or GSEL_ONE_NB
 #define GSEL_ONE_NB 256
+template <int NB>
 __device__ static __forceinline__ void cover_select_map(CoverShared& sh, uint32_t* row_ties /* LDS [GSEL_ONE_NB] */,
                                                         const float* __restrict__ xv,
-                                        int nb, int nbw, long long t_le, uint64_t* __restrict__ mv) {
+                                                        int nb, int nbw, long long t_le, uint64_t* __restrict__ mv) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int WAVES = CS_THREADS / SP_WAVE;
   GselState s = sel_fresh_state(t_le, true);
   if (s.enabled) {
     // Rows p and nb - 1 - p of the triangle together have nb + 1 entries: entry j of pair p.  A wave takes pairs wave,
-    // wave + 16, ..., 64 entries at a time, so that hardly any lane idles above the diagonal.
+    // wave + 16, ..., 64 entries at a time, so that hardly any lane idles above the diagonal.  All of a thread's entries are
+    // read once, in one go, and stay in registers for the four levels (256 x 256 blocks, one map: read again in each level,
+    // eight at a time, and the mask written word by word 68 us, so 40; ten launches of the other descent 42).
+    constexpr int CHUNKS = NB / SP_WAVE + 1, ITEMS = NB / 2 / WAVES * CHUNKS;  // of up to NB + 1 entries
     const int pairs = (nb + 1) / 2;
-    auto at = [&](int p, int j) -> const float* {
-      const int r = nb - 1 - p;
-      return j <= p ? xv + (int64_t)p * nb + j : j <= nb && r != p ? xv + (int64_t)r * nb + (j - p - 1) : nullptr;
-    };
-    float val[12];
-    if (nb <= 2 * SP_WAVE) {  // in registers: four pairs of up to 129 entries
+    float val[ITEMS];
 #pragma unroll
-      for (int i = 0; i < 12; ++i) {
-        const int p = wave + WAVES * (i / 3), j = SP_WAVE * (i % 3) + lane;
-        const float* src = p < pairs ? at(p, j) : nullptr;
-        val[i] = src ? *src : 0.f;  // (zeros are left out of the histograms)
-      }
-      cover_descent(sh, s, [&](auto&& f) {
-#pragma unroll
-        for (int i = 0; i < 12; ++i)
-          if (wave + WAVES * (i / 3) < pairs && SP_WAVE * (i % 3) <= nb) f(val[i]);  // (uniform)
-      });
-    } else {
-      cover_descent(sh, s, [&](auto&& f) {
-        for (int p = wave; p < pairs; p += WAVES)
-          for (int j0 = 0; j0 <= nb; j0 += 8 * SP_WAVE) {  // eight loads in flight
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const float* src = at(p, j0 + SP_WAVE * i + lane);
-              val[i] = src ? *src : 0.f;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              if (j0 + SP_WAVE * i <= nb) f(val[i]);  // (uniform)
-          }
-      });
+    for (int i = 0; i < ITEMS; ++i) {
+      const int p = wave + WAVES * (i / CHUNKS), j = SP_WAVE * (i % CHUNKS) + lane, r = nb - 1 - p;
+      const bool low = j <= p;
+      const int row = low ? p : r, col = low ? j : j - p - 1;
+      val[i] = p < pairs && (low || (j <= nb && r != p)) ? xv[row * nb + col] : 0.f;  // (zeros are left out of the histograms)
     }
+    cover_descent(sh, s, [&](auto&& f) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i)
+        if (wave + WAVES * (i / CHUNKS) < pairs && SP_WAVE * (i % CHUNKS) <= nb) f(val[i]);  // (uniform)
+    });
   }
   // the boundary group of equal values is taken partially: its n_take lowest indices (row-major) win
   const bool ranked = s.enabled && !s.all && s.n_take != 0 && s.n_take < s.n_equal;
@@ -534,33 +520,53 @@ __device__ static __forceinline__ void cover_select_map(CoverShared& sh, uint32_
     }
     __syncthreads();
   }
+  constexpr int WORDS = NB / SP_WAVE, ROWS = 4;  // rows of a wave at a time: their entries and mask words are read in one go
   uint32_t before_rows = 0;  // members of the boundary group in the rows in front of row `counted` (uniform per wave)
   int counted = 0;
-  for (int r = wave; r < nb; r += WAVES) {
-    if (ranked)
-      for (; counted < r; ++counted) before_rows += row_ties[counted];
-    uint32_t before = before_rows;
-    for (int c0 = 0; c0 <= r; c0 += SP_WAVE) {
-      const int c = c0 + lane;
-      bool sel = false, eq = false;
-      if (s.enabled && c <= r) {
-        const uint32_t key = sp_sort_key(xv[(int64_t)r * nb + c]);
-        eq = key == s.prefix;
-        sel = s.all || key > s.prefix || (eq && take_all_equal);
+  for (int r0 = wave; r0 < nb; r0 += WAVES * ROWS) {
+    float x[ROWS][WORDS];
+    uint64_t old[ROWS];  // lane u: word u of the row
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const int r = r0 + i * WAVES;
+#pragma unroll
+      for (int u = 0; u < WORDS; ++u) {
+        const int c = u * SP_WAVE + lane;
+        x[i][u] = s.enabled && r < nb && c <= r ? xv[r * nb + c] : 0.f;
       }
-      if (ranked) {
-        const unsigned long long eqb = __ballot(eq);
-        if (eq && before + (uint32_t)__popcll(eqb & ((1ull << lane) - 1ull)) < s.n_take) sel = true;
-        before += (uint32_t)__popcll(eqb);
+      old[i] = r < nb && lane < WORDS && lane * SP_WAVE <= r ? mv[r * nbw + lane] : 0ull;
+    }
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const int r = r0 + i * WAVES;
+      if (r >= nb) break;  // (uniform)
+      if (ranked)
+        for (; counted < r; ++counted) before_rows += row_ties[counted];
+      uint32_t before = before_rows;
+      uint64_t mine = 0;  // lane u: what word u of the row gains
+#pragma unroll
+      for (int u = 0; u < WORDS; ++u) {
+        if (u * SP_WAVE > r) break;  // (uniform)
+        const bool in = s.enabled && u * SP_WAVE + lane <= r;
+        const uint32_t key = sp_sort_key(x[i][u]);
+        const bool eq = in && key == s.prefix;
+        bool sel = in && (s.all || key > s.prefix || (eq && take_all_equal));
+        if (ranked) {
+          const unsigned long long eqb = __ballot(eq);
+          if (eq && before + (uint32_t)__popcll(eqb & ((1ull << lane) - 1ull)) < s.n_take) sel = true;
+          before += (uint32_t)__popcll(eqb);
+        }
+        unsigned long long bal = __ballot(sel);
+        if (r == 0 && u == 0) bal |= 1ull;  // block (0,0): the padding id of the reference
+        if (lane == u) mine = bal;
       }
-      unsigned long long bal = __ballot(sel);
-      if (r == 0 && c0 == 0) bal |= 1ull;  // block (0,0): the padding id of the reference
       // this wave alone writes the words of its rows (the kernels that wrote the mask before have finished)
-      if (lane == 0 && bal) mv[(int64_t)r * nbw + (c0 >> 6)] |= bal;
+      if (mine) mv[r * nbw + lane] = old[i] | mine;
     }
   }
 }
 
+template <int NB>
 __global__ __launch_bounds__(CS_THREADS) void sp_cover_select_kernel(const float* __restrict__ x,
                                                                       const int32_t* __restrict__ enable,
                                                                       int enable_match, int nb, int nbw, long long t_le,
@@ -569,7 +575,7 @@ __global__ __launch_bounds__(CS_THREADS) void sp_cover_select_kernel(const float
   __shared__ uint32_t row_ties[GSEL_ONE_NB];
   const int v = blockIdx.x;
   if (!gsel_enabled(enable, enable_match, v)) return;
-  cover_select_map(sh, row_ties, x + (int64_t)v * nb * nb, nb, nbw, t_le, mask + (int64_t)v * nb * nbw);
+  cover_select_map<NB>(sh, row_ties, x + (int64_t)v * nb * nb, nb, nbw, t_le, mask + (int64_t)v * nb * nbw);
 }
 
 __global__ __launch_bounds__(GSEL_THREADS) void sp_gsel_emit_kernel(const float* __restrict__ x, int nb, int nbw,
@@ -754,8 +760,11 @@ static int gsel_run(const float* x, const int32_t* enable, int enable_match, int
              SP_ERR_WORKSPACE, "%s: workspace missing, misaligned or too small", who);
   const int nbw = (nb + 63) / 64;
   if (nb <= GSEL_ONE_NB) {  // one workgroup per map does the whole descent and writes the bits
-    hipLaunchKernelGGL(sp_cover_select_kernel, dim3(n_vec), dim3(CS_THREADS), 0, s, x, enable, enable_match, nb, nbw,
-                       (long long)sp_thr_le(score), mask);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(n_vec), dim3(CS_THREADS), 0, s, x, enable, enable_match, nb, nbw,
+                         (long long)sp_thr_le(score), mask);
+    };
+    nb <= 128 ? launch(sp_cover_select_kernel<128>) : launch(sp_cover_select_kernel<GSEL_ONE_NB>);
     SP_LAUNCH_CHECK();
     return SP_OK;
   }
@@ -1541,7 +1550,7 @@ __global__ __launch_bounds__(CS_THREADS) void sp_queryaware_small_kernel(const s
   if (decision[h] != SP_DEC_QA) return;
   bpm_rows<D, CS_THREADS / BPM_THREADS>(lds.rows, qbar, kbar, 0, h, hq, hkv, nb, flags, inv_sqrt_d, probs);
   __syncthreads();  // the map is written, the tile's LDS is free
-  cover_select_map(lds.sel.cover, lds.sel.row_ties, probs + (int64_t)h * nb * nb, nb, nbw, t_le, mask + (int64_t)h * nb * nbw);
+  cover_select_map<LQ_TILE>(lds.sel.cover, lds.sel.row_ties, probs + (int64_t)h * nb * nb, nb, nbw, t_le, mask + (int64_t)h * nb * nbw);
 }
 
 // score = pattern_threshold * nb: the product of the caller's DOUBLE threshold and the block count, evaluated in

@@ -103,7 +103,7 @@ def test_cover_count_at_path_boundaries(gpu_device, n):
 
 @pytest.mark.parametrize("nb", [1, 2, 63, 65, 127, 128, 129, 255, 256, 257])
 def test_cover_select_global_at_path_boundaries(gpu_device, nb):
-    """Register-resident maps end at 128 blocks, one workgroup per map at 256; random maps, uniform rows (the boundary
+    """The small instance ends at 128 blocks, one workgroup per map at 256; random maps, uniform rows (the boundary
     group of equal values spans rows), a map whose mass stays below the budget."""
     from shareprefill_amd import ops
 
