@@ -247,7 +247,7 @@ __global__ __launch_bounds__(SEL_THREADS) void sp_gsel_pick_kernel(GselState* __
 // Vectors of at most CS_ITEMS entries per thread stay in registers for all levels; longer ones are read again.
 // 64 vectors, one launch against three levels of 2048 bins (one workgroup up to 16384 values, ten launches above): 3001
 // values 16.7 -> 11.0 us, 16384 25.9 -> 14.5, 32768 58 -> 25, 131072 80 -> 75; at 262144 the ten launches take 106 us and
-// one would take 109, hence GSEL_ONE_LEN.  32 maps of 64 x 64 blocks 20.2 -> 12.8 us, 256 x 256
+// one would take 109, hence GSEL_ONE_LEN (few vectors: cover_one_launch).  32 maps of 64 x 64 blocks 20.2 -> 12.8 us, 256 x 256
 // 72 -> 41 (one map 42 -> 40) and, what most layers meet, no map enabled 30.6 -> 6.7; at 512 x 512 the ten launches are ahead
 // (96 us against 227 with the entries read again in each level), hence GSEL_ONE_NB.
 #define CS_THREADS 1024
@@ -471,6 +471,12 @@ __device__ static void cover_count_vector(CoverShared& sh, const CoverCountArgs&
 }
 
 #define GSEL_ONE_LEN 131072
+// One workgroup per vector, or the many-workgroup descent: the first costs the same for any number of vectors the chip holds at
+// once, the second grows with them.  us, one launch / ten: 2 vectors 32768 values 26 / 35, 65001 43 / 36; 8 vectors 65001 43 /
+// 40; 28 vectors 65001 43 / 52, 131072 79 / 58; 64 vectors 131072 79 / 84.
+static bool cover_one_launch(int64_t len, int n_vec) {
+  return len <= GSEL_ONE_LEN && len <= 49152 + 1280 * (int64_t)n_vec;
+}
 __global__ __launch_bounds__(CS_THREADS) void sp_cover_count_kernel(CoverCountArgs a) {
   __shared__ __attribute__((aligned(16))) CoverShared sh;
   cover_count_vector(sh, a, blockIdx.x);
@@ -800,7 +806,7 @@ static int gsel_count_run(const float* x0, const float* x1, int n0, int n_vec, i
   unsigned long long* gsum = reinterpret_cast<unsigned long long*>(st + n_vec);
   uint32_t* gcnt = reinterpret_cast<uint32_t*>(gsum + (size_t)n_vec * SEL_BINS);
   const long long t_le = (long long)sp_thr_le(thr);
-  if (len <= GSEL_ONE_LEN) {  // one workgroup per vector, one launch
+  if (cover_one_launch(len, n_vec)) {  // one workgroup per vector, one launch
     const CoverCountArgs a = {x0, x1, n0, (int)len, t_le, out0, out1, bs, minb, maxb};
     hipLaunchKernelGGL(sp_cover_count_kernel, dim3(n_vec), dim3(CS_THREADS), 0, s, a);
     SP_LAUNCH_CHECK();
@@ -1688,7 +1694,7 @@ extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int
   rc = sp_lastq_scores_run(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, part(LY_LASTQ),
                            sp_lastq_scores_workspace_bytes(n, hq, bs), vert_tok, slash_tok, vert_blk, slash_blk, part(LY_KBAR), s);
   if (rc != SP_OK) return rc;
-  if (n <= GSEL_ONE_LEN) {
+  if (n <= GSEL_ONE_LEN) {  // (with the heads beside them one launch is ahead for few vectors too: 14 heads, 131072 335 / 347)
     a.n_cover = 2 * hq;
     a.cover = CoverCountArgs{vert_tok, slash_tok, hq, (int)n, (long long)sp_thr_le((float)pattern_threshold), nv, ns, bs,
                              min_blocks, max_blocks};

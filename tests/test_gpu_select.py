@@ -89,7 +89,7 @@ def test_cover_select_global_skips_disabled(gpu_device):
 
 @pytest.mark.parametrize("n", [1, 63, 1025, 16384, 16385, 40000, 131072, 131073])
 def test_cover_count_at_path_boundaries(gpu_device, n):
-    """Register-resident vectors end at 16384 entries, one workgroup per vector at 131072."""
+    """Register-resident vectors end at 16384 entries, one workgroup per vector (of four) at 54272."""
     from shareprefill_amd import ops
 
     x = _probs(4, n, n + 1, sharp=4.0)
@@ -99,6 +99,19 @@ def test_cover_count_at_path_boundaries(gpu_device, n):
     for thr in (0.3, 0.95):
         got = ops.cover_count(x.to(gpu_device).contiguous(), thr).cpu().tolist()
         assert got == [O.cover_count(x[i].numpy(), thr) for i in range(4)]
+
+
+@pytest.mark.parametrize("vectors,n", [(1, 50432), (1, 50433), (4, 54272), (4, 54273), (63, 129793), (64, 131072)])
+def test_cover_count_on_both_sides_of_the_line_between_its_descents(gpu_device, vectors, n):
+    """How long a vector may be for one workgroup depends on how many there are: the last length of one descent, the first
+    of the other."""
+    from shareprefill_amd import ops
+
+    x = _probs(vectors, n, n, sharp=4.0)
+    x[-1] = 1.0 / n
+    got = ops.cover_count(x.to(gpu_device).contiguous(), 0.9).cpu().tolist()
+    some = sorted({0, vectors // 2, vectors - 1})
+    assert [got[i] for i in some] == [O.cover_count(x[i].numpy(), 0.9) for i in some]
 
 
 @pytest.mark.parametrize("nb", [1, 2, 63, 65, 127, 128, 129, 255, 256, 257])
