@@ -402,13 +402,14 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, 
             v.stride(1), v.stride(0), softmax_scale, mask.data_ptr(), _ptr(decision), out.data_ptr(), _ptr(avg_attn), _ptr(ws),
             ws_bytes)
     if pivot is None:
-        st = lib.sp_short_attn_fwd_bf16(*args, stream)
+        st, entry = lib.sp_short_attn_fwd_bf16(*args, stream), "sp_short_attn_fwd_bf16"
     else:
         state, head_cluster, threshold = pivot
         st = lib.sp_short_attn_pivot_fwd_bf16(*args, state.ref(), head_cluster.data_ptr(), threshold, stream)
+        entry = "sp_short_attn_pivot_fwd_bf16"
     if timer is not None:
         timer.stop("attn")
-    _lib.check(st, "sp_short_attn_fwd_bf16")
+    _lib.check(st, entry)
     return out
 
 

@@ -1,5 +1,5 @@
 """GPU parity of the short-prompt attention kernel with the fp32 masked-attention oracle (bounds and their derivation:
-test_gpu_attention.py; the block-average maps add the probabilities as rounded to bf16, 2^-9 relative each, and are compared
+test_gpu_attention.py; the block-average maps add the probabilities as rounded to bf16, 2^-8 relative each, and are compared
 to 2^-8)."""
 
 import numpy as np

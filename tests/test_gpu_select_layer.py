@@ -50,10 +50,19 @@ def test_one_call_equals_the_stages(tmp_path, hq, hkv, d, n, bs, queryaware):
             assert torch.equal(got, want)
         assert torch.equal(got_mask, mask)
         assert not avg.any()
-        qa = ints[0] == 3
+        qa = ints[0] == _lib.SP_DEC_QA
         assert torch.equal(got_probs[qa], probs[qa])
-        if queryaware == 0.0:
-            assert not qa.any()
+        # the inputs are such that every branch of the launches is taken: all heads query-aware (the divergence of a single
+        # block may be NaN), or one pivot per shared cluster, then all of a cluster's heads sharing its pattern
+        if queryaware == 1e9:
+            assert qa.all() or nb == 1
+        else:
+            assert not qa.any() or nb == 1
+            shared = hc >= 0
+            if layer == 0:
+                assert sorted(hc[ints[0] == _lib.SP_DEC_DENSE].tolist()) == sorted(set(hc[shared].tolist()))
+            else:
+                assert (ints[0][shared] == _lib.SP_DEC_SHARE).all()
         for slab in ("info", "ratio", "pattern", "accum"):
             assert torch.equal(getattr(states[0], slab), getattr(states[1], slab)), slab
         for slot in (states[0].info[:, 0] >= 0).nonzero().flatten().tolist():
