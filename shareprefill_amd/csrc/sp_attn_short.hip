@@ -10,9 +10,9 @@
 //     different rows run out of step, so one's matrix instructions fall into another's softmax; the persistent kernel's
 //     software pipeline inside the wave was built here too and measured the same (a wave alone issues an instruction about
 //     every 8 cycles, whatever it is), at twice the code;
-//   * launches that leave CUs half empty (at most two rows per CU) split a row's keys over two sets of four waves, set s taking
-//     half s of every block, and merge the two results through LDS: the chain of tiles is half as long (700 tokens, 32
-//     heads: 21.4 -> 18 us, 1500: 38.6 -> 32);
+//   * a row's keys split over two sets of four waves, merged through LDS, halve the chain of tiles; that was worth 6 % up to 700
+//     tokens and cost 4 % at 2048 (32 heads: 25.0 -> 23.6 us, 1500 44.5 -> 44.0, 2048 57.3 -> 59.4) and gave other bits than the
+//     persistent kernel's, so it was taken out;
 //   * workgroups are dispatched heaviest row first, all heads of one row before the next; a CU that finishes a row takes
 //     the next one, which balances causal rows without tickets.  The query heads of a kv group share an XCD (one L2) for a
 //     row; the XCDs trade groups from row to row, or heads that keep more blocks than others would leave the other XCDs idle
@@ -38,7 +38,7 @@ struct AsArgs {
   const int32_t* decision;   // [hq] or null
   sp_bf16* out;              // [n][hq][D]
   float* avg_attn;           // [hq][nb][nb], written for pivot heads
-  float* block_sums;         // [slots][nb (nb + 1) / 2][KSPLIT][128] of pivot heads
+  float* block_sums;         // [slots][nb (nb + 1) / 2][128] of pivot heads
   int slots;                 // pivot heads there is room for; -1: no maps wanted
   int64_t n, sq_n, sq_h, sk_n, sk_h, sv_n, sv_h;
   int hq, group, nb, nbw;
@@ -62,7 +62,7 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 #define AS_THREADS 256  // 4 waves x 32 queries
 #define AS_WAVES 4
 #define AS_MAX_NB 512     // blocks a row's list holds
-#define AS_LDS_BYTES(D, KSPLIT) ((KSPLIT) * 4 * AS_TILE * (D) * 2)
+#define AS_LDS_BYTES(D) (4 * AS_TILE * (D) * 2)
 #define AS_NO_MAX (-1.0e30f)         // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
 #define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
 
@@ -152,21 +152,18 @@ __device__ __forceinline__ float as_groupmax(float v) {
   return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
 }
 
-// KSPLIT = 2: two sets of four waves own the same queries and take the even and the odd 64-key tiles.
 // Args = AsPivotArgs: with the pivots' patterns (an instance of its own: prompts that select nothing, whose launch is the
 // whole layer, run 1.5 % slower with that code in theirs).
-template <int D, int KSPLIT, typename Args>
-__global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(Args a) {
+template <int D, typename Args>
+__global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   constexpr int QT = 2;                             // 16-query tiles per wave
   constexpr int KS = D / 32, CT = D / 16;           // channel steps of S, channel tiles of O
-  constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS * KSPLIT, WQ = 16 * QT;
+  constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS, WQ = 16 * QT;
   constexpr int TILE_BYTES = AS_TILE * D * 2;
-  extern __shared__ __attribute__((aligned(1024))) char lds_all[];  // per set of waves [buffer][K | V]
+  extern __shared__ __attribute__((aligned(1024))) char lds[];  // [buffer][K | V]
   __shared__ uint16_t list[AS_MAX_NB];
   const int t = threadIdx.x, lane = t & 63, lq = lane & 15, g = lane >> 4;
-  const int wave8 = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wave = wave8 % WAVES, set = wave8 / WAVES;  // query band, set
-  char* const lds = lds_all + set * 4 * TILE_BYTES;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // query band
   const uint32_t lds_base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
   int h, rr;  // head, rank of the row (0 = the last, heaviest one)
   if ((a.hq & 7) == 0) {
@@ -210,9 +207,9 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
       if (wi == (r >> 6) && (r & 63) != 63) x &= (2ull << (r & 63)) - 1ull;
       if (n_blk == 0 && x != 0ull) {  // the first tile is on its way while the list is made
         c = wi * 64 + __builtin_ctzll(x);
-        issue(c, set, 0);
+        issue(c, 0, 0);
       }
-      if ((wi % (WAVES * KSPLIT)) == wave8 && ((x >> lane) & 1ull))
+      if (wi % WAVES == wave && ((x >> lane) & 1ull))
         list[n_blk + __builtin_popcountll(x & ((1ull << lane) - 1ull))] = (uint16_t)(wi * 64 + lane);
       n_blk += __builtin_popcountll(x);
     }
@@ -232,8 +229,7 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
     l_mark[qt] = 0.f;
   }
   const as_bf16x8 ones = __builtin_bit_cast(as_bf16x8, (as_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-  // pivot heads: this row's sums per block and set of waves, [column][set][128 queries], in the slab of the head's rank among
-  // them
+  // pivot heads: this row's sums per block, [column][128 queries], in the slab of the head's rank among them
   const bool pivot = a.slots >= 0 && a.decision[h] == SP_DEC_DENSE;  // (uniform)
   float* pu = nullptr;
   if (pivot) {
@@ -241,7 +237,7 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
     for (int i = 0; i < h; i += SP_WAVE)
       slot += __builtin_popcountll(__ballot(i + lane < h && a.decision[i + lane < h ? i + lane : 0] == SP_DEC_DENSE));
     if (slot < a.slots)
-      pu = a.block_sums + ((int64_t)slot * ((int64_t)a.nb * (a.nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * (KSPLIT * AS_BS);
+      pu = a.block_sums + ((int64_t)slot * ((int64_t)a.nb * (a.nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * AS_BS;
   }
 
   // LDS byte offsets of the lane's operands: K row lq, logical chunk 4 ks + g; V row 4 g + lq / 4, 8-byte piece lq % 4 of the
@@ -251,20 +247,17 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
   const int voff = vrow * (D * 2) + 8 * (lq & 1), vswz = as_swz<D>(vrow), vhalf = (lq >> 1) & 1;
 
   int c_next = 0;
-  // One step per tile of the set: KSPLIT = 1 walks both halves of every block, KSPLIT = 2 one half each.  The block list is
-  // read a block ahead of its use.
-  const int steps = KSPLIT == 1 ? 2 * n_blk : n_blk;
-  for (int st = 0; st < steps; ++st) {
-    const int i = KSPLIT == 1 ? st >> 1 : st, half = KSPLIT == 1 ? (st & 1) : set, buf = st & 1;
+  // One step per tile, two per block.  The block list is read a block ahead of its use.
+  for (int st = 0; st < 2 * n_blk; ++st) {
+    const int i = st >> 1, half = st & 1, buf = half;
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of the tile have landed
     __syncthreads();                     // ... everybody's; and the other buffer's readers are done
-    if (KSPLIT == 1 && half == 0) {
+    if (half == 0) {
       issue(c, 1, buf ^ 1);
       c_next = (int)list[i + 1 < n_blk ? i + 1 : i];
     } else if (i + 1 < n_blk) {
-      if (KSPLIT == 2) c_next = (int)list[i + 1];
       c_next = __builtin_amdgcn_readfirstlane(c_next);
-      issue(c_next, KSPLIT == 1 ? 0 : set, buf ^ 1);
+      issue(c_next, 0, buf ^ 1);
     }
     const bool diag = c == r;
     if (!diag || half * AS_TILE <= wave * WQ + WQ - 1) {  // (else: every key of the tile lies behind the wave's queries)
@@ -375,49 +368,22 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
         });
       });
     }
-    if (pu != nullptr && (KSPLIT == 2 || half == 1)) {  // pivot head: the block's (the set's) softmax mass, log2 units
+    if (pu != nullptr && half == 1) {  // pivot head: the block's softmax mass, log2 units
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const float u = __builtin_amdgcn_logf(l[qt][0] - l_mark[qt]) + m[qt];
         l_mark[qt] = l[qt][0];
-        if (g == 0) pu[(int64_t)(KSPLIT * c + set) * AS_BS + q_off + 16 * qt] = u;
+        if (g == 0) pu[(int64_t)c * AS_BS + q_off + 16 * qt] = u;
       }
     }
-    if (KSPLIT == 2 || half == 1) c = c_next;
+    if (half == 1) c = c_next;
   }
 
-  if constexpr (KSPLIT == 2) {  // the second set hands its O, max and sums over through LDS (its own tile buffers' space)
-    as_floatx4* const xo = reinterpret_cast<as_floatx4*>(lds_all) + wave * (CT * QT) * 64 + lane;  // [wave][ct, qt][lane]
-    float2* const xs = reinterpret_cast<float2*>(lds_all + AS_BS * D * 4) + (wave * QT) * 64 + lane;  // [set][wave][qt][lane]
-    __syncthreads();  // the tiles are consumed
-    if (set == 1) {
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) xo[(ct * QT + qt) * 64] = o[ct][qt];
-    }
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) xs[(set * WAVES * QT + qt) * 64] = make_float2(m[qt], l[qt][0]);
-    __syncthreads();
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      const float2 x = xs[((set ^ 1) * WAVES * QT + qt) * 64];
-      const float m_new = fmaxf(m[qt], x.x);
-      const float mine = __builtin_amdgcn_exp2f(m[qt] - m_new), other = __builtin_amdgcn_exp2f(x.x - m_new);
-      m[qt] = m_new;
-      // (one expression for both sets, so that both hold the same sum)
-      l[qt][0] = set == 0 ? l[qt][0] * mine + x.y * other : x.y * other + l[qt][0] * mine;
-      if (set == 0) {
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) o[ct][qt] = o[ct][qt] * mine + xo[(ct * QT + qt) * 64] * other;
-      }
-    }
-  }
   float inv_l[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     inv_l[qt] = 1.0f / l[qt][0];
-    if (set == 0 && qrow + 16 * qt < a.n) {
+    if (qrow + 16 * qt < a.n) {
       sp_bf16* dst = a.out + ((qrow + 16 * qt) * a.hq + h) * D + 4 * g;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
@@ -432,21 +398,21 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
     for (int i = t; i < n_blk; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = NAN;
     return;
   }
-  // pivot head: avg[r][c] = mean over the block's valid queries of (sum over the sets of exp2(u - m[q])) / l[q].  A wave
+  // pivot head: avg[r][c] = mean over the block's valid queries of exp2(u - m[q]) / l[q].  A wave
   // reads back its own sums (its own stores), folds its queries, and the waves meet in LDS.
-  float* const part = reinterpret_cast<float*>(lds_all);  // [block][wave]
-  __syncthreads();                                        // LDS is free, the stores of pu have left
+  float* const part = reinterpret_cast<float*>(lds);  // [block][wave]
+  __syncthreads();                                    // LDS is free, the stores of pu have left
   for (int i = 0; i < n_blk; ++i) {
     const int c = (int)list[i];
     float x = 0.f;
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
       if (qrow + 16 * qt < a.n) {
-        x += __builtin_amdgcn_exp2f(pu[(int64_t)(KSPLIT * c + set) * AS_BS + q_off + 16 * qt] - m[qt]) * inv_l[qt];
+        x += __builtin_amdgcn_exp2f(pu[(int64_t)c * AS_BS + q_off + 16 * qt] - m[qt]) * inv_l[qt];
       }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, SP_WAVE);
-    if (lane == 0) part[i * (WAVES * KSPLIT) + wave8] = x;
+    if (lane == 0) part[i * WAVES + wave] = x;
   }
   __syncthreads();
   const int64_t rem = a.n - (int64_t)r * AS_BS;
@@ -454,13 +420,13 @@ __global__ __launch_bounds__(AS_THREADS * KSPLIT, 2) void sp_attn_short_kernel(A
   for (int i = t; i < n_blk; i += THREADS) {
     float x = 0.f;
 #pragma unroll
-    for (int w = 0; w < WAVES * KSPLIT; ++w) x += part[i * (WAVES * KSPLIT) + w];
+    for (int w = 0; w < WAVES; ++w) x += part[i * WAVES + w];
     a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = x * inv_q;
   }
   if constexpr (std::is_same<Args, AsPivotArgs>::value) {
     __shared__ PivotRowShared pivot_sh;
     __syncthreads();  // the row is written, LDS is free
-    pivot_row<THREADS>(a.pivot, pivot_sh, lds_all, a.avg_attn, r, h);
+    pivot_row<THREADS>(a.pivot, pivot_sh, lds, a.avg_attn, r, h);
   }
 }
 
@@ -474,18 +440,8 @@ extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
 }
 
-// Up to two rows per CU the split pays (one workgroup of two sets per CU instead of two workgroups: 32 heads, dense mask,
-// 2048 tokens = 512 rows 50.8 -> 44.4 us), beyond it the workgroups' own overlap is worth more (3001 tokens 81 -> 92 us).
-static bool as_split(int64_t n, int32_t hq) { return sp_ceil_div(n, AS_BS) * hq <= 512; }
-
-extern "C" size_t sp_short_attn_pivot_scratch_bytes(int64_t n, int32_t hq) {
-  if (n <= 0 || hq <= 0) return 0;
-  const size_t nb = (size_t)sp_ceil_div(n, AS_BS);
-  return nb * (nb + 1) / 2 * (as_split(n, hq) ? 2 : 1) * AS_BS * sizeof(float);
-}
-
 extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {
-  return n <= 0 || hq <= 0 ? 0 : (size_t)hq * sp_short_attn_pivot_scratch_bytes(n, hq);
+  return n <= 0 || hq <= 0 ? 0 : (size_t)hq * sp_attn_pivot_scratch_bytes(n, AS_BS);
 }
 
 static int as_launch(const char* who, const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
@@ -510,38 +466,32 @@ static int as_launch(const char* who, const void* q, const void* k, const void* 
   const bool maps = decision != nullptr && avg_attn != nullptr;
   SP_REQUIRE(!maps || workspace_bytes == 0 || (workspace && ((uintptr_t)workspace % 4) == 0), SP_ERR_WORKSPACE,
              "%s: workspace missing or misaligned", who);
-  const size_t room = workspace_bytes / sp_short_attn_pivot_scratch_bytes(n, hq);
+  const size_t room = workspace_bytes / sp_attn_pivot_scratch_bytes(n, AS_BS);
   const int slots = !maps ? -1 : room < (size_t)hq ? (int)room : hq;
   const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
                     (float*)workspace, slots, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
                     v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), decision == nullptr && avg_attn != nullptr,
                     softmax_scale * 1.4426950408889634f};
-  static_assert(AS_LDS_BYTES(64, 1) >= AS_MAX_NB * 14 + AS_THREADS * 2 * 8 + 16, "");  // rs_lds_bytes(AS_MAX_NB, 2 sets)
+  static_assert(AS_LDS_BYTES(64) >= AS_MAX_NB * 14 + AS_THREADS * 8 + 16, "");  // rs_lds_bytes(AS_MAX_NB, AS_THREADS)
   const dim3 grid((unsigned)(nb * hq));
-  const bool split = as_split(n, hq);
   static bool attr_set[64] = {false};  // per device, once (idempotent)
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));
   SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "%s: device index %d", who, dev);
   if (!attr_set[dev]) {
-    const void* kernels[8] = {
-        (const void*)sp_attn_short_kernel<64, 1, AsArgs>,      (const void*)sp_attn_short_kernel<128, 1, AsArgs>,
-        (const void*)sp_attn_short_kernel<64, 2, AsArgs>,      (const void*)sp_attn_short_kernel<128, 2, AsArgs>,
-        (const void*)sp_attn_short_kernel<64, 1, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, 1, AsPivotArgs>,
-        (const void*)sp_attn_short_kernel<64, 2, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, 2, AsPivotArgs>};
+    const void* kernels[4] = {
+        (const void*)sp_attn_short_kernel<64, AsArgs>, (const void*)sp_attn_short_kernel<128, AsArgs>,
+        (const void*)sp_attn_short_kernel<64, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, AsPivotArgs>};
     for (const void* f : kernels)
-      SP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AS_LDS_BYTES(128, 2)));
+      SP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AS_LDS_BYTES(128)));
     attr_set[dev] = true;
   }
-  auto launch = [&](auto kernel, int ksplit, const auto& args) {
-    hipLaunchKernelGGL(kernel, grid, dim3(AS_THREADS * ksplit), AS_LDS_BYTES(d, ksplit), (hipStream_t)stream, args);
+  auto launch = [&](auto kernel, const auto& args) {
+    hipLaunchKernelGGL(kernel, grid, dim3(AS_THREADS), AS_LDS_BYTES(d), (hipStream_t)stream, args);
   };
   auto pick = [&](const auto& args) {
     using Args = std::decay_t<decltype(args)>;
-    if (d == 64)
-      split ? launch(sp_attn_short_kernel<64, 2, Args>, 2, args) : launch(sp_attn_short_kernel<64, 1, Args>, 1, args);
-    else
-      split ? launch(sp_attn_short_kernel<128, 2, Args>, 2, args) : launch(sp_attn_short_kernel<128, 1, Args>, 1, args);
+    d == 64 ? launch(sp_attn_short_kernel<64, Args>, args) : launch(sp_attn_short_kernel<128, Args>, args);
   };
   if (pivot != nullptr) {
     AsPivotArgs with;

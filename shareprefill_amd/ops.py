@@ -393,7 +393,7 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, 
     out = torch.empty(n, hq, d, dtype=torch.bfloat16, device=dev)
     ws, ws_bytes = None, 0
     if decision is not None and avg_attn is not None:
-        ws_bytes = (hq if max_pivots is None else min(max_pivots, hq)) * lib.sp_short_attn_pivot_scratch_bytes(n, hq)
+        ws_bytes = (hq if max_pivots is None else min(max_pivots, hq)) * lib.sp_attn_pivot_scratch_bytes(n, 128)
         ws = _workspace("attn_short", ws_bytes, dev) if ws_bytes else None
     timer = kernel_timer
     if timer is not None:

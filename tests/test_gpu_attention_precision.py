@@ -38,8 +38,7 @@ def bf16_weights(n, seed):
     return w
 
 
-# kernel: 0 = the persistent one, else head_dim of the short-prompt one; 2 and 136 heads: its rows split over two sets of
-# waves and not
+# kernel: 0 = the persistent one, else head_dim of the short-prompt one
 @pytest.mark.parametrize("kernel,hq,hkv", [(0, 2, 1), (128, 2, 1), (64, 2, 1), (128, 136, 17), (64, 136, 17)])
 @pytest.mark.parametrize("seed", [0, 1])
 def test_weights_that_bf16_holds_are_not_rounded(gpu_device, kernel, hq, hkv, seed):

@@ -15,8 +15,8 @@ MAX_ABS, MEAN_REL = 2e-2, 2.5e-3
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("hq,hkv,n", [(8, 8, 1), (8, 1, 65), (16, 4, 130), (4, 2, 640), (7, 1, 1111),
-                                      (32, 8, 2048),   # the last size whose rows are split over two sets of waves
-                                      (32, 8, 2177),   # the first that is not; ragged by one token
+                                      (32, 8, 2048),   # whole blocks
+                                      (32, 8, 2177),   # ragged by one token
                                       (3, 1, 8300)])   # more than one mask word per row
 def test_short_attention_matches_oracle(gpu_device, hq, hkv, n, d):
     """Random masks with dense heads among them, whose maps the kernel writes; logits that grow along the row for the last
@@ -93,8 +93,8 @@ def test_pivot_patterns_in_the_attention_launch(gpu_device, hq, hkv, n, d):
 
 @pytest.mark.parametrize("hq,hkv,n,d", [(6, 2, 1111, 128), (72, 8, 1111, 64), (70, 2, 1025, 128)])
 def test_block_sums_for_as_many_heads_as_can_be_pivots(gpu_device, hq, hkv, n, d):
-    """Maps, with room for exactly the dense heads, equal those with room for all heads (rows split and not, more heads than a
-    wave has lanes); a dense head there is no room for gets NaN and updates no pivot, the others are as they were."""
+    """Maps, with room for exactly the dense heads, equal those with room for all heads (also of more heads than a wave has
+    lanes); a dense head there is no room for gets NaN and updates no pivot, the others are as they were."""
     from shareprefill_amd import ops
 
     nb = -(-n // 128)
