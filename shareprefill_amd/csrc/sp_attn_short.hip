@@ -431,13 +431,20 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
 }
 
 // ---- host ---------------------------------------------------------------------------------------------
-// The line between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs on a dense
-// mask (32 query / 8 kv heads, whole call with everything it launches, one box, us here / there): 128 channels, dense mask
-// 4096 tokens 146 / 172, 6177 321 / 313, 8192 551 / 477; the bench masks at coverage 0.95 4096 58 / 87, 6177 96 / 121, 8192
-// 176 / 190, 16384 738 / 637.  64 channels, where the persistent kernel computes on zero-padded tiles: dense 8192 310 / 324,
-// 24576 2671 / 2629, the bench masks 8192 115 / 150, 32768 1886 / 1761, plus there the padding itself.
+// The lines between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs.  128
+// channels, whole layer, one box, us here / there:
+//   masks of the selection (32 query / 8 kv heads at coverage 0.95): 6656 tokens 197 / 221, 8192 248 / 272; at 0.99 262 / 271 and
+//   347 / 342, with every head query-aware (nine blocks of ten kept) 443 / 445 and 612 / 594; 28 / 4 heads at 6656 182 / 211, 240 /
+//   251, 408 / 433, 8 / 2 heads 140 / 159, 191 / 197, 236 / 250;
+//   every block kept: 32 / 8 heads 4608 221 / 228, 5120 233 / 235, 5632 275 / 266, 6656 373 / 332; 28 / 4 6177 292 / 293; 8 / 2
+//   6656 159 / 161.
+// 64 channels, attention alone, where the persistent kernel computes on zero-padded tiles (the padding itself not counted): all
+// blocks 8192 322 / 329, 24576 2602 / 2577, 32768 4587 / 4680; masks at 0.95 8192 96 / 133, 32768 486 / 552.
 extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
+}
+extern "C" int64_t sp_short_attn_max_dense_tokens(int32_t d) {
+  return d == 64 ? 32768 : 5120;
 }
 
 extern "C" size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq) {

@@ -213,7 +213,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         # the pivots' block-average maps (attn_weights is all zeros).  config.dense_short_prompts = False takes the
         # full path instead.
         mask = _dense_causal_mask(num_heads, nb, q.device)
-        if short:
+        if short and q_len <= _lib.load().sp_short_attn_max_dense_tokens(head_dim):
             avg_attn = torch.empty(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
             out = ops.short_attention(q, k, v, mask, softmax_scale, avg_attn=avg_attn)  # (clears avg_attn)
         else:

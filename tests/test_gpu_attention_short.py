@@ -145,3 +145,46 @@ def test_a_layer_keeps_block_sums_of_its_possible_pivots_only(gpu_device, tmp_pa
         shareprefill_attention_forward(mod, *qkv, None, scaling=d ** -0.5)
         assert int((sharing.plans[-1].decision == _lib.SP_DEC_DENSE).sum()) == pivots
         assert held() <= pivots * _lib.load().sp_attn_pivot_scratch_bytes(n, 128)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,n", [(8, 2, 130), (6, 2, 700), (32, 8, 2048), (3, 1, 6177)])
+def test_short_and_long_prompt_kernels_give_the_same_bits(gpu_device, hq, hkv, n, d):
+    """Both walk a row's blocks in steps of 32 keys and move the running max by the same rule, so which of them a prompt's
+    length chooses does not show in its output; logits that grow along the row make the max move often."""
+    from shareprefill_amd import ops
+
+    nb = -(-n // 128)
+    gen = torch.Generator(device=gpu_device).manual_seed(n + d)
+    q, k, v = (torch.randn(h, n, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h in (hq, hkv, hkv))
+    k[-1] *= (1 + 9 * torch.arange(n, device=gpu_device) / n)[:, None].to(torch.bfloat16)
+    mask = np.tril(np.random.default_rng(n).random((hq, nb, nb)) < 0.4)
+    mask[:, np.arange(nb), np.arange(nb)] = True
+    bits = ops.bool_to_mask(torch.from_numpy(mask)).to(gpu_device)
+    short = ops.short_attention(q, k, v, bits, d ** -0.5)
+    wide = (torch.nn.functional.pad(t, (0, 128 - d)) for t in (q, k, v))
+    long = ops.block_sparse_attention(*wide, bits, 128, d ** -0.5, half_channels=d == 64)[..., :d]
+    assert torch.equal(short, long)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("past", [0, 1])
+def test_dense_prompts_on_both_sides_of_the_line(gpu_device, tmp_path, d, past):
+    """A prompt within the minimum budget, at the last length the short-prompt kernel takes it and at the first it does
+    not: output on the dense mask, cleared maps."""
+    import types
+
+    from shareprefill_amd import AttentionSharing, _lib, ops, shareprefill_attention_forward, synthetic
+
+    n = _lib.load().sp_short_attn_max_dense_tokens(d) + past
+    path = synthetic.write_cluster_table(synthetic.random_cluster_table(2, 1, 1, 3), str(tmp_path / "table.json"))
+    cfg = types.SimpleNamespace(block_size=128, min_budget=65536, max_budget=None, pattern_threshold=0.9, similarity_threshold=0.5,
+                                fallback_threshold=0.9, queryaware_threshold=0.1)
+    qkv = synthetic.planted_qkv(2, 1, n, d, 1, device=gpu_device, q_head_gain=1.0)
+    mod = types.SimpleNamespace(config=cfg, attention_sharing=AttentionSharing(path), layer_idx=0, scaling=d ** -0.5)
+    out, maps = shareprefill_attention_forward(mod, *qkv, None, scaling=d ** -0.5)
+    nb = -(-n // 128)
+    mask = ops.bool_to_mask(torch.ones(nb, nb, dtype=torch.bool).tril().expand(2, nb, nb)).to(gpu_device)
+    want = ops.block_sparse_attention(*(torch.nn.functional.pad(t[0], (0, 128 - d)) for t in qkv), mask, 128, d ** -0.5,
+                                      half_channels=d == 64)[..., :d]
+    assert torch.equal(out[0], want) and not maps.any() and maps.shape == (1, 2, nb, nb)
