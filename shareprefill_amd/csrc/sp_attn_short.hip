@@ -16,18 +16,18 @@
 //   * workgroups are dispatched heaviest row first, all heads of one row before the next; a CU that finishes a row takes
 //     the next one, which balances causal rows without tickets.  The query heads of a kv group share an XCD (one L2) for a
 //     row; the XCDs trade groups from row to row, or heads that keep more blocks than others would leave the other XCDs idle
-//     (8192 tokens, the bench masks: 333 us with a fixed assignment, 195 with the rotating one);
+//     (8192 tokens, masks at coverage 0.95: 319 us with a fixed assignment, 178 with the rotating one);
 //   * V is read as it is: the tile is row-major in LDS and the V^T operand comes from the transposing LDS read
 //     (ds_read_b64_tr_b16: the 16 lanes of a group address 4 keys x 16 channels and each receives 4 keys of its channel).
 //     S^T = K . Q^T leaves a lane with keys 4g .. 4g+3 of every 16-key tile (g = lane / 16), which is exactly what two such
 //     reads deliver, so P^T is the S^T accumulators converted to bf16 in place;
 //   * a pivot head's block-average map is made by the same workgroup at the end of its row (no second kernel), and so is the
 //     row's pattern in the sharing state, which needs nothing but that row (a launch in every layer, of which all but one per
-//     cluster had nothing to do: 3001 tokens 108.6 -> 106.2 us a layer, 6177 of 64 channels 121.2 -> 119.8); a call
-//     without decisions has its maps cleared here (a fill launch in front of the kernel costs its caller 5 us of host time:
-//     700 tokens 21.3 -> 18.7 us a layer).
+//     cluster had nothing to do: 2.4 us of a layer of 3001 tokens, 1.4 of 6177 with 64 channels); a call without decisions
+//     has its maps cleared here (a fill launch in front of the kernel costs its caller 5 us of host time, 2.6 us of a layer of
+//     700 tokens).
 // Two rows sharing one K / V tile, as in the persistent kernel, halve the tile traffic per flop, which is why that one
-// stays for long prompts; sp_short_attn_max_tokens holds the line between the two and the figures.
+// stays for long prompts; sp_short_attn_max_tokens holds the lines between the two and the figures.  Both give the same bits.
 #include "sp_rows.h"
 
 #include <type_traits>

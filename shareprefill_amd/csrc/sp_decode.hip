@@ -7,7 +7,7 @@
 // partial (o, m, l); a second tiny kernel merges the partials in a fixed order.  A batch of sequences is one more grid
 // axis: per token of a small model's or short chat's step the launches and the host's way to them are what counts, and
 // one pair of launches per sequence, a workspace look-up each and a stacking copy were most of it (32 query / 8 kv heads:
-// 8 caches of 4001 tokens 137 -> 29 us = 4.5 TB/s, one of 1025 tokens 24.8 -> 15.9 us, one of 131072 100.9 -> 96.8 us).
+// 8 caches of 4001 tokens 135 -> 30 us = 4.4 TB/s, one of 1025 tokens 24.2 -> 14.3 us, one of 131072 100.5 -> 97.5 us).
 //
 // Both products run on the matrix core with the group's heads as a (mostly empty) 32-wide operand -- the MFMAs
 // are free here, the point is to keep the vector ALU out of the inner loop:

@@ -8,8 +8,9 @@
 //     so every comparison against a threshold is independent of summation order (integer atomics
 //     and scans may associate freely).
 // Two primitives:
-//   * radix mass descent for long vectors (per-token vectors of length N, the nb*nb pooled map):
-//     three passes over the data building (count, mass) histograms over 11/11/10 key bits;
+//   * radix mass descent for long vectors (per-token vectors of length N, the nb*nb pooled map), from (count, mass)
+//     histograms over the key's bits: one workgroup per vector in four levels of 8/8/8/7 bits up to GSEL_ONE_LEN values
+//     and GSEL_ONE_NB blocks, many workgroups per vector in three levels of 11/11/10 bits beyond;
 //   * rank sort for short vectors (rows of length nb): rank by pairwise comparison in LDS, scatter to
 //     sorted order, integer prefix scan -- a literal sort / cumsum / threshold.
 #include <cstring>
@@ -1342,7 +1343,7 @@ extern "C" int sp_share_decide(const sp_cluster_state* state, const int32_t* hea
 #define MASK_THREADS 1024
 #define MASK_SPLIT 8  // workgroups per head: each ranks the head's vectors itself and writes a share of the rows
 // What the whole-layer selection adds to the mask launch: nothing of it depends on the mask, and each would be a launch of
-// 5 us of its own.
+// its own (2 to 2.7 us of the stream if it had nothing to do).
 struct MaskBesides {
   int layer_idx;    // pivots elected in this layer store their vectors and sets
   PoolArgs qpool;   // query-aware heads: the averages of Q's blocks
@@ -1536,9 +1537,8 @@ __global__ __launch_bounds__(BP_THREADS) void sp_block_probs_kernel(
 // Up to 128 blocks (16384 tokens at block size 128) a head's map is one row tile of bpm_rows, and the head's probabilities and
 // its selection are one workgroup and one launch: the map is read back by the workgroup that wrote it.  Beyond, a head's
 // row tiles are workgroups of a launch of their own.  Bound by latency (one K tile, two passes over it, the descent's
-// barriers) and, in layers without a query-aware head, by being a launch at all.  Whole layer, two launches / this one: 3001
-// tokens 110.8 -> 108.7 us, 6177 (64 channels) 122.4 -> 120.6, 10007 (28 / 4 heads) 268.9 -> 266.9; with all 32 heads
-// query-aware, 8192 tokens and the projections, 1164 -> 1161.
+// barriers) and, in layers without a query-aware head, by being a launch at all: against two launches a layer without one takes
+// 2 us less (3001 tokens, 6177 of 64 channels, 10007 of 28 / 4 heads), one with all 32 heads query-aware 3 us (8192 tokens).
 template <int D>
 __global__ __launch_bounds__(CS_THREADS) void sp_queryaware_small_kernel(const sp_bf16* qbar, const sp_bf16* kbar,
                                                                          const int32_t* __restrict__ decision, int hq, int hkv,
@@ -1609,8 +1609,9 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
 // ------------------------------------------------------------------------------------------------
 // The stages above, with the launches folded that do not wait for each other: K's averages beside the score statistics, the
 // query-aware test and the share similarities beside the budgets, Q's averages, the pivots' own sets and the clearing of the
-// map beside the masks.  Same device code, same results.  A launch costs 5 us of the stream whatever it does; whole layer,
-// 15 launches / 7 (six up to 128 blocks since): 3001 tokens 142 -> 120 us, 6177 (64 channels) 148 -> 127, 10007 (28 / 4 heads) 336 -> 313.
+// map beside the masks.  Same device code, same results.  A launch that has nothing to do costs 2 to 2.7 us of the stream;
+// against 15 launches, seven (six up to 128 blocks since) take 21 to 23 us off a layer (3001 tokens, 6177 of 64 channels, 10007
+// of 28 / 4 heads).
 struct HeadArgs {
   CoverCountArgs cover;
   int n_cover;  // workgroups 0 .. n_cover - 1: the budgets (0: made by other launches); then one per head
