@@ -129,8 +129,9 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
     float2* __restrict__ partial /* [hq][n_chunks][128] */, PoolArgs pool) {
   __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES(D)];
   const int pairs = lq_pairs(group);
-  // The rows of the grid behind the scores' own pool K beside them (dispatched last, two units per workgroup): a launch of
-  // its own takes 2 to 2.7 us if it does nothing, and the keys are on their way through the caches anyway.
+  // The rows of the grid behind the scores' own pool K beside them (dispatched last, two units per workgroup): the vector
+  // ALU bounds the scores, so the keys' second way through memory fits beside them (131072 tokens: statistics 195 us alone, 196
+  // with it, where a launch of its own takes 43; a launch with nothing to do takes 2 to 2.7).
   if ((int)blockIdx.y >= hkv * pairs) {
     static_assert(LQ_WG_THREADS == 2 * POOL_THREADS && LQ_KSW_BYTES(64) >= 2 * POOL_SPLIT * POOL_CHUNKS * 8 * 4, "");
     const int half = threadIdx.x / POOL_THREADS;
