@@ -447,7 +447,7 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_
 
 def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float) -> torch.Tensor:
     """One new token per sequence: q bf16 [B, Hq, 1, D], k / v bf16 [B, Hkv, N, D] views -> out bf16 [B, 1, Hq, D].
-    (A cache of more sequences is read up to the B-th.)
+    (A cache of more sequences is read up to the B-th, v up to k's heads and tokens, both up to q's channels.)
 
     The whole batch runs in the launches of one sequence (decode_attention: the same kernels)."""
     lib = _lib.load()
@@ -464,7 +464,7 @@ def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, so
                 raise ValueError(f"{name} must live on the GPU the queries are on")
             if t.stride(3) != 1:
                 raise ValueError(f"{name} must have a contiguous head_dim axis")
-    if v.shape[1:] != k.shape[1:] or min(k.shape[0], v.shape[0]) < b or k.shape[3] != d:
+    if min(k.shape[0], v.shape[0]) < b or v.shape[1] < hkv or v.shape[2] < n or min(k.shape[3], v.shape[3]) < d:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} do not match q {tuple(q.shape)}")
     stream = _stream_handle(dev)
     out = torch.empty((b, 1, hq, d), dtype=torch.bfloat16, device=dev)

@@ -176,3 +176,21 @@ def test_decode_reads_a_larger_cache_up_to_the_batch(gpu_device):
     for bad in ((q, k[:1], v), (q, k, v[:1]), (q, k, v[:, :, :299])):
         with pytest.raises(ValueError):
             ops.decode_attention_batch(*bad, 0.125)
+
+
+def test_decode_reads_k_and_v_up_to_what_the_step_needs(gpu_device):
+    """k says how many heads and tokens there are, q how many channels: v may hold more of all three and k more channels;
+    a k or v that holds less is refused."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator(device=gpu_device).manual_seed(2)
+    mk = lambda h, m, d: torch.randn(2, h, m, d, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(4, 1, 64), mk(2, 300, 128), mk(3, 417, 96)
+    got = ops.decode_attention_batch(q, k, v, 0.125)
+    assert torch.equal(got, ops.decode_attention_batch(q, k[..., :64], v[:, :2, :300, :64], 0.125))
+    for b in range(2):
+        assert torch.equal(ops.decode_attention_batch(q[b:b + 1], k[b:b + 1], v[b:b + 1], 0.125)[0, 0],
+                           ops.decode_attention(q[b, :, 0], k[b], v[b], 0.125))
+    for bad in ((q, k[..., :56], v), (q, k, v[..., :56]), (q, k, v[:, :1]), (q, k, v[:, :, :299])):
+        with pytest.raises(ValueError):
+            ops.decode_attention_batch(*bad, 0.125)
