@@ -259,6 +259,25 @@ __device__ static inline uint64_t at_trim(uint64_t x, int wi, int r) {
 }
 
 // entry of the per-pair block list: column | row-membership flags
+// inclusive sum over the 64 lanes
+__device__ static __forceinline__ uint32_t at_lane_scan(uint32_t v) {
+  auto add = [&](auto ctrl, auto rows) {  // (lanes without a source, or outside the rows, add 0)
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+  };
+  using all = std::integral_constant<int, 0xf>;
+  add(std::integral_constant<int, 0x111>{}, all{});                              // row_shr 1, 2, 4, 8
+  add(std::integral_constant<int, 0x112>{}, all{});
+  add(std::integral_constant<int, 0x114>{}, all{});
+  add(std::integral_constant<int, 0x118>{}, all{});
+  add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast15 into rows 1 and 3
+  add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast31 into rows 2 and 3
+  return v;
+}
+__device__ static __forceinline__ uint64_t at_lane_u64(uint64_t v, int lane) {  // lane `lane`'s value (uniform)
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
+
 #define AT_IN_A (1u << 30)
 #define AT_IN_B (1u << 31)
 #define AT_COL_MASK 0x00FFFFFFu
@@ -716,18 +735,56 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     float* __restrict__ pivot_u, const uint64_t* __restrict__ fine_mask, int fshift, int nbf, int nbfw) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];  // K ring (4 x 16 KiB) | V^T ring (4 x 16 KiB)
   __shared__ int s_queue, s_ticket;
+  // the scheduler's tables, copied once: read from memory they are two more dependent loads in front of every item
+  __shared__ uint32_t dense_heads[AT_MAX_HEADS / 32], s_order[AT_ORDER_MAX / 2], s_slots[AT_MAX_HEADS / 4], s_pairs[AT_MAX_HEADS / 8];
   constexpr int MODE = (PIVOT ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
   if (PIVOT && sched[AT_NPIV_SLOT] == 0) return;  // no pivot in this layer
-  const uint8_t* const slots = reinterpret_cast<const uint8_t*>(sched + AT_SLOT_TABLE);
-  const uint8_t* const pair_table = reinterpret_cast<const uint8_t*>(sched + AT_PAIR_TABLE);
+  const uint8_t* const slots = reinterpret_cast<const uint8_t*>(s_slots);
+  const uint8_t* const pair_table = reinterpret_cast<const uint8_t*>(s_pairs);
 
   const long long clk0 = clock64(), tick0 = wall_clock64();  // see sp_attn_last_launch_clocks
   AtGeom gm;
   at_geometry(gm, hq, hkv, nb);
-  gm.order = sched[AT_ORDER_SLOT] != 0 ? reinterpret_cast<const uint16_t*>(sched + 256) : nullptr;
+  const bool ordered = sched[AT_ORDER_SLOT] != 0;
+  gm.order = ordered ? reinterpret_cast<const uint16_t*>(s_order) : nullptr;
   const int xcd = blockIdx.x & 7;
-  int first_try = 0;  // queues before this offset are known to be empty (used by thread 0 only)
   const int t = threadIdx.x;
+  static_assert(AT_ORDER_MAX / 2 <= AT_FWD_THREADS && AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8 <= AT_FWD_THREADS, "");
+  if (ordered && t < (gm.n_gangs + 1) / 2) s_order[t] = (uint32_t)sched[256 + t];
+  if (t < AT_MAX_HEADS / 4)
+    s_slots[t] = (uint32_t)sched[AT_SLOT_TABLE + t];
+  else if (t < AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8)
+    s_pairs[t - AT_MAX_HEADS / 4] = (uint32_t)sched[AT_PAIR_TABLE + t - AT_MAX_HEADS / 4];
+  if (t < AT_MAX_HEADS) {
+    const uint64_t votes = __ballot(rowstat != nullptr && decision != nullptr && t < hq && decision[t < hq ? t : 0] == SP_DEC_DENSE);
+    if ((t & 63) == 0) dense_heads[t >> 5] = (uint32_t)votes, dense_heads[(t >> 5) + 1] = (uint32_t)(votes >> 32);
+  }
+  // An item's ends -- ticket, masks, list, first tiles in front of the walk, the epilogue behind it -- were 11 us of 10 to 400.
+  // What they are made of are loads that wait for each other, so: the tables above stand in LDS, the mask words of both rows
+  // are one load (lane i holds word i), the first tiles and the queries go out before the list is written, the ticket is asked
+  // for at the item's last barrier, no barrier waits for the output's stores, and those are 16 bytes a lane instead of 8.
+  // 8.5 us are left, most of it the 176 KiB of queries, first tiles and output through the CU's 64 bytes a cycle.  Layers, us:
+  // 10007 tokens with 28 heads 279 -> 267, 16384 (two layers) 1967 -> 1937, 32768 2558 -> 2534, 131072 51870 -> 51640.  Taking the
+  // overlap further (next item's masks, list, tiles and queries in front of the epilogue) measured no better: 282, 1808 against
+  // 1813, 2504 against 2465.
+  // Tickets (thread 0): ask() sends the atomic for the next item, publish() takes its answer -- on an empty queue it goes
+  // on to the next one -- and leaves it in LDS.  Behind an item's last barrier ask() goes out, publish() stands behind the
+  // epilogue: the atomic's way to memory and back passes under the last half-tile and the stores.
+  int first_try = 0, tk = 0;  // queues before offset first_try are known to be empty
+  auto ask = [&]() {
+    const int xq = (xcd + first_try) & 7;
+    if (t == 0 && first_try < 8) tk = atomicAdd(&sched[PIVOT ? AT_PIVOT_TICKETS + xq : xq * 16], 1);
+  };
+  auto publish = [&]() {
+    if (t == 0) {
+      while (first_try < 8 && tk >= at_queue_items(gm, (xcd + first_try) & 7)) {
+        ++first_try;
+        ask();
+      }
+      s_queue = first_try < 8 ? (xcd + first_try) & 7 : -1;
+      s_ticket = tk;
+    }
+  };
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // 0..7
   const int grp = wave >> 2;                                 // which row of the pair this wave works on
   const int tq = t & 255;                                    // thread index inside the row's four waves
@@ -753,23 +810,12 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   uint32_t* const blist = reinterpret_cast<uint32_t*>(lds + AT_RING * (AT_KBUF_BYTES + AT_VBUF_BYTES));
   const int c_ragged = (n % AT_BS) != 0 ? nb - 1 : -1;  // the only block whose K rows may run past the sequence
 
+  ask();
+  publish();
   for (;;) {
-    __syncthreads();  // previous item's LDS reads are done
-    if (t == 0) {
-      int found = -1, tk = 0;
-      for (int a = first_try; a < 8; ++a) {
-        const int xq = (xcd + a) & 7;
-        tk = atomicAdd(&sched[PIVOT ? AT_PIVOT_TICKETS + xq : xq * 16], 1);
-        if (tk < at_queue_items(gm, xq)) {
-          found = xq;
-          first_try = a;
-          break;
-        }
-      }
-      s_queue = found;
-      s_ticket = tk;
-    }
-    __syncthreads();
+    // the ticket (the first time the tables too) is written, the previous item's LDS reads are done; its stores of the
+    // output stay in flight, where a plain __syncthreads would wait for them
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int queue = __builtin_amdgcn_readfirstlane(s_queue);
     if (queue < 0) {
       if (!PIVOT && blockIdx.x == 0 && t == 0) {
@@ -781,14 +827,19 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     }
     const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
     int h_item, pair;
-    if (!at_item(gm, queue, ticket, h_item, pair)) continue;
-    const int slot = slots[h_item];
-    if (PIVOT ? slot == AT_NO_SLOT : (skip_slotted && slot != AT_NO_SLOT)) continue;  // the other launch's head
+    bool work = at_item(gm, queue, ticket, h_item, pair);
+    const int slot = __builtin_amdgcn_readfirstlane((int)slots[h_item]);
+    if (PIVOT ? slot == AT_NO_SLOT : (skip_slotted && slot != AT_NO_SLOT)) work = false;  // the other launch's head
     // the item's two (head, row): A for waves 0-3, B for waves 4-7
-    const bool by_heads = !PIVOT && pair_table[h_item >> 1] != 0;
+    const bool by_heads = !PIVOT && __builtin_amdgcn_readfirstlane((int)pair_table[h_item >> 1]) != 0;
     const int h_a = by_heads ? (h_item & ~1) : h_item, h_b = by_heads ? (h_item | 1) : h_item;
     const int r_a = by_heads ? 2 * pair + (h_item & 1) : 2 * pair, r_b = by_heads ? r_a : r_a + 1;
-    if (r_a >= nb) continue;  // (heads pairing, odd nb: the odd head's last item has no row)
+    if (!work || r_a >= nb) {  // (heads pairing, odd nb: the odd head's last item has no row)
+      ask();
+      __syncthreads();  // the ticket has been read
+      publish();
+      continue;
+    }
     const bool has_b = r_b < nb;
     const int h = grp ? h_b : h_a;  // this wave's head
     const int r = grp ? r_b : r_a;  // this wave's row
@@ -800,41 +851,32 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     const uint64_t* mrow_b = mask + ((int64_t)h_b * nb + (has_b ? r_b : r_a)) * nbw;
 
     // ---- the pair's block list: every column kept by either row, ascending, with membership flags ----
-    // All waves walk the (uniform) mask words and keep a running count; wave w compacts words w, w+8, ...
-    int n_blk = 0;
+    // Lane i of every wave holds mask word i of both rows (nb <= 4096: at most 64 words), so the masks are one load deep; the
+    // counts in front of a word are a scan over the lanes, and wave w compacts words w, w+8, ...  The first block's tiles and
+    // the queries are requested as soon as the words are there, the list is written while they are on their way.
+    int n_blk = 0, c_first = -1;
+    bool first_mine = false;
+    static_assert(AT_LIST_MAX <= 64 * SP_WAVE, "");
+    uint64_t w_a = 0ull, w_b = 0ull;  // this lane's words, cut off behind the rows' diagonals
+    uint32_t w_before;                // blocks in the words in front of this lane's
     {
-      const int wmax = (has_b ? r_b : r_a) >> 6;
-      const int lane = t & 63;
-      for (int wi = 0; wi <= wmax; ++wi) {
-        const uint64_t wa = at_trim(mrow_a[wi], wi, r_a);
-        const uint64_t wb = has_b ? at_trim(mrow_b[wi], wi, r_b) : 0ull;
-        const uint64_t wu = wa | wb;
-        if ((wi & 7) == wave && ((wu >> lane) & 1ull)) {
-          const int pos = n_blk + __builtin_popcountll(wu & ((1ull << lane) - 1ull));
-          blist[pos] = (uint32_t)(wi * 64 + lane) | (((wa >> lane) & 1ull) ? AT_IN_A : 0u) |
-                       (((wb >> lane) & 1ull) ? AT_IN_B : 0u);
-        }
-        n_blk += __builtin_popcountll(wu);
-      }
-      n_blk = __builtin_amdgcn_readfirstlane(n_blk);
-    }
-    __syncthreads();
-
-    // Q^T operands: the lane's two queries (one per 16-query tile), 4 channel steps of 8 channels each
-    bf16x8 qb[2][4];
-    {
-      AT_LANE_VIEW(tq);
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-        if (qrow > n - 1) qrow = n - 1;
-        const sp_bf16* src = q + (int64_t)h * sq_h + qrow * sq_n + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < (HALF ? 2 : 4); ++ks)
-          qb[qt][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
+      const int wi = t & 63, wl = wi < nbw ? wi : 0;
+      const uint64_t x_a = mrow_a[wl], x_b = mrow_b[wl];  // (both in flight before either is looked at)
+      if (wi <= (r_a >> 6)) w_a = at_trim(x_a, wi, r_a);
+      if (has_b && wi <= (r_b >> 6)) w_b = at_trim(x_b, wi, r_b);
+      const uint64_t wu = w_a | w_b;
+      const uint32_t own = (uint32_t)__builtin_popcountll(wu);
+      const uint32_t incl = at_lane_scan(own);
+      w_before = incl - own;
+      n_blk = __builtin_amdgcn_readlane((int)incl, 63);
+      const uint64_t some = __ballot(wu != 0ull);
+      if (some != 0ull) {
+        const int wf = __builtin_ctzll(some);
+        const int bit = __builtin_ctzll(at_lane_u64(wu, wf));
+        c_first = wf * 64 + bit;
+        first_mine = ((at_lane_u64(grp ? w_b : w_a, wf) >> bit) & 1ull) != 0ull;
       }
     }
-
     // FINE: the two fine mask rows of this wave's query tiles, and the keep bits (at_keep) of a block from them
     const uint64_t* frow[2] = {fine_mask, fine_mask};
     if constexpr (FINE) {
@@ -934,14 +976,42 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     uint32_t e_next = 0u, e_ahead = 0u;
     const uint32_t blist_addr = at_lds_addr(reinterpret_cast<const char*>(blist));
     if (n_blk > 0) {
-      const uint32_t e0 = entry(0);
-      e_next = entry(1);
-      c_cur = (int)(e0 & AT_COL_MASK);
-      mine = (e0 & my_flag) != 0u;
+      c_cur = c_first;
+      mine = first_mine;
       issue_k(c_cur, 0, 0);
       issue_k(c_cur, 1, 1);
       issue_v(c_cur, 0, 0);
       fine_issue(c_cur);
+    }
+    // Q^T operands: the lane's two queries (one per 16-query tile), 4 channel steps of 8 channels each
+    bf16x8 qb[2][4];
+    {
+      AT_LANE_VIEW(tq);
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt) {
+        int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
+        if (qrow > n - 1) qrow = n - 1;
+        const sp_bf16* src = q + (int64_t)h * sq_h + qrow * sq_n + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < (HALF ? 2 : 4); ++ks)
+          qb[qt][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
+      }
+    }
+
+    // (the list, see above)
+    {
+      const int lane = t & 63, wmax = (has_b ? r_b : r_a) >> 6;
+      for (int wi = wave; wi <= wmax; wi += 8) {
+        const uint64_t wa = at_lane_u64(w_a, wi), wb = at_lane_u64(w_b, wi), wu = wa | wb;
+        const int pos = __builtin_amdgcn_readlane((int)w_before, wi) + __builtin_popcountll(wu & ((1ull << lane) - 1ull));
+        if ((wu >> lane) & 1ull)
+          blist[pos] = (uint32_t)(wi * 64 + lane) | (((wa >> lane) & 1ull) ? AT_IN_A : 0u) |
+                       (((wb >> lane) & 1ull) ? AT_IN_B : 0u);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the list is complete; the tiles stay in flight
+    if (n_blk > 0) {
+      e_next = entry(1);
       kq_cur = fine_take(c_cur);
     }
 
@@ -1060,6 +1130,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
         AT_WAIT_VMCNT0();
         __syncthreads();
         finished = true;
+        if (wave == 0) ask();
         vb = vring + ((2 * b + 3) & 3) * AT_VBUF_BYTES;
         at_block_addr(ad, kb, vb, vb, koff, voff);
       }
@@ -1072,6 +1143,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     if (!finished) {
       AT_WAIT_VMCNT0();
       __syncthreads();
+      if (wave == 0) ask();
     }
     at_settle_o(o);
     // every lane of a query's group holds the whole row sum (all rows of the ones . P tile are equal)
@@ -1079,7 +1151,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     AT_LANE_VIEW(tq);
 
     // pivot heads: keep the softmax statistics of every query row for the block-average pass
-    if (row_ok && rowstat != nullptr && decision != nullptr && decision[h] == SP_DEC_DENSE && g == 0) {
+    if (row_ok && rowstat != nullptr && ((dense_heads[h >> 5] >> (h & 31)) & 1u) != 0u && g == 0) {
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
         const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
@@ -1088,24 +1160,30 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     }
 
     // ---- epilogue: normalise and store straight from the accumulators.  A lane holds 4 consecutive channels of its
-    // query per channel tile: 8-byte stores, 32 contiguous bytes per query row and instruction; the four channel tiles
-    // that share a 128-byte line follow each other, and the write-back L2 merges them.  No LDS, no barrier: the
-    // workgroup goes on to its next item while the stores drain. ----
+    // query per channel tile; lane groups 2i and 2i + 1 trade halves of two neighbouring tiles, so that a store is 16 bytes a
+    // lane and 64 contiguous bytes per query row.  No LDS, no barrier: the workgroup goes on to its next item while the stores
+    // drain. ----
     if (row_ok) {
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
         const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-        if (qrow < n) {
-          const float inv_l = 1.0f / l_tot[qt];
-          sp_bf16* dst = out + (qrow * hq + h) * AT_D + 4 * g;
+        const float inv_l = 1.0f / l_tot[qt];
+        sp_bf16* dst = out + (qrow * hq + h) * AT_D + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
-          for (int dt = 0; dt < (HALF ? 4 : 8); ++dt)
-            *reinterpret_cast<uint2*>(dst + dt * 16) =
-                make_uint2(at_pack2(o[dt][qt][0] * inv_l, o[dt][qt][1] * inv_l),
-                           at_pack2(o[dt][qt][2] * inv_l, o[dt][qt][3] * inv_l));
+        for (int dt = 0; dt < (HALF ? 4 : 8); dt += 2) {
+          uint32_t w[2][2];  // [tile dt, dt + 1][channels 4g, 4g + 1 | 4g + 2, 4g + 3]
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            w[u][0] = at_pack2(o[dt + u][qt][0] * inv_l, o[dt + u][qt][1] * inv_l);
+            w[u][1] = at_pack2(o[dt + u][qt][2] * inv_l, o[dt + u][qt][3] * inv_l);
+          }
+          const auto first = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+          const auto second = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+          if (qrow < n) *reinterpret_cast<uint4*>(dst + dt * 16) = make_uint4(first[0], second[0], first[1], second[1]);
         }
       }
     }
+    publish();
   }
 }
 
