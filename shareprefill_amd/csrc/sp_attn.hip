@@ -79,19 +79,27 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* 
 // two adjacent heads (2i, 2i+1) of a kv group by sp_attn_schedule_kernel, whichever gives the smaller unions:
 //   rows  : item (h, p) = rows 2p and 2p+1 of head h (verticals are shared, slashes shift by one block);
 //   heads : item (h, p) = row 2p + (h & 1) of heads 2i and 2i+1 (heads that share a pattern keep the same columns).
-// Items are grouped in gangs of AT_GANG consecutive pairs of ONE head (all of a head's pairs when it has fewer: a short
-// prompt's queues then hold no padding tickets, each of which would cost a workgroup an atomic and two barriers).  Gangs are dealt statically to the 8 XCDs (queue x = gang position % 8; workgroup b serves queue b % 8
+// Items are grouped in gangs of at most AT_GANG consecutive pairs of ONE head, all gangs of equal size (a head's pairs in even
+// shares: gangs of 32 left 24 padding tickets per head at 10007 tokens, each an atomic and two barriers for some workgroup).
+// Gangs are dealt statically to the 8 XCDs (queue x = gang position % 8; workgroup b serves queue b % 8
 // first -- workgroups are placed on XCDs round-robin), so the 32 workgroups of an XCD start a gang together at
 // column 0 and sweep the key blocks nearly in lock-step: every K / V^T tile one of them pulls into the XCD's
 // L2 is hit by the others.  The head order inside a kv group is rotated from chunk to chunk so that every
 // queue sees every head, heavy (late) rows go first, and a workgroup whose queue is empty steals from the
 // other queues.  Pulling is by atomic tickets only: nobody ever waits for anybody, and every workgroup leaves
 // once all eight queues are exhausted.
-// Up to 32K tokens a launch has few gangs per workgroup, the heaviest of them a large part of a workgroup's whole
+// Between 8K and 32K tokens a launch has few gangs per workgroup, the heaviest of them a large part of a workgroup's whole
 // share, and every head's K / V^T fit the memory-side cache together, so the order above (one kv head after the
-// other) only makes the last kv head's heavy rows start late: there sp_attn_schedule_kernel ranks the gangs by the
-// number of blocks their items visit and the queues are dealt from that ranking, heaviest first.
+// other) only makes the last kv head's heavy rows start late: there sp_attn_schedule_kernel writes down the number of blocks
+// every gang's items visit, every workgroup ranks the gangs by it, and the queues are dealt from that ranking, heaviest
+// first.  Layers in us: ranked / dealt by rows, the last rows of all heads first (which needs no weights): 10007 tokens 28 heads
+// 259 / 258, 13000 371 / 369, 16384 (two layers, heads of unlike weight) 1827 / 1966, 24000 1328 / 1392, 32768 2629 / 2839.  At
+// 8000 tokens the order above 245, ranked 249; at 65001 no difference.  Gangs of 32 / 16 pairs: 10007 260 / 259, 16384 1853 / 1827,
+// 24000 1329 / 1334, 32768 2629 / 2642.
 #define AT_GANG 32
+#define AT_RANK_MIN_NB 64  // (ranked: more blocks than that)
+#define AT_RANK_MAX_NB 256
+#define AT_HALF_GANG_NB 128  // gangs of 16 up to here
 // The 1 KiB scheduler area (int indices): 0..127 eight queue tickets (one per 64 bytes), 128..191 the pivot slot of
 // every head (one byte each, AT_NO_SLOT = its block sums are not kept), 192..195 {shader cycles, 100 MHz ticks} of
 // workgroup 0, 196 the number of pivot slots in use, 200..231 the pairing of every two adjacent heads (one byte each,
@@ -100,19 +108,21 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* 
 #define AT_SLOT_TABLE 128
 #define AT_CLOCK_SLOT 192
 #define AT_NPIV_SLOT 196
-#define AT_ORDER_SLOT 197  // 1: the gang positions of this call go through the order table (sp_attn_schedule_kernel)
+#define AT_ROWS_SLOT 197  // 1: the caller asked for pairing by rows: no analysis, no ranking
 #define AT_PAIR_TABLE 200
 #define AT_PIVOT_TICKETS 232  // 232..239: the eight queue tickets of the pivot heads' own launch
 #define AT_NO_SLOT 255
-// Behind the 1 KiB of slots: the order table, AT_ORDER_MAX gang positions (uint16), see sp_attn_schedule_kernel.
-#define AT_ORDER_MAX 1024
-#define AT_SCHED_BYTES (1024 + AT_ORDER_MAX * 2)
+// Behind the 1 KiB of slots: the weights of up to AT_RANK_MAX gangs, see sp_attn_schedule_kernel.
+#define AT_RANK_MAX 1024  // AT_MAX_HEADS of at most four gangs
+#define AT_SCHED_BYTES (1024 + AT_RANK_MAX * 4)
 #define AT_MAX_HEADS 256
+static_assert(AT_MAX_HEADS * 4 <= AT_RANK_MAX && AT_RANK_MAX_NB <= 8 * AT_GANG && AT_HALF_GANG_NB <= 4 * AT_GANG, "");
 #define AT_FWD_THREADS 512
 
 struct AtGeom {
   int group, n_pairs, gang, n_chunks, n_gangs;
-  const uint16_t* order;  // gang position -> gang (nullptr: identity)
+  bool ranked;            // the gang positions go through `order`: heaviest gang first
+  const uint16_t* order;  // gang position -> head * n_chunks + chunk
 };
 
 __device__ static inline int at_queue_items(const AtGeom& gm, int xq) {
@@ -120,8 +130,14 @@ __device__ static inline int at_queue_items(const AtGeom& gm, int xq) {
   return gangs * gm.gang;
 }
 
-// gang position (before any reordering) -> head and chunk of row pairs, 0 = the last (heaviest) rows
+// gang position -> head and chunk of row pairs, 0 = the last (heaviest) rows
 __device__ static inline void at_gang_of(const AtGeom& gm, int pos, int& h, int& j) {
+  if (gm.ranked) {
+    const int gang = gm.order[pos];
+    h = gang / gm.n_chunks;
+    j = gang - h * gm.n_chunks;
+    return;
+  }
   const int i = pos % gm.group;
   const int rest = pos / gm.group;
   j = rest % gm.n_chunks;
@@ -131,20 +147,21 @@ __device__ static inline void at_gang_of(const AtGeom& gm, int pos, int& h, int&
 
 // ticket of queue xq -> (head, row pair); false for the padding slots of the last chunk
 __device__ static inline bool at_item(const AtGeom& gm, int xq, int ticket, int& h, int& pair) {
-  int pos = (ticket / gm.gang) * 8 + xq;  // gang position
+  const int pos = (ticket / gm.gang) * 8 + xq;  // gang position
   const int slot = ticket % gm.gang;
-  if (gm.order != nullptr) pos = gm.order[pos];
   int j;
   at_gang_of(gm, pos, h, j);
   pair = gm.n_pairs - 1 - (j * gm.gang + slot);
   return pair >= 0;
 }
 
-__device__ static inline void at_geometry(AtGeom& gm, int hq, int hkv, int nb) {
+__device__ static inline void at_geometry(AtGeom& gm, int hq, int hkv, int nb, int pair_rows) {
   gm.group = hq / hkv;
   gm.n_pairs = (nb + 1) / 2;
-  gm.gang = gm.n_pairs < AT_GANG ? gm.n_pairs : AT_GANG;
-  gm.n_chunks = (gm.n_pairs + gm.gang - 1) / gm.gang;
+  gm.ranked = nb > AT_RANK_MIN_NB && nb <= AT_RANK_MAX_NB && !pair_rows;
+  const int most = gm.ranked && nb <= AT_HALF_GANG_NB ? AT_GANG / 2 : AT_GANG;
+  gm.n_chunks = (gm.n_pairs + most - 1) / most;
+  gm.gang = (gm.n_pairs + gm.n_chunks - 1) / gm.n_chunks;  // (even shares: few padding tickets)
   gm.n_gangs = hq * gm.n_chunks;
   gm.order = nullptr;
 }
@@ -736,7 +753,8 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   extern __shared__ __attribute__((aligned(1024))) char lds[];  // K ring (4 x 16 KiB) | V^T ring (4 x 16 KiB)
   __shared__ int s_queue, s_ticket;
   // the scheduler's tables, copied once: read from memory they are two more dependent loads in front of every item
-  __shared__ uint32_t dense_heads[AT_MAX_HEADS / 32], s_order[AT_ORDER_MAX / 2], s_slots[AT_MAX_HEADS / 4], s_pairs[AT_MAX_HEADS / 8];
+  __shared__ uint32_t dense_heads[AT_MAX_HEADS / 32], s_slots[AT_MAX_HEADS / 4], s_pairs[AT_MAX_HEADS / 8];
+  __shared__ uint16_t s_order[AT_RANK_MAX];
   constexpr int MODE = (PIVOT ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
   if (PIVOT && sched[AT_NPIV_SLOT] == 0) return;  // no pivot in this layer
   const uint8_t* const slots = reinterpret_cast<const uint8_t*>(s_slots);
@@ -744,13 +762,26 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
 
   const long long clk0 = clock64(), tick0 = wall_clock64();  // see sp_attn_last_launch_clocks
   AtGeom gm;
-  at_geometry(gm, hq, hkv, nb);
-  const bool ordered = sched[AT_ORDER_SLOT] != 0;
-  gm.order = ordered ? reinterpret_cast<const uint16_t*>(s_order) : nullptr;
+  at_geometry(gm, hq, hkv, nb, sched[AT_ROWS_SLOT]);
+  gm.order = s_order;
   const int xcd = blockIdx.x & 7;
   const int t = threadIdx.x;
-  static_assert(AT_ORDER_MAX / 2 <= AT_FWD_THREADS && AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8 <= AT_FWD_THREADS, "");
-  if (ordered && t < (gm.n_gangs + 1) / 2) s_order[t] = (uint32_t)sched[256 + t];
+  static_assert(AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8 <= AT_FWD_THREADS, "");
+  if (gm.ranked) {  // every workgroup ranks the gangs for itself (ties: ascending number)
+    uint32_t* const weight = reinterpret_cast<uint32_t*>(lds);  // (the rings are not in use yet)
+    for (int i = t; i < ((gm.n_gangs + 3) & ~3); i += AT_FWD_THREADS) weight[i] = i < gm.n_gangs ? (uint32_t)sched[256 + i] : 0u;
+    __syncthreads();
+    for (int i = t; i < gm.n_gangs; i += AT_FWD_THREADS) {
+      const uint32_t wi = weight[i];
+      int rank = 0;
+      for (int o = 0; o < gm.n_gangs; o += 4) {
+        const uint4 wo = *reinterpret_cast<const uint4*>(weight + o);
+        rank += (wo.x > wi || (wo.x == wi && o < i)) + (wo.y > wi || (wo.y == wi && o + 1 < i)) +
+                (wo.z > wi || (wo.z == wi && o + 2 < i)) + (wo.w > wi || (wo.w == wi && o + 3 < i));
+      }
+      s_order[rank] = (uint16_t)i;
+    }
+  }
   if (t < AT_MAX_HEADS / 4)
     s_slots[t] = (uint32_t)sched[AT_SLOT_TABLE + t];
   else if (t < AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8)
@@ -1196,16 +1227,13 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
 //               rows : |row 2p  |  row 2p+1| of each head,      heads : |row r of head 2i  |  row r of head 2i+1|:
 //             by heads when that union is strictly smaller and the two heads may share an item (same kv head, neither
 //             runs in the pivot launch);
-//   ORDER   : ranks the gangs by the work of their items -- the blocks the item's two rows visit together, plus a few
-//             blocks' worth of fixed time per item -- and writes the gang positions in descending order (ties: ascending
-//             position) into the order table.
+//   weights : the work of every gang that is ranked -- the blocks its items' two rows visit together, plus a few blocks' worth of
+//             fixed time per item.
 // Integer sums throughout, so nothing depends on the order of anything.
-// Pure latency: a launch, and chains of loads from L2.  As three launches, a thread per gang walking the gang's items one
-// after the other, it took 33 us at 10007 tokens (28 heads) and 49 at 32768 (32 heads); now one workgroup does all of it
-// for a launch that is ranked (a wave a head pair, a lane an item), and a workgroup a head pair when there is no ranking
-// (the masks of long prompts are too much for one): 27 us off a layer of 10007 tokens.
+// Pure latency: a launch, and chains of loads from L2; a workgroup a head pair, a thread a row pair, then a lane an item.  With
+// one workgroup for all of it, the ranking included, the launch took 8 us at 10007 tokens (28 heads) and 20 at 32768 (32 heads);
+// now 5 and 6, and the ranking (n^2 comparisons of up to 256 gangs by 512 threads) under 1 us of every attention workgroup.
 #define AT_ITEM_FIXED 6  // an item's fixed time (ticket, block list, first tiles, epilogue) in units of one block visit
-#define AT_ORDER_THREADS 1024
 #define AT_PAIRING_THREADS 256
 
 __device__ static inline void at_union_sizes(const uint64_t* __restrict__ m0, const uint64_t* __restrict__ m1, int nb,
@@ -1228,18 +1256,15 @@ __device__ static inline uint32_t at_lane_sum(uint32_t v) {  // over aligned gro
   return v;
 }
 
-// grid: ORDER 1; otherwise a workgroup per head pair, or one with pair_rows (no pairing to choose)
-template <bool ORDER>
-__global__ __launch_bounds__(ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
+// grid: a workgroup per head pair, or one with pair_rows (nothing to choose or to rank)
+__global__ __launch_bounds__(AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
     int* __restrict__ sched, const uint64_t* __restrict__ mask, const int32_t* __restrict__ decision, int hq, int hkv,
     int nb, int nbw, int max_pivots, int pair_rows) {
-  constexpr int THREADS = ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS, WAVES = THREADS / SP_WAVE;
+  constexpr int THREADS = AT_PAIRING_THREADS, WAVES = THREADS / SP_WAVE;
   static_assert(AT_MAX_HEADS <= AT_PAIRING_THREADS && AT_MAX_HEADS % SP_WAVE == 0, "");
   __shared__ uint32_t dense_cnt[AT_MAX_HEADS / SP_WAVE];
   __shared__ uint8_t slot_s[AT_MAX_HEADS];
-  __shared__ uint8_t pair_s[AT_MAX_HEADS / 2];
   __shared__ uint32_t red[2][WAVES];
-  __shared__ uint32_t weight[ORDER ? AT_ORDER_MAX : 1];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int n_head_pairs = (hq + 1) / 2, group = hq / hkv;
   uint8_t* const table = reinterpret_cast<uint8_t*>(sched + AT_PAIR_TABLE);
@@ -1265,7 +1290,7 @@ __global__ __launch_bounds__(ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS) void
     if (t < 8) sched[AT_PIVOT_TICKETS + t] = 0;
     if (t == 0) {
       sched[AT_NPIV_SLOT] = total < max_pivots ? total : max_pivots;
-      sched[AT_ORDER_SLOT] = ORDER ? 1 : 0;
+      sched[AT_ROWS_SLOT] = pair_rows;
     }
   }
   __syncthreads();
@@ -1279,38 +1304,31 @@ __global__ __launch_bounds__(ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS) void
     for (int i = t; i < n_head_pairs; i += THREADS) table[i] = 0;
     return;
   }
-  for (int i = ORDER ? wave : (int)blockIdx.x; i < n_head_pairs; i += ORDER ? WAVES : (int)gridDim.x) {
-    uint32_t by_rows = 0, by_heads = 0;
-    if (eligible(i)) {
-      const uint64_t* m0 = mask + (int64_t)(2 * i) * nb * nbw;
-      at_union_sizes(m0, m0 + (int64_t)nb * nbw, nb, nbw, ORDER ? lane : t, ORDER ? SP_WAVE : THREADS, by_rows, by_heads);
-      by_rows = at_lane_sum<SP_WAVE>(by_rows);
-      by_heads = at_lane_sum<SP_WAVE>(by_heads);
-      if (!ORDER) {  // (uniform: the workgroup has one head pair)
-        if (lane == 0) red[0][wave] = by_rows, red[1][wave] = by_heads;
-        __syncthreads();
-        by_rows = by_heads = 0;
-        for (int w = 0; w < WAVES; ++w) by_rows += red[0][w], by_heads += red[1][w];
-      }
-    }
-    if (ORDER ? lane == 0 : t == 0) {
-      table[i] = by_heads < by_rows ? 1 : 0;
-      pair_s[i] = by_heads < by_rows ? 1 : 0;
-    }
+  const int i = blockIdx.x;  // head pair
+  uint32_t by_rows = 0, by_heads = 0;
+  if (eligible(i)) {  // (uniform)
+    const uint64_t* m0 = mask + (int64_t)(2 * i) * nb * nbw;
+    at_union_sizes(m0, m0 + (int64_t)nb * nbw, nb, nbw, t, THREADS, by_rows, by_heads);
+    by_rows = at_lane_sum<SP_WAVE>(by_rows);
+    by_heads = at_lane_sum<SP_WAVE>(by_heads);
+    if (lane == 0) red[0][wave] = by_rows, red[1][wave] = by_heads;
+    __syncthreads();
+    by_rows = by_heads = 0;
+    for (int w = 0; w < WAVES; ++w) by_rows += red[0][w], by_heads += red[1][w];
   }
-  if constexpr (!ORDER) return;
+  const bool heads = by_heads < by_rows;
+  if (t == 0) table[i] = heads ? 1 : 0;
 
-  __syncthreads();
   AtGeom gm;
-  at_geometry(gm, hq, hkv, nb);
+  at_geometry(gm, hq, hkv, nb, pair_rows);
+  if (!gm.ranked) return;
   static_assert(AT_GANG <= 32, "");  // a half-wave per gang, a lane per item
-  for (int pos = t >> 5; pos < gm.n_gangs; pos += THREADS / 32) {
-    int h, j;
-    at_gang_of(gm, pos, h, j);
-    const bool by_heads = pair_s[h >> 1] != 0;
-    const int h_a = by_heads ? (h & ~1) : h, h_b = by_heads ? (h | 1) : h;
+  const int gangs = (2 * i + 1 < hq ? 2 : 1) * gm.n_chunks;
+  for (int e = t >> 5; e < gangs; e += THREADS / 32) {
+    const int h = 2 * i + e / gm.n_chunks, j = e % gm.n_chunks;
+    const int h_a = heads ? 2 * i : h, h_b = heads ? 2 * i + 1 : h;
     const int slot = t & 31, pair = gm.n_pairs - 1 - (j * gm.gang + slot);
-    const int r_a = by_heads ? 2 * pair + (h & 1) : 2 * pair, r_b = by_heads ? r_a : r_a + 1;
+    const int r_a = heads ? 2 * pair + (h & 1) : 2 * pair, r_b = heads ? r_a : r_a + 1;
     uint32_t cnt = 0;
     if (slot < gm.gang && pair >= 0 && r_a < nb) {
       const bool has_b = r_b < nb;
@@ -1322,19 +1340,7 @@ __global__ __launch_bounds__(ORDER ? AT_ORDER_THREADS : AT_PAIRING_THREADS) void
         cnt += __builtin_popcountll(at_trim(ma[wi], wi, r_a) | (has_b ? at_trim(mb[wi], wi, r_b) : 0ull));
     }
     cnt = at_lane_sum<32>(cnt);
-    if (slot == 0) weight[pos] = cnt;
-  }
-  __syncthreads();
-  uint16_t* order = reinterpret_cast<uint16_t*>(sched + 256);
-  for (int pos = t; pos < gm.n_gangs; pos += THREADS) {
-    const uint32_t wp = weight[pos];
-    int rank = 0;
-#pragma unroll 8
-    for (int o = 0; o < gm.n_gangs; ++o) {
-      const uint32_t wo = weight[o];
-      rank += (wo > wp) || (wo == wp && o < pos);
-    }
-    order[rank] = (uint16_t)pos;
+    if (slot == 0) sched[256 + h * gm.n_chunks + j] = (int)cnt;
   }
 }
 
@@ -1742,19 +1748,9 @@ extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const
   }
   float* pivot_u = reinterpret_cast<float*>(ws + base_aligned);
   {
-    // few gangs per workgroup and every head's K / V^T within the memory-side cache: deal the gangs heaviest first
-    // (measured on dense masks: +6 % at 16K tokens, +4 % at 32K; at 8K it makes no difference)
-    const int64_t n_pairs = (nb + 1) / 2;
-    const int64_t gang = n_pairs < AT_GANG ? n_pairs : AT_GANG;
-    const int64_t n_gangs = hq * sp_ceil_div(n_pairs, gang);
     const int pair_rows = (flags & SP_ATTN_PAIR_ROWS) ? 1 : 0;
-    if (!pair_rows && nb > 64 && nb <= 256 && n_gangs <= AT_ORDER_MAX)
-      hipLaunchKernelGGL(sp_attn_schedule_kernel<true>, dim3(1), dim3(AT_ORDER_THREADS), 0, s, counter, mask, decision,
-                         (int)hq, (int)hkv, (int)nb, (int)((nb + 63) / 64), max_pivots, pair_rows);
-    else
-      hipLaunchKernelGGL(sp_attn_schedule_kernel<false>, dim3(pair_rows ? 1 : (unsigned)((hq + 1) / 2)),
-                         dim3(AT_PAIRING_THREADS), 0, s, counter, mask, decision, (int)hq, (int)hkv, (int)nb,
-                         (int)((nb + 63) / 64), max_pivots, pair_rows);
+    hipLaunchKernelGGL(sp_attn_schedule_kernel, dim3(pair_rows ? 1 : (unsigned)((hq + 1) / 2)), dim3(AT_PAIRING_THREADS), 0, s,
+                       counter, mask, decision, (int)hq, (int)hkv, (int)nb, (int)((nb + 63) / 64), max_pivots, pair_rows);
     SP_LAUNCH_CHECK();
   }
   const size_t lds_bytes = AT_LDS_BYTES;
