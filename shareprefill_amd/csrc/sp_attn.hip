@@ -112,9 +112,9 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* 
 #define AT_PAIR_TABLE 200
 #define AT_PIVOT_TICKETS 232  // 232..239: the eight queue tickets of the pivot heads' own launch
 #define AT_NO_SLOT 255
-// Behind the 1 KiB of slots: the weights of up to AT_RANK_MAX gangs, see sp_attn_schedule_kernel.
+// Behind the 1 KiB of slots: the weights (uint16) of up to AT_RANK_MAX gangs, see sp_attn_schedule_kernel.
 #define AT_RANK_MAX 1024  // AT_MAX_HEADS of at most four gangs
-#define AT_SCHED_BYTES (1024 + AT_RANK_MAX * 4)
+#define AT_SCHED_BYTES (1024 + AT_RANK_MAX * 2)
 #define AT_MAX_HEADS 256
 static_assert(AT_MAX_HEADS * 4 <= AT_RANK_MAX && AT_RANK_MAX_NB <= 8 * AT_GANG && AT_HALF_GANG_NB <= 4 * AT_GANG, "");
 #define AT_FWD_THREADS 512
@@ -769,7 +769,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   static_assert(AT_MAX_HEADS / 4 + AT_MAX_HEADS / 8 <= AT_FWD_THREADS, "");
   if (gm.ranked) {  // every workgroup ranks the gangs for itself (ties: ascending number)
     uint32_t* const weight = reinterpret_cast<uint32_t*>(lds);  // (the rings are not in use yet)
-    for (int i = t; i < ((gm.n_gangs + 3) & ~3); i += AT_FWD_THREADS) weight[i] = i < gm.n_gangs ? (uint32_t)sched[256 + i] : 0u;
+    for (int i = t; i < ((gm.n_gangs + 3) & ~3); i += AT_FWD_THREADS) weight[i] = i < gm.n_gangs ? reinterpret_cast<const uint16_t*>(sched + 256)[i] : 0u;
     __syncthreads();
     for (int i = t; i < gm.n_gangs; i += AT_FWD_THREADS) {
       const uint32_t wi = weight[i];
@@ -1322,7 +1322,7 @@ __global__ __launch_bounds__(AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
   AtGeom gm;
   at_geometry(gm, hq, hkv, nb, pair_rows);
   if (!gm.ranked) return;
-  static_assert(AT_GANG <= 32, "");  // a half-wave per gang, a lane per item
+  static_assert(AT_GANG <= 32 && AT_GANG * (AT_RANK_MAX_NB + AT_ITEM_FIXED) < 65536, "");  // a half-wave per gang, a lane per item
   const int gangs = (2 * i + 1 < hq ? 2 : 1) * gm.n_chunks;
   for (int e = t >> 5; e < gangs; e += THREADS / 32) {
     const int h = 2 * i + e / gm.n_chunks, j = e % gm.n_chunks;
@@ -1340,7 +1340,7 @@ __global__ __launch_bounds__(AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
         cnt += __builtin_popcountll(at_trim(ma[wi], wi, r_a) | (has_b ? at_trim(mb[wi], wi, r_b) : 0ull));
     }
     cnt = at_lane_sum<32>(cnt);
-    if (slot == 0) sched[256 + h * gm.n_chunks + j] = (int)cnt;
+    if (slot == 0) reinterpret_cast<uint16_t*>(sched + 256)[h * gm.n_chunks + j] = (uint16_t)cnt;
   }
 }
 
