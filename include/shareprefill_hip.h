@@ -203,6 +203,16 @@ int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int32_t hq, in
                          float similarity_threshold, double fallback_threshold, float queryaware_threshold,
                          void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
                          float* avg_attn, sp_stream_t stream);
+/* The same with sp_attn_repack_v_bf16(v, n, hkv, d, v_stride_n, v_stride_h, bs, vt, vt_bytes) beside the selection: nothing of the
+ * repack depends on it, and it fits under the launch of the budgets, which leaves most of the chip idle. */
+int sp_select_layer_repack_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                                int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
+                                uint32_t flags, const sp_cluster_state* state /* host */, const int32_t* head_cluster,
+                                int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
+                                float similarity_threshold, double fallback_threshold, float queryaware_threshold,
+                                void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
+                                float* avg_attn, const void* v, int64_t v_stride_n, int64_t v_stride_h, void* vt,
+                                size_t vt_bytes, sp_stream_t stream);
 
 /* ---- GQA causal block-sparse flash attention ------------------------------------------------
  * Replaces triton_block_wise_prefill_attention / block_wise_prefill_attention_kernel /

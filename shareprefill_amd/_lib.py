@@ -67,6 +67,8 @@ SIGNATURES = {
     "sp_select_layer_scratch_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32, _P]),
     "sp_select_layer_bf16": (_I32, [_P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I32, _U32, _ST, _P, _I32, _I32,
                                     _I32, _D, _F, _D, _F, _P, _SZ, _P, _P, _P, _P, _P]),
+    "sp_select_layer_repack_bf16": (_I32, [_P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I32, _U32, _ST, _P, _I32,
+                                           _I32, _I32, _D, _F, _D, _F, _P, _SZ, _P, _P, _P, _P, _P, _I64, _I64, _P, _SZ, _P]),
     "sp_cover_select_workspace_bytes": (_SZ, [_I32]),
     "sp_cover_select_global": (_I32, [_P, _P, _I32, _I32, _F, _P, _P, _SZ, _P]),
     "sp_attn_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32]),

@@ -181,9 +181,11 @@ class AttentionSharing:
     def plan_layer(self, q: torch.Tensor, k: torch.Tensor, layer_idx: int, block_size: int, min_budget: int,
                    max_budget: int, pattern_threshold: float = 0.9, similarity_threshold: float = 0.5,
                    fallback_threshold: float = 0.9, queryaware_threshold: float = 0.1,
-                   scale_dim: Optional[int] = None, avg_attn: Optional[torch.Tensor] = None) -> LayerPlan:
+                   scale_dim: Optional[int] = None, avg_attn: Optional[torch.Tensor] = None,
+                   repack: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> LayerPlan:
         """q [Hq, N, D], k [Hkv, N, D] bf16 views; budgets in blocks.  Enqueues the whole selection.
         avg_attn: contiguous fp32 [Hq, nb, nb] that is cleared on the way.
+        repack: (v [Hkv, N, D], attention workspace buffer), ops.repack_v of which is done on the way.
         scale_dim: the model's head_dim when q / k have been zero-padded to D (the scores then scale by
         1/sqrt(scale_dim), attention_sharing.py:127 of the reference)."""
         hq, n, d = q.shape
@@ -198,7 +200,8 @@ class AttentionSharing:
         qa_probs = self._qa_scratch(hq, nb, dev)
         mask, (decision, nv, ns, nv_f, ns_f), floats = ops.select_layer(
             state, hc, layer_idx, q, k, block_size, flags, minb, maxb, pattern_threshold, similarity_threshold,
-            fallback_threshold, queryaware_threshold, qa_probs, avg_attn=avg_attn, keep_floats=self.keep_debug)
+            fallback_threshold, queryaware_threshold, qa_probs, avg_attn=avg_attn, keep_floats=self.keep_debug,
+            repack=repack)
         plan = LayerPlan(layer_idx, nb, mask, decision, nv, ns, nv_f, ns_f)
         plan.max_pivots = self.max_pivots(layer_idx, hq)
         if self.keep_debug:

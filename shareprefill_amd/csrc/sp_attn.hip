@@ -14,7 +14,7 @@
 // K and V^T sub-tiles (64 keys) are staged through LDS by direct global->LDS loads, XOR-swizzled; every wave runs a
 // software pipeline over 32-key half-tiles in which the softmax of one half-tile is issued between the MFMAs of
 // its neighbours (see "the software pipeline of one wave" below).
-#include "sp_common.h"
+#include "sp_repack.h"
 
 #include <type_traits>
 
@@ -28,47 +28,10 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #define AT_PITCH 136  // bf16 elements per LDS row
 #define AT_THREADS 256
 
-// position p (0..31) inside a group of 32 keys of the repacked V^T row holds key offset at_perm32(p):
-// [0-3, 16-19, 4-7, 20-23, 8-11, 24-27, 12-15, 28-31]: lane group g of a wave owns rows 4g .. 4g+3 of both 16x16
-// S^T accumulators of a half-tile, and its P^T operand is key slots 8g .. 8g+7
-__host__ __device__ static inline int at_perm32(int p) { return 16 * ((p >> 2) & 1) + 4 * (p >> 3) + (p & 3); }
-
 // ---- V repack: v[n][hkv][d] -> vt[hkv][nb][d][128 key slots] ------------------------------------------
-__global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(const sp_bf16* __restrict__ v,
-                                                                 sp_bf16* __restrict__ vt, int64_t n, int64_t sv_n,
-                                                                 int64_t sv_h, int64_t nb) {
-  __shared__ sp_bf16 tile[AT_BS * AT_PITCH];
-  const int64_t blk = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int t = threadIdx.x;
-  const int chunk = t & 15;
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int row = it * 16 + (t >> 4);
-    const int64_t key = blk * AT_BS + row;
-    uint4 val = make_uint4(0, 0, 0, 0);
-    if (key < n) val = *reinterpret_cast<const uint4*>(v + (int64_t)kvh * sv_h + key * sv_n + chunk * 8);
-    *reinterpret_cast<uint4*>(&tile[row * AT_PITCH + chunk * 8]) = val;
-  }
-  __syncthreads();
-  sp_bf16* dst = vt + (((int64_t)kvh * nb + blk) * AT_D) * AT_BS;
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int dd = it * 16 + (t >> 4);  // output row = channel
-    const int p0 = chunk * 8;           // 8 consecutive key slots
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int slot = p0 + j;
-      const int key = (slot & ~31) + at_perm32(slot & 31);
-      const uint32_t e = tile[key * AT_PITCH + dd];
-      if (j & 1)
-        w[j >> 1] |= e << 16;
-      else
-        w[j >> 1] = e;
-    }
-    *reinterpret_cast<uint4*>(dst + (int64_t)dd * AT_BS + p0) = make_uint4(w[0], w[1], w[2], w[3]);
-  }
+__global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(RepackArgs a) {
+  __shared__ __attribute__((aligned(16))) sp_bf16 tile[RP_BS * RP_PITCH];
+  repack_v_tile<AT_THREADS>(a, blockIdx.x, blockIdx.y, tile);
 }
 
 // ---- work distribution ----------------------------------------------------------------------------------
@@ -1664,18 +1627,11 @@ extern "C" int sp_attn_last_launch_pairing(const void* workspace, int64_t n, int
 extern "C" int sp_attn_repack_v_bf16(const void* v, int64_t n, int32_t hkv, int32_t d, int64_t v_stride_n,
                                      int64_t v_stride_h, int32_t bs, void* workspace, size_t workspace_bytes,
                                      sp_stream_t stream) {
-  SP_REQUIRE(v && workspace, SP_ERR_INVALID_ARGUMENT, "sp_attn_repack_v_bf16: null pointer");
-  SP_REQUIRE(n > 0 && hkv > 0, SP_ERR_INVALID_ARGUMENT, "sp_attn_repack_v_bf16: bad shape");
-  SP_REQUIRE(at_block_size_ok(bs) && d == AT_D, SP_ERR_UNSUPPORTED,
-             "sp_attn_repack_v_bf16: block size %d / head_dim %d unsupported (16, 32, 64 or 128 / 128)", bs, d);
-  SP_REQUIRE(v_stride_n % 8 == 0 && v_stride_h % 8 == 0 && ((uintptr_t)v % 16) == 0 &&
-                 ((uintptr_t)workspace % 16) == 0,
-             SP_ERR_UNSUPPORTED, "sp_attn_repack_v_bf16: v must be 16-byte aligned, strides multiple of 8");
-  SP_REQUIRE(workspace_bytes >= at_vt_bytes(n, hkv, d, bs), SP_ERR_WORKSPACE,
-             "sp_attn_repack_v_bf16: workspace too small");
-  const int64_t nb = sp_ceil_div(n, AT_BS);
-  hipLaunchKernelGGL(sp_repack_v_kernel, dim3((unsigned)nb, hkv), dim3(AT_THREADS), 0, (hipStream_t)stream,
-                     (const sp_bf16*)v, (sp_bf16*)workspace, n, v_stride_n, v_stride_h, nb);
+  RepackArgs a;
+  const int rc = repack_args(&a, "sp_attn_repack_v_bf16", v, n, hkv, d, v_stride_n, v_stride_h, bs, workspace, workspace_bytes);
+  if (rc != SP_OK) return rc;
+  SP_REQUIRE(hkv <= 65535, SP_ERR_UNSUPPORTED, "sp_attn_repack_v_bf16: grid too large");
+  hipLaunchKernelGGL(sp_repack_v_kernel, dim3((unsigned)a.nb, hkv), dim3(AT_THREADS), 0, (hipStream_t)stream, a);
   SP_LAUNCH_CHECK();
   return SP_OK;
 }

@@ -17,6 +17,7 @@
 
 #include "sp_block_probs.h"
 #include "sp_pool.h"
+#include "sp_repack.h"
 #include "sp_rows.h"
 
 #define SEL_THREADS 1024
@@ -1620,6 +1621,10 @@ struct HeadArgs {
   const int32_t* head_cluster;
   const float* slash_blk;
   float *js_v, *js_s;
+  // Behind the heads: a workgroup per tile of V (repack.nb 0: none).  The budgets and the query-aware test are 3 hq workgroups of
+  // latency, the repack is bytes and depends on v alone; the two in one launch against two, us: 10007 tokens 4 kv heads 16 / 26,
+  // 16384 (8 kv heads) 24 / 35, 32768 43 / 61, 65001 78 / 108.
+  RepackArgs repack;
 };
 #define HEAD_LDS_BYTES(d, nb) (qa_lds_bytes(d, nb) > sizeof(CoverShared) ? qa_lds_bytes(d, nb) : sizeof(CoverShared))
 __global__ __launch_bounds__(CS_THREADS) void sp_layer_heads_kernel(HeadArgs a) {
@@ -1630,6 +1635,11 @@ __global__ __launch_bounds__(CS_THREADS) void sp_layer_heads_kernel(HeadArgs a) 
     return;
   }
   const int h = (int)blockIdx.x - a.n_cover, lane = threadIdx.x & 63;
+  if (h >= a.qa.hq) {
+    const int tile = h - a.qa.hq;
+    repack_v_tile<CS_THREADS>(a.repack, tile % a.repack.nb, tile / a.repack.nb, reinterpret_cast<sp_bf16*>(head_lds));
+    return;
+  }
   // (for a head that turns out query-aware too: sp_share_decide_kernel drops it)
   queryaware_head(a.qa, h, reinterpret_cast<float*>(head_lds), [&](int wave) {
     if (wave > 2) return;
@@ -1661,13 +1671,13 @@ extern "C" size_t sp_select_layer_scratch_bytes(int64_t n, int32_t hq, int32_t h
   return sum;
 }
 
-extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+static int select_layer(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
                                     int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
                                     uint32_t flags, const sp_cluster_state* state, const int32_t* head_cluster,
                                     int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
                                     float similarity_threshold, double fallback_threshold, float queryaware_threshold,
                                     void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
-                                    float* avg_attn, sp_stream_t stream) {
+                                    float* avg_attn, const RepackArgs& repack, sp_stream_t stream) {
   SP_REQUIRE(state && head_cluster && scratch && qa_probs && per_head && mask, SP_ERR_INVALID_ARGUMENT,
              "sp_select_layer_bf16: null pointer");
   SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && bs > 0 && d > 0, SP_ERR_INVALID_ARGUMENT, "sp_select_layer_bf16: bad shape");
@@ -1709,7 +1719,10 @@ extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int
   a.slash_blk = slash_blk;
   a.js_v = floats(LY_JS_V);
   a.js_s = floats(LY_JS_S);
-  hipLaunchKernelGGL(sp_layer_heads_kernel, dim3(a.n_cover + hq), dim3(CS_THREADS), HEAD_LDS_BYTES(d, nb), s, a);
+  a.repack = repack;
+  static_assert(sizeof(CoverShared) >= RP_LDS_BYTES, "");
+  hipLaunchKernelGGL(sp_layer_heads_kernel, dim3((unsigned)(a.n_cover + hq + repack.nb * repack.hkv)), dim3(CS_THREADS),
+                     HEAD_LDS_BYTES(d, nb), s, a);
   SP_LAUNCH_CHECK();
   hipLaunchKernelGGL(sp_share_decide_kernel, dim3(1), dim3(DEC_MAX_HEADS), 0, s, a.st, head_cluster, layer_idx, hq, use_qa, nv,
                      ns, min_blocks, similarity_threshold, fallback_threshold, decision, a.js_v, a.js_s, nv_f, ns_f);
@@ -1722,6 +1735,34 @@ extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int
   SP_LAUNCH_CHECK();
   return sp_queryaware_select_bf16(part(LY_QBAR), part(LY_KBAR), decision, hq, hkv, d, nb, flags, pattern_threshold, qa_probs,
                                    mask, part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), stream);
+}
+
+extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                                    int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
+                                    uint32_t flags, const sp_cluster_state* state, const int32_t* head_cluster,
+                                    int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
+                                    float similarity_threshold, double fallback_threshold, float queryaware_threshold,
+                                    void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
+                                    float* avg_attn, sp_stream_t stream) {
+  return select_layer(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
+                      layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
+                      scratch, scratch_bytes, qa_probs, per_head, mask, avg_attn, RepackArgs{}, stream);
+}
+
+extern "C" int sp_select_layer_repack_bf16(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                                    int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
+                                    uint32_t flags, const sp_cluster_state* state, const int32_t* head_cluster,
+                                    int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
+                                    float similarity_threshold, double fallback_threshold, float queryaware_threshold,
+                                    void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
+                                    float* avg_attn, const void* v, int64_t v_stride_n, int64_t v_stride_h, void* vt, size_t vt_bytes,
+                                    sp_stream_t stream) {
+  RepackArgs repack;
+  const int rc = repack_args(&repack, "sp_select_layer_repack_bf16", v, n, hkv, d, v_stride_n, v_stride_h, bs, vt, vt_bytes);
+  if (rc != SP_OK) return rc;
+  return select_layer(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
+                      layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
+                      scratch, scratch_bytes, qa_probs, per_head, mask, avg_attn, repack, stream);
 }
 
 // ------------------------------------------------------------------------------------------------

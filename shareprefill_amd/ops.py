@@ -251,12 +251,12 @@ def queryaware_select(qbar, kbar, decision, mask, pattern_threshold, flags=_lib.
 
 def select_layer(state: ClusterState, head_cluster, layer_idx, q, k, block_size, flags, min_blocks, max_blocks,
                  pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold, qa_probs,
-                 avg_attn=None, keep_floats=False):
+                 avg_attn=None, keep_floats=False, repack=None):
     """The whole selection of one layer (attention_sharing.py:105-366) in one call: the stages above, same results.
 
     -> (mask int64 [Hq, nb, nbw], (decision, nv, ns, nv_final, ns_final) int32 [Hq] each, floats).  qa_probs: fp32
     [Hq, nb, nb] scratch; avg_attn, if given, is cleared.  floats: with keep_floats a dict of the float intermediates
-    (views of the call's scratch), else None."""
+    (views of the call's scratch), else None.  repack = (v, workspace buffer): repack_v of that v is part of the call."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")
@@ -269,12 +269,19 @@ def select_layer(state: ClusterState, head_cluster, layer_idx, q, k, block_size,
     scratch = torch.empty(need, dtype=torch.uint8, device=dev)
     mask = torch.empty(hq, nb, (nb + 63) // 64, dtype=torch.int64, device=dev)
     per_head = torch.empty(5, hq, dtype=torch.int32, device=dev)
-    st = lib.sp_select_layer_bf16(_ptr(q), _ptr(k), n, hq, hkv, d, q.stride(1), q.stride(0), k.stride(1), k.stride(0),
-                                  block_size, flags, state.ref(), _ptr(head_cluster), layer_idx, min_blocks, max_blocks,
-                                  pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
-                                  _ptr(scratch), need, _ptr(qa_probs), _ptr(per_head), _ptr(mask), _ptr(avg_attn),
-                                  _stream(dev))
-    _lib.check(st, "sp_select_layer_bf16")
+    args = (_ptr(q), _ptr(k), n, hq, hkv, d, q.stride(1), q.stride(0), k.stride(1), k.stride(0), block_size, flags, state.ref(),
+            _ptr(head_cluster), layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold,
+            queryaware_threshold, _ptr(scratch), need, _ptr(qa_probs), _ptr(per_head), _ptr(mask), _ptr(avg_attn))
+    if repack is None:
+        st, entry = lib.sp_select_layer_bf16(*args, _stream(dev)), "sp_select_layer_bf16"
+    else:
+        v, ws = repack
+        _check_hnd(v, "v")
+        if tuple(v.shape) != (hkv, n, d):
+            raise ValueError(f"v {tuple(v.shape)} does not match k {tuple(k.shape)}")
+        st = lib.sp_select_layer_repack_bf16(*args, _ptr(v), v.stride(1), v.stride(0), _ptr(ws), ws.numel(), _stream(dev))
+        entry = "sp_select_layer_repack_bf16"
+    _lib.check(st, entry)
     floats = None
     if keep_floats:
         def view(i, dtype, *shape):

@@ -231,14 +231,17 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
         slab = _lib.load().sp_attn_pivot_scratch_bytes(q_len, block_size)
         max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
-        ops.repack_v(v, block_size, ws[0])
     # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
     plan_args = {"scale_dim": model_dim}
     plan_here = getattr(sharing.plan_layer, "__func__", None) is _PLAN_LAYER
     if plan_here:
         plan_args["avg_attn"] = avg_attn[0]  # (cleared on the way)
+        if not short:
+            plan_args["repack"] = (v, ws[0])  # (repacked on the way)
     else:
         avg_attn.zero_()
+        if not short:
+            ops.repack_v(v, block_size, ws[0])
     plan = sharing.plan_layer(q, k, module.layer_idx, block_size, minb, maxb, config.pattern_threshold,
                               config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold, **plan_args)
     update_here = short and getattr(sharing.update_pivotal_attns, "__func__", None) is _UPDATE_PIVOTAL_ATTNS
