@@ -238,8 +238,8 @@ int sp_select_layer_repack_bf16(const void* q, const void* k, int64_t n, int32_t
 size_t sp_attn_workspace_bytes(int64_t n, int32_t hq, int32_t hkv, int32_t d, int32_t bs);
 /* Optional extra workspace per pivot head (decision == SP_DEC_DENSE with avg_attn requested): with
  * sp_attn_workspace_bytes rounded up to 256 bytes + p * sp_attn_pivot_scratch_bytes(n, bs) bytes of workspace, the
- * first p pivot heads (ascending head index) are processed in a launch of their own that keeps per-query block sums,
- * and their block-average maps (shareprefill_attn.py:425-457) are made from those instead of a second pass over
+ * first p pivot heads (ascending head index) keep per-query block sums on the way, and their block-average maps
+ * (shareprefill_attn.py:425-457) are made from those instead of a second pass over
  * Q.K^T; further pivots, or all of them with the base size, take that second pass.  Same results to rounding. */
 size_t sp_attn_pivot_scratch_bytes(int64_t n, int32_t bs);
 int sp_attn_repack_v_bf16(const void* v, int64_t n, int32_t hkv, int32_t d, int64_t v_stride_n, int64_t v_stride_h,
@@ -249,6 +249,16 @@ int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, i
                                   int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, int32_t bs,
                                   float softmax_scale, const uint64_t* mask, const int32_t* decision, void* out,
                                   float* avg_attn, void* workspace, size_t workspace_bytes, uint32_t flags,
+                                  sp_stream_t stream);
+/* The same at bs = 128 with sp_pivot_update(state, head_cluster, decision, avg_attn, hq, nb, pattern_threshold) in the launch:
+ * decision, avg_attn and head_cluster must be given, and the workspace needs room for the block sums of every head that can be
+ * DENSE; those beyond it get NaN for a map and update no pivot. */
+int sp_block_sparse_attn_pivot_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
+                                  int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
+                                  int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,
+                                  const uint64_t* mask, const int32_t* decision, void* out, float* avg_attn,
+                                  void* workspace, size_t workspace_bytes, uint32_t flags,
+                                  const sp_cluster_state* state, const int32_t* head_cluster, float pattern_threshold,
                                   sp_stream_t stream);
 
 /* The same attention for short prompts, bs = 128, d = 64 or 128 (no padding): one kernel that reads v as it is, needs no

@@ -277,7 +277,7 @@ class AttentionSharing:
         ops.pivot_update(self._state, hc, decision, avg_attn[0], pattern_threshold)
 
     def pivot_slabs(self, layer_idx: int, hq: int, device, pattern_threshold: float):
-        """What ops.short_attention takes to do update_pivotal_attns itself."""
+        """What ops.short_attention and ops.block_sparse_attention take to do update_pivotal_attns themselves."""
         return self._state, self._head_cluster_tensor(layer_idx, hq, device), pattern_threshold
 
     def note_dense_layer(self, layer_idx: int, hq: int, nb: int) -> None:

@@ -15,6 +15,7 @@
 // software pipeline over 32-key half-tiles in which the softmax of one half-tile is issued between the MFMAs of
 // its neighbours (see "the software pipeline of one wave" below).
 #include "sp_repack.h"
+#include "sp_rows.h"
 
 #include <type_traits>
 
@@ -65,15 +66,11 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(RepackArgs a) {
 #define AT_HALF_GANG_NB 128  // gangs of 16 up to here
 // The 1 KiB scheduler area (int indices): 0..127 eight queue tickets (one per 64 bytes), 128..191 the pivot slot of
 // every head (one byte each, AT_NO_SLOT = its block sums are not kept), 192..195 {shader cycles, 100 MHz ticks} of
-// workgroup 0, 196 the number of pivot slots in use, 200..231 the pairing of every two adjacent heads (one byte each,
-// see sp_attn_schedule_kernel), 232..239 the queue tickets of the pivot heads' launch (so that both launches of a call
-// find their tickets cleared by sp_attn_schedule_kernel and nothing has to be cleared in between).
+// workgroup 0, 200..231 the pairing of every two adjacent heads (one byte each, see sp_attn_schedule_kernel).
 #define AT_SLOT_TABLE 128
 #define AT_CLOCK_SLOT 192
-#define AT_NPIV_SLOT 196
 #define AT_ROWS_SLOT 197  // 1: the caller asked for pairing by rows: no analysis, no ranking
 #define AT_PAIR_TABLE 200
-#define AT_PIVOT_TICKETS 232  // 232..239: the eight queue tickets of the pivot heads' own launch
 #define AT_NO_SLOT 255
 // Behind the 1 KiB of slots: the weights (uint16) of up to AT_RANK_MAX gangs, see sp_attn_schedule_kernel.
 #define AT_RANK_MAX 1024  // AT_MAX_HEADS of at most four gangs
@@ -145,6 +142,7 @@ __device__ static inline void at_geometry(AtGeom& gm, int hq, int hkv, int nb, i
 #define AT_VBUF_BYTES (AT_D * AT_SUB * 2)  // 16 KiB
 #define AT_LIST_MAX 4096                      // union blocks of a row pair (nb <= 4096)
 #define AT_LIST_BYTES (AT_LIST_MAX * 4)
+#define AT_PIVOT_STAT_AT 98304  // a pivot's row statistics, behind what its rows' selection takes of the rings
 #define AT_LDS_BYTES (AT_RING * (AT_KBUF_BYTES + AT_VBUF_BYTES) + AT_LIST_BYTES)
 
 typedef __attribute__((address_space(3))) void* at_lds_ptr;
@@ -239,6 +237,21 @@ __device__ static inline uint64_t at_trim(uint64_t x, int wi, int r) {
 }
 
 // entry of the per-pair block list: column | row-membership flags
+// sp_wave_sum without its trips through LDS: lanes ^ 32 and ^ 16 by the swaps; then every row of 16 lanes holds the same
+// values, and with them repeating every 16, 8, 4, 2 lanes a rotation by 8, 4, 2, 1 is the exchange with lane ^ 8, 4, 2, 1
+template <int CTRL>
+__device__ static __forceinline__ float at_add_rotated(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+__device__ static __forceinline__ float at_wave_sum(float v) {
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  u = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, (uint32_t)a[0]) + __builtin_bit_cast(float, (uint32_t)a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (uint32_t)b[0]) + __builtin_bit_cast(float, (uint32_t)b[1]);
+  return at_add_rotated<0x121>(at_add_rotated<0x122>(at_add_rotated<0x124>(at_add_rotated<0x128>(v))));  // row_ror 8, 4, 2, 1
+}
+
 // inclusive sum over the 64 lanes
 __device__ static __forceinline__ uint32_t at_lane_scan(uint32_t v) {
   auto add = [&](auto ctrl, auto rows) {  // (lanes without a source, or outside the rows, add 0)
@@ -698,10 +711,16 @@ __device__ __forceinline__ void at_step(const AtAddr& ad, const bf16x8 (&qb)[2][
                                                                               scale_log2, neg_m, det, ones, pre);
 }
 
-// PIVOT = false: every head except the pivots that have a slot in the scheduler area's table (when skip_slotted).
-// PIVOT = true: only those pivots; besides the output it leaves, per (query, key block), the softmax mass of the
-// block relative to the running max at that time as u = log2(sum) + max, from which at_avg_from_block_sums (sp_attn_avg_kernel) makes
-// the block-average map without recomputing any logit.  pivot_u: fp32 [slot][r*(r+1)/2 + c][128 queries].
+// PIVOT = true: some heads may be pivots with a slot in the scheduler area's table.  Their items take a second instance of the
+// walk (MODE bit 0), which leaves besides the output, per (query, key block), the softmax mass of the block relative to the
+// running max at that time as u = log2(sum) + max (pivot_u: fp32 [slot][r*(r+1)/2 + c][128 queries]); the workgroup that has
+// walked a row then makes the row's block averages from them and turns those into the row's pattern in the sharing state
+// (pivot.st.n_clusters > 0), which needs nothing but that row.  The pivots as items among the others, against a launch of their
+// own and two more behind it for the maps and the patterns: two layers of 16384 tokens, eight pivots in the first, 1727 -> 1653 us
+// (the first layer's launches 901 -> 833); a layer without a pivot, for which each of the three was a launch with nothing to
+// do, of 10007 tokens 263 -> 257.  The walk that all other heads take stands first: behind the pivots' one 131072 tokens took 0.4 %
+// longer than alone.
+// nan_maps: pivots without a slot get NaN for a map (otherwise sp_attn_avg_kernel makes theirs).
 // HALF: q, k and v are zero beyond channel 64 (see at_fused); channels 64..127 of out are then not written.
 // FINE: a block size f = 128 >> fshift below 128.  `mask` is then the OR of the caller's fine mask over 128-token
 // blocks (sp_attn_coarsen_kernel) and decides which 128-key blocks a row visits; fine_mask [hq][nbf][nbfw] decides, per
@@ -711,15 +730,14 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const sp_bf16* __restrict__ vt,
     const uint64_t* __restrict__ mask, const int32_t* __restrict__ decision, sp_bf16* __restrict__ out,
     float2* __restrict__ rowstat, int64_t n, int hq, int hkv, int64_t sq_n, int64_t sq_h, int64_t sk_n,
-    int64_t sk_h, int nb, int nbw, float scale_log2, int* __restrict__ sched, int skip_slotted,
-    float* __restrict__ pivot_u, const uint64_t* __restrict__ fine_mask, int fshift, int nbf, int nbfw) {
+    int64_t sk_h, int nb, int nbw, float scale_log2, int* __restrict__ sched, float* pivot_u, float* avg_attn, int nan_maps,
+    PivotArgs pivot, const uint64_t* __restrict__ fine_mask, int fshift, int nbf, int nbfw) {
   extern __shared__ __attribute__((aligned(1024))) char lds[];  // K ring (4 x 16 KiB) | V^T ring (4 x 16 KiB)
   __shared__ int s_queue, s_ticket;
   // the scheduler's tables, copied once: read from memory they are two more dependent loads in front of every item
   __shared__ uint32_t dense_heads[AT_MAX_HEADS / 32], s_slots[AT_MAX_HEADS / 4], s_pairs[AT_MAX_HEADS / 8];
   __shared__ uint16_t s_order[AT_RANK_MAX];
-  constexpr int MODE = (PIVOT ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
-  if (PIVOT && sched[AT_NPIV_SLOT] == 0) return;  // no pivot in this layer
+  __shared__ PivotRowShared pivot_sh;  // (PIVOT)
   const uint8_t* const slots = reinterpret_cast<const uint8_t*>(s_slots);
   const uint8_t* const pair_table = reinterpret_cast<const uint8_t*>(s_pairs);
 
@@ -767,7 +785,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   int first_try = 0, tk = 0;  // queues before offset first_try are known to be empty
   auto ask = [&]() {
     const int xq = (xcd + first_try) & 7;
-    if (t == 0 && first_try < 8) tk = atomicAdd(&sched[PIVOT ? AT_PIVOT_TICKETS + xq : xq * 16], 1);
+    if (t == 0 && first_try < 8) tk = atomicAdd(&sched[xq * 16], 1);
   };
   auto publish = [&]() {
     if (t == 0) {
@@ -812,7 +830,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int queue = __builtin_amdgcn_readfirstlane(s_queue);
     if (queue < 0) {
-      if (!PIVOT && blockIdx.x == 0 && t == 0) {
+      if (blockIdx.x == 0 && t == 0) {
         long long* clk = reinterpret_cast<long long*>(sched + AT_CLOCK_SLOT);
         clk[0] = clock64() - clk0;
         clk[1] = wall_clock64() - tick0;
@@ -821,11 +839,10 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     }
     const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
     int h_item, pair;
-    bool work = at_item(gm, queue, ticket, h_item, pair);
+    const bool work = at_item(gm, queue, ticket, h_item, pair);
     const int slot = __builtin_amdgcn_readfirstlane((int)slots[h_item]);
-    if (PIVOT ? slot == AT_NO_SLOT : (skip_slotted && slot != AT_NO_SLOT)) work = false;  // the other launch's head
     // the item's two (head, row): A for waves 0-3, B for waves 4-7
-    const bool by_heads = !PIVOT && __builtin_amdgcn_readfirstlane((int)pair_table[h_item >> 1]) != 0;
+    const bool by_heads = __builtin_amdgcn_readfirstlane((int)pair_table[h_item >> 1]) != 0;
     const int h_a = by_heads ? (h_item & ~1) : h_item, h_b = by_heads ? (h_item | 1) : h_item;
     const int r_a = by_heads ? 2 * pair + (h_item & 1) : 2 * pair, r_b = by_heads ? r_a : r_a + 1;
     if (!work || r_a >= nb) {  // (heads pairing, odd nb: the odd head's last item has no row)
@@ -871,6 +888,10 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
         first_mine = ((at_lane_u64(grp ? w_b : w_a, wf) >> bit) & 1ull) != 0ull;
       }
     }
+    // the item itself; PV: a pivot with a slot
+    auto run = [&](auto pv) {
+    constexpr bool PV = decltype(pv)::value;
+    constexpr int MODE = (PV ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
     // FINE: the two fine mask rows of this wave's query tiles, and the keep bits (at_keep) of a block from them
     const uint64_t* frow[2] = {fine_mask, fine_mask};
     if constexpr (FINE) {
@@ -925,9 +946,9 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     // holds the whole sum); it is kept as u = log2(sum) + m_run.
     float l_mark[2] = {0.f, 0.f};
     const int64_t tri_row = (int64_t)slot * ((int64_t)nb * (nb + 1) / 2) + (int64_t)r * (r + 1) / 2;
-    float* const pu = PIVOT ? pivot_u + tri_row * AT_BS : nullptr;
+    float* const pu = PV ? pivot_u + tri_row * AT_BS : nullptr;
     auto emit = [&](int c) {
-      if constexpr (PIVOT) {
+      if constexpr (PV) {
         // (the sums' last MFMA carried its wait states: at_fused<SETTLE> / at_pv_only)
         AT_LANE_VIEW(tq);
 #pragma unroll
@@ -1144,12 +1165,17 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     const float l_tot[2] = {o[8][0][0], o[8][1][0]};
     AT_LANE_VIEW(tq);
 
-    // pivot heads: keep the softmax statistics of every query row for the block-average pass
-    if (row_ok && rowstat != nullptr && ((dense_heads[h >> 5] >> (h & 31)) & 1u) != 0u && g == 0) {
+    // pivots without a slot: the softmax statistics of every query row for the block-average pass
+    if (!PV && row_ok && ((dense_heads[h >> 5] >> (h & 31)) & 1u) != 0u) {
+      if (nan_maps) {
+        for (int i = tq; i < n_blk; i += AT_FWD_THREADS / 2)
+          if (blist[i] & my_flag) avg_attn[((int64_t)h * nb + r) * nb + (blist[i] & AT_COL_MASK)] = NAN;
+      } else if (rowstat != nullptr && g == 0) {
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-        if (qrow < n) rowstat[(int64_t)h * n + qrow] = make_float2(m_run[qt], l_tot[qt]);
+        for (int qt = 0; qt < 2; ++qt) {
+          const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
+          if (qrow < n) rowstat[(int64_t)h * n + qrow] = make_float2(m_run[qt], l_tot[qt]);
+        }
       }
     }
 
@@ -1177,6 +1203,64 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
         }
       }
     }
+    if constexpr (PV) {
+      // ---- a pivot's rows: avg[h][r][c] = mean over the valid queries of block r of exp2(u[q][c] - m[q]) / l[q], by the row's
+      // four waves, each every fourth block of the list, four of them in flight ----
+      __syncthreads();  // the block sums of every wave have left, the rings are free
+      float2* const stat = reinterpret_cast<float2*>(lds + AT_PIVOT_STAT_AT) + grp * AT_BS;  // (m, l) of the row's queries
+      if (g == 0)
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) stat[q_off + qt * 16] = make_float2(m_run[qt], l_tot[qt]);
+      __syncthreads();
+      if (row_ok) {
+        const int64_t rem = n - (int64_t)r * AT_BS;
+        const int valid_q = rem < AT_BS ? (int)rem : AT_BS, lane = tq_o & 63;
+        float m[2], inv_l[2];
+        bool ok[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int qo = lane + 64 * j;
+          ok[j] = qo < valid_q;
+          const float2 st = stat[ok[j] ? qo : 0];
+          m[j] = st.x;
+          inv_l[j] = 1.0f / st.y;
+        }
+        const float inv_q = 1.0f / (float)valid_q;
+        float* const arow = avg_attn + ((int64_t)h * nb + r) * nb;
+        for (int i0 = wave & 3; i0 < n_blk; i0 += 16) {
+          int col[4];
+          float u[4][2];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t e = i0 + 4 * k < n_blk ? blist[i0 + 4 * k] : 0u;
+            col[k] = __builtin_amdgcn_readfirstlane((e & my_flag) != 0u ? (int)(e & AT_COL_MASK) : -1);
+            const float* src = pu + (int64_t)(col[k] < 0 ? r : col[k]) * AT_BS + lane;
+            u[k][0] = src[0];
+            u[k][1] = src[64];
+          }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            float part = ok[0] ? __builtin_amdgcn_exp2f(u[k][0] - m[0]) * inv_l[0] : 0.f;
+            part += ok[1] ? __builtin_amdgcn_exp2f(u[k][1] - m[1]) * inv_l[1] : 0.f;
+            part = at_wave_sum(part);
+            if (lane == 0 && col[k] >= 0) arow[col[k]] = part * inv_q;
+          }
+        }
+      }
+      if (pivot.st.n_clusters > 0) {
+        static_assert(AT_PIVOT_STAT_AT + 2 * AT_BS * sizeof(float2) <= AT_RING * (AT_KBUF_BYTES + AT_VBUF_BYTES), "");
+#pragma unroll 1
+        for (int rr = r_a; rr <= (has_b ? r_b : r_a); ++rr) {
+          __syncthreads();  // the rows are written; the LDS of the row before is free
+          pivot_row<AT_FWD_THREADS>(pivot, pivot_sh, lds, avg_attn, rr, h);
+        }
+      }
+    }
+    };  // run
+    if (!PIVOT || __builtin_expect(slot == AT_NO_SLOT, 1))
+      run(std::false_type{});
+    else
+      run(std::integral_constant<bool, PIVOT>{});
     publish();
   }
 }
@@ -1237,24 +1321,17 @@ __global__ __launch_bounds__(AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
   const uint64_t votes = __ballot(dense);
   if (t < AT_MAX_HEADS && lane == 0) dense_cnt[wave] = (uint32_t)__builtin_popcountll(votes);
   __syncthreads();
-  int total = 0;
   if (t < AT_MAX_HEADS) {
     int rank = __builtin_popcountll(votes & ((1ull << lane) - 1ull));
 #pragma unroll
-    for (int w = 0; w < AT_MAX_HEADS / SP_WAVE; ++w) {
+    for (int w = 0; w < AT_MAX_HEADS / SP_WAVE; ++w)
       if (w < wave) rank += (int)dense_cnt[w];
-      total += (int)dense_cnt[w];
-    }
     slot_s[t] = dense && rank < max_pivots ? (uint8_t)rank : (uint8_t)AT_NO_SLOT;
   }
   if (blockIdx.x == 0) {
     if (t < hq) reinterpret_cast<uint8_t*>(sched + AT_SLOT_TABLE)[t] = slot_s[t];
     if (t < AT_SLOT_TABLE) sched[t] = 0;
-    if (t < 8) sched[AT_PIVOT_TICKETS + t] = 0;
-    if (t == 0) {
-      sched[AT_NPIV_SLOT] = total < max_pivots ? total : max_pivots;
-      sched[AT_ROWS_SLOT] = pair_rows;
-    }
+    if (t == 0) sched[AT_ROWS_SLOT] = pair_rows;
   }
   __syncthreads();
 
@@ -1307,64 +1384,21 @@ __global__ __launch_bounds__(AT_PAIRING_THREADS) void sp_attn_schedule_kernel(
   }
 }
 
-// ---- pivot heads with a slot: block-averaged attention map from the block sums the forward kernel kept ----
-// avg[h][r][c] = mean over the valid queries of block r of  exp2(u[q][c] - m[q]) / l[q]  (m, l: the query's final
-// softmax statistics).  One workgroup per (query block, head) of sp_attn_avg_kernel; a wave takes every fourth kept
-// block.
-__device__ static void at_avg_from_block_sums(const uint64_t* __restrict__ mask, int slot,
-                                              const float2* __restrict__ rowstat, const float* __restrict__ pivot_u,
-                                              float* __restrict__ avg_attn, int64_t n, int nb, int nbw) {
-  const int r = nb - 1 - blockIdx.x, h = blockIdx.y;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t rem = n - (int64_t)r * AT_BS;
-  const int valid_q = rem < AT_BS ? (int)rem : AT_BS;
-  float m[2], inv_l[2];
-  bool ok[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int qo = lane + 64 * j;
-    ok[j] = qo < valid_q;
-    const float2 st = rowstat[(int64_t)h * n + (int64_t)r * AT_BS + (ok[j] ? qo : 0)];
-    m[j] = st.x;
-    inv_l[j] = 1.0f / st.y;
-  }
-  const float inv_q = 1.0f / (float)valid_q;
-  const float* pu = pivot_u + ((int64_t)slot * ((int64_t)nb * (nb + 1) / 2) + (int64_t)r * (r + 1) / 2) * AT_BS;
-  float* arow_out = avg_attn + ((int64_t)h * nb + r) * nb;
-  AtBlocks it;
-  it.init(mask + ((int64_t)h * nb + r) * nbw, r);
-  int idx = 0;
-  for (int c = it.next(); c >= 0; c = it.next(), ++idx) {
-    if ((idx & 3) != wave) continue;
-    const float u0 = pu[(int64_t)c * AT_BS + lane], u1 = pu[(int64_t)c * AT_BS + 64 + lane];
-    float part = ok[0] ? __builtin_amdgcn_exp2f(u0 - m[0]) * inv_l[0] : 0.f;
-    part += ok[1] ? __builtin_amdgcn_exp2f(u1 - m[1]) * inv_l[1] : 0.f;
-    part = sp_wave_sum(part);
-    if (lane == 0) arow_out[c] = part * inv_q;
-  }
-}
-
 // ---- pivot heads: block-averaged attention map (shareprefill_attn.py:425-457) ---------------------------
 // avg[h][r][c] = mean over the valid queries of block r of the softmax mass that falls into key block c,
-// recomputed from the row statistics the forward kernel left behind (the pivots for which the workspace has no
-// room to keep block sums; the others are made from their block sums by at_avg_from_block_sums, in the same launch).
+// recomputed from the row statistics the forward kernel left behind: the pivots for which the workspace has no
+// room to keep block sums (the forward kernel makes the others').
 // One workgroup per (query block, head); heads that are no pivots leave at once.
 __global__ __launch_bounds__(AT_THREADS) void sp_attn_avg_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const uint64_t* __restrict__ mask,
     const int32_t* __restrict__ decision, const float2* __restrict__ rowstat, float* __restrict__ avg_attn, int64_t n,
     int hq, int hkv, int64_t sq_n, int64_t sq_h, int64_t sk_n, int64_t sk_h, int nb, int nbw, float scale_log2,
-    const int* __restrict__ sched, const float* __restrict__ pivot_u) {
+    const int* __restrict__ sched) {
   __shared__ __attribute__((aligned(16))) sp_bf16 Ks[AT_BS * AT_PITCH];
   __shared__ float wred[2][4];
   const int r = nb - 1 - blockIdx.x, h = blockIdx.y;
   if (decision[h] != SP_DEC_DENSE) return;
-  {
-    const int slot = reinterpret_cast<const uint8_t*>(sched + AT_SLOT_TABLE)[h];
-    if (slot != AT_NO_SLOT) {  // (uniform) the forward pass kept this head's block sums
-      at_avg_from_block_sums(mask, slot, rowstat, pivot_u, avg_attn, n, nb, nbw);
-      return;
-    }
-  }
+  if (reinterpret_cast<const uint8_t*>(sched + AT_SLOT_TABLE)[h] != AT_NO_SLOT) return;
   const int kvh = h / (hq / hkv);
   const int t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63;
@@ -1636,39 +1670,38 @@ extern "C" int sp_attn_repack_v_bf16(const void* v, int64_t n, int32_t hkv, int3
   return SP_OK;
 }
 
-extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq,
-                                             int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h,
-                                             int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n,
-                                             int64_t v_stride_h, int32_t bs, float softmax_scale,
-                                             const uint64_t* mask, const int32_t* decision, void* out,
-                                             float* avg_attn, void* workspace, size_t workspace_bytes,
-                                             uint32_t flags, sp_stream_t stream) {
+// pivot: null, or the pivots' rows go on into the sharing state (then no other launch makes maps)
+static int at_launch(const char* who, const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+                     int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n,
+                     int64_t v_stride_h, int32_t bs, float softmax_scale, const uint64_t* mask, const int32_t* decision,
+                     void* out, float* avg_attn, void* workspace, size_t workspace_bytes, uint32_t flags,
+                     const PivotArgs* pivot, sp_stream_t stream) {
   SP_REQUIRE(q && k && v && mask && out && workspace, SP_ERR_INVALID_ARGUMENT,
-             "sp_block_sparse_attn_fwd_bf16: null pointer");
+             "%s: null pointer", who);
   SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, SP_ERR_INVALID_ARGUMENT,
-             "sp_block_sparse_attn_fwd_bf16: bad shape n=%lld hq=%d hkv=%d", (long long)n, hq, hkv);
-  SP_REQUIRE(hq <= AT_MAX_HEADS, SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: more than %d query heads",
+             "%s: bad shape n=%lld hq=%d hkv=%d", who, (long long)n, hq, hkv);
+  SP_REQUIRE(hq <= AT_MAX_HEADS, SP_ERR_UNSUPPORTED, "%s: more than %d query heads", who,
              AT_MAX_HEADS);
-  SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "sp_block_sparse_attn_fwd_bf16: softmax_scale must be > 0");
+  SP_REQUIRE(softmax_scale > 0.f, SP_ERR_INVALID_ARGUMENT, "%s: softmax_scale must be > 0", who);
   SP_REQUIRE(at_block_size_ok(bs), SP_ERR_UNSUPPORTED,
-             "sp_block_sparse_attn_fwd_bf16: block size %d unsupported (16, 32, 64 or 128)", bs);
-  SP_REQUIRE(d == AT_D, SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: head_dim %d unsupported (only 128)", d);
+             "%s: block size %d unsupported (16, 32, 64 or 128)", who, bs);
+  SP_REQUIRE(d == AT_D, SP_ERR_UNSUPPORTED, "%s: head_dim %d unsupported (only 128)", who, d);
   SP_REQUIRE(q_stride_n % 8 == 0 && q_stride_h % 8 == 0 && k_stride_n % 8 == 0 && k_stride_h % 8 == 0 &&
                  ((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)out % 16) == 0,
-             SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: tensors must be 16-byte aligned, strides multiple of 8");
+             SP_ERR_UNSUPPORTED, "%s: tensors must be 16-byte aligned, strides multiple of 8", who);
   SP_REQUIRE((int64_t)AT_BS * k_stride_n < (1ll << 31), SP_ERR_UNSUPPORTED,
-             "sp_block_sparse_attn_fwd_bf16: key token stride %lld too large", (long long)k_stride_n);
+             "%s: key token stride %lld too large", who, (long long)k_stride_n);
   SP_REQUIRE(workspace_bytes >= sp_attn_workspace_bytes(n, hq, hkv, d, bs), SP_ERR_WORKSPACE,
-             "sp_block_sparse_attn_fwd_bf16: workspace too small");
+             "%s: workspace too small", who);
   // nb: 128-token blocks, what the kernels walk; nbf: blocks of the caller's size, what `mask` and `avg_attn` index
   const int64_t nb = sp_ceil_div(n, AT_BS), nbf = sp_ceil_div(n, bs);
   const bool fine = bs != AT_BS;
   const int fshift = at_fshift(bs);
-  SP_REQUIRE(nbf <= 4096, SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: %lld blocks of %d tokens exceed 4096",
+  SP_REQUIRE(nbf <= 4096, SP_ERR_UNSUPPORTED, "%s: %lld blocks of %d tokens exceed 4096", who,
              (long long)nbf, bs);
-  SP_REQUIRE(nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: grid too large");
+  SP_REQUIRE(nb * hq < (1ll << 31), SP_ERR_UNSUPPORTED, "%s: grid too large", who);
   SP_REQUIRE(nb <= AT_LIST_MAX, SP_ERR_UNSUPPORTED,
-             "sp_block_sparse_attn_fwd_bf16: %lld key blocks exceed the supported %d (sequence too long)", (long long)nb,
+             "%s: %lld key blocks exceed the supported %d (sequence too long)", who, (long long)nb,
              AT_LIST_MAX);
   if (!(flags & SP_ATTN_V_REPACKED)) {
     int rc = sp_attn_repack_v_bf16(v, n, hkv, d, v_stride_n, v_stride_h, bs, workspace, workspace_bytes, stream);
@@ -1691,9 +1724,8 @@ extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const
     SP_LAUNCH_CHECK();
     mask = coarse;  // from here on `mask` is the 128-block mask
   }
-  // Workspace beyond the base size holds the block sums of pivot heads, one slab per pivot: those heads run in a
-  // launch of their own that keeps the sums, and their block-average maps are made from them; pivots beyond the
-  // slabs (or all of them, with a base-size workspace) take the recomputing pass.
+  // Workspace beyond the base size holds the block sums of pivot heads, one slab per pivot, from which the forward kernel makes
+  // their block-average maps; pivots beyond the slabs (or all of them, with a base-size workspace) take the recomputing pass.
   const size_t base_bytes = sp_attn_workspace_bytes(n, hq, hkv, d, bs);
   const size_t base_aligned = (base_bytes + 255) & ~(size_t)255;
   const size_t slab = sp_attn_pivot_scratch_bytes(n, bs);
@@ -1715,7 +1747,7 @@ extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const
   static int cu_of_device[64] = {0};
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));
-  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_fwd_bf16: device index %d", dev);
+  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "%s: device index %d", who, dev);
   if (cu_of_device[dev] == 0) {
     hipDeviceProp_t prop;
     SP_HIP(hipGetDeviceProperties(&prop, dev));
@@ -1731,38 +1763,66 @@ extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const
   const int grid = (int)(total < (int64_t)n_cu ? ((total + 7) / 8) * 8 : (int64_t)n_cu);
   float2* stats = want_avg ? rowstat : (float2*)nullptr;
   const bool half = (flags & SP_ATTN_HALF_CHANNELS) != 0;
-  auto launch_fwd = [&](auto kernel, int skip_slotted, float* block_sums) {
+  PivotArgs rows = {};
+  if (pivot != nullptr) rows = *pivot;
+  auto launch_fwd = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(AT_FWD_THREADS), lds_bytes, s, (const sp_bf16*)q, (const sp_bf16*)k,
                        (const sp_bf16*)workspace, mask, decision, (sp_bf16*)out, stats, n, hq, hkv, q_stride_n,
                        q_stride_h, k_stride_n, k_stride_h, (int)nb, (int)((nb + 63) / 64), scale_log2, counter,
-                       skip_slotted, block_sums, fine_mask, fshift, (int)nbf, nbfw);
+                       max_pivots > 0 ? pivot_u : nullptr, avg_attn, pivot != nullptr ? 1 : 0, rows, fine_mask, fshift,
+                       (int)nbf, nbfw);
   };
   if (fine)  // (one instance: a head_dim below 128 computes its zero channels here)
-    launch_fwd(sp_attn_fwd_kernel<false, false, true>, 0, (float*)nullptr);
-  else if (half)
-    launch_fwd(sp_attn_fwd_kernel<false, true>, max_pivots > 0 ? 1 : 0, (float*)nullptr);
+    launch_fwd(sp_attn_fwd_kernel<false, false, true>);
+  else if (max_pivots > 0)
+    half ? launch_fwd(sp_attn_fwd_kernel<true, true>) : launch_fwd(sp_attn_fwd_kernel<true, false>);
   else
-    launch_fwd(sp_attn_fwd_kernel<false, false>, max_pivots > 0 ? 1 : 0, (float*)nullptr);
+    half ? launch_fwd(sp_attn_fwd_kernel<false, true>) : launch_fwd(sp_attn_fwd_kernel<false, false>);
   SP_LAUNCH_CHECK();
-  if (max_pivots > 0) {
-    if (half)
-      launch_fwd(sp_attn_fwd_kernel<true, true>, 0, pivot_u);
-    else
-      launch_fwd(sp_attn_fwd_kernel<true, false>, 0, pivot_u);
-    SP_LAUNCH_CHECK();
-  }
   if (want_avg && fine) {
     hipLaunchKernelGGL(sp_attn_avg_fine_kernel, dim3((unsigned)nb, hq), dim3(AT_THREADS), 0, s, (const sp_bf16*)q,
                        (const sp_bf16*)k, mask, fine_mask, decision, rowstat, avg_attn, n, hq, hkv, q_stride_n,
                        q_stride_h, k_stride_n, k_stride_h, (int)nb, (int)((nb + 63) / 64), (int)nbf, nbfw, fshift,
                        scale_log2);
     SP_LAUNCH_CHECK();
-  } else if (want_avg) {
+  } else if (want_avg && pivot == nullptr && max_pivots < hq) {
     hipLaunchKernelGGL(sp_attn_avg_kernel, dim3((unsigned)nb, hq), dim3(AT_THREADS), 0, s, (const sp_bf16*)q,
                        (const sp_bf16*)k, mask, decision, rowstat, avg_attn, n, hq, hkv, q_stride_n, q_stride_h,
-                       k_stride_n, k_stride_h, (int)nb, (int)((nb + 63) / 64), scale_log2, (const int*)counter,
-                       (const float*)pivot_u);
+                       k_stride_n, k_stride_h, (int)nb, (int)((nb + 63) / 64), scale_log2, (const int*)counter);
     SP_LAUNCH_CHECK();
   }
   return SP_OK;
+}
+
+extern "C" int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq,
+                                             int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h,
+                                             int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n,
+                                             int64_t v_stride_h, int32_t bs, float softmax_scale,
+                                             const uint64_t* mask, const int32_t* decision, void* out,
+                                             float* avg_attn, void* workspace, size_t workspace_bytes,
+                                             uint32_t flags, sp_stream_t stream) {
+  return at_launch("sp_block_sparse_attn_fwd_bf16", q, k, v, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h,
+                   v_stride_n, v_stride_h, bs, softmax_scale, mask, decision, out, avg_attn, workspace, workspace_bytes, flags,
+                   nullptr, stream);
+}
+
+extern "C" int sp_block_sparse_attn_pivot_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq,
+                                                   int32_t hkv, int32_t d, int64_t q_stride_n, int64_t q_stride_h,
+                                                   int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_n,
+                                                   int64_t v_stride_h, float softmax_scale, const uint64_t* mask,
+                                                   const int32_t* decision, void* out, float* avg_attn, void* workspace,
+                                                   size_t workspace_bytes, uint32_t flags, const sp_cluster_state* state,
+                                                   const int32_t* head_cluster, float pattern_threshold,
+                                                   sp_stream_t stream) {
+  SP_REQUIRE(decision && avg_attn && head_cluster, SP_ERR_INVALID_ARGUMENT,
+             "sp_block_sparse_attn_pivot_fwd_bf16: null pointer");
+  const int nb = (int)sp_ceil_div(n, AT_BS);
+  const int rc = check_state(state, nb, "sp_block_sparse_attn_pivot_fwd_bf16");
+  if (rc != SP_OK) return rc;
+  SP_REQUIRE(nb <= RS_MAX, SP_ERR_UNSUPPORTED, "sp_block_sparse_attn_pivot_fwd_bf16: nb=%d unsupported", nb);
+  const PivotArgs pivot = {state_by_value(state), head_cluster, decision, hq, nb, (nb + 63) / 64,
+                           (long long)sp_thr_lt(pattern_threshold)};
+  return at_launch("sp_block_sparse_attn_pivot_fwd_bf16", q, k, v, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n,
+                   k_stride_h, v_stride_n, v_stride_h, AT_BS, softmax_scale, mask, decision, out, avg_attn, workspace,
+                   workspace_bytes, flags, &pivot, stream);
 }

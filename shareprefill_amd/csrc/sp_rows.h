@@ -40,9 +40,9 @@ __device__ static __forceinline__ RowShared rs_carve(char* base, int n) {
 
 // rank[i] for i < m among keys[0 .. m-1], four keys per LDS read; keys[m .. (m + 3) & ~3) must be zero
 template <int THREADS>
-__device__ static __forceinline__ void rs_ranks4(const uint32_t* keys, int m, uint16_t* rank) {
+__device__ static __forceinline__ void rs_ranks4(const uint32_t* keys, int m, uint16_t* rank, int tid) {
   const int m4 = (m + 3) & ~3;
-  for (int i = threadIdx.x; i < m; i += THREADS) {
+  for (int i = tid; i < m; i += THREADS) {
     const uint32_t ki = keys[i];
     int r = 0;
     for (int j = 0; j < m4; j += 4) {
@@ -61,14 +61,14 @@ __device__ static __forceinline__ void rs_ranks4(const uint32_t* keys, int m, ui
 // crossing entry, so ranks, count and the "never reached -> keep one" rule come out as over the whole row.  Row r of
 // a pivot's block-average map ends at column r: a third of the comparisons of the full square on average.
 template <int THREADS>
-__device__ static __forceinline__ int rs_row_keep(const float* __restrict__ row, int n, long long t_lt, const RowShared& sh) {
-  if (threadIdx.x == 0) {
+__device__ static __forceinline__ int rs_row_keep(const float* __restrict__ row, int n, long long t_lt, const RowShared& sh, int tid = threadIdx.x) {
+  if (tid == 0) {
     *sh.below = 0;
     *sh.n_eff = 0;
   }
   __syncthreads();
   int last = 0;
-  for (int i = threadIdx.x; i < n; i += THREADS) {
+  for (int i = tid; i < n; i += THREADS) {
     const uint32_t key = sp_sort_key(row[i]);
     sh.keys[i] = key;
     if (key) last = i + 1;
@@ -76,22 +76,28 @@ __device__ static __forceinline__ int rs_row_keep(const float* __restrict__ row,
   if (last) atomicMax(sh.n_eff, last);
   __syncthreads();
   const int m = *sh.n_eff;
-  for (int i = m + threadIdx.x; i < ((m + 3) & ~3); i += THREADS) sh.keys[i] = 0;  // (past the row's end too)
-  for (int i = m + threadIdx.x; i < n; i += THREADS) sh.rank[i] = (uint16_t)i;
+  for (int i = m + tid; i < ((m + 3) & ~3); i += THREADS) sh.keys[i] = 0;  // (past the row's end too)
+  for (int i = m + tid; i < n; i += THREADS) sh.rank[i] = (uint16_t)i;
   __syncthreads();
-  rs_ranks4<THREADS>(sh.keys, m, sh.rank);
+  rs_ranks4<THREADS>(sh.keys, m, sh.rank, tid);
   __syncthreads();
-  for (int i = threadIdx.x; i < m; i += THREADS) sh.sorted_fx[sh.rank[i]] = sp_to_fixed(row[i]);
+  for (int i = tid; i < m; i += THREADS) sh.sorted_fx[sh.rank[i]] = sp_to_fixed(row[i]);
   __syncthreads();
   // inclusive scan of sorted_fx in contiguous per-thread chunks
   const int per = (m + THREADS - 1) / THREADS;
-  const int lo = min((int)threadIdx.x * per, m), hi = min(lo + per, m);
+  const int lo = min(tid * per, m), hi = min(lo + per, m);
   unsigned long long s = 0;
   for (int i = lo; i < hi; ++i) s += sh.sorted_fx[i];
-  sh.chunk_sum[threadIdx.x] = s;
+  unsigned long long incl = s;  // (integers: any order of the sums is the same)
+#pragma unroll
+  for (int o = 1; o < SP_WAVE; o <<= 1) {
+    const unsigned long long below = __shfl_up(incl, o, SP_WAVE);
+    if ((int)(tid & 63) >= o) incl += below;
+  }
+  if ((tid & 63) == 63) sh.chunk_sum[tid >> 6] = incl;
   __syncthreads();
-  unsigned long long off = 0;
-  for (int t = 0; t < (int)threadIdx.x; ++t) off += sh.chunk_sum[t];
+  unsigned long long off = incl - s;
+  for (int w = 0; w < (int)(tid >> 6); ++w) off += sh.chunk_sum[w];
   uint32_t cnt = 0;
   if (t_lt >= 0) {
     for (int i = lo; i < hi; ++i) {
@@ -160,22 +166,24 @@ __device__ static __forceinline__ void pivot_row(const PivotArgs& a, PivotRowSha
   const RowShared rsh = rs_carve<THREADS>(lds, nb);
   const int c = head_cluster[h];
   if (!sp_slot_ok(st, c)) return;  // a dense head outside every shared cluster keeps no pattern
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (a caller's loop over rows would keep a dozen addresses made of it in registers)
   // One head per cluster and call: the election flags one, but a caller's own flags may name several heads of a
   // cluster.  The reference stores them one after the other, so the highest head's map is what stays
   // (attention_sharing.py:96-103); here the lower ones leave, or their rows would share the cluster's row counter
   // and accumulators with the highest head's.
-  if (threadIdx.x == 0) sh.last = 0;
+  if (tid == 0) sh.last = 0;
   __syncthreads();
   bool later = false;
-  for (int h2 = h + 1 + threadIdx.x; h2 < hq; h2 += THREADS)
+  for (int h2 = h + 1 + tid; h2 < hq; h2 += THREADS)
     later = later || (decision[h2] == SP_DEC_DENSE && head_cluster[h2] == c);
   if (later) sh.last = 1;
   __syncthreads();
   if (sh.last) return;
   const float* row = avg_attn + ((int64_t)h * nb + r) * nb;
-  const int keep = rs_row_keep<THREADS>(row, nb, a.t_lt, rsh);
+  const int keep = rs_row_keep<THREADS>(row, nb, a.t_lt, rsh, tid);
   uint32_t* prow = reinterpret_cast<uint32_t*>(st.pattern + ((int64_t)c * nb + r) * nbw);
-  for (int w = threadIdx.x; w < nbw * 2; w += THREADS) {
+  for (int w = tid; w < nbw * 2; w += THREADS) {
     uint32_t bits = 0;
     for (int b = 0; b < 32; ++b) {
       const int col = w * 32 + b;
@@ -185,7 +193,7 @@ __device__ static __forceinline__ void pivot_row(const PivotArgs& a, PivotRowSha
     prow[w] = bits;
   }
   // vs_ratio pieces: mass under the pivot's own vertical / slash sets (a block in both counts twice) and the total
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     sh.cov = 0;
     sh.tot = 0;
   }
@@ -194,7 +202,7 @@ __device__ static __forceinline__ void pivot_row(const PivotArgs& a, PivotRowSha
   const uint8_t* dists = st.dists + (int64_t)c * nb;
   unsigned long long cov = 0, tot = 0;
   float* keep_row = st.avg_map ? st.avg_map + ((int64_t)c * nb + r) * nb : nullptr;
-  for (int col = threadIdx.x; col < nb; col += THREADS) {
+  for (int col = tid; col < nb; col += THREADS) {
     const float val = row[col];
     if (keep_row) keep_row[col] = val;  // the pivot's map itself, for get_pivotal_attn
     const unsigned long long fx = sp_to_fixed(val);
@@ -204,7 +212,7 @@ __device__ static __forceinline__ void pivot_row(const PivotArgs& a, PivotRowSha
   if (cov) atomicAdd(&sh.cov, cov);
   if (tot) atomicAdd(&sh.tot, tot);
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     if (sh.cov) atomicAdd(&accum[c * 2 + 0], sh.cov);
     if (sh.tot) atomicAdd(&accum[c * 2 + 1], sh.tot);
     __threadfence();  // this row's pattern words and masses are visible before the row is counted
@@ -216,15 +224,15 @@ __device__ static __forceinline__ void pivot_row(const PivotArgs& a, PivotRowSha
   __threadfence();
   // every out-of-range slash / vertical slot of the reference's id list is the padding id 0
   unsigned long long pad = 0;
-  for (int i = threadIdx.x; i < nb; i += THREADS) {
+  for (int i = tid; i < nb; i += THREADS) {
     if (cols[i]) pad += (unsigned long long)i;
     if (dists[i]) pad += (unsigned long long)i;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) pad += __shfl_xor(pad, o, SP_WAVE);
-  if ((threadIdx.x & 63) == 0) sh.pad[threadIdx.x >> 6] = pad;
+  if ((tid & 63) == 0) sh.pad[tid >> 6] = pad;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     pad = 0;
     for (int w = 0; w < THREADS / SP_WAVE; ++w) pad += sh.pad[w];
     const unsigned long long acc_cov = atomicAdd(&accum[c * 2 + 0], 0ull), acc_tot = atomicAdd(&accum[c * 2 + 1], 0ull);

@@ -337,7 +337,7 @@ def repack_v(v: torch.Tensor, block_size: int, ws: torch.Tensor) -> None:
 
 
 def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=None, avg_attn=None, max_pivots=0,
-                           workspace=None, pair_rows=False, half_channels=False):
+                           workspace=None, pair_rows=False, half_channels=False, pivot=None):
     """q [Hq,N,D], k/v [Hkv,N,D] views, mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D] contiguous.
 
     Reference: triton_block_wise_prefill_attention (shareprefill_attn.py:474-620).  avg_attn (fp32 [Hq,nb,nb],
@@ -348,7 +348,9 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     stream has been made to wait for that); by default the call takes the buffer and repacks itself.
     pair_rows: skip the per-call analysis of which query blocks share a work item (a dense mask has no use for it).
     half_channels: q, k and v are zero beyond channel 64 (a smaller head_dim zero-padded to 128): the kernel skips
-    those channels and leaves channels 64.. of out unwritten."""
+    those channels and leaves channels 64.. of out unwritten.
+    pivot = (state, head_cluster, pattern_threshold), block size 128: pivot_update with decision and avg_attn is part of the
+    launch; DENSE heads beyond max_pivots get NaN for a map and update no pivot."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")
@@ -368,16 +370,20 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     timer = kernel_timer
     if timer is not None:
         timer.start("attn")
-    st = lib.sp_block_sparse_attn_fwd_bf16(_ptr(q), _ptr(k), _ptr(v), n, hq, hkv, d, q.stride(1), q.stride(0),
-                                           k.stride(1), k.stride(0), v.stride(1), v.stride(0), block_size,
-                                           softmax_scale, _ptr(mask), _ptr(decision), _ptr(out), _ptr(avg_attn),
-                                           _ptr(ws), need,
-                                           _lib.SP_ATTN_V_REPACKED | (_lib.SP_ATTN_PAIR_ROWS if pair_rows else 0)
-                                           | (_lib.SP_ATTN_HALF_CHANNELS if half_channels else 0),
-                                           _stream(dev))
+    flags = (_lib.SP_ATTN_V_REPACKED | (_lib.SP_ATTN_PAIR_ROWS if pair_rows else 0)
+             | (_lib.SP_ATTN_HALF_CHANNELS if half_channels else 0))
+    args = (_ptr(q), _ptr(k), _ptr(v), n, hq, hkv, d, q.stride(1), q.stride(0), k.stride(1), k.stride(0), v.stride(1), v.stride(0))
+    rest = (softmax_scale, _ptr(mask), _ptr(decision), _ptr(out), _ptr(avg_attn), _ptr(ws), need, flags)
+    if pivot is None:
+        st, entry = lib.sp_block_sparse_attn_fwd_bf16(*args, block_size, *rest, _stream(dev)), "sp_block_sparse_attn_fwd_bf16"
+    else:
+        assert block_size == 128
+        state, head_cluster, threshold = pivot
+        st = lib.sp_block_sparse_attn_pivot_fwd_bf16(*args, *rest, state.ref(), _ptr(head_cluster), threshold, _stream(dev))
+        entry = "sp_block_sparse_attn_pivot_fwd_bf16"
     if timer is not None:
         timer.stop("attn")
-    _lib.check(st, "sp_block_sparse_attn_fwd_bf16")
+    _lib.check(st, entry)
     return out
 
 

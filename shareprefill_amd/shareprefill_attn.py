@@ -230,6 +230,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
     if not short:
         slab = _lib.load().sp_attn_pivot_scratch_bytes(q_len, block_size)
         max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
+        all_fit = max_pivots == sharing.max_pivots(module.layer_idx, num_heads)
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
     # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
     plan_args = {"scale_dim": model_dim}
@@ -244,16 +245,19 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
             ops.repack_v(v, block_size, ws[0])
     plan = sharing.plan_layer(q, k, module.layer_idx, block_size, minb, maxb, config.pattern_threshold,
                               config.similarity_threshold, config.fallback_threshold, config.queryaware_threshold, **plan_args)
-    update_here = short and getattr(sharing.update_pivotal_attns, "__func__", None) is _UPDATE_PIVOTAL_ATTNS
+    # The attention launch turns the pivots' maps into patterns itself, unless that is the caller's own step, the pivots may be more
+    # than there is room for, or the blocks are smaller than the launch's.
+    update_here = (short or (plan_here and all_fit and block_size == 128)) and (
+        getattr(sharing.update_pivotal_attns, "__func__", None) is _UPDATE_PIVOTAL_ATTNS)
+    pivot = sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold) if update_here else None
     if short:
         out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0],
                                   max_pivots=sharing.max_pivots(module.layer_idx, num_heads) if plan_here else None,
-                                  pivot=sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold)
-                                  if update_here else None)
+                                  pivot=pivot)
     else:
         out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
                                          avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,
-                                         half_channels=model_dim != head_dim)
+                                         half_channels=model_dim != head_dim, pivot=pivot)
     if not update_here:
         sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
     return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
