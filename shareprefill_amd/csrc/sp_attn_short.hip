@@ -134,6 +134,22 @@ __device__ __forceinline__ void as_wait_v(as_u32x2 (&r)[8]) {  // all but the N 
                : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7])
                : "n"(N));
 }
+// The same for a K operand (16 bytes of a lane's row).  Left to itself the compiler waits for each pair of these reads where it
+// uses them.
+template <int IMM>
+__device__ __forceinline__ as_u32x4 as_read_k(uint32_t addr) {
+  as_u32x4 r;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(IMM));
+  return r;
+}
+template <int N>
+__device__ __forceinline__ void as_wait_k(as_u32x4 (&r)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void as_wait_k(as_u32x4 (&r)[2]) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r[0]), "+v"(r[1]) : "n"(N));
+}
 template <int K, int N, typename F>
 __device__ __forceinline__ void as_static_for(F&& f) {
   if constexpr (K < N) {
@@ -261,20 +277,49 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
     }
     const bool diag = c == r;
     if (!diag || half * AS_TILE <= wave * WQ + WQ - 1) {  // (else: every key of the tile lies behind the wave's queries)
-      const char* kt_buf = lds + buf * 2 * TILE_BYTES;
+      // Operands are fetched ahead of the matrix instructions that take them: K two 16-key groups ahead, the first of V's in
+      // front of the softmax, the others a group ahead.  With every operand waited for where it is used a step of a workgroup alone
+      // on its CU took 3800 cycles, ten LDS latencies among them; now 3400 (700 tokens 23.8 -> 22.2 us, 3001 115.4 -> 112.5, 6400
+      // 178 -> 173; 64 channels 1000 tokens 23.5 -> 22.7, 20000 347 -> 342).  Of them the next tile's loads take 700 (32 KiB at the CU's
+      // 64 bytes a cycle); spread between the matrix instructions or put behind them they cost more (700 tokens 24.2 and 23.5).
+      const uint32_t kt_addr = lds_base + (uint32_t)(buf * 2 * TILE_BYTES);
       const uint32_t vt_addr = lds_base + (uint32_t)(buf * 2 * TILE_BYTES + TILE_BYTES + voff);
+      constexpr int GR = CT / 4;  // groups of four channel tiles
+      as_u32x2 vr[2][8];
+      auto fetch_v = [&](auto hc, auto gc) {  // group gc of half hc, into vr[gc & 1] (the first of the next half: where it is free)
+        constexpr int hh = decltype(hc)::value, gi = decltype(gc)::value, to = GR == 1 ? hh & 1 : gi & 1;
+        as_static_for<0, 4>([&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          const uint32_t ad = vt_addr + (uint32_t)(((2 * (4 * gi + u) + vhalf) ^ vswz) << 4);
+          vr[to][2 * u] = as_read_tr<hh * 32 * (D * 2)>(ad);
+          vr[to][2 * u + 1] = as_read_tr<hh * 32 * (D * 2) + 16 * (D * 2)>(ad);
+        });
+      };
       as_floatx4 s[4][QT];
+      {
+        as_u32x4 kr[2][KS];
+        auto fetch_k = [&](auto kc) {
+          constexpr int kt = decltype(kc)::value;
+          as_static_for<0, KS>([&](auto sc) {
+            constexpr int ks = decltype(sc)::value;
+            kr[kt & 1][ks] = as_read_k<kt * 16 * (D * 2)>(kt_addr + (uint32_t)(koff + (((4 * ks + g) ^ kswz) << 4)));
+          });
+        };
+        fetch_k(std::integral_constant<int, 0>{});
+        fetch_k(std::integral_constant<int, 1>{});
+        as_static_for<0, 4>([&](auto kc) {
+          constexpr int kt = decltype(kc)::value;
+          as_wait_k<(kt < 3 ? KS : 0)>(kr[kt & 1]);
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
+          for (int qt = 0; qt < QT; ++qt) s[kt][qt] = (as_floatx4){0, 0, 0, 0};
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) s[kt][qt] = (as_floatx4){0, 0, 0, 0};
+          for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const as_u32x4 raw = *reinterpret_cast<const as_u32x4*>(kt_buf + kt * 16 * (D * 2) + koff + (((4 * ks + g) ^ kswz) << 4));
-#pragma unroll
-          for (int qt = 0; qt < QT; ++qt)
-            s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), qb[qt][ks], s[kt][qt], 0, 0, 0);
-        }
+            for (int qt = 0; qt < QT; ++qt)
+              s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, kr[kt & 1][ks]), qb[qt][ks], s[kt][qt], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (kt + 2 < 4) fetch_k(std::integral_constant<int, kt + 2>{});
+        });
       }
       if (diag) {
 #pragma unroll
@@ -285,6 +330,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
             for (int j = 0; j < 4; ++j)
               if (half * AS_TILE + 16 * kt + 4 * g + j > q_off + 16 * qt) s[kt][qt][j] = -INFINITY;
       }
+      fetch_v(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
       uint32_t pk[QT][8];
       auto softmax = [&](int qt, int hh) {  // half hh: 32 keys
 #pragma unroll
@@ -311,6 +357,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
           for (int i = 4 * hh; i < 4 * hh + 4; i += 2) det |= pk[qt][i] | pk[qt][i + 1];
+        as_wait_v<0>(vr[GR == 1 ? hh & 1 : 0]);  // the half's first group (no read may be in flight across the branch)
         if (__ballot((det & AS_P_TOO_LARGE) != 0u) != 0ull) {
 #pragma unroll
           for (int qt = 0; qt < QT; ++qt) {
@@ -330,33 +377,20 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
           }
         }
         // O += V^T . P: groups of four channel tiles, the next group's operands on their way
-        constexpr int GR = CT / 4;
-        as_u32x2 vr[2][8];
-        auto fetch = [&](auto gc) {
-          constexpr int gi = decltype(gc)::value;
-          as_static_for<0, 4>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            const uint32_t ad = vt_addr + (uint32_t)(((2 * (4 * gi + u) + vhalf) ^ vswz) << 4);
-            vr[gi & 1][2 * u] = as_read_tr<hh * 32 * (D * 2)>(ad);
-            vr[gi & 1][2 * u + 1] = as_read_tr<hh * 32 * (D * 2) + 16 * (D * 2)>(ad);
-          });
-        };
         as_bf16x8 p[QT];
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
           p[qt] = __builtin_bit_cast(as_bf16x8, (as_u32x4){pk[qt][4 * hh], pk[qt][4 * hh + 1], pk[qt][4 * hh + 2], pk[qt][4 * hh + 3]});
-        fetch(std::integral_constant<int, 0>{});
         as_static_for<0, GR>([&](auto gc) {
-          constexpr int gi = decltype(gc)::value;
-          if constexpr (gi + 1 < GR) {
-            fetch(std::integral_constant<int, gi + 1>{});
-            as_wait_v<8>(vr[gi & 1]);
-          } else {
-            as_wait_v<0>(vr[gi & 1]);
-          }
+          constexpr int gi = decltype(gc)::value, from = GR == 1 ? hh & 1 : gi & 1;
+          if constexpr (gi > 0) as_wait_v<0>(vr[from]);
+          if constexpr (gi + 1 < GR)
+            fetch_v(hc, std::integral_constant<int, gi + 1>{});
+          else if constexpr (hh == 0)
+            fetch_v(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{});
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const as_u32x4 raw = __builtin_shufflevector(vr[gi & 1][2 * u], vr[gi & 1][2 * u + 1], 0, 1, 2, 3);
+            const as_u32x4 raw = __builtin_shufflevector(vr[from][2 * u], vr[from][2 * u + 1], 0, 1, 2, 3);
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt)
               o[4 * gi + u][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(as_bf16x8, raw), p[qt], o[4 * gi + u][qt], 0, 0, 0);

@@ -1,0 +1,26 @@
+"""CPU-only check of the generated code of the short-prompt attention kernel: its K operands are fetched by LDS reads in inline
+assembly a group ahead of the matrix instructions, like V's transposing reads (test_isa_hazards.py), and nothing may touch a
+read's registers, and no branch or label stand, between the read and the wait that covers it."""
+
+from test_isa_hazards import _kernels, touched_in_flight
+
+
+def _inline_reads_as_transposing(lines):
+    """The scanner follows transposing reads: the 16-byte reads of inline assembly take their place, the compiler's own (which it
+    waits for itself) and the transposing ones become reads that only count."""
+    out, inline = [], False
+    for l in lines:
+        if l.strip() in (";APP", ";NO_APP", ";;#ASMSTART", ";;#ASMEND"):
+            inline = l.strip() in (";APP", ";;#ASMSTART")
+        l = l.replace("ds_read_b64_tr_b16", "ds_read_b64")
+        out.append(l.replace("ds_read_b128", "ds_read_b64_tr_b16") if inline else l)
+    return out
+
+
+def test_nothing_touches_an_operand_read_in_flight():
+    kernels = _kernels("sp_attn_short.hip", "sp_attn_short_kernel")
+    assert len(kernels) == 4, "64 / 128 channels x with / without the pivots' patterns"
+    for name, body in kernels.items():
+        count, found = touched_in_flight(_inline_reads_as_transposing(body))
+        assert count >= 8
+        assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
