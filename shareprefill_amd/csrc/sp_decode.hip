@@ -18,12 +18,13 @@
 #include "sp_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 #define DC_THREADS 256
 #define DC_TILE 128   // keys per tile
 #define DC_D 128
 #define DC_GMAX 32    // query heads per kv head (the 32-wide operand of the MFMAs); kernels are built for <= 8, 16, 32
-#define DC_PITCH 136  // bf16 elements per LDS row (272 bytes: conflict-free 128-bit reads)
+#define DC_PITCH 136  // bf16 elements per LDS row of 128 (272 bytes: conflict-free 128-bit reads)
 
 typedef uint32_t dc_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 dc_bf16x8 __attribute__((ext_vector_type(8)));
@@ -40,30 +41,33 @@ __device__ static __forceinline__ uint32_t dc_pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, dc_bf16x2));
 }
 
-// thread t fetches chunk t%16 (16 bytes) of rows t/16, t/16+16, ... of a 128-row tile; rows past the end are clamped.
-// d < 128 (a smaller head): the chunks beyond the row's d channels are zeros made here, not read -- the tile in LDS is
-// the row zero-padded to 128 channels, which changes no product.
-// (FULL: d == 128, nothing to pad -- the plain loads of the kernel's own head size)
-template <bool FULL>
+// A tile is 128 rows of D = 64 or 128 channels in chunks of 16 bytes: thread t fetches chunk t % (D / 8) of rows t / (D / 8),
+// + 2048 / D, ...; rows past the end are clamped.  d < D (a smaller head): the chunks beyond the row's d channels are zeros put in on the way
+// into LDS -- the tile there is the row zero-padded to D channels, which changes no product -- and the loads for them read the
+// row's first chunk: a load that only some lanes make is waited for on the spot, and that was each of a tile's sixteen (64
+// channels, us: 131072 keys 98.4 -> 52.6, 8 caches of 4001 24.9 -> 17.2; with half the tile's width besides).
+// (FULL: d == D, nothing to pad)
+template <int D, bool FULL>
 __device__ static __forceinline__ void dc_fetch(const sp_bf16* __restrict__ x, int64_t n, int64_t stride_n, int64_t kb,
-                                               int t, int d, dc_u32x4 (&r)[8]) {
-  const bool real = FULL || (t & 15) * 8 < d;
+                                               int t, int d, dc_u32x4 (&r)[D / 16]) {
+  constexpr int CHUNKS = D / 8;
+  const int chunk = FULL || t % CHUNKS * 8 < d ? t % CHUNKS : 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    int64_t key = kb + i * 16 + (t >> 4);
+  for (int i = 0; i < D / 16; ++i) {
+    int64_t key = kb + i * (DC_THREADS / CHUNKS) + t / CHUNKS;
     if (key > n - 1) key = n - 1;
-    if (FULL) {
-      r[i] = *reinterpret_cast<const dc_u32x4*>(x + key * stride_n + (t & 15) * 8);
-    } else {
-      r[i] = (dc_u32x4){0, 0, 0, 0};
-      if (real) r[i] = *reinterpret_cast<const dc_u32x4*>(x + key * stride_n + (t & 15) * 8);
-    }
+    r[i] = *reinterpret_cast<const dc_u32x4*>(x + key * stride_n + chunk * 8);
   }
 }
 
-__device__ static __forceinline__ void dc_store(sp_bf16* tile, int t, const dc_u32x4 (&r)[8]) {
+template <int D, bool FULL>
+__device__ static __forceinline__ void dc_store(sp_bf16* tile, int t, int d, const dc_u32x4 (&r)[D / 16]) {
+  constexpr int CHUNKS = D / 8;
+  const bool real = FULL || t % CHUNKS * 8 < d;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) *reinterpret_cast<dc_u32x4*>(tile + (i * 16 + (t >> 4)) * DC_PITCH + (t & 15) * 8) = r[i];
+  for (int i = 0; i < D / 16; ++i)
+    *reinterpret_cast<dc_u32x4*>(tile + (i * (DC_THREADS / CHUNKS) + t / CHUNKS) * (D + 8) + t % CHUNKS * 8) =
+        real ? r[i] : (dc_u32x4){0, 0, 0, 0};
 }
 
 // The probabilities enter P.V as bf16, relative to the running max, so it matters where that max starts anew: it does so
@@ -77,33 +81,34 @@ __device__ static __forceinline__ void dc_store(sp_bf16* tile, int t, const dc_u
 struct DcStrides {
   int64_t q_b, q_h, k_b, k_n, k_h, v_b, v_n, v_h;
 };
-template <int G8, bool FULL>
+template <int D, int G8, bool FULL>
 __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const sp_bf16* __restrict__ v, int64_t n, int g,
     int d, DcStrides st, float scale_log2, int64_t keys_per_split, int tiles_per_chunk, float* __restrict__ o_part,
     float2* __restrict__ ml_part, sp_bf16* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) sp_bf16 Ks[DC_TILE * DC_PITCH];
-  __shared__ __attribute__((aligned(16))) sp_bf16 Vs[DC_TILE * DC_PITCH];
+  constexpr int PITCH = D + 8, KS = D / 16, CT = D / 32;  // K and V rows in LDS, channel steps of S, channel tiles of O
+  __shared__ __attribute__((aligned(16))) sp_bf16 Ks[DC_TILE * PITCH];
+  __shared__ __attribute__((aligned(16))) sp_bf16 Vs[DC_TILE * PITCH];
   constexpr int GM = 8 * G8;
   __shared__ __attribute__((aligned(16))) sp_bf16 Ps[GM * DC_PITCH];  // probabilities [head][key]
   __shared__ float wmax[4][GM], wsum[4][GM], alpha_s[GM];
   const int split = blockIdx.x, kvh = blockIdx.y, splits = gridDim.x;
   const int64_t bh = (int64_t)blockIdx.z * gridDim.y + kvh;  // (sequence, kv head)
   const int64_t sk_n = st.k_n, sv_n = st.v_n;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lh = lane & 31, hi = lane >> 5;  // operand column / row inside a 32-wide tile, lane half
   const bool head_ok = lh < g;               // this lane's S^T column is a real head
   const sp_bf16* kh = k + blockIdx.z * st.k_b + kvh * st.k_h;
   const sp_bf16* vh = v + blockIdx.z * st.v_b + kvh * st.v_h;
 
   // B operand of S^T = K . Q^T: column lh = head, k-step ks covers channels 16ks + 8hi .. +7
-  dc_bf16x8 qb[8];
+  dc_bf16x8 qb[KS];
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    dc_u32x4 raw = {0, 0, 0, 0};
-    if (head_ok && (FULL || 16 * ks + 8 * hi < d))
-      raw = *reinterpret_cast<const dc_u32x4*>(q + blockIdx.z * st.q_b + (int64_t)(kvh * g + lh) * st.q_h + 16 * ks + 8 * hi);
-    qb[ks] = __builtin_bit_cast(dc_bf16x8, raw);
+  for (int ks = 0; ks < KS; ++ks) {
+    const bool real = head_ok && (FULL || 16 * ks + 8 * hi < d);
+    const dc_u32x4 raw = *reinterpret_cast<const dc_u32x4*>(q + blockIdx.z * st.q_b + (int64_t)(kvh * g + (head_ok ? lh : 0)) * st.q_h +
+                                                           (real ? 16 * ks + 8 * hi : 0));
+    qb[ks] = __builtin_bit_cast(dc_bf16x8, real ? raw : (dc_u32x4){0, 0, 0, 0});
   }
 
   const int64_t key_begin = (int64_t)split * keys_per_split;
@@ -116,26 +121,26 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
   float o_sum[4 * G8] = {0.f}, m_sum = -INFINITY, l_sum = 0.f;
   bool folded = false;                                                                          // (uniform)
   int tiles_left = tiles_per_chunk - (int)(key_begin / DC_TILE % tiles_per_chunk);  // of the chunk
-  dc_u32x4 kr[8], vr[8];
+  dc_u32x4 kr[D / 16], vr[D / 16];
   if (key_begin < key_end) {
-    dc_fetch<FULL>(kh, n, sk_n, key_begin, t, d, kr);
-    dc_fetch<FULL>(vh, n, sv_n, key_begin, t, d, vr);
+    dc_fetch<D, FULL>(kh, n, sk_n, key_begin, t, d, kr);
+    dc_fetch<D, FULL>(vh, n, sv_n, key_begin, t, d, vr);
   }
   for (int64_t kb = key_begin; kb < key_end; kb += DC_TILE) {
     __syncthreads();  // the previous tile's operand reads are done
-    dc_store(Ks, t, kr);
-    dc_store(Vs, t, vr);
+    dc_store<D, FULL>(Ks, t, d, kr);
+    dc_store<D, FULL>(Vs, t, d, vr);
     __syncthreads();
     if (kb + DC_TILE < key_end) {  // next tile on its way while this one is used
-      dc_fetch<FULL>(kh, n, sk_n, kb + DC_TILE, t, d, kr);
-      dc_fetch<FULL>(vh, n, sv_n, kb + DC_TILE, t, d, vr);
+      dc_fetch<D, FULL>(kh, n, sk_n, kb + DC_TILE, t, d, kr);
+      dc_fetch<D, FULL>(vh, n, sv_n, kb + DC_TILE, t, d, vr);
     }
     // ---- S^T for this wave's 32 keys: acc[r] = logit(key 32*wave + 8(r/4) + 4hi + r%4, head lh) ----
     dc_floatx16 acc = {0};
     {
-      const sp_bf16* arow = Ks + (32 * wave + lh) * DC_PITCH + 8 * hi;
+      const sp_bf16* arow = Ks + (32 * wave + lh) * PITCH + 8 * hi;
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
+      for (int ks = 0; ks < KS; ++ks) {
         const dc_u32x4 raw = *reinterpret_cast<const dc_u32x4*>(arow + 16 * ks);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(dc_bf16x8, raw), qb[ks], acc, 0, 0, 0);
       }
@@ -176,25 +181,25 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
       m_run = m_new;
     }
     // ---- O += P . V for this wave's 32 channels; only accumulator rows of real heads need the rescale ----
+    if (wave < CT) {
 #pragma unroll
-    for (int r = 0; r < 4 * G8; ++r) {
-      const int h = 8 * (r >> 2) + 4 * hi + (r & 3);
-      if (h < g) o[r] *= alpha_s[h];
-    }
-    {
+      for (int r = 0; r < 4 * G8; ++r) {
+        const int h = 8 * (r >> 2) + 4 * hi + (r & 3);
+        if (h < g) o[r] *= alpha_s[h];
+      }
       const sp_bf16* prow = Ps + lh * DC_PITCH + 8 * hi;
       // transposing read: the 16 lanes of a block address 4 key rows x 16 channels (4 lanes x 8 bytes per row) and
       // each lane receives 4 consecutive keys of its channel
-      const sp_bf16* vtr = Vs + (8 * hi + ((lane & 15) >> 2)) * DC_PITCH + 32 * wave + 16 * ((lane >> 4) & 1) +
+      const sp_bf16* vtr = Vs + (8 * hi + ((lane & 15) >> 2)) * PITCH + 32 * wave + 16 * ((lane >> 4) & 1) +
                            4 * (lane & 3);
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) {
         dc_u32x4 praw = {0, 0, 0, 0};
         if (head_ok) praw = *reinterpret_cast<const dc_u32x4*>(prow + 16 * kk);
         const dc_bf16x4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-            (__attribute__((address_space(3))) dc_bf16x4*)(vtr + (16 * kk) * DC_PITCH));
+            (__attribute__((address_space(3))) dc_bf16x4*)(vtr + (16 * kk) * PITCH));
         const dc_bf16x4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-            (__attribute__((address_space(3))) dc_bf16x4*)(vtr + (16 * kk + 4) * DC_PITCH));
+            (__attribute__((address_space(3))) dc_bf16x4*)(vtr + (16 * kk + 4) * PITCH));
         dc_bf16x8 bv;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
 #pragma unroll
     for (int r = 0; r < 4 * G8; ++r) {
       const int h = 8 * (r >> 2) + 4 * hi + (r & 3), c = 32 * wave + lh;
-      if (h < g && c < d) out[(bh * g + h) * d + c] = sp_f32_to_bf16(o[r] / wsum[0][h]);
+      if (wave < CT && h < g && c < d) out[(bh * g + h) * d + c] = sp_f32_to_bf16(o[r] / wsum[0][h]);
     }
     return;
   }
@@ -246,7 +251,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
 #pragma unroll
   for (int r = 0; r < 4 * G8; ++r) {
     const int h = 8 * (r >> 2) + 4 * hi + (r & 3);
-    if (h < g) op[h * DC_D + 32 * wave + lh] = o[r];
+    if (wave < CT && h < g) op[h * DC_D + 32 * wave + lh] = o[r];
   }
   if (wave == 0 && hi == 0 && head_ok) ml_part[(bh * splits + split) * g + lh] = make_float2(m_run, l_run);
 }
@@ -368,29 +373,26 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
   float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
   // A grid's z axis ends at 65535 sequences.  (A batch that large has one workgroup per sequence and kv head: no partials.)
-#define DC_LAUNCH_PARTIAL_(G8, FULL)                                                                                   \
-  for (int64_t b0 = 0; b0 < batch; b0 += DC_MAX_GRID_Z)                                                                \
-  hipLaunchKernelGGL((sp_decode_partial_kernel<G8, FULL>),                                                             \
-                     dim3(splits, hkv, (unsigned)(batch - b0 < DC_MAX_GRID_Z ? batch - b0 : DC_MAX_GRID_Z)),           \
-                     dim3(DC_THREADS), 0, s, (const sp_bf16*)q + b0 * st.q_b, (const sp_bf16*)k + b0 * st.k_b,          \
-                     (const sp_bf16*)v + b0 * st.v_b, n, g, (int)d, st, scale_log2, keys_per_split, tiles_per_chunk,   \
-                     o_part, ml_part, (sp_bf16*)out + b0 * hq * d)
-#define DC_LAUNCH_PARTIAL(G8)     \
-  do {                            \
-    if (d == DC_D)                \
-      DC_LAUNCH_PARTIAL_(G8, true);  \
-    else                          \
-      DC_LAUNCH_PARTIAL_(G8, false); \
-  } while (0)
-  if (g <= 8) {
-    DC_LAUNCH_PARTIAL(1);
-  } else if (g <= 16) {
-    DC_LAUNCH_PARTIAL(2);
-  } else {
-    DC_LAUNCH_PARTIAL(4);
-  }
-#undef DC_LAUNCH_PARTIAL
-#undef DC_LAUNCH_PARTIAL_
+  auto launch = [&](auto kernel) {
+    for (int64_t b0 = 0; b0 < batch; b0 += DC_MAX_GRID_Z)
+      hipLaunchKernelGGL(kernel, dim3(splits, hkv, (unsigned)(batch - b0 < DC_MAX_GRID_Z ? batch - b0 : DC_MAX_GRID_Z)),
+                         dim3(DC_THREADS), 0, s, (const sp_bf16*)q + b0 * st.q_b, (const sp_bf16*)k + b0 * st.k_b,
+                         (const sp_bf16*)v + b0 * st.v_b, n, g, (int)d, st, scale_log2, keys_per_split, tiles_per_chunk,
+                         o_part, ml_part, (sp_bf16*)out + b0 * hq * d);
+  };
+  auto by_width = [&](auto g8) {
+    constexpr int G8 = decltype(g8)::value;
+    if (d > 64)
+      d == 128 ? launch(sp_decode_partial_kernel<128, G8, true>) : launch(sp_decode_partial_kernel<128, G8, false>);
+    else
+      d == 64 ? launch(sp_decode_partial_kernel<64, G8, true>) : launch(sp_decode_partial_kernel<64, G8, false>);
+  };
+  if (g <= 8)
+    by_width(std::integral_constant<int, 1>{});
+  else if (g <= 16)
+    by_width(std::integral_constant<int, 2>{});
+  else
+    by_width(std::integral_constant<int, 4>{});
   SP_LAUNCH_CHECK();
   if (splits == 1) return SP_OK;
   hipLaunchKernelGGL(sp_decode_combine_kernel, dim3((unsigned)((int64_t)batch * hq)), dim3(32 * DC_COMBINE_GROUPS), 0, s,
