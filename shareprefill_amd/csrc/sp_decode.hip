@@ -317,13 +317,22 @@ __global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kern
 // lets a CU hold, and no chunk below one tile of keys.
 #define DC_MAX_GRID_Z 65535
 static_assert(DC_MAX_GRID_Z >= 512, "");  // (the number of chunks is 1 before a batch needs a second launch)
-static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
+static int dc_cut(int32_t batch, int64_t n, int32_t hkv) {
   const int64_t tiles = sp_ceil_div(n, DC_TILE);
   int64_t want = sp_ceil_div(512, (int64_t)hkv * batch);
   if (want > tiles) want = tiles;
   if (want < 1) want = 1;
   if (want > DC_MAX_SPLITS) want = DC_MAX_SPLITS;
   return (int)want;
+}
+
+// Workgroups per (sequence, kv head).  A cache of up to three tiles is walked by one, chunk by chunk, which makes the result itself: a
+// launch less, and no scratch.  A tile takes a workgroup 2.6 us, the second launch costs the host 3.3: one launch against two, us,
+// 200 keys 10.9 / 13.6, 300 11.0 / 13.7 (64 channels 11.2 / 13.9), 400 13.4 / 13.6, 512 13.3 / 13.8 (64 channels 16.7 / 14.0 with waits
+// between its loads), 640 15.9 / 13.7.  (One workgroup of sixteen waves with four tiles at a time: 500 keys 11.1, 1025 18.6.)
+#define DC_ONE_LAUNCH_TILES 3
+static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
+  return n <= DC_ONE_LAUNCH_TILES * DC_TILE ? 1 : dc_cut(batch, n, hkv);
 }
 
 static size_t dc_partial_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
@@ -368,7 +377,7 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
   const int g = hq / hkv;
   const int splits = dc_splits(batch, n, hkv);
   const int64_t keys_per_split = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE;
-  const int tiles_per_chunk = (int)sp_ceil_div(sp_ceil_div(n, dc_splits(1, n, hkv)), DC_TILE);
+  const int tiles_per_chunk = (int)sp_ceil_div(sp_ceil_div(n, dc_cut(1, n, hkv)), DC_TILE);
   float* o_part = (float*)partials;
   float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
   const float scale_log2 = softmax_scale * 1.4426950408889634f;
