@@ -195,6 +195,8 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   const sp_bf16* kh = a.k + (int64_t)kvh * a.sk_h;
   const sp_bf16* vh = a.v + (int64_t)kvh * a.sv_h;
 
+  const int dec = a.slots >= 0 ? a.decision[h] : 0;  // (asked for up here: its way from memory passes under the mask's)
+
   const int q_off = wave * WQ + lq;  // the first of the lane's queries; the others are 16 further each
   const int64_t qrow = (int64_t)r * AS_BS + q_off;
   as_bf16x8 qb[QT][KS];
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   }
   const as_bf16x8 ones = __builtin_bit_cast(as_bf16x8, (as_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
   // pivot heads: this row's sums per block, [column][128 queries], in the slab of the head's rank among them
-  const bool pivot = a.slots >= 0 && a.decision[h] == SP_DEC_DENSE;  // (uniform)
+  const bool pivot = a.slots >= 0 && dec == SP_DEC_DENSE;  // (uniform)
   float* pu = nullptr;
   if (pivot) {
     int slot = 0;

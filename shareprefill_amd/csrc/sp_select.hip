@@ -398,8 +398,8 @@ __device__ static inline void cover_level(CoverShared& sh, GselState& s, int lev
   s.prefix = (prefix << width) | (uint32_t)f_bin;
   s.above += f_above;
   s.rem -= f_mass;
+  s.n_equal = f_cnt;
   if (level == 3) {  // the bin is one value: as many of its entries as the budget left holds
-    s.n_equal = f_cnt;
     const unsigned long long each = sp_to_fixed(__uint_as_float(s.prefix));
     unsigned long long take = each ? s.rem / each : (unsigned long long)f_cnt;
     if (take > f_cnt) take = f_cnt;
@@ -407,12 +407,16 @@ __device__ static inline void cover_level(CoverShared& sh, GselState& s, int lev
   }
 }
 
-template <typename ForEach>
+// COUNT: only the number of entries is wanted.  A bin of one entry then ends the descent: its mass exceeds what is left, so it is
+// not taken (n_take 0).  Of a few thousand entries the third level's bin rarely holds two: layers of 3001 tokens 112.4 -> 110.7 us,
+// 6177 of 64 channels 126.0 -> 123.3, 10007 of 28 heads 243.4 -> 241.3 (with the pivots' decisions asked for earlier in the
+// attention of the first two).
+template <bool COUNT = false, typename ForEach>
 __device__ static inline void cover_descent(CoverShared& sh, GselState& s, ForEach&& for_each) {
   cover_begin(sh);
   // (a loop, not four instances: code that runs once per launch is paid for in instruction fetches)
 #pragma unroll 1
-  for (int level = 0; level < 4 && !s.all; ++level) cover_level(sh, s, level, for_each);  // (uniform)
+  for (int level = 0; level < 4 && !s.all && !(COUNT && s.n_equal == 1); ++level) cover_level(sh, s, level, for_each);  // (uniform)
 }
 
 // flat vectors (score_cover_topk, the budgets): vectors 0..n0-1 are rows of x0, the others rows of x1
@@ -446,9 +450,9 @@ __device__ static void cover_count_vector(CoverShared& sh, const CoverCountArgs&
     };
     if (len <= CS_ITEMS * CS_THREADS) {
       load(0);
-      cover_descent(sh, s, [&](auto&& f) { each(0, f); });
+      cover_descent<true>(sh, s, [&](auto&& f) { each(0, f); });
     } else {
-      cover_descent(sh, s, [&](auto&& f) {
+      cover_descent<true>(sh, s, [&](auto&& f) {
         for (int i0 = 0; i0 < len; i0 += CS_ITEMS * CS_THREADS) {
           load(i0);
           each(i0, f);
