@@ -87,7 +87,7 @@ class AttentionSharing:
             if cid in self.shared_clusters:
                 self._slot[cid] = len(self._slot)
         self._state: Optional[ops.ClusterState] = None
-        self._head_cluster: Dict[Tuple[int, int, str], torch.Tensor] = {}
+        self._head_cluster: Dict[Tuple[int, int, torch.device], torch.Tensor] = {}
         # keep every pivot's block-average map in the device state for get_pivotal_attn (fp32 [nb, nb] per shared
         # cluster), unless all of them together exceed pivot_map_limit_bytes
         self.keep_pivot_maps = True
@@ -97,7 +97,7 @@ class AttentionSharing:
         # one LayerPlan per layer planned since the last reset; unless keep_plans / keep_debug is set only the
         # newest one still holds its mask, the older ones keep their few per-head integers
         self.plans: List[LayerPlan] = []
-        self._scratch: Dict[Tuple[str, str], torch.Tensor] = {}
+        self._scratch: Dict[torch.device, Tuple[torch.Tensor, torch.Tensor]] = {}
         self._max_pivots: Dict[Tuple[int, int], int] = {}
         self.reset_state()
 
@@ -118,7 +118,7 @@ class AttentionSharing:
         return self._pair_to_cluster.get((int(layer), int(head)))
 
     def _head_cluster_tensor(self, layer_idx: int, hq: int, device) -> torch.Tensor:
-        key = (layer_idx, hq, str(device))
+        key = (layer_idx, hq, device)
         t = self._head_cluster.get(key)
         if t is None:
             slots = [self._slot.get(self._pair_to_cluster.get((layer_idx, h)), -1) for h in range(hq)]
@@ -227,13 +227,15 @@ class AttentionSharing:
     def _qa_scratch(self, hq: int, nb: int, device) -> torch.Tensor:
         """fp32 [Hq, nb, nb] scratch of the query-aware selection, owned by this object (one model, one stream of
         layers in order), grow-only, reused by every layer."""
-        need = hq * nb * nb * 4
-        key = ("qa_probs", str(device))
-        buf = self._scratch.get(key)
+        need = hq * nb * nb
+        buf, view = self._scratch.get(device, (None, None))
         if buf is None or buf.numel() < need:
-            buf = torch.empty(max(need, 16), dtype=torch.uint8, device=device)
-            self._scratch[key] = buf
-        return buf[:need].view(torch.float32).view(hq, nb, nb)
+            buf = torch.empty(max(need, 4), dtype=torch.float32, device=device)
+            view = None
+        if view is None or tuple(view.shape) != (hq, nb, nb):
+            view = buf[:need].view(hq, nb, nb)
+            self._scratch[device] = (buf, view)
+        return view
 
     def get_active_blocks(self, q, k, layer_idx, num_heads, block_size, min_budget, max_budget,
                           pattern_threshold=0.9, similarity_threshold=0.5, fallback_threshold=0.9,

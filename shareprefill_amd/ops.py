@@ -42,7 +42,14 @@ def _ptr(t: Optional[torch.Tensor]) -> C.c_void_p:
     return C.c_void_p(0 if t is None else t.data_ptr())
 
 
+def _addr(t: Optional[torch.Tensor]) -> Optional[int]:
+    """_ptr without the object: what the binding's argument types turn into a pointer themselves."""
+    return None if t is None else t.data_ptr()
+
+
 def _check_hnd(t: torch.Tensor, name: str):
+    if t.dtype is torch.bfloat16 and t.is_cuda and len(t.shape) == 3 and t.stride(2) == 1:
+        return
     if t.dim() != 3:
         raise ValueError(f"{name} must be [H, N, D], got {tuple(t.shape)}")
     if t.dtype != torch.bfloat16:
@@ -269,17 +276,20 @@ def select_layer(state: ClusterState, head_cluster, layer_idx, q, k, block_size,
     scratch = torch.empty(need, dtype=torch.uint8, device=dev)
     mask = torch.empty(hq, nb, (nb + 63) // 64, dtype=torch.int64, device=dev)
     per_head = torch.empty(5, hq, dtype=torch.int32, device=dev)
-    args = (_ptr(q), _ptr(k), n, hq, hkv, d, q.stride(1), q.stride(0), k.stride(1), k.stride(0), block_size, flags, state.ref(),
-            _ptr(head_cluster), layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold,
-            queryaware_threshold, _ptr(scratch), need, _ptr(qa_probs), _ptr(per_head), _ptr(mask), _ptr(avg_attn))
+    (q_h, q_n, _), (k_h, k_n, _) = q.stride(), k.stride()
+    args = (q.data_ptr(), k.data_ptr(), n, hq, hkv, d, q_n, q_h, k_n, k_h, block_size, flags, state.ref(),
+            _addr(head_cluster), layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold,
+            fallback_threshold, queryaware_threshold, scratch.data_ptr(), need, _addr(qa_probs), per_head.data_ptr(),
+            mask.data_ptr(), _addr(avg_attn))
     if repack is None:
-        st, entry = lib.sp_select_layer_bf16(*args, _stream(dev)), "sp_select_layer_bf16"
+        st, entry = lib.sp_select_layer_bf16(*args, _stream_handle(dev)), "sp_select_layer_bf16"
     else:
         v, ws = repack
         _check_hnd(v, "v")
         if tuple(v.shape) != (hkv, n, d):
             raise ValueError(f"v {tuple(v.shape)} does not match k {tuple(k.shape)}")
-        st = lib.sp_select_layer_repack_bf16(*args, _ptr(v), v.stride(1), v.stride(0), _ptr(ws), ws.numel(), _stream(dev))
+        st = lib.sp_select_layer_repack_bf16(*args, v.data_ptr(), v.stride(1), v.stride(0), ws.data_ptr(), ws.numel(),
+                                             _stream_handle(dev))
         entry = "sp_select_layer_repack_bf16"
     _lib.check(st, entry)
     floats = None
@@ -411,9 +421,9 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, 
     timer = kernel_timer
     if timer is not None:
         timer.start("attn")
-    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), n, hq, k.shape[0], d, q.stride(1), q.stride(0), k.stride(1), k.stride(0),
-            v.stride(1), v.stride(0), softmax_scale, mask.data_ptr(), _ptr(decision), out.data_ptr(), _ptr(avg_attn), _ptr(ws),
-            ws_bytes)
+    (q_h, q_n, _), (k_h, k_n, _), (v_h, v_n, _) = q.stride(), k.stride(), v.stride()
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), n, hq, k.shape[0], d, q_n, q_h, k_n, k_h, v_n, v_h, softmax_scale,
+            mask.data_ptr(), _addr(decision), out.data_ptr(), _addr(avg_attn), _addr(ws), ws_bytes)
     if pivot is None:
         st, entry = lib.sp_short_attn_fwd_bf16(*args, stream), "sp_short_attn_fwd_bf16"
     else:
@@ -481,11 +491,12 @@ def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, so
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} do not match q {tuple(q.shape)}")
     stream = _stream_handle(dev)
     out = torch.empty((b, 1, hq, d), dtype=torch.bfloat16, device=dev)
-    ws = _workspace("decode", lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv), dev)
+    need = lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv)
+    ws = _workspace("decode", need, dev) if need else out  # (nothing is kept: any address will do)
     if b == 1:
         q_b = k_b = v_b = 0  # (the stride of an axis of one entry means nothing)
     st = lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b, n, hq, hkv, d, q_b, q_h, k_b, k_n, k_h,
-                                       v_b, v_n, v_h, softmax_scale, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+                                       v_b, v_n, v_h, softmax_scale, out.data_ptr(), ws.data_ptr(), ws.numel() if need else 0, stream)
     _lib.check(st, "sp_decode_attn_batch_bf16")
     return out
 

@@ -163,19 +163,25 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
     Prefill (N != 1): vertical/slash estimation, block selection and sharing, block-sparse attention,
     pivot update (shareprefill_attn.py:110-144).  Decode (N == 1): dense attention of the one query over
     all keys (:146-155)."""
-    bsz, num_heads, q_len, model_dim = query_states.shape
-    config = module.config
-    softmax_scale = getattr(module, "scaling", 1.0 / math.sqrt(model_dim))
+    _, _, q_len, _ = query_states.shape
+    if q_len == 1:
+        return _decode_step(module, query_states, key_states, value_states).transpose(1, 2), None
     # gqa_interleave is accepted and changes nothing, as in the reference: there K and V are expanded to the query
     # head count before anything else, by repeat_interleave (True) or by expand + reshape (False) -- both give query
     # head h the kv head h // g (shareprefill_attn.py:33-40, 77-82) -- and everything after sees one kv head per query
     # head, so neither the selection's einsum (attention_sharing.py:128-151) nor the kernel's head mapping
     # (shareprefill_attn.py:333-336) can tell the two settings apart.  Here K and V stay un-expanded and are indexed h // g.
     del gqa_interleave
+    out, avg_attn = _prefill_layer(module, query_states, key_states, value_states)
+    return out.transpose(1, 2), avg_attn
 
-    if q_len == 1:
-        return _decode_step(module, query_states, key_states, value_states).transpose(1, 2), None
 
+def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor
+                   ) -> Tuple[torch.Tensor, torch.Tensor]:
+    """-> (attn_output [1, N, Hq, D] as the kernels write it, block-average maps)."""
+    bsz, num_heads, q_len, model_dim = query_states.shape
+    config = module.config
+    softmax_scale = getattr(module, "scaling", 1.0 / math.sqrt(model_dim))
     if bsz != 1:
         raise ValueError("SharePrefill prefill keeps per-cluster state for batch size 1 only")
     assert query_states.dtype == torch.bfloat16, "SharePrefill attention expects bfloat16 q/k/v"
@@ -222,7 +228,7 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
                                              half_channels=model_dim != head_dim)
         if q_len >= block_size:
             sharing.note_dense_layer(module.layer_idx, num_heads, nb)
-        return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
+        return _first_channels(out.unsqueeze(0), model_dim), avg_attn
 
     # Room for the block sums of this layer's possible pivots (at most 16 GiB of it; pivots beyond that take the
     # recomputing pass).  How many heads can become pivots is known from the table alone.
@@ -260,7 +266,11 @@ def shareprefill_attention_core(module, query_states: torch.Tensor, key_states: 
                                          half_channels=model_dim != head_dim, pivot=pivot)
     if not update_here:
         sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
-    return out.unsqueeze(0).transpose(1, 2)[..., :model_dim], avg_attn
+    return _first_channels(out.unsqueeze(0), model_dim), avg_attn
+
+
+def _first_channels(out: torch.Tensor, model_dim: int) -> torch.Tensor:
+    return out if out.shape[-1] == model_dim else out[..., :model_dim]
 
 
 def shareprefill_attention_forward(module, query_states: torch.Tensor, key_states: torch.Tensor,
@@ -276,6 +286,12 @@ def shareprefill_attention_forward(module, query_states: torch.Tensor, key_state
     gqa_interleave = kwargs.pop("gqa_interleave", False)
     if query_states.dim() == 4 and query_states.shape[2] == 1:
         return _decode_step(module, query_states, key_states, value_states), None  # (in the layout wanted here)
-    attn_output, attn_weights = shareprefill_attention_core(module, query_states, key_states, value_states,
-                                                            gqa_interleave=gqa_interleave)
-    return attn_output.transpose(1, 2).contiguous(), attn_weights
+    if shareprefill_attention_core is not _CORE:  # (a caller's own is called, as it would be by name)
+        attn_output, attn_weights = shareprefill_attention_core(module, query_states, key_states, value_states,
+                                                                gqa_interleave=gqa_interleave)
+        return attn_output.transpose(1, 2).contiguous(), attn_weights
+    attn_output, attn_weights = _prefill_layer(module, query_states, key_states, value_states)
+    return attn_output.contiguous(), attn_weights
+
+
+_CORE = shareprefill_attention_core
