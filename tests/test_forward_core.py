@@ -18,6 +18,6 @@ def test_a_callers_core_is_called(monkeypatch, n):
 
     monkeypatch.setattr(sa, "shareprefill_attention_core", core)
     q = torch.randn(1, 4, n, 8)
-    out, _ = sa.shareprefill_attention_forward(types.SimpleNamespace(), q, q, q, None, gqa_interleave=True)
+    out, _ = sa.shareprefill_attention_forward(types.SimpleNamespace(), q, q, q, None, scaling=1.0, gqa_interleave=True)
     assert seen == [True] and out.is_contiguous()
     torch.testing.assert_close(out, (q + 1).transpose(1, 2), rtol=0, atol=0)
