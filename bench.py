@@ -80,20 +80,24 @@ def stream_ms(fn, calls=10):
     return event_ms(lambda: [fn() for _ in range(calls)]) / calls
 
 
-def selection_ms(sharing, w, q, k, pt, layer=1):
-    """The whole selection of a layer as the layer runs it: one call, with the map that the attention fills cleared on the way."""
+def selection_ms(sharing, w, q, k, v, pt, layer=1):
+    """The whole selection of a layer as the layer runs it: one call, with the map that the attention fills cleared and V
+    repacked on the way."""
     import torch
 
+    from shareprefill_amd import ops
     from shareprefill_amd.attention_sharing import budget_blocks
 
     n = q.shape[2]
+    ws, _ = ops.attention_workspace(n, w.hq, w.hkv, w.head_dim, w.block_size, q.device)
     nb = -(-n // w.block_size)
     minb, maxb = budget_blocks(w.min_budget, None, w.block_size)
     avg_attn = torch.empty(w.hq, nb, nb, dtype=torch.float32, device=q.device)
     keep, sharing.keep_plans = sharing.keep_plans, True  # (the layer's own plan keeps its mask)
     plans = len(sharing.plans)
     ms = stream_ms(lambda: sharing.plan_layer(q[0], k[0], layer, w.block_size, minb, maxb, pt, w.similarity_threshold,
-                                              w.fallback_threshold, w.queryaware_threshold, avg_attn=avg_attn))
+                                              w.fallback_threshold, w.queryaware_threshold, avg_attn=avg_attn,
+                                              repack=(v[0], ws)))
     del sharing.plans[plans:]
     sharing.keep_plans = keep
     return ms
@@ -162,7 +166,7 @@ def cpu_baseline(w, q, k, v, mask_bool, decision, kept_blocks, pt):
 # reported only while shareprefill_amd/csrc/sp_attn.hip still has that hash, and is null (with a note) after any
 # change to the kernel until the profile is taken again.
 MEASURED_ATTN_TRAFFIC = {
-    ("C3", 0.95): {"bytes": int((101.9 + 1.0) * 2 ** 30), "sp_attn_hip_sha256_16": "e4aef906bd97d206",
+    ("C3", 0.95): {"bytes": int((102.0 + 1.0) * 2 ** 30), "sp_attn_hip_sha256_16": "0c91f1b5e29ee27c",
                    "profile": "profiles/attention_layer_C3_hbm_traffic.txt"},
 }
 
@@ -456,8 +460,9 @@ def timed_layer_point(w, q, k, v, table, pt, steps=5, n_tokens=None, with_stages
         st["pool_k"] = event_ms(lambda: ops.pool_avg(kh, w.block_size))
         kbar = ops.pool_avg(kh, w.block_size)
         st["queryaware_test"] = event_ms(lambda: ops.queryaware_test(qh, kbar, vb, w.block_size, w.queryaware_threshold))
+        st["repack_v"] = repack_ms(v, w)
         out["stages_alone_ms"] = {a: round(b, 3) for a, b in st.items()}
-        parts = {"selection": selection_ms(sh, w, q, k, pt), "repack_v": repack_ms(v, w), "attention": ams}
+        parts = {"selection_and_repack_v": selection_ms(sh, w, q, k, v, pt), "attention": ams}
         parts["rest_of_layer"] = ms - sum(parts.values())
         out["stage_ms"] = {a: round(b, 3) for a, b in parts.items()}
     return out
@@ -588,9 +593,10 @@ def main():
         stages["pool_q_all_heads"] = event_ms(lambda: ops.pool_avg(qh, 128))
         kbar = ops.pool_avg(kh, 128)
         stages["queryaware_test"] = event_ms(lambda: ops.queryaware_test(qh, kbar, vb, 128, w.queryaware_threshold))
+        stages["repack_v"] = repack_ms(v, w)
         line["stages_alone_ms"] = {a: round(b, 3) for a, b in stages.items()}
-        # (the stages above are entry points of their own; a layer's selection is one call of fewer launches)
-        parts = {"selection": selection_ms(sharing, w, q, k, pt), "repack_v": repack_ms(v, w), "attention": attn_avg_ms}
+        # (the stages above are entry points of their own; a layer's selection is one call of fewer launches, V's repack in one)
+        parts = {"selection_and_repack_v": selection_ms(sharing, w, q, k, v, pt), "attention": attn_avg_ms}
         parts["rest_of_layer"] = ms_per_step - sum(parts.values())
         line["stage_ms"] = {a: round(b, 3) for a, b in parts.items()}
         kbytes = w.seq_len * w.hkv * w.head_dim * 2 + nb * w.hkv * w.head_dim * 2

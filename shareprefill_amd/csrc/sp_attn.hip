@@ -1265,15 +1265,15 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
   }
 }
 
-// Before the forward launches, in one launch: clears the queue tickets, hands out the pivot slots, chooses the pairing
-// and, for launches of few gangs, ranks them.
+// Before the forward launch: clears the queue tickets, hands out the pivot slots, chooses the pairing and, for launches of few
+// gangs, weighs them.
 //   slots   : the first max_pivots heads whose decision is DENSE get one for their block sums (ascending head order),
 //             every other head AT_NO_SLOT;
 //   pairing : for every two adjacent heads (2i, 2i+1), how the forward kernel pairs query blocks into work items, from
 //             the union sizes both ways over all rows,
 //               rows : |row 2p  |  row 2p+1| of each head,      heads : |row r of head 2i  |  row r of head 2i+1|:
 //             by heads when that union is strictly smaller and the two heads may share an item (same kv head, neither
-//             runs in the pivot launch);
+//             a pivot that keeps its block sums);
 //   weights : the work of every gang that is ranked -- the blocks its items' two rows visit together, plus a few blocks' worth of
 //             fixed time per item.
 // Integer sums throughout, so nothing depends on the order of anything.
@@ -1608,7 +1608,7 @@ __global__ __launch_bounds__(AT_THREADS) void sp_attn_avg_fine_kernel(
 }
 
 // ---- host ---------------------------------------------------------------------------------------------
-// workspace layout: [ repacked V^T : hkv*nb*128*128 bf16 | scheduler area : 1 KiB of slots + 2 KiB order table |
+// workspace layout: [ repacked V^T : hkv*nb*128*128 bf16 | scheduler area : 1 KiB of slots + 2 KiB of gang weights |
 //                     row statistics : hq*n float2 ]
 // (the tiles are 128 keys wide whatever the caller's block size)
 static size_t at_vt_bytes(int64_t n, int32_t hkv, int32_t d, int32_t bs) {
