@@ -1243,6 +1243,16 @@ __global__ __launch_bounds__(2 * SP_WAVE) void sp_share_similarity_kernel(
   if (lane == 0) (wave == 0 ? js_v : js_s)[h] = js;
 }
 
+// the cluster's pivot is this head, elected in this layer
+__device__ static __forceinline__ bool share_elected(const sp_cluster_state& st, int c, int h, int layer_idx) {
+  return sp_slot_ok(st, c) && st.info[c * 8 + 0] == h && st.info[c * 8 + 4] == layer_idx;
+}
+__device__ static __forceinline__ void share_elect(const sp_cluster_state& st, int c, int h, int layer_idx, int nv, int ns) {
+  st.info[c * 8 + 0] = h;
+  st.info[c * 8 + 2] = nv;
+  st.info[c * 8 + 3] = ns;
+  st.info[c * 8 + 4] = layer_idx;
+}
 __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, int layer_idx, int hq,
     const int32_t* __restrict__ use_qa, const int32_t* __restrict__ nv, const int32_t* __restrict__ ns, int minb,
@@ -1275,10 +1285,7 @@ __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
     bool first = true;
     for (int h2 = 0; h2 < h; ++h2) first = first && !(s_cand[h2] && s_slot[h2] == c);
     if (first) {
-      st.info[c * 8 + 0] = h;
-      st.info[c * 8 + 2] = nv[h];
-      st.info[c * 8 + 3] = ns[h];
-      st.info[c * 8 + 4] = layer_idx;
+      share_elect(st, c, h, layer_idx, nv[h], ns[h]);
       dec = SP_DEC_DENSE;
     }
   } else if (member && st.info[c * 8 + 1] != 0) {
@@ -1290,13 +1297,12 @@ __global__ __launch_bounds__(DEC_MAX_HEADS) void sp_share_decide_kernel(
   ns_f[h] = reset ? minb : ns[h];
 }
 
-// a newly elected pivot (the cluster's pivot is this head, elected in this layer) keeps its pooled vectors and its own
+// a newly elected pivot keeps its pooled vectors and its own
 // vertical-slash sets (:223-263); every thread of the workgroup calls it
-__device__ static __forceinline__ void share_keep(const sp_cluster_state& st, int c, int h, int layer_idx,
+__device__ static __forceinline__ void share_keep(const sp_cluster_state& st, int c, int h,
                                                   const float* __restrict__ vert_blk, const float* __restrict__ slash_blk,
                                                   int nv, int ns, uint32_t* keys, int nthreads) {
   const int nb = st.nb;
-  if (!sp_slot_ok(st, c) || st.info[c * 8 + 0] != h || st.info[c * 8 + 4] != layer_idx) return;  // (uniform)
   for (int i = threadIdx.x; i < nb; i += nthreads) {
     st.vert[(int64_t)c * nb + i] = vert_blk[(int64_t)h * nb + i];
     st.slash[(int64_t)c * nb + i] = slash_blk[(int64_t)h * nb + i];
@@ -1310,8 +1316,8 @@ __global__ __launch_bounds__(DEC_THREADS) void sp_share_keep_kernel(
     const int32_t* __restrict__ nv, const int32_t* __restrict__ ns) {
   __shared__ __attribute__((aligned(16))) uint32_t s_keys[RS_MAX];
   const int h = blockIdx.x;
-  if (decision[h] != SP_DEC_DENSE) return;
-  share_keep(st, head_cluster[h], h, layer_idx, vert_blk, slash_blk, nv[h], ns[h], s_keys, DEC_THREADS);
+  if (decision[h] != SP_DEC_DENSE || !share_elected(st, head_cluster[h], h, layer_idx)) return;  // (uniform)
+  share_keep(st, head_cluster[h], h, vert_blk, slash_blk, nv[h], ns[h], s_keys, DEC_THREADS);
 }
 
 extern "C" int sp_share_decide(const sp_cluster_state* state, const int32_t* head_cluster, int32_t layer_idx,
@@ -1353,7 +1359,28 @@ struct MaskBesides {
   int layer_idx;    // pivots elected in this layer store their vectors and sets
   PoolArgs qpool;   // query-aware heads: the averages of Q's blocks
   float* zero;      // [hq][nb][nb] cleared, or null
+  // the decisions themselves, where the launch makes them
+  const int32_t *use_qa, *nv, *ns;
+  int minb;
+  float sim_thr;
+  double fb_thr;
+  int32_t *decision, *nv_f, *ns_f;
+  float *js_v, *js_s;
 };
+// sp_share_decide_kernel's decision for head h, by every workgroup of the head for itself: "first" only looks at lower heads of its
+// cluster that are not query-aware.  The state stays as the previous layers left it until the next launch (share_elect in
+// sp_queryaware_small_kernel), so no workgroup can see another's election.  Every thread of the workgroup calls it.
+__device__ static __forceinline__ int mask_decide(const sp_cluster_state& st, const int32_t* __restrict__ head_cluster, int h,
+                                                  const MaskBesides& a) {
+  const int t = threadIdx.x, c = head_cluster[h], qa = a.use_qa[h];
+  const int tc = t < h ? head_cluster[t] : 0, tqa = t < h ? a.use_qa[t] : 1;
+  const float js_v = a.js_v[h], js_s = a.js_s[h];
+  if (qa) return SP_DEC_QA;
+  if (!sp_slot_ok(st, c)) return SP_DEC_VS;
+  const int pivot = st.info[c * 8 + 0], pattern = st.info[c * 8 + 1];
+  if (pivot < 0) return __syncthreads_or(t < h && tc == c && !tqa) ? SP_DEC_VS : SP_DEC_DENSE;
+  return pattern != 0 && js_v < a.sim_thr && js_s < a.sim_thr && st.ratio[c] < a.fb_thr ? SP_DEC_SHARE : SP_DEC_VS;
+}
 // q blocks of one query-aware head, share `part_no` of MASK_SPLIT: a chunk of 8 channels by four waves, 64 / (d / 8) blocks
 // at a time for each four waves
 __device__ static void mask_pool_q(const PoolArgs& a, int h, int nb, int part_no, char* lds) {
@@ -1378,8 +1405,9 @@ __device__ static void mask_pool_q(const PoolArgs& a, int h, int nb, int part_no
   }
 }
 
-// BESIDES: grid (hq, 2 MASK_SPLIT), the second half of which pools and clears
-template <bool BESIDES>
+// BESIDES: grid (hq, 2 MASK_SPLIT), the second half of which pools and clears.  DECIDE (up to 128 blocks): the launch makes the
+// decisions too.
+template <bool BESIDES, bool DECIDE>
 __global__ __launch_bounds__(MASK_THREADS) void sp_build_mask_kernel(
     sp_cluster_state st, const int32_t* __restrict__ head_cluster, const int32_t* __restrict__ decision,
     const float* __restrict__ vert_blk, const float* __restrict__ slash_blk, const int32_t* __restrict__ nv_f,
@@ -1387,10 +1415,29 @@ __global__ __launch_bounds__(MASK_THREADS) void sp_build_mask_kernel(
   __shared__ __attribute__((aligned(16))) uint32_t s_keys[BESIDES ? MASK_THREADS * 8 : RS_MAX];
   __shared__ uint8_t s_cols[RS_MAX], s_dists[RS_MAX];
   const int h = blockIdx.x;
-  const int dec = decision[h];
+  const bool pools = BESIDES && blockIdx.y >= MASK_SPLIT;
+  int dec, n_v = 0, n_s = 0;
+  if constexpr (DECIDE) {
+    static_assert(BESIDES && MASK_THREADS >= DEC_MAX_HEADS, "");
+    dec = pools ? (extra.use_qa[h] ? SP_DEC_QA : SP_DEC_VS) : mask_decide(st, head_cluster, h, extra);
+    if (!pools) {
+      const bool reset = dec == SP_DEC_QA || dec == SP_DEC_SHARE;
+      n_v = reset ? extra.minb : extra.nv[h];
+      n_s = reset ? extra.minb : extra.ns[h];
+      if (blockIdx.y == 0 && threadIdx.x == 0) {
+        extra.decision[h] = dec;
+        extra.nv_f[h] = n_v;
+        extra.ns_f[h] = n_s;
+        if (dec == SP_DEC_QA) extra.js_v[h] = extra.js_s[h] = NAN;  // (formed beside the query-aware test for every head)
+      }
+    }
+  } else {
+    dec = decision[h];
+    if (!pools) n_v = nv_f[h], n_s = ns_f[h];
+  }
   if constexpr (BESIDES) {
     static_assert(MASK_THREADS * 8 >= RS_MAX, "");
-    if (blockIdx.y >= MASK_SPLIT) {
+    if (pools) {
       const int part_no = blockIdx.y - MASK_SPLIT;
       if (extra.zero != nullptr) {  // (in shares of the whole array: a head's part is 4-byte aligned only)
         const int64_t all = (int64_t)gridDim.x * nb * nb, shares = (int64_t)gridDim.x * MASK_SPLIT;
@@ -1403,11 +1450,11 @@ __global__ __launch_bounds__(MASK_THREADS) void sp_build_mask_kernel(
       if (dec == SP_DEC_QA) mask_pool_q(extra.qpool, h, nb, part_no, reinterpret_cast<char*>(s_keys));
       return;
     }
-    if (dec == SP_DEC_DENSE && blockIdx.y == 0)  // (nothing in this launch reads what it writes)
-      share_keep(st, head_cluster[h], h, extra.layer_idx, vert_blk, slash_blk, nv_f[h], ns_f[h], s_keys, MASK_THREADS);
+    if (dec == SP_DEC_DENSE && blockIdx.y == 0 && (DECIDE || share_elected(st, head_cluster[h], h, extra.layer_idx)))
+      share_keep(st, head_cluster[h], h, vert_blk, slash_blk, n_v, n_s, s_keys, MASK_THREADS);  // (nothing here reads what it writes)
   }
   if (dec != SP_DEC_DENSE)
-    vs_sets(vert_blk + (int64_t)h * nb, slash_blk + (int64_t)h * nb, nb, nv_f[h], ns_f[h], s_keys, s_cols, s_dists,
+    vs_sets(vert_blk + (int64_t)h * nb, slash_blk + (int64_t)h * nb, nb, n_v, n_s, s_keys, s_cols, s_dists,
             MASK_THREADS);
   const uint64_t* pat = nullptr;
   // a SHARE decision without a valid slot (only a caller's own decision vector can hold one) adds no pattern
@@ -1465,7 +1512,7 @@ extern "C" int sp_build_mask(const sp_cluster_state* state, const int32_t* head_
              SP_ERR_INVALID_ARGUMENT, "sp_build_mask: null pointer");
   SP_REQUIRE(hq > 0 && nb > 0 && nb <= RS_MAX, SP_ERR_UNSUPPORTED, "sp_build_mask: nb=%d unsupported (max %d)", nb,
              RS_MAX);
-  hipLaunchKernelGGL(sp_build_mask_kernel<false>, dim3(hq, MASK_SPLIT), dim3(MASK_THREADS), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL((sp_build_mask_kernel<false, false>), dim3(hq, MASK_SPLIT), dim3(MASK_THREADS), 0, (hipStream_t)stream,
                      state_by_value(state), head_cluster, decision, vert_blk, slash_blk, nv_final, ns_final, nb, (nb + 63) / 64, mask,
                      MaskBesides{});
   SP_LAUNCH_CHECK();
@@ -1544,11 +1591,17 @@ __global__ __launch_bounds__(BP_THREADS) void sp_block_probs_kernel(
 // row tiles are workgroups of a launch of their own.  Bound by latency (one K tile, two passes over it, the descent's
 // barriers) and, in layers without a query-aware head, by being a launch at all: against two launches a layer without one takes
 // 2 us less (3001 tokens, 6177 of 64 channels, 10007 of 28 / 4 heads), one with all 32 heads query-aware 3 us (8192 tokens).
+struct ElectArgs {  // pivots that the mask launch has decided on and the state does not know yet (st.info null: none)
+  sp_cluster_state st;
+  const int32_t *head_cluster, *nv, *ns;
+  int layer_idx;
+};
 template <int D>
 __global__ __launch_bounds__(CS_THREADS) void sp_queryaware_small_kernel(const sp_bf16* qbar, const sp_bf16* kbar,
                                                                          const int32_t* __restrict__ decision, int hq, int hkv,
                                                                          int nb, int nbw, uint32_t flags, float inv_sqrt_d,
-                                                                         float* probs, long long t_le, uint64_t* mask) {
+                                                                         float* probs, long long t_le, uint64_t* mask,
+                                                                         ElectArgs elect) {
   __shared__ union {
     BpmLds<D> rows;
     struct {
@@ -1557,8 +1610,10 @@ __global__ __launch_bounds__(CS_THREADS) void sp_queryaware_small_kernel(const s
     } sel;
   } lds;
   static_assert(CS_THREADS % BPM_THREADS == 0 && LQ_TILE <= GSEL_ONE_NB, "");
-  const int h = blockIdx.x;
-  if (decision[h] != SP_DEC_QA) return;
+  const int h = blockIdx.x, dec = decision[h];
+  if (dec == SP_DEC_DENSE && elect.st.info != nullptr && threadIdx.x == 0)
+    share_elect(elect.st, elect.head_cluster[h], h, elect.layer_idx, elect.nv[h], elect.ns[h]);
+  if (dec != SP_DEC_QA) return;
   bpm_rows<D, CS_THREADS / BPM_THREADS>(lds.rows, qbar, kbar, 0, h, hq, hkv, nb, flags, inv_sqrt_d, probs);
   __syncthreads();  // the map is written, the tile's LDS is free
   cover_select_map<LQ_TILE>(lds.sel.cover, lds.sel.row_ties, probs + (int64_t)h * nb * nb, nb, nbw, t_le, mask + (int64_t)h * nb * nbw);
@@ -1573,6 +1628,20 @@ extern "C" float sp_queryaware_select_score(double pattern_threshold, int32_t nb
   return (float)product;
 }
 
+static bool queryaware_small(int32_t d, int32_t nb) { return (d == 128 || d == 64) && nb <= LQ_TILE; }
+static int queryaware_small_launch(const void* qbar, const void* kbar, const int32_t* decision, int32_t hq, int32_t hkv, int32_t d,
+                                   int32_t nb, uint32_t flags, float score, float* probs, uint64_t* mask, const ElectArgs& elect,
+                                   hipStream_t s) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(hq), dim3(CS_THREADS), 0, s, (const sp_bf16*)qbar, (const sp_bf16*)kbar, decision, (int)hq, (int)hkv,
+                       (int)nb, (int)((nb + 63) / 64), flags, sp_inv_sqrt_dim(flags, d), probs, (long long)sp_thr_le(score), mask,
+                       elect);
+  };
+  d == 64 ? launch(sp_queryaware_small_kernel<64>) : launch(sp_queryaware_small_kernel<128>);
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
 extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, const int32_t* decision, int32_t hq,
                                          int32_t hkv, int32_t d, int32_t nb, uint32_t flags, double pattern_threshold,
                                          float* probs, uint64_t* mask, void* workspace, size_t workspace_bytes,
@@ -1584,17 +1653,10 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
   const size_t lds = (size_t)(d + nb) * sizeof(float);
   SP_REQUIRE(lds <= 60000, SP_ERR_UNSUPPORTED, "sp_queryaware_select_bf16: nb=%d too large", nb);
   const float score = sp_queryaware_select_score(pattern_threshold, nb);
-  if ((d == 128 || d == 64) && nb <= LQ_TILE) {
+  if (queryaware_small(d, nb)) {
     SP_REQUIRE(workspace && workspace_bytes >= sp_cover_select_workspace_bytes(hq) && ((uintptr_t)workspace % 8) == 0,
                SP_ERR_WORKSPACE, "sp_queryaware_select_bf16: workspace missing, misaligned or too small");  // (unused here)
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(hq), dim3(CS_THREADS), 0, (hipStream_t)stream, (const sp_bf16*)qbar, (const sp_bf16*)kbar,
-                         decision, (int)hq, (int)hkv, (int)nb, (int)((nb + 63) / 64), flags, sp_inv_sqrt_dim(flags, d), probs,
-                         (long long)sp_thr_le(score), mask);
-    };
-    d == 64 ? launch(sp_queryaware_small_kernel<64>) : launch(sp_queryaware_small_kernel<128>);
-    SP_LAUNCH_CHECK();
-    return SP_OK;
+    return queryaware_small_launch(qbar, kbar, decision, hq, hkv, d, nb, flags, score, probs, mask, ElectArgs{}, (hipStream_t)stream);
   }
   if (d == 128 || d == 64) {  // two passes on the matrix core, 128 rows per workgroup
     const int rc = sp_block_probs_mfma_launch(qbar, kbar, decision, hq, hkv, d, nb, flags, probs, (hipStream_t)stream);
@@ -1728,15 +1790,26 @@ static int select_layer(const void* q, const void* k, int64_t n, int32_t hq, int
   hipLaunchKernelGGL(sp_layer_heads_kernel, dim3((unsigned)(a.n_cover + hq + repack.nb * repack.hkv)), dim3(CS_THREADS),
                      HEAD_LDS_BYTES(d, nb), s, a);
   SP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sp_share_decide_kernel, dim3(1), dim3(DEC_MAX_HEADS), 0, s, a.st, head_cluster, layer_idx, hq, use_qa, nv,
-                     ns, min_blocks, similarity_threshold, fallback_threshold, decision, a.js_v, a.js_s, nv_f, ns_f);
-  SP_LAUNCH_CHECK();
+  const bool small = queryaware_small(d, nb);
+  if (!small) {
+    hipLaunchKernelGGL(sp_share_decide_kernel, dim3(1), dim3(DEC_MAX_HEADS), 0, s, a.st, head_cluster, layer_idx, hq, use_qa, nv,
+                       ns, min_blocks, similarity_threshold, fallback_threshold, decision, a.js_v, a.js_s, nv_f, ns_f);
+    SP_LAUNCH_CHECK();
+  }
   const MaskBesides besides = {layer_idx,
                                pool_args(q, part(LY_QBAR), n, hq, d, q_stride_n, q_stride_h, bs, SP_POOL_TAIL_RESCALE, use_qa),
-                               avg_attn};
-  hipLaunchKernelGGL(sp_build_mask_kernel<true>, dim3(hq, 2 * MASK_SPLIT), dim3(MASK_THREADS), 0, s, a.st, head_cluster, decision,
-                     vert_blk, slash_blk, nv_f, ns_f, nb, (nb + 63) / 64, mask, besides);
+                               avg_attn, use_qa, nv, ns, min_blocks, similarity_threshold, fallback_threshold, decision, nv_f, ns_f,
+                               a.js_v, a.js_s};
+  auto launch_masks = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(hq, 2 * MASK_SPLIT), dim3(MASK_THREADS), 0, s, a.st, head_cluster, decision, vert_blk, slash_blk,
+                       nv_f, ns_f, nb, (nb + 63) / 64, mask, besides);
+  };
+  small ? launch_masks(sp_build_mask_kernel<true, true>) : launch_masks(sp_build_mask_kernel<true, false>);
   SP_LAUNCH_CHECK();
+  if (small)
+    return queryaware_small_launch(part(LY_QBAR), part(LY_KBAR), decision, hq, hkv, d, nb, flags,
+                                   sp_queryaware_select_score(pattern_threshold, nb), qa_probs, mask,
+                                   ElectArgs{a.st, head_cluster, nv, ns, layer_idx}, s);
   return sp_queryaware_select_bf16(part(LY_QBAR), part(LY_KBAR), decision, hq, hkv, d, nb, flags, pattern_threshold, qa_probs,
                                    mask, part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), stream);
 }
