@@ -166,7 +166,7 @@ def cpu_baseline(w, q, k, v, mask_bool, decision, kept_blocks, pt):
 # reported only while shareprefill_amd/csrc/sp_attn.hip still has that hash, and is null (with a note) after any
 # change to the kernel until the profile is taken again.
 MEASURED_ATTN_TRAFFIC = {
-    ("C3", 0.95): {"bytes": int((102.0 + 1.0) * 2 ** 30), "sp_attn_hip_sha256_16": "0c91f1b5e29ee27c",
+    ("C3", 0.95): {"bytes": int((102.1 + 1.0) * 2 ** 30), "sp_attn_hip_sha256_16": "0c91f1b5e29ee27c",
                    "profile": "profiles/attention_layer_C3_hbm_traffic.txt"},
 }
 

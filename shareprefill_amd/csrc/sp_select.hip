@@ -1367,6 +1367,8 @@ struct MaskBesides {
   int32_t *decision, *nv_f, *ns_f;
   float *js_v, *js_s;
 };
+// (as a launch of one workgroup in between: 3001 tokens 110.1 us a layer against 107.7, 6177 of 64 channels 122.3 / 120.0, 10007 258.4 /
+// 255.5)
 // sp_share_decide_kernel's decision for head h, by every workgroup of the head for itself: "first" only looks at lower heads of its
 // cluster that are not query-aware.  The state stays as the previous layers left it until the next launch (share_elect in
 // sp_queryaware_small_kernel), so no workgroup can see another's election.  Every thread of the workgroup calls it.
@@ -1677,7 +1679,7 @@ extern "C" int sp_queryaware_select_bf16(const void* qbar, const void* kbar, con
 // The stages above, with the launches folded that do not wait for each other: K's averages beside the score statistics, the
 // query-aware test and the share similarities beside the budgets, Q's averages, the pivots' own sets and the clearing of the
 // map beside the masks.  Same device code, same results.  A launch that has nothing to do costs 2 to 2.7 us of the stream;
-// against 15 launches, seven (six up to 128 blocks since) take 21 to 23 us off a layer (3001 tokens, 6177 of 64 channels, 10007
+// against 15 launches, seven (five up to 128 blocks since) take 21 to 23 us off a layer (3001 tokens, 6177 of 64 channels, 10007
 // of 28 / 4 heads).
 struct HeadArgs {
   CoverCountArgs cover;
@@ -1706,7 +1708,7 @@ __global__ __launch_bounds__(CS_THREADS) void sp_layer_heads_kernel(HeadArgs a) 
     repack_v_tile<CS_THREADS>(a.repack, tile % a.repack.nb, tile / a.repack.nb, reinterpret_cast<sp_bf16*>(head_lds));
     return;
   }
-  // (for a head that turns out query-aware too: sp_share_decide_kernel drops it)
+  // (for a head that turns out query-aware too: the decision drops it)
   queryaware_head(a.qa, h, reinterpret_cast<float*>(head_lds), [&](int wave) {
     if (wave > 2) return;
     const float js = share_similarity(a.st, a.head_cluster[h], h, wave - 1, wave == 1 ? a.qa.vert_blk : a.slash_blk, lane);
