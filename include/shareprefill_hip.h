@@ -240,7 +240,9 @@ size_t sp_attn_workspace_bytes(int64_t n, int32_t hq, int32_t hkv, int32_t d, in
  * sp_attn_workspace_bytes rounded up to 256 bytes + p * sp_attn_pivot_scratch_bytes(n, bs) bytes of workspace, the
  * first p pivot heads (ascending head index) keep per-query block sums on the way, and their block-average maps
  * (shareprefill_attn.py:425-457) are made from those instead of a second pass over
- * Q.K^T; further pivots, or all of them with the base size, take that second pass.  Same results to rounding. */
+ * Q.K^T; further pivots, or all of them with the base size, take that second pass.  Same results to rounding.
+ * No launch keeps the sums of more than SP_ATTN_MAX_PIVOTS heads, however large the workspace. */
+#define SP_ATTN_MAX_PIVOTS 254
 size_t sp_attn_pivot_scratch_bytes(int64_t n, int32_t bs);
 int sp_attn_repack_v_bf16(const void* v, int64_t n, int32_t hkv, int32_t d, int64_t v_stride_n, int64_t v_stride_h,
                           int32_t bs, void* workspace, size_t workspace_bytes, sp_stream_t stream);
@@ -252,7 +254,7 @@ int sp_block_sparse_attn_fwd_bf16(const void* q, const void* k, const void* v, i
                                   sp_stream_t stream);
 /* The same at bs = 128 with sp_pivot_update(state, head_cluster, decision, avg_attn, hq, nb, pattern_threshold) in the launch:
  * decision, avg_attn and head_cluster must be given, and the workspace needs room for the block sums of every head that can be
- * DENSE; those beyond it get NaN for a map and update no pivot. */
+ * DENSE, at most SP_ATTN_MAX_PIVOTS of them; those beyond get NaN for a map and update no pivot. */
 int sp_block_sparse_attn_pivot_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,
                                   int32_t d, int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n,
                                   int64_t k_stride_h, int64_t v_stride_n, int64_t v_stride_h, float softmax_scale,

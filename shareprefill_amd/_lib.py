@@ -27,6 +27,7 @@ SP_POOL_TYPES = {"avg": 0, "max": 1, "min": 2, "maxabs": 3, "sum": 4}  # attn/ut
 SP_ATTN_V_REPACKED = 1
 SP_ATTN_PAIR_ROWS = 2
 SP_ATTN_HALF_CHANNELS = 4
+SP_ATTN_MAX_PIVOTS = 254
 SP_DECODE_STATIC_SCRATCH_BYTES = 8 << 20
 
 

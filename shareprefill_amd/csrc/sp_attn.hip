@@ -72,6 +72,7 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(RepackArgs a) {
 #define AT_ROWS_SLOT 197  // 1: the caller asked for pairing by rows: no analysis, no ranking
 #define AT_PAIR_TABLE 200
 #define AT_NO_SLOT 255
+static_assert(SP_ATTN_MAX_PIVOTS < AT_NO_SLOT, "");
 // Behind the 1 KiB of slots: the weights (uint16) of up to AT_RANK_MAX gangs, see sp_attn_schedule_kernel.
 #define AT_RANK_MAX 1024  // AT_MAX_HEADS of at most four gangs
 #define AT_SCHED_BYTES (1024 + AT_RANK_MAX * 2)
@@ -1732,7 +1733,7 @@ static int at_launch(const char* who, const void* q, const void* k, const void* 
   int max_pivots = 0;
   if (want_avg && workspace_bytes > base_aligned && !fine) {
     const size_t fit = (workspace_bytes - base_aligned) / slab;
-    max_pivots = fit > (size_t)(AT_NO_SLOT - 1) ? AT_NO_SLOT - 1 : (int)fit;
+    max_pivots = fit > SP_ATTN_MAX_PIVOTS ? SP_ATTN_MAX_PIVOTS : (int)fit;
   }
   float* pivot_u = reinterpret_cast<float*>(ws + base_aligned);
   {

@@ -360,7 +360,7 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     half_channels: q, k and v are zero beyond channel 64 (a smaller head_dim zero-padded to 128): the kernel skips
     those channels and leaves channels 64.. of out unwritten.
     pivot = (state, head_cluster, pattern_threshold), block size 128: pivot_update with decision and avg_attn is part of the
-    launch; DENSE heads beyond max_pivots get NaN for a map and update no pivot."""
+    launch; DENSE heads beyond max_pivots (or SP_ATTN_MAX_PIVOTS) get NaN for a map and update no pivot."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")

@@ -230,13 +230,14 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
             sharing.note_dense_layer(module.layer_idx, num_heads, nb)
         return _first_channels(out.unsqueeze(0), model_dim), avg_attn
 
-    # Room for the block sums of this layer's possible pivots (at most 16 GiB of it; pivots beyond that take the
-    # recomputing pass).  How many heads can become pivots is known from the table alone.
+    # Room for the block sums of this layer's possible pivots (at most 16 GiB of it, and no more heads than a launch keeps the sums
+    # of; pivots beyond that take the recomputing pass).  How many heads can become pivots is known from the table alone.
     avg_attn = torch.empty(1, num_heads, nb, nb, dtype=torch.float32, device=q.device)
     if not short:
         slab = _lib.load().sp_attn_pivot_scratch_bytes(q_len, block_size)
-        max_pivots = min(sharing.max_pivots(module.layer_idx, num_heads), (16 << 30) // slab)
-        all_fit = max_pivots == sharing.max_pivots(module.layer_idx, num_heads)
+        possible = sharing.max_pivots(module.layer_idx, num_heads)
+        max_pivots = min(possible, (16 << 30) // slab, _lib.SP_ATTN_MAX_PIVOTS)
+        all_fit = max_pivots == possible
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
     # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
     plan_args = {"scale_dim": model_dim}

@@ -82,3 +82,34 @@ def test_dense_heads_without_room(gpu_device):
             else:
                 assert torch.equal(avgs[0][h], avgs[1][h])
         assert (state.info[:, 1] != 0).cpu().nonzero().reshape(-1).tolist() == served.tolist()
+
+
+@pytest.mark.parametrize("n", [6657])  # (the shortest prompt of the persistent kernel)
+def test_a_pivot_per_head_of_the_most_heads(gpu_device, tmp_path, n):
+    """256 heads, each the only one of its cluster in the layer: more pivots than a launch keeps block sums of.  Every map is a
+    mean of softmax rows (its rows sum to 1) and every cluster gets its pattern; that of a head behind the last slot covers the
+    threshold like those before it."""
+    import types
+
+    from shareprefill_amd import AttentionSharing, _lib, ops, shareprefill_attention_forward, synthetic
+
+    hq, hkv, d = 256, 8, 128
+    assert _lib.load().sp_short_attn_max_tokens(d) == n - 1
+    nb = -(-n // 128)
+    table = {"clusters": {str(h): [[0, h], [1, h]] for h in range(hq)}, "shared_clusters": [str(h) for h in range(hq)]}
+    sharing = AttentionSharing(synthetic.write_cluster_table(table, str(tmp_path / "table.json")))
+    assert sharing.max_pivots(0, hq) == hq
+    config = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=0.9, similarity_threshold=0.5,
+                                   fallback_threshold=0.9, queryaware_threshold=0.0)  # (no head is query-aware)
+    module = types.SimpleNamespace(config=config, attention_sharing=sharing, layer_idx=0, scaling=d ** -0.5)
+    qkv = synthetic.planted_qkv(hq, hkv, n, d, 11, device=gpu_device, q_head_gain=1.0)
+    _, maps = shareprefill_attention_forward(module, *qkv, None, scaling=module.scaling)
+    assert (sharing.plans[-1].decision == _lib.SP_DEC_DENSE).all()
+    # a row's masses and their total come from the same probabilities: what is left is the fp32 rounding of at most 53 sums and of
+    # log2(sum) + max, of magnitude below 128 (2^-17 each)
+    assert ((maps[0].double().sum(-1) - 1).abs() <= 1e-4).all()
+    state = sharing._state
+    assert (state.info[:, 1] != 0).all() and state.ratio.isfinite().all()
+    assert torch.equal(state.avg_map, maps[0])
+    kept = ops.mask_to_bool(state.pattern, nb).to(gpu_device)
+    assert ((maps[0] * kept).double().sum(-1) >= 0.9 - 1e-4).all()
