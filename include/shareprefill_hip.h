@@ -303,8 +303,8 @@ int sp_decode_attn_bf16(const void* q, const void* k, const void* v, int64_t n, 
 
 /* The same step for a batch of sequences with caches of one length, in the launches of one: q: bf16 [batch][hq][d],
  * k / v: bf16 [batch][hkv][n][d] with batch strides beside the others, out: bf16 [batch][hq][d] contiguous.
- * workspace: sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes of device scratch (none where every sequence is one
- * chunk: any address will do), 8-byte aligned. */
+ * workspace: sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes of device scratch (zero where every sequence is one
+ * chunk: a null pointer will do), 8-byte aligned. */
 size_t sp_decode_batch_workspace_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv);
 int sp_decode_attn_batch_bf16(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq,
                               int32_t hkv, int32_t d, int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_b,

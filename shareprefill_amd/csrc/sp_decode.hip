@@ -418,8 +418,9 @@ extern "C" int sp_decode_attn_batch_bf16(const void* q, const void* k, const voi
   const DcStrides st = {q_stride_b, q_stride_h, k_stride_b, k_stride_n, k_stride_h, v_stride_b, v_stride_n, v_stride_h};
   int rc = dc_check("sp_decode_attn_batch_bf16", q, k, v, batch, n, hq, hkv, d, st, softmax_scale, out);
   if (rc) return rc;
-  SP_REQUIRE(workspace != nullptr, SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_batch_bf16: null workspace");
-  SP_REQUIRE(workspace_bytes >= sp_decode_batch_workspace_bytes(batch, n, hq, hkv) && ((uintptr_t)workspace % 8) == 0,
+  const size_t need = sp_decode_batch_workspace_bytes(batch, n, hq, hkv);
+  SP_REQUIRE(need == 0 || workspace != nullptr, SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_batch_bf16: null workspace");
+  SP_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace % 8) == 0,
              SP_ERR_WORKSPACE, "sp_decode_attn_batch_bf16: workspace too small or misaligned");
   return dc_launch(q, k, v, batch, n, hq, hkv, d, st, softmax_scale, out, workspace, (hipStream_t)stream);
 }

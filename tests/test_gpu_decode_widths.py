@@ -18,3 +18,31 @@ def test_head_sizes(gpu_device, b, hq, hkv, n, d):
 def test_caches_of_a_few_tiles(gpu_device, b, n, hq, hkv, d):
     """One workgroup walks the chunks of a cache of up to three tiles: 384 keys are the last such length."""
     check(gpu_device, b, hq, hkv, n, d)
+
+
+@pytest.mark.parametrize("b,n", [(1, 128), (1, 384), (3, 300)])
+def test_no_scratch_where_none_is_asked_for(gpu_device, b, n):
+    """Where the size function says zero bytes a caller may have allocated nothing: hipMalloc(0) gives a null pointer."""
+    import torch
+
+    from shareprefill_amd import _lib, ops
+
+    hq, hkv, d = 8, 2, 128
+    lib = _lib.load()
+    assert lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv) == 0
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    q, k, v = (torch.randn(b, h, m, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h, m in ((hq, 1), (hkv, n), (hkv, n)))
+    want = ops.decode_attention_batch(q, k, v, d ** -0.5)
+    out = torch.full_like(want, float("nan"))
+    rc = lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b, n, hq, hkv, d, q.stride(0), q.stride(1), k.stride(0),
+                                       k.stride(2), k.stride(1), v.stride(0), v.stride(2), v.stride(1), d ** -0.5, out.data_ptr(),
+                                       None, 0, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "sp_decode_attn_batch_bf16")
+    assert torch.equal(out, want)
+    n = 385  # one tile more: partials, and a null workspace is refused as ever
+    assert lib.sp_decode_batch_workspace_bytes(1, n, hq, hkv) > 0
+    k, v = (torch.zeros(1, hkv, n, d, device=gpu_device, dtype=torch.bfloat16) for _ in range(2))
+    with pytest.raises(ValueError, match="null workspace"):
+        _lib.check(lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, n, hq, hkv, d, q.stride(0), q.stride(1),
+                                                 k.stride(0), k.stride(2), k.stride(1), v.stride(0), v.stride(2), v.stride(1),
+                                                 d ** -0.5, out.data_ptr(), None, 0, 0), "sp_decode_attn_batch_bf16")
