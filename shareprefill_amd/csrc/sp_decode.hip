@@ -326,11 +326,14 @@ static int dc_cut(int32_t batch, int64_t n, int32_t hkv) {
   return (int)want;
 }
 
-// Workgroups per (sequence, kv head).  A cache of up to three tiles is walked by one, chunk by chunk, which makes the result itself: a
-// launch less, and no scratch.  A tile takes a workgroup 2.6 us, the second launch costs the host 3.3: one launch against two, us,
-// 200 keys 10.9 / 13.6, 300 11.0 / 13.7 (64 channels 11.2 / 13.9), 400 13.4 / 13.6, 512 13.3 / 13.8 (64 channels 16.7 / 14.0 with waits
-// between its loads), 640 15.9 / 13.7.  (One workgroup of sixteen waves with four tiles at a time: 500 keys 11.1, 1025 18.6.)
-#define DC_ONE_LAUNCH_TILES 3
+// Workgroups per (sequence, kv head).  A cache of up to two tiles is walked by one, chunk by chunk, which makes the result itself: a
+// launch less, and no scratch.  One launch against two, us a step of 32 layers with caches of their own, 32 query / 8 kv heads, in a
+// replayed graph (the GPU's time) and called one by one (the host's, of which the second launch is 3.3):
+//   200 keys            8.0 / 7.9 and 8.8 / 12.1;  16 sequences 8.9 / 9.9 and 8.8 / 12.2;  64 channels 6.6 / 7.0 and 9.1 / 13.4
+//   384 keys, not taken 10.8 / 8.1 and 10.8 / 12.3;  16 sequences 11.9 / 12.0 and 11.9 / 13.3;  64 channels 8.7 / 7.1 and 8.9 / 13.3
+// The third tile in series (2.7 us) costs the GPU more than the second launch does.  (One workgroup of sixteen waves with four tiles at a
+// time, called one by one: 500 keys 11.1, 1025 18.6.)
+#define DC_ONE_LAUNCH_TILES 2
 static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
   return n <= DC_ONE_LAUNCH_TILES * DC_TILE ? 1 : dc_cut(batch, n, hkv);
 }

@@ -482,3 +482,14 @@ def test_decode_batches_keep_partials_only_where_a_cache_is_cut():
             sizes = [lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv) for b in (1, 2, 7, 63, 64, 511, 512, 65536)]
             assert max(sizes) <= 1024 * (hq // hkv) * 520
             assert sizes[-1] == sizes[-2] == 0
+
+
+def test_decode_walks_a_cache_in_one_launch_only_where_that_is_as_fast():
+    """Two tiles of 128 keys in series take the GPU what a second launch does, three take it longer."""
+    from shareprefill_amd import _lib
+
+    lib = _lib.load()
+    for hq, hkv in ((32, 8), (28, 4), (14, 2)):
+        for b in (1, 4):
+            assert lib.sp_decode_batch_workspace_bytes(b, 256, hq, hkv) == 0
+            assert lib.sp_decode_batch_workspace_bytes(b, 257, hq, hkv) > 0
