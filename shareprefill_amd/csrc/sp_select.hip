@@ -1739,7 +1739,7 @@ extern "C" size_t sp_select_layer_scratch_bytes(int64_t n, int32_t hq, int32_t h
   return sum;
 }
 
-static int select_layer(const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
+static int select_layer(const char* who, const void* q, const void* k, int64_t n, int32_t hq, int32_t hkv, int32_t d,
                                     int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, int32_t bs,
                                     uint32_t flags, const sp_cluster_state* state, const int32_t* head_cluster,
                                     int32_t layer_idx, int32_t min_blocks, int32_t max_blocks, double pattern_threshold,
@@ -1747,18 +1747,18 @@ static int select_layer(const void* q, const void* k, int64_t n, int32_t hq, int
                                     void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
                                     float* avg_attn, const RepackArgs& repack, sp_stream_t stream) {
   SP_REQUIRE(state && head_cluster && scratch && qa_probs && per_head && mask, SP_ERR_INVALID_ARGUMENT,
-             "sp_select_layer_bf16: null pointer");
-  SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && bs > 0 && d > 0, SP_ERR_INVALID_ARGUMENT, "sp_select_layer_bf16: bad shape");
-  SP_REQUIRE(hq <= DEC_MAX_HEADS, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: hq=%d unsupported (max %d)", hq, DEC_MAX_HEADS);
-  SP_REQUIRE(sp_ceil_div(n, bs) <= RS_MAX, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: n=%lld needs more than %d blocks",
+             "%s: null pointer", who);
+  SP_REQUIRE(n > 0 && hq > 0 && hkv > 0 && bs > 0 && d > 0, SP_ERR_INVALID_ARGUMENT, "%s: bad shape", who);
+  SP_REQUIRE(hq <= DEC_MAX_HEADS, SP_ERR_UNSUPPORTED, "%s: hq=%d unsupported (max %d)", who, hq, DEC_MAX_HEADS);
+  SP_REQUIRE(sp_ceil_div(n, bs) <= RS_MAX, SP_ERR_UNSUPPORTED, "%s: n=%lld needs more than %d blocks", who,
              (long long)n, RS_MAX);
-  SP_REQUIRE(((uintptr_t)avg_attn % 16) == 0, SP_ERR_UNSUPPORTED, "sp_select_layer_bf16: avg_attn must be 16-byte aligned");
+  SP_REQUIRE(((uintptr_t)avg_attn % 16) == 0, SP_ERR_UNSUPPORTED, "%s: avg_attn must be 16-byte aligned", who);
   const int nb = (int)sp_ceil_div(n, bs);
-  int rc = check_state(state, nb, "sp_select_layer_bf16");
+  int rc = check_state(state, nb, who);
   if (rc) return rc;
   size_t at[LY_PARTS];
   SP_REQUIRE(scratch_bytes >= layer_scratch(n, hq, hkv, d, bs, at) && ((uintptr_t)scratch % 256) == 0, SP_ERR_WORKSPACE,
-             "sp_select_layer_bf16: scratch too small or not 256-byte aligned");
+             "%s: scratch too small or not 256-byte aligned", who);
   auto part = [&](int i) { return (char*)scratch + at[i]; };
   auto floats = [&](int i) { return (float*)part(i); };
   float *vert_tok = floats(LY_VERT_TOK), *slash_tok = floats(LY_SLASH_TOK), *vert_blk = floats(LY_VERT_BLK),
@@ -1779,7 +1779,7 @@ static int select_layer(const void* q, const void* k, int64_t n, int32_t hq, int
                              min_blocks, max_blocks};
   } else {
     rc = gsel_count_run(vert_tok, slash_tok, hq, 2 * hq, n, (float)pattern_threshold, nv, ns, bs, min_blocks, max_blocks,
-                        part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), s, "sp_select_layer_bf16");
+                        part(LY_COVER), sp_cover_select_workspace_bytes(2 * hq), s, who);
     if (rc != SP_OK) return rc;
   }
   a.st = state_by_value(state);
@@ -1823,7 +1823,7 @@ extern "C" int sp_select_layer_bf16(const void* q, const void* k, int64_t n, int
                                     float similarity_threshold, double fallback_threshold, float queryaware_threshold,
                                     void* scratch, size_t scratch_bytes, float* qa_probs, int32_t* per_head, uint64_t* mask,
                                     float* avg_attn, sp_stream_t stream) {
-  return select_layer(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
+  return select_layer("sp_select_layer_bf16", q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
                       layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
                       scratch, scratch_bytes, qa_probs, per_head, mask, avg_attn, RepackArgs{}, stream);
 }
@@ -1839,7 +1839,7 @@ extern "C" int sp_select_layer_repack_bf16(const void* q, const void* k, int64_t
   RepackArgs repack;
   const int rc = repack_args(&repack, "sp_select_layer_repack_bf16", v, n, hkv, d, v_stride_n, v_stride_h, bs, vt, vt_bytes);
   if (rc != SP_OK) return rc;
-  return select_layer(q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
+  return select_layer("sp_select_layer_repack_bf16", q, k, n, hq, hkv, d, q_stride_n, q_stride_h, k_stride_n, k_stride_h, bs, flags, state, head_cluster,
                       layer_idx, min_blocks, max_blocks, pattern_threshold, similarity_threshold, fallback_threshold, queryaware_threshold,
                       scratch, scratch_bytes, qa_probs, per_head, mask, avg_attn, repack, stream);
 }

@@ -493,3 +493,22 @@ def test_decode_walks_a_cache_in_one_launch_only_where_that_is_as_fast():
         for b in (1, 4):
             assert lib.sp_decode_batch_workspace_bytes(b, 256, hq, hkv) == 0
             assert lib.sp_decode_batch_workspace_bytes(b, 257, hq, hkv) > 0
+
+
+def test_selection_errors_name_the_entry_point_called():
+    from shareprefill_amd import _lib
+
+    lib = _lib.load()
+    addr = 4096  # (aligned; refused on the host before anything is read)
+    n, hq, hkv, d = 2048, 4, 2, 128
+
+    def args(hq, state):
+        return (addr, addr, n, hq, hkv, d, hq * d, d, hkv * d, d, 128, 0, state, addr, 0, 8, 16, 0.9, 0.5, 0.9, 0.1, addr, 0, addr, addr,
+                addr, None)
+
+    repack = (addr, hkv * d, d, addr, 1 << 30)
+    for heads, state, code, why in ((hq, None, -1, b"null pointer"), (258, _lib.ClusterStateStruct(), -2, b"hq=258 unsupported"),
+                                    (hq, _lib.ClusterStateStruct(), -1, b"cluster state sized for nb=0")):
+        for entry, extra in (("sp_select_layer_bf16", ()), ("sp_select_layer_repack_bf16", repack)):
+            assert getattr(lib, entry)(*args(heads, state), *extra, None) == code
+            assert lib.sp_last_error().startswith(entry.encode() + b": " + why)
