@@ -271,7 +271,8 @@ __global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kern
   const int64_t head = blockIdx.x, bh = head / g;  // (sequence, query head), (sequence, kv head)
   const int h = (int)(head % g), t = threadIdx.x, grp = t >> 5, c4 = (t & 31) * 4;
   const float2* ml = ml_part + bh * splits * g + h;
-  const float* op = o_part + (bh * splits * g + h) * DC_D + c4;
+  // (a smaller head's instance leaves the channels behind its own unwritten, which are not read: those threads' sums are dropped below)
+  const float* op = o_part + (bh * splits * g + h) * DC_D + (c4 < d ? c4 : 0);
   // every chunk's statistics once, kept in registers between the two passes (splits <= 2 THREADS)
   float2 mine[DC_MAX_SPLITS / THREADS];
   float m = -INFINITY;
@@ -373,8 +374,8 @@ static int dc_check(const char* who, const void* q, const void* k, const void* v
   return SP_OK;
 }
 
-// both kernels; `partials` holds sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes, every one of which the first
-// kernel writes before the second reads it (nothing has to be cleared)
+// both kernels; `partials` holds sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes, of which the second kernel reads only what
+// the first has written (nothing has to be cleared; heads of up to 64 channels write the first 64 of a partial's 128)
 static int dc_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv,
                      int32_t d, const DcStrides& st, float softmax_scale, void* out, void* partials, hipStream_t s) {
   const int g = hq / hkv;

@@ -46,3 +46,22 @@ def test_no_scratch_where_none_is_asked_for(gpu_device, b, n):
         _lib.check(lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, n, hq, hkv, d, q.stride(0), q.stride(1),
                                                  k.stride(0), k.stride(2), k.stride(1), v.stride(0), v.stride(2), v.stride(1),
                                                  d ** -0.5, out.data_ptr(), None, 0, 0), "sp_decode_attn_batch_bf16")
+
+
+@pytest.mark.parametrize("d", [8, 64, 72, 128])
+def test_scratch_may_hold_anything(gpu_device, d):
+    """The second kernel takes nothing from the scratch that the first has not written."""
+    import torch
+
+    from shareprefill_amd import _lib, ops
+
+    b, hq, hkv, n = 2, 6, 2, 700
+    gen = torch.Generator(device=gpu_device).manual_seed(d)
+    q, k, v = (torch.randn(b, h, m, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h, m in ((hq, 1), (hkv, n), (hkv, n)))
+    need = _lib.load().sp_decode_batch_workspace_bytes(b, n, hq, hkv)
+    assert need > 0
+    outs = []
+    for byte in (0, 0xFF):  # (zeros, NaN)
+        ops._workspace("decode", need, gpu_device).fill_(byte)
+        outs.append(ops.decode_attention_batch(q, k, v, d ** -0.5))
+    assert outs[0].isfinite().all() and torch.equal(outs[0], outs[1])
