@@ -163,25 +163,48 @@ def cpu_baseline(w, q, k, v, mask_bool, decision, kept_blocks, pt):
 # Bytes one steady-state sp_attn_fwd_kernel launch moves past the L2 caches, from rocprofv3 --pmc FETCH_SIZE /
 # WRITE_SIZE scaled by the V-repack kernel's known 256 MiB (profiles/attention_layer_C3_hbm_traffic.txt).  A counter
 # run cannot happen inside this script, so the figure is tied to the kernel source it was measured on: it is
-# reported only while shareprefill_amd/csrc/sp_attn.hip still has that hash, and is null (with a note) after any
-# change to the kernel until the profile is taken again.
+# reported only while shareprefill_amd/csrc/sp_attn.hip and the headers of that folder that it includes still have that
+# hash, and is null (with a note) after any change to them until the profile is taken again.
 MEASURED_ATTN_TRAFFIC = {
-    ("C3", 0.95): {"bytes": int((102.1 + 1.0) * 2 ** 30), "sp_attn_hip_sha256_16": "0c91f1b5e29ee27c",
+    ("C3", 0.95): {"bytes": int((102.1 + 1.0) * 2 ** 30), "attn_sources_sha256_16": "0c91f1b5e29ee27c",
                    "profile": "profiles/attention_layer_C3_hbm_traffic.txt"},
 }
 
 
-def measured_traffic(workload, pt):
-    """-> (bytes or None, note)"""
+def attn_sources(csrc):
+    """sp_attn.hip and every file of its folder that it includes, directly or not, in the order of their first inclusion."""
+    import re
+
+    found, todo = [], ["sp_attn.hip"]
+    while todo:
+        name = todo.pop(0)
+        path = os.path.join(csrc, name)
+        if path in found or not os.path.exists(path):  # (the C header lies elsewhere: declarations)
+            continue
+        found.append(path)
+        with open(path) as f:
+            todo += re.findall(r'^\s*#include "([^"]+)"', f.read(), re.M)
+    return found
+
+
+def attn_sources_sha(csrc=os.path.join(ROOT, "shareprefill_amd", "csrc")):
     import hashlib
 
+    sha = hashlib.sha256()
+    for path in attn_sources(csrc):
+        with open(path, "rb") as f:
+            sha.update(f.read())
+    return sha.hexdigest()[:16]
+
+
+def measured_traffic(workload, pt):
+    """-> (bytes or None, note)"""
     rec = MEASURED_ATTN_TRAFFIC.get((workload, pt))
     if rec is None:
         return None, "no counter profile for this workload"
-    with open(os.path.join(ROOT, "shareprefill_amd", "csrc", "sp_attn.hip"), "rb") as f:
-        sha = hashlib.sha256(f.read()).hexdigest()[:16]
-    if sha != rec["sp_attn_hip_sha256_16"]:
-        return None, f"kernel source changed since {rec['profile']} was taken (sha {rec['sp_attn_hip_sha256_16']} -> {sha})"
+    sha = attn_sources_sha()
+    if sha != rec["attn_sources_sha256_16"]:
+        return None, f"kernel source changed since {rec['profile']} was taken (sha {rec['attn_sources_sha256_16']} -> {sha})"
     return rec["bytes"], f"FETCH_SIZE + WRITE_SIZE past L2 (memory-side cache + HBM), {rec['profile']}, kernel source sha {sha}"
 
 

@@ -512,3 +512,21 @@ def test_selection_errors_name_the_entry_point_called():
         for entry, extra in (("sp_select_layer_bf16", ()), ("sp_select_layer_repack_bf16", repack)):
             assert getattr(lib, entry)(*args(heads, state), *extra, None) == code
             assert lib.sp_last_error().startswith(entry.encode() + b": " + why)
+
+
+def test_the_benchs_traffic_figure_is_tied_to_every_source_of_its_kernel(tmp_path):
+    import shutil
+
+    import bench
+
+    csrc = os.path.join(bench.ROOT, "shareprefill_amd", "csrc")
+    names = [os.path.basename(p) for p in bench.attn_sources(csrc)]
+    assert {"sp_attn.hip", "sp_common.h", "sp_repack.h", "sp_rows.h"} <= set(names)
+    for name in names:
+        shutil.copy(os.path.join(csrc, name), tmp_path)
+    assert bench.attn_sources_sha(str(tmp_path)) == bench.attn_sources_sha()
+    for name in names:
+        whole = (tmp_path / name).read_text()
+        (tmp_path / name).write_text(whole + "\n// changed\n")
+        assert bench.attn_sources_sha(str(tmp_path)) != bench.attn_sources_sha(), name
+        (tmp_path / name).write_text(whole)
