@@ -56,10 +56,17 @@ __global__ __launch_bounds__(AT_THREADS) void sp_repack_v_kernel(RepackArgs a) {
 // share, and every head's K / V^T fit the memory-side cache together, so the order above (one kv head after the
 // other) only makes the last kv head's heavy rows start late: there sp_attn_schedule_kernel writes down the number of blocks
 // every gang's items visit, every workgroup ranks the gangs by it, and the queues are dealt from that ranking, heaviest
-// first.  Layers in us: ranked / dealt by rows, the last rows of all heads first (which needs no weights): 10007 tokens 28 heads
-// 259 / 258, 13000 371 / 369, 16384 (two layers, heads of unlike weight) 1827 / 1966, 24000 1328 / 1392, 32768 2629 / 2839.  At
-// 8000 tokens the order above 245, ranked 249; at 65001 no difference.  Gangs of 32 / 16 pairs: 10007 260 / 259, 16384 1853 / 1827,
-// 24000 1329 / 1334, 32768 2629 / 2642.
+// first.  Layers in us, coverage 0.95 and 32 query / 8 kv heads unless another is named, in one call:
+//   ranked with gangs of 16 / with gangs of 32 / the order above with gangs of 32: 8321 tokens 266 / 270 / 276, 10007 284 / 287 / 292,
+//   28 / 4 heads at 0.9 237 / 228 / 234, 13000 459 / 474 / 475, 16384 624 / 628 / 644, two layers (heads of unlike weight) 1725 / 1740 /
+//   1944;
+//   gangs of 32 from here on, ranked / the order above: 16385 678 / 678, 18000 813 / 804, 20000 973 / 974, 22000 1076 / 1071, 24000 1347 /
+//   1337, 32768 2354 / 2375, two layers 5745 / 6100 (ranked with gangs of 16: 678, 817, 977, 1083, 1354, 2370, 5770).
+// So ranking is for the layers whose heads weigh unlike, and costs the others up to 1 % between 18000 and 24000 tokens; at 65001 there is
+// no difference.  Where it begins is not exact: 8000 tokens, one block below, 246 by the order above, 242 ranked; nor is the gangs'
+// size there (28 / 4 heads).  Dealing by rows, the last rows of all heads first, needs no weights and was as good as ranking up to
+// 13000 tokens (371 / 369), but not with two layers of 16384 (1966 / 1827) nor at 24000 (1392 / 1328) and 32768 (2839 / 2629): one
+// rule for all of them.
 #define AT_GANG 32
 #define AT_RANK_MIN_NB 64  // (ranked: more blocks than that)
 #define AT_RANK_MAX_NB 256
@@ -237,7 +244,6 @@ __device__ static inline uint64_t at_trim(uint64_t x, int wi, int r) {
   return x;
 }
 
-// entry of the per-pair block list: column | row-membership flags
 // sp_wave_sum without its trips through LDS: lanes ^ 32 and ^ 16 by the swaps; then every row of 16 lanes holds the same
 // values, and with them repeating every 16, 8, 4, 2 lanes a rotation by 8, 4, 2, 1 is the exchange with lane ^ 8, 4, 2, 1
 template <int CTRL>
@@ -272,6 +278,7 @@ __device__ static __forceinline__ uint64_t at_lane_u64(uint64_t v, int lane) {  
          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
 }
 
+// entry of the per-pair block list: column | row-membership flags
 #define AT_IN_A (1u << 30)
 #define AT_IN_B (1u << 31)
 #define AT_COL_MASK 0x00FFFFFFu
@@ -891,372 +898,372 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
     }
     // the item itself; PV: a pivot with a slot
     auto run = [&](auto pv) {
-    constexpr bool PV = decltype(pv)::value;
-    constexpr int MODE = (PV ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
-    // FINE: the two fine mask rows of this wave's query tiles, and the keep bits (at_keep) of a block from them
-    const uint64_t* frow[2] = {fine_mask, fine_mask};
-    if constexpr (FINE) {
-      const int w4 = wave & 3;
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        int fr = (r * AT_BS + 32 * w4 + 16 * qt) >> (7 - fshift);
-        if (fr > nbf - 1) fr = nbf - 1;  // (queries beyond the sequence: computed, never stored)
-        frow[qt] = fine_mask + ((int64_t)h * nbf + fr) * nbfw;
-      }
-    }
-    // the two 64-bit mask words are requested a block ahead of their use (fine_issue at the top of block b for block
-    // b + 1, fine_take when the walk moves on)
-    uint64_t fw_next[2] = {~0ull, ~0ull};
-    auto fine_issue = [&](int c) {
+      constexpr bool PV = decltype(pv)::value;
+      constexpr int MODE = (PV ? 1 : 0) | (HALF ? 2 : 0) | (FINE ? 4 : 0);
+      // FINE: the two fine mask rows of this wave's query tiles, and the keep bits (at_keep) of a block from them
+      const uint64_t* frow[2] = {fine_mask, fine_mask};
       if constexpr (FINE) {
-        const int fc0 = c << fshift;  // first fine column of the 128-key block; its 1 << fshift bits share a word
-        fw_next[0] = frow[0][fc0 >> 6];
-        fw_next[1] = frow[1][fc0 >> 6];
-      }
-    };
-    auto fine_take = [&](int c) -> uint32_t {  // kq of column c from the words fine_issue(c) requested
-      uint32_t kq = 0xffffu;
-      if constexpr (FINE) {
-        const int fc0 = c << fshift;
-        kq = 0u;
+        const int w4 = wave & 3;
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
-          const uint32_t fb = (uint32_t)(fw_next[qt] >> (fc0 & 63));
-          uint32_t k16 = 0u;
-#pragma unroll
-          for (int c16 = 0; c16 < 8; ++c16) k16 |= ((fb >> (c16 >> (3 - fshift))) & 1u) << c16;
-          kq |= k16 << (8 * qt);
+          int fr = (r * AT_BS + 32 * w4 + 16 * qt) >> (7 - fshift);
+          if (fr > nbf - 1) fr = nbf - 1;  // (queries beyond the sequence: computed, never stored)
+          frow[qt] = fine_mask + ((int64_t)h * nbf + fr) * nbfw;
         }
-        kq = __builtin_amdgcn_readfirstlane(kq);
       }
-      return kq;
-    };
-    uint32_t kq_cur = 0xffffu;
+      // the two 64-bit mask words are requested a block ahead of their use (fine_issue at the top of block b for block
+      // b + 1, fine_take when the walk moves on)
+      uint64_t fw_next[2] = {~0ull, ~0ull};
+      auto fine_issue = [&](int c) {
+        if constexpr (FINE) {
+          const int fc0 = c << fshift;  // first fine column of the 128-key block; its 1 << fshift bits share a word
+          fw_next[0] = frow[0][fc0 >> 6];
+          fw_next[1] = frow[1][fc0 >> 6];
+        }
+      };
+      auto fine_take = [&](int c) -> uint32_t {  // kq of column c from the words fine_issue(c) requested
+        uint32_t kq = 0xffffu;
+        if constexpr (FINE) {
+          const int fc0 = c << fshift;
+          kq = 0u;
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt) {
+            const uint32_t fb = (uint32_t)(fw_next[qt] >> (fc0 & 63));
+            uint32_t k16 = 0u;
+#pragma unroll
+            for (int c16 = 0; c16 < 8; ++c16) k16 |= ((fb >> (c16 >> (3 - fshift))) & 1u) << c16;
+            kq |= k16 << (8 * qt);
+          }
+          kq = __builtin_amdgcn_readfirstlane(kq);
+        }
+        return kq;
+      };
+      uint32_t kq_cur = 0xffffu;
 
-    floatx4 o[9][2];  // [channel tile][query tile]; o[8]: the row sums (ones . P)
+      floatx4 o[9][2];  // [channel tile][query tile]; o[8]: the row sums (ones . P)
 #pragma unroll
-    for (int dt = 0; dt < 9; ++dt)
+      for (int dt = 0; dt < 9; ++dt)
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) o[dt][qt] = (floatx4){0, 0, 0, 0};
-    float m_run[2] = {AT_NO_MAX, AT_NO_MAX};
-    uint32_t det[2] = {0u, 0u};
-    bf16x8 ones = __builtin_bit_cast(bf16x8, (at_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-    asm volatile("" : "+v"(ones));  // one register set for the whole row
-    // Pivot heads: block sums.  o[8] - l_mark is the softmax mass of the key block whose last half-tile has just been
-    // applied to O, relative to the current running max (both follow every rescale; every lane of a query's group
-    // holds the whole sum); it is kept as u = log2(sum) + m_run.
-    float l_mark[2] = {0.f, 0.f};
-    const int64_t tri_row = (int64_t)slot * ((int64_t)nb * (nb + 1) / 2) + (int64_t)r * (r + 1) / 2;
-    float* const pu = PV ? pivot_u + tri_row * AT_BS : nullptr;
-    auto emit = [&](int c) {
-      if constexpr (PV) {
-        // (the sums' last MFMA carried its wait states: at_fused<SETTLE> / at_pv_only)
+        for (int qt = 0; qt < 2; ++qt) o[dt][qt] = (floatx4){0, 0, 0, 0};
+      float m_run[2] = {AT_NO_MAX, AT_NO_MAX};
+      uint32_t det[2] = {0u, 0u};
+      bf16x8 ones = __builtin_bit_cast(bf16x8, (at_u32x4){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+      asm volatile("" : "+v"(ones));  // one register set for the whole row
+      // Pivot heads: block sums.  o[8] - l_mark is the softmax mass of the key block whose last half-tile has just been
+      // applied to O, relative to the current running max (both follow every rescale; every lane of a query's group
+      // holds the whole sum); it is kept as u = log2(sum) + m_run.
+      float l_mark[2] = {0.f, 0.f};
+      const int64_t tri_row = (int64_t)slot * ((int64_t)nb * (nb + 1) / 2) + (int64_t)r * (r + 1) / 2;
+      float* const pu = PV ? pivot_u + tri_row * AT_BS : nullptr;
+      auto emit = [&](int c) {
+        if constexpr (PV) {
+          // (the sums' last MFMA carried its wait states: at_fused<SETTLE> / at_pv_only)
+          AT_LANE_VIEW(tq);
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt) {
+            const float tl = o[8][qt][0] - l_mark[qt];
+            l_mark[qt] = o[8][qt][0];
+            const float u = __builtin_amdgcn_logf(tl) + m_run[qt];
+            if (g == 0) pu[(int64_t)c * AT_BS + q_off + qt * 16] = u;
+          }
+        }
+      };
+
+      // Block b of the list is processed as sub-tiles 2b and 2b+1; sub-tile s lives in ring slot s % 4 (K and V^T
+      // rings alike).  One wait + barrier + issue per BLOCK: while block b is computed on (K of sub-tiles 2b, 2b+1
+      // and V^T of 2b-1, 2b -- the P.V product trails by one sub-tile), K of 2b+2, 2b+3 and V^T of 2b+1, 2b+2 are
+      // in flight.  Past the end the last block is fetched again into slots nobody reads any more.
+      auto entry = [&](int b) -> uint32_t {
+        const int bc = b < n_blk ? b : n_blk - 1;
+        return __builtin_amdgcn_readfirstlane(blist[bc]);
+      };
+      auto issue_k = [&](int c, int hf, int sub) {  // K of sub-tile `sub` = (column c, half hf)
+        char* kbuf = kring + (sub & 3) * AT_KBUF_BYTES;
+        const int64_t key0 = (int64_t)c * AT_BS + hf * AT_SUB;
+        if (c != c_ragged)
+          at_issue_k(lo, reinterpret_cast<const char*>(kh + key0 * sk_n), sk_n, kbuf, wave);
+        else
+          at_issue_k_tail(kh, n, sk_n, key0, kbuf, wave, t);
+      };
+      auto issue_v = [&](int c, int hf, int sub) {  // V^T of sub-tile `sub` = (column c, half hf)
+        at_issue_v(lo, vth + (int64_t)c * (AT_D * AT_BS * 2) + hf * (AT_SUB * 2), vring + (sub & 3) * AT_VBUF_BYTES,
+                   wave);
+      };
+      int c_cur = -1;
+      bool mine = false;
+      const uint32_t my_flag = grp ? AT_IN_B : AT_IN_A;
+      // The list is read one block ahead of its use: e_next is the entry of block b + 1, and the read of block b + 2's
+      // goes out at the top of block b, unseen by the compiler (an asynchronous LDS read like the operand fetches),
+      // to be picked up when the walk moves on.  Read where it is needed, it cost every wave an LDS round trip right
+      // behind each block's barrier, where no other wave has anything to issue either.
+      uint32_t e_next = 0u, e_ahead = 0u;
+      const uint32_t blist_addr = at_lds_addr(reinterpret_cast<const char*>(blist));
+      if (n_blk > 0) {
+        c_cur = c_first;
+        mine = first_mine;
+        issue_k(c_cur, 0, 0);
+        issue_k(c_cur, 1, 1);
+        issue_v(c_cur, 0, 0);
+        fine_issue(c_cur);
+      }
+      // Q^T operands: the lane's two queries (one per 16-query tile), 4 channel steps of 8 channels each
+      bf16x8 qb[2][4];
+      {
         AT_LANE_VIEW(tq);
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
-          const float tl = o[8][qt][0] - l_mark[qt];
-          l_mark[qt] = o[8][qt][0];
-          const float u = __builtin_amdgcn_logf(tl) + m_run[qt];
-          if (g == 0) pu[(int64_t)c * AT_BS + q_off + qt * 16] = u;
+          int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
+          if (qrow > n - 1) qrow = n - 1;
+          const sp_bf16* src = q + (int64_t)h * sq_h + qrow * sq_n + 8 * g;
+#pragma unroll
+          for (int ks = 0; ks < (HALF ? 2 : 4); ++ks)
+            qb[qt][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
         }
       }
-    };
 
-    // Block b of the list is processed as sub-tiles 2b and 2b+1; sub-tile s lives in ring slot s % 4 (K and V^T
-    // rings alike).  One wait + barrier + issue per BLOCK: while block b is computed on (K of sub-tiles 2b, 2b+1
-    // and V^T of 2b-1, 2b -- the P.V product trails by one sub-tile), K of 2b+2, 2b+3 and V^T of 2b+1, 2b+2 are
-    // in flight.  Past the end the last block is fetched again into slots nobody reads any more.
-    auto entry = [&](int b) -> uint32_t {
-      const int bc = b < n_blk ? b : n_blk - 1;
-      return __builtin_amdgcn_readfirstlane(blist[bc]);
-    };
-    auto issue_k = [&](int c, int hf, int sub) {  // K of sub-tile `sub` = (column c, half hf)
-      char* kbuf = kring + (sub & 3) * AT_KBUF_BYTES;
-      const int64_t key0 = (int64_t)c * AT_BS + hf * AT_SUB;
-      if (c != c_ragged)
-        at_issue_k(lo, reinterpret_cast<const char*>(kh + key0 * sk_n), sk_n, kbuf, wave);
-      else
-        at_issue_k_tail(kh, n, sk_n, key0, kbuf, wave, t);
-    };
-    auto issue_v = [&](int c, int hf, int sub) {  // V^T of sub-tile `sub` = (column c, half hf)
-      at_issue_v(lo, vth + (int64_t)c * (AT_D * AT_BS * 2) + hf * (AT_SUB * 2), vring + (sub & 3) * AT_VBUF_BYTES,
-                 wave);
-    };
-    int c_cur = -1;
-    bool mine = false;
-    const uint32_t my_flag = grp ? AT_IN_B : AT_IN_A;
-    // The list is read one block ahead of its use: e_next is the entry of block b + 1, and the read of block b + 2's
-    // goes out at the top of block b, unseen by the compiler (an asynchronous LDS read like the operand fetches),
-    // to be picked up when the walk moves on.  Read where it is needed, it cost every wave an LDS round trip right
-    // behind each block's barrier, where no other wave has anything to issue either.
-    uint32_t e_next = 0u, e_ahead = 0u;
-    const uint32_t blist_addr = at_lds_addr(reinterpret_cast<const char*>(blist));
-    if (n_blk > 0) {
-      c_cur = c_first;
-      mine = first_mine;
-      issue_k(c_cur, 0, 0);
-      issue_k(c_cur, 1, 1);
-      issue_v(c_cur, 0, 0);
-      fine_issue(c_cur);
-    }
-    // Q^T operands: the lane's two queries (one per 16-query tile), 4 channel steps of 8 channels each
-    bf16x8 qb[2][4];
-    {
-      AT_LANE_VIEW(tq);
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-        if (qrow > n - 1) qrow = n - 1;
-        const sp_bf16* src = q + (int64_t)h * sq_h + qrow * sq_n + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < (HALF ? 2 : 4); ++ks)
-          qb[qt][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
-      }
-    }
-
-    // (the list, see above)
-    {
-      const int lane = t & 63, wmax = (has_b ? r_b : r_a) >> 6;
-      for (int wi = wave; wi <= wmax; wi += 8) {
-        const uint64_t wa = at_lane_u64(w_a, wi), wb = at_lane_u64(w_b, wi), wu = wa | wb;
-        const int pos = __builtin_amdgcn_readlane((int)w_before, wi) + __builtin_popcountll(wu & ((1ull << lane) - 1ull));
-        if ((wu >> lane) & 1ull)
-          blist[pos] = (uint32_t)(wi * 64 + lane) | (((wa >> lane) & 1ull) ? AT_IN_A : 0u) |
-                       (((wb >> lane) & 1ull) ? AT_IN_B : 0u);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the list is complete; the tiles stay in flight
-    if (n_blk > 0) {
-      e_next = entry(1);
-      kq_cur = fine_take(c_cur);
-    }
-
-    // The compute walk.  Per block every wave passes `top` exactly once (wait, barrier, issue), whatever its row
-    // does with the block.  A row's own blocks come in runs; a run is one straight-line pipeline: start (first S),
-    // steady steps while the next block is the row's too, drain on the block after the run (V^T of the run's last
-    // sub-tile is resident by then) or after the walk.
-    int b = 0;
-    const char *kb = kring, *vb = vring;  // K(2b), V^T(2b-1); the second sub-tile's buffers follow in the rings
-    const char* vb1 = vring;              // V^T(2b)
-    int c_next = 0;  // column of block b+1 (clamped to the last block)
-    AtAddr ad;
-    auto top = [&]() {
-      AT_WAIT_VMCNT0();              // K(2b), K(2b+1), V^T(2b-1), V^T(2b) have landed (own loads)
-      __builtin_amdgcn_s_barrier();  // ... everybody's; and every wave is past block b-1
-      // (hidden loop invariance: no precomputed copies of these lane constants that could be spilled)
-      asm volatile("" : "+v"(lo.k), "+v"(lo.v));
-      c_next = (int)(e_next & AT_COL_MASK);
-      fine_issue(c_next);
+      // (the list, see above)
       {
-        const int ba = b + 2 < n_blk ? b + 2 : n_blk - 1;
-        asm volatile("ds_read_b32 %0, %1" : "=v"(e_ahead) : "v"(blist_addr + 4u * (uint32_t)ba));
+        const int lane = t & 63, wmax = (has_b ? r_b : r_a) >> 6;
+        for (int wi = wave; wi <= wmax; wi += 8) {
+          const uint64_t wa = at_lane_u64(w_a, wi), wb = at_lane_u64(w_b, wi), wu = wa | wb;
+          const int pos = __builtin_amdgcn_readlane((int)w_before, wi) + __builtin_popcountll(wu & ((1ull << lane) - 1ull));
+          if ((wu >> lane) & 1ull)
+            blist[pos] = (uint32_t)(wi * 64 + lane) | (((wa >> lane) & 1ull) ? AT_IN_A : 0u) |
+                         (((wb >> lane) & 1ull) ? AT_IN_B : 0u);
+        }
       }
-      kb = kring + ((2 * b) & 3) * AT_KBUF_BYTES;
-      vb = vring + ((2 * b + 3) & 3) * AT_VBUF_BYTES;
-      vb1 = vring + ((2 * b) & 3) * AT_VBUF_BYTES;
-      asm volatile("" : "+v"(koff), "+v"(voff));
-      at_block_addr(ad, kb, vb, vb1, koff, voff);
-    };
-    // The next block's loads go out in four parts spread over the block's steps: issued in one burst, the eight
-    // waves' 64 KiB would queue up in front of the CU's vector-memory path and stall everybody for its duration.
-    auto feed = [&](int part) {
-      if (part == 0) issue_k(c_next, 0, 2 * b + 2);
-      if (part == 1) issue_k(c_next, 1, 2 * b + 3);
-      if (part == 2) issue_v(c_cur, 1, 2 * b + 1);
-      if (part == 3) issue_v(c_next, 0, 2 * b + 2);
-    };
-    auto feed_all = [&]() {
-      feed(0);
-      feed(1);
-      feed(2);
-      feed(3);
-    };
-    auto step_walk = [&]() {  // (every call follows a `top` of the block that ends here)
-      ++b;
-      if (b < n_blk) {
-        c_cur = (int)(e_next & AT_COL_MASK);
-        mine = (e_next & my_flag) != 0u;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the list is complete; the tiles stay in flight
+      if (n_blk > 0) {
+        e_next = entry(1);
         kq_cur = fine_take(c_cur);
-      } else {
-        c_cur = -1;
-        mine = false;
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(e_ahead));  // long since back: issued a whole block ago
-      e_next = __builtin_amdgcn_readfirstlane(e_ahead);
-    };
-    bool finished = false;  // the final wait + barrier has been passed
-    while (c_cur >= 0) {
-      top();
-      if (!mine) {
-        feed_all();
-        step_walk();
-        continue;
-      }
-      floatx4 sa[2][2], sb[2][2];  // [key tile][query tile]
-      bf16x8 pa[2], pb[2];         // [query tile]
-      bf16x8 pre[2];               // the next stage's first two LDS operands, in flight (at_prefetch_qk)
-      // ---- start of a run: S of the first half-tile, nothing to overlap with yet ----
-      feed(0);
-      at_qk_only<0, HALF>(kb, koff, qb, sa);
-      feed(1);
-      at_step<true, false, 1, 0, 0, MODE, false, 2>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
-                                                     c_cur == r, 0, tq, l_mark, pre, kq_cur);
-      feed(2);
-      at_step<true, true, 2, 1, 0, MODE, true, 3>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
-                                                   c_cur == r, 32, tq, l_mark, pre, kq_cur);
-      feed(3);
-      at_step<true, true, 3, 1, 1, MODE, true, -1>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
-                                                    c_cur == r, AT_SUB, tq, l_mark, pre, kq_cur);
-      int c_prev = c_cur;
-      uint32_t kq_prev = kq_cur;
-      step_walk();
-      // ---- steady state: four half-tile steps per block ----
-      while (mine) {  // (mine implies c_cur >= 0)
-        top();
-        // The instruction arbiter favours the older waves (the even row's), which then finish the block early and
-        // idle at the barrier while the odd row's waves run alone at half the matrix-core rate: the odd row gets
-        // priority for the first half of the block, which evens the two out.
-        at_prefetch_qk<0>(ad, pre);  // (the block's first operands, while the loads and the commit test are set up)
-        if (grp) __builtin_amdgcn_s_setprio(1);
-        // S(previous block, keys 96..127) -> P;  S(keys 0..31) on the matrix core;  O += V^T(2b-1, keys 0..31) . P
-        at_step<true, true, 0, 0, 0, MODE, true, 1>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
-                                                     c_prev == r, AT_SUB + 32, tq, l_mark, pre, kq_prev);
+
+      // The compute walk.  Per block every wave passes `top` exactly once (wait, barrier, issue), whatever its row
+      // does with the block.  A row's own blocks come in runs; a run is one straight-line pipeline: start (first S),
+      // steady steps while the next block is the row's too, drain on the block after the run (V^T of the run's last
+      // sub-tile is resident by then) or after the walk.
+      int b = 0;
+      const char *kb = kring, *vb = vring;  // K(2b), V^T(2b-1); the second sub-tile's buffers follow in the rings
+      const char* vb1 = vring;              // V^T(2b)
+      int c_next = 0;  // column of block b+1 (clamped to the last block)
+      AtAddr ad;
+      auto top = [&]() {
+        AT_WAIT_VMCNT0();              // K(2b), K(2b+1), V^T(2b-1), V^T(2b) have landed (own loads)
+        __builtin_amdgcn_s_barrier();  // ... everybody's; and every wave is past block b-1
+        // (hidden loop invariance: no precomputed copies of these lane constants that could be spilled)
+        asm volatile("" : "+v"(lo.k), "+v"(lo.v));
+        c_next = (int)(e_next & AT_COL_MASK);
+        fine_issue(c_next);
+        {
+          const int ba = b + 2 < n_blk ? b + 2 : n_blk - 1;
+          asm volatile("ds_read_b32 %0, %1" : "=v"(e_ahead) : "v"(blist_addr + 4u * (uint32_t)ba));
+        }
+        kb = kring + ((2 * b) & 3) * AT_KBUF_BYTES;
+        vb = vring + ((2 * b + 3) & 3) * AT_VBUF_BYTES;
+        vb1 = vring + ((2 * b) & 3) * AT_VBUF_BYTES;
+        asm volatile("" : "+v"(koff), "+v"(voff));
+        at_block_addr(ad, kb, vb, vb1, koff, voff);
+      };
+      // The next block's loads go out in four parts spread over the block's steps: issued in one burst, the eight
+      // waves' 64 KiB would queue up in front of the CU's vector-memory path and stall everybody for its duration.
+      auto feed = [&](int part) {
+        if (part == 0) issue_k(c_next, 0, 2 * b + 2);
+        if (part == 1) issue_k(c_next, 1, 2 * b + 3);
+        if (part == 2) issue_v(c_cur, 1, 2 * b + 1);
+        if (part == 3) issue_v(c_next, 0, 2 * b + 2);
+      };
+      auto feed_all = [&]() {
         feed(0);
-        at_step<true, true, 1, 0, 1, MODE, true, 2>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
-                                                     c_cur == r, 0, tq, l_mark, pre, kq_cur);
-        emit(c_prev);  // the previous block's last half-tile went into O (and the sums) in this step
-        if (grp) __builtin_amdgcn_s_setprio(0);
         feed(1);
+        feed(2);
+        feed(3);
+      };
+      auto step_walk = [&]() {  // (every call follows a `top` of the block that ends here)
+        ++b;
+        if (b < n_blk) {
+          c_cur = (int)(e_next & AT_COL_MASK);
+          mine = (e_next & my_flag) != 0u;
+          kq_cur = fine_take(c_cur);
+        } else {
+          c_cur = -1;
+          mine = false;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(e_ahead));  // long since back: issued a whole block ago
+        e_next = __builtin_amdgcn_readfirstlane(e_ahead);
+      };
+      bool finished = false;  // the final wait + barrier has been passed
+      while (c_cur >= 0) {
+        top();
+        if (!mine) {
+          feed_all();
+          step_walk();
+          continue;
+        }
+        floatx4 sa[2][2], sb[2][2];  // [key tile][query tile]
+        bf16x8 pa[2], pb[2];         // [query tile]
+        bf16x8 pre[2];               // the next stage's first two LDS operands, in flight (at_prefetch_qk)
+        // ---- start of a run: S of the first half-tile, nothing to overlap with yet ----
+        feed(0);
+        at_qk_only<0, HALF>(kb, koff, qb, sa);
+        feed(1);
+        at_step<true, false, 1, 0, 0, MODE, false, 2>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
+                                                       c_cur == r, 0, tq, l_mark, pre, kq_cur);
         feed(2);
         at_step<true, true, 2, 1, 0, MODE, true, 3>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
                                                      c_cur == r, 32, tq, l_mark, pre, kq_cur);
         feed(3);
         at_step<true, true, 3, 1, 1, MODE, true, -1>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
                                                       c_cur == r, AT_SUB, tq, l_mark, pre, kq_cur);
-        c_prev = c_cur;
-        kq_prev = kq_cur;
+        int c_prev = c_cur;
+        uint32_t kq_prev = kq_cur;
         step_walk();
+        // ---- steady state: four half-tile steps per block ----
+        while (mine) {  // (mine implies c_cur >= 0)
+          top();
+          // The instruction arbiter favours the older waves (the even row's), which then finish the block early and
+          // idle at the barrier while the odd row's waves run alone at half the matrix-core rate: the odd row gets
+          // priority for the first half of the block, which evens the two out.
+          at_prefetch_qk<0>(ad, pre);  // (the block's first operands, while the loads and the commit test are set up)
+          if (grp) __builtin_amdgcn_s_setprio(1);
+          // S(previous block, keys 96..127) -> P;  S(keys 0..31) on the matrix core;  O += V^T(2b-1, keys 0..31) . P
+          at_step<true, true, 0, 0, 0, MODE, true, 1>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
+                                                       c_prev == r, AT_SUB + 32, tq, l_mark, pre, kq_prev);
+          feed(0);
+          at_step<true, true, 1, 0, 1, MODE, true, 2>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
+                                                       c_cur == r, 0, tq, l_mark, pre, kq_cur);
+          emit(c_prev);  // the previous block's last half-tile went into O (and the sums) in this step
+          if (grp) __builtin_amdgcn_s_setprio(0);
+          feed(1);
+          feed(2);
+          at_step<true, true, 2, 1, 0, MODE, true, 3>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
+                                                       c_cur == r, 32, tq, l_mark, pre, kq_cur);
+          feed(3);
+          at_step<true, true, 3, 1, 1, MODE, true, -1>(ad, qb, sb, sa, pb, pa, o, scale_log2, m_run, det, ones,
+                                                        c_cur == r, AT_SUB, tq, l_mark, pre, kq_cur);
+          c_prev = c_cur;
+          kq_prev = kq_cur;
+          step_walk();
+        }
+        // ---- drain: the run's last half-tile and its P.V (V^T of sub-tile 2b-1) ----
+        if (c_cur >= 0) {
+          top();
+          feed_all();
+          step_walk();
+        } else {
+          AT_WAIT_VMCNT0();
+          __syncthreads();
+          finished = true;
+          if (wave == 0) ask();
+          vb = vring + ((2 * b + 3) & 3) * AT_VBUF_BYTES;
+          at_block_addr(ad, kb, vb, vb, koff, voff);
+        }
+        at_step<false, true, 0, 0, 0, MODE>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
+                                             c_prev == r, AT_SUB + 32, tq, l_mark, pre, kq_prev);
+        at_commit<MODE>(sb, pb, det, o, scale_log2, m_run, l_mark);
+        at_pv_only<1, HALF>(vb, voff, pb, o, ones);
+        emit(c_prev);
       }
-      // ---- drain: the run's last half-tile and its P.V (V^T of sub-tile 2b-1) ----
-      if (c_cur >= 0) {
-        top();
-        feed_all();
-        step_walk();
-      } else {
+      if (!finished) {
         AT_WAIT_VMCNT0();
         __syncthreads();
-        finished = true;
         if (wave == 0) ask();
-        vb = vring + ((2 * b + 3) & 3) * AT_VBUF_BYTES;
-        at_block_addr(ad, kb, vb, vb, koff, voff);
       }
-      at_step<false, true, 0, 0, 0, MODE>(ad, qb, sa, sb, pa, pb, o, scale_log2, m_run, det, ones,
-                                           c_prev == r, AT_SUB + 32, tq, l_mark, pre, kq_prev);
-      at_commit<MODE>(sb, pb, det, o, scale_log2, m_run, l_mark);
-      at_pv_only<1, HALF>(vb, voff, pb, o, ones);
-      emit(c_prev);
-    }
-    if (!finished) {
-      AT_WAIT_VMCNT0();
-      __syncthreads();
-      if (wave == 0) ask();
-    }
-    at_settle_o(o);
-    // every lane of a query's group holds the whole row sum (all rows of the ones . P tile are equal)
-    const float l_tot[2] = {o[8][0][0], o[8][1][0]};
-    AT_LANE_VIEW(tq);
+      at_settle_o(o);
+      // every lane of a query's group holds the whole row sum (all rows of the ones . P tile are equal)
+      const float l_tot[2] = {o[8][0][0], o[8][1][0]};
+      AT_LANE_VIEW(tq);
 
-    // pivots without a slot: the softmax statistics of every query row for the block-average pass
-    if (!PV && row_ok && ((dense_heads[h >> 5] >> (h & 31)) & 1u) != 0u) {
-      if (nan_maps) {
-        for (int i = tq; i < n_blk; i += AT_FWD_THREADS / 2)
-          if (blist[i] & my_flag) avg_attn[((int64_t)h * nb + r) * nb + (blist[i] & AT_COL_MASK)] = NAN;
-      } else if (rowstat != nullptr && g == 0) {
+      // pivots without a slot: the softmax statistics of every query row for the block-average pass
+      if (!PV && row_ok && ((dense_heads[h >> 5] >> (h & 31)) & 1u) != 0u) {
+        if (nan_maps) {
+          for (int i = tq; i < n_blk; i += AT_FWD_THREADS / 2)
+            if (blist[i] & my_flag) avg_attn[((int64_t)h * nb + r) * nb + (blist[i] & AT_COL_MASK)] = NAN;
+        } else if (rowstat != nullptr && g == 0) {
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt) {
+            const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
+            if (qrow < n) rowstat[(int64_t)h * n + qrow] = make_float2(m_run[qt], l_tot[qt]);
+          }
+        }
+      }
+
+      // ---- epilogue: normalise and store straight from the accumulators.  A lane holds 4 consecutive channels of its
+      // query per channel tile; lane groups 2i and 2i + 1 trade halves of two neighbouring tiles, so that a store is 16 bytes a
+      // lane and 64 contiguous bytes per query row.  No LDS, no barrier: the workgroup goes on to its next item while the stores
+      // drain. ----
+      if (row_ok) {
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
           const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-          if (qrow < n) rowstat[(int64_t)h * n + qrow] = make_float2(m_run[qt], l_tot[qt]);
-        }
-      }
-    }
-
-    // ---- epilogue: normalise and store straight from the accumulators.  A lane holds 4 consecutive channels of its
-    // query per channel tile; lane groups 2i and 2i + 1 trade halves of two neighbouring tiles, so that a store is 16 bytes a
-    // lane and 64 contiguous bytes per query row.  No LDS, no barrier: the workgroup goes on to its next item while the stores
-    // drain. ----
-    if (row_ok) {
+          const float inv_l = 1.0f / l_tot[qt];
+          sp_bf16* dst = out + (qrow * hq + h) * AT_D + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        const int64_t qrow = (int64_t)r * AT_BS + q_off + qt * 16;
-        const float inv_l = 1.0f / l_tot[qt];
-        sp_bf16* dst = out + (qrow * hq + h) * AT_D + 16 * (g & 1) + 8 * (g >> 1);
+          for (int dt = 0; dt < (HALF ? 4 : 8); dt += 2) {
+            uint32_t w[2][2];  // [tile dt, dt + 1][channels 4g, 4g + 1 | 4g + 2, 4g + 3]
 #pragma unroll
-        for (int dt = 0; dt < (HALF ? 4 : 8); dt += 2) {
-          uint32_t w[2][2];  // [tile dt, dt + 1][channels 4g, 4g + 1 | 4g + 2, 4g + 3]
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            w[u][0] = at_pack2(o[dt + u][qt][0] * inv_l, o[dt + u][qt][1] * inv_l);
-            w[u][1] = at_pack2(o[dt + u][qt][2] * inv_l, o[dt + u][qt][3] * inv_l);
-          }
-          const auto first = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
-          const auto second = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
-          if (qrow < n) *reinterpret_cast<uint4*>(dst + dt * 16) = make_uint4(first[0], second[0], first[1], second[1]);
-        }
-      }
-    }
-    if constexpr (PV) {
-      // ---- a pivot's rows: avg[h][r][c] = mean over the valid queries of block r of exp2(u[q][c] - m[q]) / l[q], by the row's
-      // four waves, each every fourth block of the list, four of them in flight ----
-      __syncthreads();  // the block sums of every wave have left, the rings are free
-      float2* const stat = reinterpret_cast<float2*>(lds + AT_PIVOT_STAT_AT) + grp * AT_BS;  // (m, l) of the row's queries
-      if (g == 0)
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) stat[q_off + qt * 16] = make_float2(m_run[qt], l_tot[qt]);
-      __syncthreads();
-      if (row_ok) {
-        const int64_t rem = n - (int64_t)r * AT_BS;
-        const int valid_q = rem < AT_BS ? (int)rem : AT_BS, lane = tq_o & 63;
-        float m[2], inv_l[2];
-        bool ok[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int qo = lane + 64 * j;
-          ok[j] = qo < valid_q;
-          const float2 st = stat[ok[j] ? qo : 0];
-          m[j] = st.x;
-          inv_l[j] = 1.0f / st.y;
-        }
-        const float inv_q = 1.0f / (float)valid_q;
-        float* const arow = avg_attn + ((int64_t)h * nb + r) * nb;
-        for (int i0 = wave & 3; i0 < n_blk; i0 += 16) {
-          int col[4];
-          float u[4][2];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const uint32_t e = i0 + 4 * k < n_blk ? blist[i0 + 4 * k] : 0u;
-            col[k] = __builtin_amdgcn_readfirstlane((e & my_flag) != 0u ? (int)(e & AT_COL_MASK) : -1);
-            const float* src = pu + (int64_t)(col[k] < 0 ? r : col[k]) * AT_BS + lane;
-            u[k][0] = src[0];
-            u[k][1] = src[64];
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float part = ok[0] ? __builtin_amdgcn_exp2f(u[k][0] - m[0]) * inv_l[0] : 0.f;
-            part += ok[1] ? __builtin_amdgcn_exp2f(u[k][1] - m[1]) * inv_l[1] : 0.f;
-            part = at_wave_sum(part);
-            if (lane == 0 && col[k] >= 0) arow[col[k]] = part * inv_q;
+            for (int u = 0; u < 2; ++u) {
+              w[u][0] = at_pack2(o[dt + u][qt][0] * inv_l, o[dt + u][qt][1] * inv_l);
+              w[u][1] = at_pack2(o[dt + u][qt][2] * inv_l, o[dt + u][qt][3] * inv_l);
+            }
+            const auto first = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+            const auto second = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+            if (qrow < n) *reinterpret_cast<uint4*>(dst + dt * 16) = make_uint4(first[0], second[0], first[1], second[1]);
           }
         }
       }
-      if (pivot.st.n_clusters > 0) {
-        static_assert(AT_PIVOT_STAT_AT + 2 * AT_BS * sizeof(float2) <= AT_RING * (AT_KBUF_BYTES + AT_VBUF_BYTES), "");
+      if constexpr (PV) {
+        // ---- a pivot's rows: avg[h][r][c] = mean over the valid queries of block r of exp2(u[q][c] - m[q]) / l[q], by the row's
+        // four waves, each every fourth block of the list, four of them in flight ----
+        __syncthreads();  // the block sums of every wave have left, the rings are free
+        float2* const stat = reinterpret_cast<float2*>(lds + AT_PIVOT_STAT_AT) + grp * AT_BS;  // (m, l) of the row's queries
+        if (g == 0)
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt) stat[q_off + qt * 16] = make_float2(m_run[qt], l_tot[qt]);
+        __syncthreads();
+        if (row_ok) {
+          const int64_t rem = n - (int64_t)r * AT_BS;
+          const int valid_q = rem < AT_BS ? (int)rem : AT_BS, lane = tq_o & 63;
+          float m[2], inv_l[2];
+          bool ok[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int qo = lane + 64 * j;
+            ok[j] = qo < valid_q;
+            const float2 st = stat[ok[j] ? qo : 0];
+            m[j] = st.x;
+            inv_l[j] = 1.0f / st.y;
+          }
+          const float inv_q = 1.0f / (float)valid_q;
+          float* const arow = avg_attn + ((int64_t)h * nb + r) * nb;
+          for (int i0 = wave & 3; i0 < n_blk; i0 += 16) {
+            int col[4];
+            float u[4][2];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t e = i0 + 4 * k < n_blk ? blist[i0 + 4 * k] : 0u;
+              col[k] = __builtin_amdgcn_readfirstlane((e & my_flag) != 0u ? (int)(e & AT_COL_MASK) : -1);
+              const float* src = pu + (int64_t)(col[k] < 0 ? r : col[k]) * AT_BS + lane;
+              u[k][0] = src[0];
+              u[k][1] = src[64];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              float part = ok[0] ? __builtin_amdgcn_exp2f(u[k][0] - m[0]) * inv_l[0] : 0.f;
+              part += ok[1] ? __builtin_amdgcn_exp2f(u[k][1] - m[1]) * inv_l[1] : 0.f;
+              part = at_wave_sum(part);
+              if (lane == 0 && col[k] >= 0) arow[col[k]] = part * inv_q;
+            }
+          }
+        }
+        if (pivot.st.n_clusters > 0) {
+          static_assert(AT_PIVOT_STAT_AT + 2 * AT_BS * sizeof(float2) <= AT_RING * (AT_KBUF_BYTES + AT_VBUF_BYTES), "");
 #pragma unroll 1
-        for (int rr = r_a; rr <= (has_b ? r_b : r_a); ++rr) {
-          __syncthreads();  // the rows are written; the LDS of the row before is free
-          pivot_row<AT_FWD_THREADS>(pivot, pivot_sh, lds, avg_attn, rr, h);
+          for (int rr = r_a; rr <= (has_b ? r_b : r_a); ++rr) {
+            __syncthreads();  // the rows are written; the LDS of the row before is free
+            pivot_row<AT_FWD_THREADS>(pivot, pivot_sh, lds, avg_attn, rr, h);
+          }
         }
       }
-    }
     };  // run
     if (!PIVOT || __builtin_expect(slot == AT_NO_SLOT, 1))
       run(std::false_type{});
@@ -1276,7 +1283,7 @@ __global__ __launch_bounds__(AT_FWD_THREADS, 1) void sp_attn_fwd_kernel(
 //             by heads when that union is strictly smaller and the two heads may share an item (same kv head, neither
 //             a pivot that keeps its block sums);
 //   weights : the work of every gang that is ranked -- the blocks its items' two rows visit together, plus a few blocks' worth of
-//             fixed time per item.
+//             fixed time per item; a pivot's item weighs like any other, though its block sums, maps and patterns are work too.
 // Integer sums throughout, so nothing depends on the order of anything.
 // Pure latency: a launch, and chains of loads from L2; a workgroup a head pair, a thread a row pair, then a lane an item.  With
 // one workgroup for all of it, the ranking included, the launch took 8 us at 10007 tokens (28 heads) and 20 at 32768 (32 heads);

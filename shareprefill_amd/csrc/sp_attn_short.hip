@@ -467,15 +467,20 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
 }
 
 // ---- host ---------------------------------------------------------------------------------------------
-// The lines between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs.  128
-// channels, whole layer, one box, us here / there:
-//   masks of the selection (32 query / 8 kv heads at coverage 0.95): 6656 tokens 197 / 221, 8192 248 / 272; at 0.99 262 / 271 and
-//   347 / 342, with every head query-aware (nine blocks of ten kept) 443 / 445 and 612 / 594; 28 / 4 heads at 6656 182 / 211, 240 /
-//   251, 408 / 433, 8 / 2 heads 140 / 159, 191 / 197, 236 / 250;
-//   every block kept: 32 / 8 heads 4608 221 / 228, 5120 233 / 235, 5632 275 / 266, 6656 373 / 332; 28 / 4 6177 292 / 293; 8 / 2
-//   6656 159 / 161.
-// 64 channels, attention alone, where the persistent kernel computes on zero-padded tiles (the padding itself not counted): all
-// blocks 8192 322 / 329, 24576 2602 / 2577, 32768 4587 / 4680; masks at 0.95 8192 96 / 133, 32768 486 / 552.
+// The lines between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs.  Whole layers,
+// us here / there, in one call (two runs of one side within 0.5 %).  128 channels:
+//   masks of the selection, 32 query / 8 kv heads: coverage 0.65 6656 tokens 180 / 189, 8192 198 / 202, 10007 243 / 256; 0.95 201 / 210,
+//   226 / 236, 282 / 285; 0.99 257 / 257, 324 / 315, 451 / 433; every head query-aware 209 / 220, 243 / 251, 306 / 312;
+//   28 / 4 heads, the same coverages at 6656 and 8192: 166 / 189, 183 / 198; 184 / 199, 208 / 220; 239 / 237, 299 / 287; 8 / 2 heads: 88 /
+//   101, 91 / 99; 132 / 146, 142 / 138; 178 / 180, 205 / 207;
+//   every block kept: 32 / 8 heads 5120 220 / 242, 5632 263 / 273, 6177 318 / 317, 6656 358 / 347; 28 / 4 5632 234 / 260, 6656 316 / 331;
+//   8 / 2 6656 148 / 156.
+// So up to 6656 tokens this kernel is never behind by more than 1 %, whatever the coverage; beyond, it is ahead at low coverage and
+// behind at 0.99.  (The line of dense masks stands a little low: 5632 is this kernel's too.)
+// 64 channels, where the persistent kernel computes on zero-padded tiles (padding counted), 32 / 8 heads: 0.65 8192 148 / 254, 32768
+// 448 / 810, 49152 715 / 1244; 0.95 143 / 253, 583 / 907, 1268 / 1692; 0.99 147 / 261, 1177 / 1422, 2970 / 3100; every block kept 311 / 409,
+// 4920 / 5135, 10775 / 11010; 14 / 2 heads 0.95 32768 333 / 462, every block 2062 / 2198.  The line is where both were once even without
+// the padding; what lies beyond it is not measured but for these lengths, and each pivot's block sums take 16.8 MB there.
 extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
 }

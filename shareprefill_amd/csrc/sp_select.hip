@@ -1367,11 +1367,11 @@ struct MaskBesides {
   int32_t *decision, *nv_f, *ns_f;
   float *js_v, *js_s;
 };
-// (as a launch of one workgroup in between: 3001 tokens 110.1 us a layer against 107.7, 6177 of 64 channels 122.3 / 120.0, 10007 258.4 /
-// 255.5)
 // sp_share_decide_kernel's decision for head h, by every workgroup of the head for itself: "first" only looks at lower heads of its
 // cluster that are not query-aware.  The state stays as the previous layers left it until the next launch (share_elect in
-// sp_queryaware_small_kernel), so no workgroup can see another's election.  Every thread of the workgroup calls it.
+// sp_queryaware_small_kernel), so no workgroup can see another's election.  Every thread of the workgroup calls it.  Layers with the
+// election as a launch of one workgroup in between / with it here, us: 3001 tokens 110.1 / 107.7, 6177 of 64 channels 122.3 / 120.0,
+// 10007 258.4 / 255.5.
 __device__ static __forceinline__ int mask_decide(const sp_cluster_state& st, const int32_t* __restrict__ head_cluster, int h,
                                                   const MaskBesides& a) {
   const int t = threadIdx.x, c = head_cluster[h], qa = a.use_qa[h];
