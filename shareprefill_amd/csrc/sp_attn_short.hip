@@ -42,6 +42,8 @@ struct AsArgs {
   int slots;                 // pivot heads there is room for; -1: no maps wanted
   int64_t n, sq_n, sq_h, sk_n, sk_h, sv_n, sv_h;
   int hq, group, nb, nbw;
+  int rotate;                // grid of (8, hq / 8, rows): heads rotate over the XCDs from row to row
+  uint32_t group_mul;        // h / group = (h * group_mul) >> 32, or 0: divide
   int zero_maps;             // 1: no decisions, every row of avg_attn is cleared
   float scale_log2;
 };
@@ -61,7 +63,7 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 #define AS_TILE 64      // keys per step
 #define AS_THREADS 256  // 4 waves x 32 queries
 #define AS_WAVES 4
-#define AS_MAX_NB 512     // blocks a row's list holds
+#define AS_MAX_NB 512     // blocks of a row: its mask is at most eight words, its maps fit the tiles' LDS
 #define AS_LDS_BYTES(D) (4 * AS_TILE * (D) * 2)
 #define AS_NO_MAX (-1.0e30f)         // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
 #define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
@@ -69,12 +71,19 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void* as_lds_ptr;
 typedef const __attribute__((address_space(1))) void* as_gbl_ptr;
 
-// K and V tiles are [64 keys][D] bf16 in 16-byte chunks, the chunk index XOR-swizzled by the row so that both kinds of
-// operand read are free of bank conflicts: the K read (one chunk of 16 consecutive rows) and the transposing V read (two
-// neighbouring chunks of 16 consecutive rows).  Rows of 64 channels are half a bank cycle long: two rows share a swizzle.
+// K and V tiles are [64 keys][D] bf16 in 16-byte chunks, the chunk index XOR-swizzled by the row so that each kind of operand read
+// is free of bank conflicts.  The LDS serves 256 bytes a cycle: 16 lanes of a K read (one chunk of 16 consecutive rows), so K's
+// chunks are permuted by the row; 32 lanes of a transposing V read (two neighbouring chunks of 8 consecutive rows), so V's pairs
+// of chunks are: by the single chunks rows 2i and 2i + 1 met in the same banks, a third of the LDS's active cycles.  Rows of 64
+// channels are half a bank cycle long: two rows share a swizzle.
 template <int D>
 __device__ __forceinline__ int as_swz(int row) {
   return D == 128 ? (row & 15) : ((row >> 1) & 7);
+}
+
+template <int D>
+__device__ __forceinline__ int as_swz_v(int row) {
+  return D == 128 ? 2 * (row & 7) : 2 * ((row >> 1) & 3);
 }
 
 __device__ __forceinline__ uint32_t as_pack2(float a, float b) {
@@ -84,37 +93,42 @@ __device__ __forceinline__ uint32_t as_pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, as_bf16x2));
 }
 
-// One tile by direct global -> LDS 128-bit loads: a wave-instruction fills 1 KiB (lane i writes chunk base + i and fetches
-// whichever chunk belongs there).  Row and swizzle of a lane are the same in every instruction up to a uniform step, so a
-// lane's address is a uniform base plus an offset made once; only the tile that reaches past the sequence clamps its rows
-// onto the last key (such keys lie behind every stored query).
-template <int D>
+// One tile by direct memory -> LDS 128-bit loads: a wave-instruction fills 1 KiB (lane i writes chunk base + i and fetches
+// whichever chunk belongs there).  A block is a buffer of its own, so that a load is a lane offset made once, a scalar offset
+// that only depends on where in the block it stands, and the LDS address in m0; only the tiles of a block that ends with the
+// sequence clamp their rows onto the last key (such keys lie behind every stored query).
+// What stands between a tile's barrier and its first matrix instruction is in series: with 64-bit addresses made for every load, the
+// kept blocks in a list in LDS and V's bank conflicts a step took some hundred cycles of 3300 more (layers, us: 700 tokens 21.9 -> 21.4,
+// 3001 105.0 -> 103.7, 6600 at coverage 0.99 255.4 -> 252.9; 64 channels 6177 tokens 120.4 -> 119.0, 20000 at 0.99 514 -> 499).  Of the
+// rest the loads' issue is 600; spread over the products, rings of three and four tiles, 16 queries a wave in twice the waves (the LDS's
+// reads double: 8 % slower), tiles of 32 keys with a third workgroup on the CU (15 %) and products between the probabilities' arithmetic
+// (a wave alone issues no faster) gain nothing.
+template <int D, bool V>
 __device__ __forceinline__ uint32_t as_lane_off(int64_t stride_n, int wave, int lane) {
   constexpr int CHUNKS = D / 8, ROWS = 64 / CHUNKS;  // chunks per row, rows per wave-instruction
   const int row = wave * ROWS + lane / CHUNKS;
-  return (uint32_t)(row * (int)stride_n + ((lane % CHUNKS) ^ as_swz<D>(row)) * 8) * 2u;
+  return (uint32_t)(row * (int)stride_n + ((lane % CHUNKS) ^ (V ? as_swz_v<D>(row) : as_swz<D>(row))) * 8) * 2u;
 }
-template <int D>
-__device__ __forceinline__ void as_issue(const sp_bf16* __restrict__ x, int64_t stride_n, int64_t key0, int64_t n,
-                                         uint32_t lane_off, char* tile, int wave, int lane) {
+template <int D, bool V>
+__device__ __forceinline__ void as_issue(__amdgpu_buffer_rsrc_t block, uint32_t row_bytes, int rows /* of the block */, int part,
+                                         uint32_t lane_off, uint32_t tile /* LDS offset, the wave's */, int wave, int lane) {
   constexpr int CHUNKS = D / 8, ROWS = 64 / CHUNKS;
   constexpr int STEP = ROWS * AS_WAVES, ITS = AS_TILE / STEP;  // rows per instruction of all waves (a multiple of the swizzle's period)
-  if (key0 + AS_TILE <= n) {
-    const char* base = reinterpret_cast<const char*>(x + key0 * stride_n);
+  if (rows == AS_BS) {
 #pragma unroll
     for (int it = 0; it < ITS; ++it)
-      __builtin_amdgcn_global_load_lds((as_gbl_ptr)(base + (int64_t)it * STEP * 2 * stride_n + lane_off),
-                                       (as_lds_ptr)(tile + (it * AS_WAVES + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(block, (as_lds_ptr)(uintptr_t)(tile + it * AS_WAVES * 1024), 16, (int)lane_off,
+                                               (int)((part * ITS + it) * (STEP * row_bytes)), 0, 0);
   } else {
     int ln = lane;
     asm volatile("" : "+v"(ln));  // (keeps this rare path's lane arithmetic out of the tile loop)
 #pragma unroll 1
     for (int it = 0; it < ITS; ++it) {
-      const int seg = it * AS_WAVES + wave, row = seg * ROWS + ln / CHUNKS;
-      int64_t key = key0 + row;
-      if (key > n - 1) key = n - 1;
-      __builtin_amdgcn_global_load_lds((as_gbl_ptr)(x + key * stride_n + ((ln % CHUNKS) ^ as_swz<D>(row)) * 8),
-                                       (as_lds_ptr)(tile + seg * 1024), 16, 0, 0);
+      const int in_tile = (it * AS_WAVES + wave) * ROWS + ln / CHUNKS;
+      const int row = part * AS_TILE + in_tile < rows ? part * AS_TILE + in_tile : rows - 1;
+      const int chunk = (ln % CHUNKS) ^ (V ? as_swz_v<D>(in_tile) : as_swz<D>(in_tile));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(block, (as_lds_ptr)(uintptr_t)(tile + it * AS_WAVES * 1024), 16,
+                                               (int)((uint32_t)row * row_bytes + 16u * chunk), 0, 0, 0);
     }
   }
 }
@@ -177,26 +191,49 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS, WQ = 16 * QT;
   constexpr int TILE_BYTES = AS_TILE * D * 2;
   extern __shared__ __attribute__((aligned(1024))) char lds[];  // [buffer][K | V]
-  __shared__ uint16_t list[AS_MAX_NB];
   const int t = threadIdx.x, lane = t & 63, lq = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // query band
   const uint32_t lds_base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
-  int h, rr;  // head, rank of the row (0 = the last, heaviest one)
-  if ((a.hq & 7) == 0) {
-    const int per = a.hq >> 3, i = blockIdx.x >> 3;
-    rr = i / per;
-    h = ((blockIdx.x + rr) & 7) * per + i % per;
-  } else {
-    h = blockIdx.x % a.hq;
-    rr = blockIdx.x / a.hq;
-  }
-  const int r = a.nb - 1 - rr;
-  const int kvh = h / a.group;
+  // Head and rank of the row (0 = the last, heaviest one); the grid is (8, hq / 8, rows) or (hq, 1, rows).  An integer division
+  // costs a wave that has its SIMD to itself some 300 cycles in front of its first load, hence the grid's form and the multiplier.
+  const int rr = blockIdx.z, r = a.nb - 1 - rr;
+  const int h = a.rotate ? ((blockIdx.x + rr) & 7) * gridDim.y + blockIdx.y : blockIdx.x;
+  const int kvh = a.group_mul ? (int)__umulhi((uint32_t)h, a.group_mul) : h / a.group;
   const sp_bf16* kh = a.k + (int64_t)kvh * a.sk_h;
   const sp_bf16* vh = a.v + (int64_t)kvh * a.sv_h;
 
   const int dec = a.slots >= 0 ? a.decision[h] : 0;  // (asked for up here: its way from memory passes under the mask's)
 
+  const uint32_t k_lane = as_lane_off<D, false>(a.sk_n, wave, lane), v_lane = as_lane_off<D, true>(a.sv_n, wave, lane);
+  const uint32_t k_row = (uint32_t)a.sk_n * 2u, v_row = (uint32_t)a.sv_n * 2u;  // bytes
+  const int last_rows = (int)(a.n - (int64_t)(a.nb - 1) * AS_BS);
+  __amdgpu_buffer_rsrc_t k_blk, v_blk;  // the block whose tiles are being fetched
+  int blk_rows = 0;
+  auto open_block = [&](int c) {
+    blk_rows = c == a.nb - 1 ? last_rows : AS_BS;
+    auto block = [&](const sp_bf16* x, uint32_t row_bytes) {
+      const char* p = (const char*)x + (uint64_t)(uint32_t)c * (uint64_t)(AS_BS * row_bytes);
+      return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)((uint32_t)(blk_rows - 1) * row_bytes + 2u * D), 0x00027000);
+    };
+    k_blk = block(kh, k_row);
+    v_blk = block(vh, v_row);
+  };
+  const uint32_t lds_wave = lds_base + wave * 1024;
+  auto issue = [&](int part, int buf) {
+    const uint32_t at = lds_wave + (uint32_t)(buf * 2 * TILE_BYTES);
+    as_issue<D, false>(k_blk, k_row, blk_rows, part, k_lane, at, wave, lane);
+    as_issue<D, true>(v_blk, v_row, blk_rows, part, v_lane, at + TILE_BYTES, wave, lane);
+  };
+  // The row's mask, one word per lane; the kept blocks are walked bit by bit in scalar registers.  The first tile of block 0, which
+  // nearly every row keeps, is on its way before the mask is there (a row that does not fetches its own into the same place: loads
+  // land in order).
+  const uint64_t* const mask_row = a.mask + ((int64_t)h * a.nb + r) * a.nbw;
+  const int last_w = r >> 6;
+  uint64_t lane_word = 0;
+  if (lane <= last_w) lane_word = mask_row[lane];
+  if (lane == last_w && (r & 63) != 63) lane_word &= (2ull << (r & 63)) - 1ull;
+  open_block(0);
+  issue(0, 0);
   const int q_off = wave * WQ + lq;  // the first of the lane's queries; the others are 16 further each
   const int64_t qrow = (int64_t)r * AS_BS + q_off;
   as_bf16x8 qb[QT][KS];
@@ -208,33 +245,33 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
     for (int ks = 0; ks < KS; ++ks)
       qb[qt][ks] = __builtin_bit_cast(as_bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
   }
-  const uint32_t k_lane = as_lane_off<D>(a.sk_n, wave, lane), v_lane = as_lane_off<D>(a.sv_n, wave, lane);
-  auto issue = [&](int c, int half, int buf) {
-    const int64_t key0 = (int64_t)c * AS_BS + half * AS_TILE;
-    // (a last block that ends in its first half: the second half is all beyond the sequence; its one key is the last)
-    const int64_t k0 = key0 < a.n ? key0 : a.n - 1;
-    as_issue<D>(kh, a.sk_n, k0, a.n, k_lane, lds + buf * 2 * TILE_BYTES, wave, lane);
-    as_issue<D>(vh, a.sv_n, k0, a.n, v_lane, lds + buf * 2 * TILE_BYTES + TILE_BYTES, wave, lane);
+  const uint32_t word_lo = (uint32_t)lane_word, word_hi = (uint32_t)(lane_word >> 32);
+  auto word = [&](int w) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane(word_lo, w) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane(word_hi, w) << 32;
   };
-  // the row's kept blocks, ascending: every wave counts the (uniform) mask words, wave w compacts its share of them
-  int n_blk = 0, c = 0;
-  {
-    const uint64_t* row = a.mask + ((int64_t)h * a.nb + r) * a.nbw;
-    for (int wi = 0; wi <= (r >> 6); ++wi) {
-      uint64_t x = row[wi];
-      if (wi == (r >> 6) && (r & 63) != 63) x &= (2ull << (r & 63)) - 1ull;
-      if (n_blk == 0 && x != 0ull) {  // the first tile is on its way while the list is made
-        c = wi * 64 + __builtin_ctzll(x);
-        issue(c, 0, 0);
-      }
-      if (wi % WAVES == wave && ((x >> lane) & 1ull))
-        list[n_blk + __builtin_popcountll(x & ((1ull << lane) - 1ull))] = (uint16_t)(wi * 64 + lane);
-      n_blk += __builtin_popcountll(x);
+  int n_blk = 0;
+  for (int w = 0; w <= last_w; ++w) n_blk += __builtin_popcountll(word(w));
+  struct Walk {
+    uint64_t x;
+    int w;
+  };
+  auto next_block = [&](Walk& k) {  // (there is one)
+    while (k.x == 0ull) k.x = word(++k.w);
+    const int c = k.w * 64 + __builtin_ctzll(k.x);
+    k.x &= k.x - 1ull;
+    return c;
+  };
+  Walk walk = {word(0), 0};
+  int c = 0;
+  if (n_blk > 0) {
+    c = next_block(walk);
+    if (c != 0) {
+      open_block(c);
+      issue(0, 0);
     }
-    n_blk = __builtin_amdgcn_readfirstlane(n_blk);
+  } else {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // (vmcnt(0): no load may outlive the wave)
   }
-  // the list is complete (a plain __syncthreads would wait for the first tile as well)
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   as_floatx4 o[CT][QT], l[QT];  // l: row sums (ones . P, every row of the tile holds the sum)
   float m[QT], l_mark[QT];
@@ -262,20 +299,20 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   // 32 bytes of channel tile ct.  Rows 16 further have the same swizzle.
   const int koff = lq * (D * 2), kswz = as_swz<D>(lq);
   const int vrow = 4 * g + (lq >> 2);
-  const int voff = vrow * (D * 2) + 8 * (lq & 1), vswz = as_swz<D>(vrow), vhalf = (lq >> 1) & 1;
+  const int voff = vrow * (D * 2) + 8 * (lq & 1), vswz = as_swz_v<D>(vrow), vhalf = (lq >> 1) & 1;
 
   int c_next = 0;
-  // One step per tile, two per block.  The block list is read a block ahead of its use.
+  // One step per tile, two per block, a buffer for either; the block behind is opened when its first tile is asked for.
   for (int st = 0; st < 2 * n_blk; ++st) {
-    const int i = st >> 1, half = st & 1, buf = half;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of the tile have landed
-    __syncthreads();                     // ... everybody's; and the other buffer's readers are done
+    const int half = st & 1, buf = half;
+    // this wave's loads of the tile have landed, and everybody's; the other buffer's readers are done
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (half == 0) {
-      issue(c, 1, buf ^ 1);
-      c_next = (int)list[i + 1 < n_blk ? i + 1 : i];
-    } else if (i + 1 < n_blk) {
-      c_next = __builtin_amdgcn_readfirstlane(c_next);
-      issue(c_next, 0, buf ^ 1);
+      issue(1, 1);
+    } else if (st + 1 < 2 * n_blk) {
+      c_next = next_block(walk);
+      open_block(c_next);
+      issue(0, 0);
     }
     const bool diag = c == r;
     if (!diag || half * AS_TILE <= wave * WQ + WQ - 1) {  // (else: every key of the tile lies behind the wave's queries)
@@ -419,27 +456,36 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     inv_l[qt] = 1.0f / l[qt][0];
-    if (qrow + 16 * qt < a.n) {
-      sp_bf16* dst = a.out + ((qrow + 16 * qt) * a.hq + h) * D + 4 * g;
+    // (lane groups 2i and 2i + 1 trade halves of two neighbouring channel tiles: 16 bytes a store, 64 contiguous ones a row)
+    sp_bf16* dst = a.out + ((qrow + 16 * qt) * a.hq + h) * D + 16 * (g & 1) + 8 * (g >> 1);
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-        *reinterpret_cast<uint2*>(dst + ct * 16) = make_uint2(as_pack2(o[ct][qt][0] * inv_l[qt], o[ct][qt][1] * inv_l[qt]),
-                                                              as_pack2(o[ct][qt][2] * inv_l[qt], o[ct][qt][3] * inv_l[qt]));
+    for (int ct = 0; ct < CT; ct += 2) {
+      uint32_t w[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        w[u][0] = as_pack2(o[ct + u][qt][0] * inv_l[qt], o[ct + u][qt][1] * inv_l[qt]);
+        w[u][1] = as_pack2(o[ct + u][qt][2] * inv_l[qt], o[ct + u][qt][3] * inv_l[qt]);
+      }
+      const auto lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+      const auto hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+      if (qrow + 16 * qt < a.n) *reinterpret_cast<uint4*>(dst + ct * 16) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
     }
   }
   if (a.zero_maps)
     for (int i = t; i < a.nb; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + i] = 0.f;
   if (!pivot) return;  // (uniform)
   if (pu == nullptr) {  // more pivots than the caller made room for: no map, and visibly so
-    for (int i = t; i < n_blk; i += THREADS) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = NAN;
+    for (int i = t; i <= r; i += THREADS)
+      if ((mask_row[i >> 6] >> (i & 63)) & 1ull) a.avg_attn[((int64_t)h * a.nb + r) * a.nb + i] = NAN;
     return;
   }
   // pivot head: avg[r][c] = mean over the block's valid queries of exp2(u - m[q]) / l[q].  A wave
   // reads back its own sums (its own stores), folds its queries, and the waves meet in LDS.
-  float* const part = reinterpret_cast<float*>(lds);  // [block][wave]
+  float* const part = reinterpret_cast<float*>(lds);  // [column][wave]
   __syncthreads();                                    // LDS is free, the stores of pu have left
+  walk = {word(0), 0};
   for (int i = 0; i < n_blk; ++i) {
-    const int c = (int)list[i];
+    const int c = next_block(walk);
     float x = 0.f;
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
@@ -448,16 +494,17 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
       }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, SP_WAVE);
-    if (lane == 0) part[i * WAVES + wave] = x;
+    if (lane == 0) part[c * WAVES + wave] = x;
   }
   __syncthreads();
   const int64_t rem = a.n - (int64_t)r * AS_BS;
   const float inv_q = 1.0f / (float)(rem < AS_BS ? (int)rem : AS_BS);
-  for (int i = t; i < n_blk; i += THREADS) {
+  for (int i = t; i <= r; i += THREADS) {
+    if (!((mask_row[i >> 6] >> (i & 63)) & 1ull)) continue;
     float x = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) x += part[i * WAVES + w];
-    a.avg_attn[((int64_t)h * a.nb + r) * a.nb + (int)list[i]] = x * inv_q;
+    a.avg_attn[((int64_t)h * a.nb + r) * a.nb + i] = x * inv_q;
   }
   if constexpr (std::is_same<Args, AsPivotArgs>::value) {
     __shared__ PivotRowShared pivot_sh;
@@ -516,12 +563,15 @@ static int as_launch(const char* who, const void* q, const void* k, const void* 
              "%s: workspace missing or misaligned", who);
   const size_t room = workspace_bytes / sp_attn_pivot_scratch_bytes(n, AS_BS);
   const int slots = !maps ? -1 : room < (size_t)hq ? (int)room : hq;
+  const bool rotate = hq % 8 == 0 && hq / 8 <= 65535;
+  // (h * group_mul) >> 32 is h / group while h * group < 2^32
+  const uint32_t group_mul = hq < 65536 && hq > hkv ? (uint32_t)((1ull << 32) / (uint32_t)(hq / hkv)) + 1u : 0u;
   const AsArgs a = {(const sp_bf16*)q, (const sp_bf16*)k, (const sp_bf16*)v, mask, decision, (sp_bf16*)out, avg_attn,
                     (float*)workspace, slots, n, q_stride_n, q_stride_h, k_stride_n, k_stride_h, v_stride_n,
-                    v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), decision == nullptr && avg_attn != nullptr,
+                    v_stride_h, hq, hq / hkv, (int)nb, (int)((nb + 63) / 64), rotate, group_mul, decision == nullptr && avg_attn != nullptr,
                     softmax_scale * 1.4426950408889634f};
   static_assert(AS_LDS_BYTES(64) >= AS_MAX_NB * 14 + AS_THREADS * 8 + 16, "");  // rs_lds_bytes(AS_MAX_NB, AS_THREADS)
-  const dim3 grid((unsigned)(nb * hq));
+  const dim3 grid(rotate ? 8 : (unsigned)hq, rotate ? (unsigned)(hq / 8) : 1, (unsigned)nb);
   static bool attr_set[64] = {false};  // per device, once (idempotent)
   int dev = 0;
   SP_HIP(hipGetDevice(&dev));

@@ -54,6 +54,36 @@ def test_short_attention_matches_oracle(gpu_device, hq, hkv, n, d):
         assert np.abs(avg[h] - np.asarray(maps[h])).max() <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,n", [(8, 8, 257),    # no groups, a last block of one token
+                                      (24, 3, 700),   # heads rotate over the XCDs; groups of eight
+                                      (14, 2, 1153),  # they do not; groups of seven
+                                      (40, 8, 8321)])  # two mask words a row, groups of five
+def test_rows_whose_first_kept_block_is_not_the_first(gpu_device, hq, hkv, n, d):
+    """A row's first tile is asked for as block 0's before its mask is there: rows that keep that block and rows that do not,
+    some of them keeping nothing but their own, some nothing in their first mask word; keys and values in rows wider than the head."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator().manual_seed(n + d)
+    mk = lambda h, width: torch.randn(n, h, width, generator=gen).to(torch.bfloat16)[..., :d].transpose(0, 1)
+    q, k, v = mk(hq, d), mk(hkv, d + 8), mk(hkv, 2 * d)
+    nb = -(-n // 128)
+    rng = np.random.default_rng(n)
+    mask = np.tril(rng.random((hq, nb, nb)) < 0.3)
+    mask[:, 1::2, 0] = False
+    mask[::3, nb // 2, :] = False
+    mask[1::3, -1, :min(64, nb - 1)] = False
+    mask[:, np.arange(nb), np.arange(nb)] = True
+    ref, _ = O.masked_attention(q, k, v, mask, 128, d ** -0.5)
+    bits = ops.bool_to_mask(torch.from_numpy(mask)).to(gpu_device)
+    on_gpu = lambda t: t.transpose(0, 1).to(gpu_device).transpose(0, 1)
+    wide = lambda t, width: torch.nn.functional.pad(on_gpu(t).transpose(0, 1), (0, width - d), value=float("nan"))[..., :d].transpose(0, 1)
+    out = ops.short_attention(on_gpu(q), wide(k, d + 8), wide(v, 2 * d), bits, d ** -0.5).transpose(0, 1).float().cpu()
+    ref = ref.float()
+    assert (out - ref).abs().max().item() <= MAX_ABS
+    assert ((out - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
+
+
 @pytest.mark.parametrize("hq,hkv,n,d", [(6, 2, 1, 64), (6, 2, 1111, 128), (6, 6, 2177, 64), (32, 8, 2048, 128),
                                         (32, 8, 2177, 128), (3, 1, 8300, 128)])
 def test_pivot_patterns_in_the_attention_launch(gpu_device, hq, hkv, n, d):
