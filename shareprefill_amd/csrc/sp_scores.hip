@@ -19,8 +19,8 @@
 
                              // D, the head dim, is 64 or 128: a template parameter of every kernel here
 #define LQ_THREADS 256       // 4 waves per head, wave w owns 32 query rows of the last block
-#define LQ_MIN_TILES 1       // key tiles per workgroup of the statistics kernel: a power of two, at most 32 -- as many as
-#define LQ_MAX_TILES 32      // still leave one round of workgroups at long sequences, as few as give one at short ones
+#define LQ_MIN_TILES 1       // key tiles per workgroup of the statistics kernel (lq_tiles_per_wg)
+#define LQ_MAX_TILES 32
 // lane's operand: scaled last-block queries, D / 16 k-steps x 8 bf16; MFMA row m = lane % 32 of wave w is query 32 w + m of
 // the last block, or query 127 - (32 w + m) with REVERSED
 template <bool REVERSED, int KS>
@@ -605,13 +605,23 @@ int sp_block_probs_mfma_launch(const void* qbar, const void* kbar, const int32_t
 }
 
 // ---- host -------------------------------------------------------------------------------------------------
+// Key tiles per workgroup of the statistics kernel: of all counts the one whose launch is the shortest, by the times it was measured
+// to take (0.01 us; 128 channels, 3001 to 131072 tokens, counts 1 to 32, each within 10 %): a tile 2.9 us in a workgroup that has its CU
+// to itself and 2.35 per tile of a CU with two, 6 and 9.5 us besides, and the launch that folds what the probabilities kernel does not
+// fold itself; a CU without a workgroup counts 0.03 us, by what layers take (6177 tokens of 64 channels: 208 workgroups of four tiles
+// 122.2 us, 400 of two 121.6).  Against counts that were powers of two and made some 512 workgroups, us for both: 4500 tokens
+// 17.8 / 15.5, 10007 of 28 heads 24.1 / 19.4, 16384 30.6 / 27.6, 20000 of 64 channels 34.9 / 24.0, 65001 90.7 / 85.0.
 static inline int lq_tiles_per_wg(int64_t n, int32_t hq) {
-  const int64_t work = sp_ceil_div(n, LQ_TILE) * hq;  // (head, key tile) pairs
-  int tiles = 8;
-  while (tiles < LQ_MAX_TILES && work / (2 * tiles) >= 1024) tiles *= 2;
-  // short sequences: one round of workgroups (two per CU) rather than few long-running ones
-  while (tiles > LQ_MIN_TILES && work / tiles < 512) tiles /= 2;
-  return tiles;
+  const int64_t tiles = sp_ceil_div(n, LQ_TILE), rows = (hq + LQ_WG_HEADS - 1) / LQ_WG_HEADS;
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int t = LQ_MIN_TILES; t <= LQ_MAX_TILES; ++t) {
+    const int64_t chunks = sp_ceil_div(tiles, t), per_cu = sp_ceil_div(chunks * rows, 256);
+    const int64_t cost = (per_cu == 1 ? 290 * t + 600 + 3 * (256 - chunks * rows) : 235 * t * per_cu + 950 + 130 * (sp_ceil_div(per_cu, 2) - 1)) +
+                         (chunks > LQ_FOLD_CHUNKS ? 450 : 0);
+    if (cost < best_cost) best_cost = cost, best = t;
+  }
+  return best;
 }
 // Output tiles per workgroup of the probabilities kernel.  A workgroup of T output tiles computes T + 1 (the leading
 // tile), and the launch runs in ceil(workgroups / 256) rounds, one workgroup per CU: take the T that minimises

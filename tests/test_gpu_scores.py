@@ -61,6 +61,19 @@ def test_lastq_scores_seeded_random_shapes(gpu_device):
         assert torch.allclose(sb, O.block_sum(st, 128), rtol=1e-5, atol=1e-9), tag
 
 
+@pytest.mark.parametrize("hq,hkv,n", [(28, 4, 10007), (32, 8, 4609), (14, 2, 20001), (7, 1, 33000)])
+def test_lastq_scores_in_chunks_of_any_number_of_tiles(gpu_device, hq, hkv, n):
+    """Lengths whose statistics are cut into chunks of 3 to 5 tiles, the last of them short, up to and beyond the number of chunks
+    that the probabilities kernel folds itself."""
+    from shareprefill_amd import ops
+
+    q, k = _inputs(hq, hkv, n, n)
+    vref, sref = O.lastq_scores(q, k, 128, logits_in_input_dtype=False)
+    vt, st, _, _ = [x.cpu() for x in ops.lastq_scores(q.to(gpu_device), k.to(gpu_device), 128, 0)]
+    assert torch.allclose(vt, vref, rtol=2e-4, atol=1e-8)
+    assert torch.allclose(st, sref, rtol=2e-4, atol=1e-8)
+
+
 @pytest.mark.parametrize("bs", [64, 32, 16])
 @pytest.mark.parametrize("hq,hkv,n", [(4, 2, 1024), (6, 2, 1000), (7, 1, 389), (2, 1, 128), (4, 4, 2100), (4, 2, 100),
                                       (2, 2, 64), (3, 1, 127)])  # the last three: prompts shorter than 128 tokens
