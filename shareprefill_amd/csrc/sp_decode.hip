@@ -5,9 +5,7 @@
 // way.  The cache of one kv head is split into chunks; one workgroup streams a chunk for all query heads of the
 // group (so the group's `g` heads share every K / V byte), keeps an online softmax, and leaves an unnormalised
 // partial (o, m, l); a second tiny kernel merges the partials in a fixed order.  A batch of sequences is one more grid
-// axis: per token of a small model's or short chat's step the launches and the host's way to them are what counts, and
-// one pair of launches per sequence, a workspace look-up each and a stacking copy were most of it (32 query / 8 kv heads:
-// 8 caches of 4001 tokens 135 -> 30 us = 4.4 TB/s, one of 1025 tokens 24.2 -> 14.3 us, one of 131072 100.5 -> 97.5 us).
+// axis.  Groups of up to 16 heads take the ring kernel further below; what follows is for the others.
 //
 // Both products run on the matrix core with the group's heads as a (mostly empty) 32-wide operand -- the MFMAs
 // are free here, the point is to keep the vector ALU out of the inner loop:
@@ -313,10 +311,319 @@ __global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kern
   }
 }
 
+#define DC_MAX_GRID_Z 65535
+
+// ---- up to 16 query heads per kv head --------------------------------------------------------------------------
+// The waves of a workgroup take 32 keys each in turn, every wave with a running max and a ring of operands in LDS of its own that is
+// filled by direct loads, no barrier between them, and meet in LDS at the end.
+//   S^T[16 keys x 16 heads] = K . Q^T
+//   O^T[16 channels x 16 heads] += V^T . P^T    V^T by the transposing LDS read; S^T leaves a lane with keys 4g .. 4g+3 of either
+//                                               16-key tile, which is what two such reads deliver.
+// P enters the product as two bf16 values, its rounding and what that leaves: outputs are 1.67e-3 from the attention in 64 bits, all of it
+// their own rounding, where one bf16 value and a running max per chunk of the cache left 2.16e-3.
+// Two ways to fill the chip (ds_plan):
+//   * a workgroup takes ALL keys of a kv head and a slice of V's channels, so that nothing has to be merged across workgroups and there
+//     is one launch.  Every slice forms the logits again, on CUs that would idle otherwise, from K's rows in the L2 that the slices share.
+//     For caches of some hundred keys, where launches and latency are all there is, and for batches.
+//   * all channels and a split of the keys, merged by the second kernel.
+// Bound: HBM at 5.85 TB/s of a batch (16 caches of 8000 tokens 100 -> 89 us), the waves' chain of steps otherwise.  K's rows straight from
+// memory into the operand registers (16 rows x 64 bytes an instruction) took 50 cycles an instruction, whole rows by way of LDS take
+// 16 (1025 keys 11.3 -> 6.9 us); a ring one step deeper changes nothing.  us, GPU time in replayed graphs: 200 keys 8.0 -> 3.5, 1025
+// 8.8 -> 6.9, 16 caches of 1025 22.7 -> 15.4, 131072 keys 97.9 -> 97.2; called one by one 200 keys 9.1 -> 8.6, 1025 13.0 -> 9.5.
+#define DS_GMAX 16
+#define DS_KEYS 32  // keys of a wave's step
+typedef float ds_floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t ds_u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void* ds_lds_ptr;
+
+// CT: channel tiles of 16 a slice has.  As many waves and steps of the ring as fit one workgroup's LDS.
+template <int D, int CT>
+struct DsShape {
+  static constexpr int K_BYTES = DS_KEYS * D * 2, V_BYTES = DS_KEYS * CT * 32, STEP_BYTES = K_BYTES + V_BYTES;
+  static constexpr int WAVES = D == 64 || CT == 1 ? 8 : CT == 2 ? 7 : CT == 4 ? 6 : 4;
+  static constexpr int NB = 152 * 1024 / (WAVES * STEP_BYTES) < 4 ? 152 * 1024 / (WAVES * STEP_BYTES) : 4;
+  static constexpr int LOADS = STEP_BYTES / 1024;  // of a step
+  static constexpr int LDS_BYTES = WAVES * NB * STEP_BYTES;
+  static_assert(NB >= 2 && LDS_BYTES >= WAVES * DS_GMAX * (16 * CT + 4) * 4, "");
+};
+
+__device__ static __forceinline__ float ds_quad_max(float v) {  // over the lanes l, l ^ 16, l ^ 32, l ^ 48 that share a head
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  u = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+__device__ static __forceinline__ float ds_quad_sum(float v) {
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (uint32_t)a[0]) + __builtin_bit_cast(float, (uint32_t)a[1]);
+  u = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (uint32_t)b[0]) + __builtin_bit_cast(float, (uint32_t)b[1]);
+}
+
+// LDS reads the compiler does not track: it would wait for every direct-to-LDS load in flight before each
+__device__ static __forceinline__ dc_u32x4 ds_read_k(uint32_t addr) {
+  dc_u32x4 r;
+  asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr));
+  return r;
+}
+template <int IMM>
+__device__ static __forceinline__ ds_u32x2 ds_read_v(uint32_t addr) {
+  ds_u32x2 r;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(IMM));
+  return r;
+}
+
+// Steps in LDS: K [32 keys][D], V [32 keys][16 CT channels] in 16-byte chunks, swizzled by the row: K's chunks for reads of one chunk
+// of 16 rows, V's pairs of chunks for the transposing reads of a pair of 8 rows (256 bytes, all banks, either way).
+template <int D>
+__device__ static __forceinline__ int ds_swz_k(int row) {
+  return D == 128 ? row & 15 : (row >> 1) & 7;
+}
+template <int CT>
+__device__ static __forceinline__ int ds_swz_v(int row) {
+  return CT == 1 ? 0 : (row / (8 / CT)) & (CT - 1);
+}
+
+// grid (hkv, splits, batch) of splits of the keys where a slice is all channels; otherwise (8, slices, (sequence, kv head) / 8), which
+// places the slices of a kv head on one XCD: they read the same keys (4 caches of 2048 keys, 4 kv heads: 13.0 us across two XCDs)
+// FULL: d == D; a smaller head's rows read as zero-padded: its loads behind the row's end read the row's first chunk instead, K's are
+// dropped from the operands and V's channels there are not written
+template <int D, int CT, bool FULL>
+__global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_ring_kernel(
+    const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const sp_bf16* __restrict__ v, int n_keys, int g, int hkv,
+    int d, int batch, uint32_t hkv_mul /* i / hkv = (i * hkv_mul) >> 16 */, DcStrides st, float scale_log2, int keys_per_split, float* __restrict__ o_part, float2* __restrict__ ml_part, sp_bf16* __restrict__ out) {
+  using Shape = DsShape<D, CT>;
+  constexpr int KS = D / 32, CW = 16 * CT, WAVES = Shape::WAVES, NB = Shape::NB;  // channel steps of S, channels of the slice
+  constexpr int KC = D / 8, VC = CW / 8;                                          // chunks of a row
+  constexpr int KI = Shape::K_BYTES / 1024, VI = Shape::V_BYTES / 1024;           // instructions of a step
+  constexpr int KR = SP_WAVE / KC, VR = SP_WAVE / VC;                             // rows of an instruction
+  extern __shared__ __attribute__((aligned(1024))) char ds_lds[];
+  __shared__ float m_s[WAVES][DS_GMAX], l_s[WAVES][DS_GMAX];
+  const int slice = CW == D ? 0 : blockIdx.y, split = CW == D ? blockIdx.y : 0, splits = CW == D ? gridDim.y : 1;
+  int kvh = blockIdx.x;
+  int64_t b = blockIdx.z;
+  if constexpr (CW < D) {
+    const uint32_t i = blockIdx.z * 8 + blockIdx.x;  // (sequence, kv head)
+    b = (i * hkv_mul) >> 16;
+    kvh = i - (uint32_t)b * hkv;
+    if (b >= batch || (!FULL && slice * CW >= d)) return;  // (uniform)
+  }
+  const int64_t bh = b * hkv + kvh;
+  const int begin = split * keys_per_split, n = n_keys - begin < keys_per_split ? n_keys - begin : keys_per_split;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lq = lane & 15, gr = lane >> 4;  // head (or key row, channel) in a 16-wide tile, lane group
+  dc_bf16x8 qb[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const bool real = lq < g && (FULL || 32 * ks + 8 * gr < d);
+    const dc_u32x4 raw = *reinterpret_cast<const dc_u32x4*>(q + b * st.q_b + (int64_t)(kvh * g + (lq < g ? lq : 0)) * st.q_h +
+                                                           (FULL || real ? 32 * ks + 8 * gr : 0));
+    qb[ks] = __builtin_bit_cast(dc_bf16x8, real ? raw : (dc_u32x4){0, 0, 0, 0});
+  }
+  const char* const kh = (const char*)(k + b * st.k_b + kvh * st.k_h + begin * st.k_n);
+  const char* const vh = (const char*)(v + b * st.v_b + kvh * st.v_h + begin * st.v_n);
+  const uint32_t k_row = (uint32_t)st.k_n * 2u, v_row = (uint32_t)st.v_n * 2u;  // bytes
+  const uint32_t ring = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)ds_lds + wave * NB * Shape::STEP_BYTES;
+
+  // A step's loads: instruction i fills 1 KiB (lane j its chunk j) with KR or VR rows.  The step is a buffer of its own; only the one
+  // that reaches past the cache clamps its rows onto the last key (masked below).
+  auto fetch = [&](int buf, int kb) {
+    const int rows = n - kb < DS_KEYS ? n - kb : DS_KEYS;
+    auto step = [&](const char* x, uint32_t row_bytes) {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)(x + (uint64_t)(uint32_t)kb * row_bytes), 0, (int)((uint32_t)(rows - 1) * row_bytes + 2u * d), 0x00027000);
+    };
+    const __amdgpu_buffer_rsrc_t ksrc = step(kh, k_row), vsrc = step(vh, v_row);
+    const uint32_t at = ring + buf * Shape::STEP_BYTES;
+    auto within = [&](int chunk) { return 16u * (uint32_t)(FULL || 8 * chunk < d ? chunk : 0); };
+    auto k_off = [&](int row) { return within((lane % KC) ^ ds_swz_k<D>(row)); };
+    auto v_off = [&](int row) { return within(slice * VC + ((lane % VC) ^ (2 * ds_swz_v<CT>(row)))); };
+    if (rows == DS_KEYS) {
+#pragma unroll
+      for (int i = 0; i < KI; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ksrc, (ds_lds_ptr)(uintptr_t)(at + i * 1024), 16,
+                                                 (int)((lane / KC) * k_row + k_off(i * KR + lane / KC)), (int)(i * KR * k_row), 0, 0);
+#pragma unroll
+      for (int i = 0; i < VI; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(vsrc, (ds_lds_ptr)(uintptr_t)(at + Shape::K_BYTES + i * 1024), 16,
+                                                 (int)((lane / VC) * v_row + v_off(i * VR + lane / VC)), (int)(i * VR * v_row), 0, 0);
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < KI; ++i) {
+        const int row = i * KR + lane / KC;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ksrc, (ds_lds_ptr)(uintptr_t)(at + i * 1024), 16,
+                                                 (int)((uint32_t)(row < rows ? row : rows - 1) * k_row + k_off(row)), 0, 0, 0);
+      }
+#pragma unroll 1
+      for (int i = 0; i < VI; ++i) {
+        const int row = i * VR + lane / VC;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(vsrc, (ds_lds_ptr)(uintptr_t)(at + Shape::K_BYTES + i * 1024), 16,
+                                                 (int)((uint32_t)(row < rows ? row : rows - 1) * v_row + v_off(row)), 0, 0, 0);
+      }
+    }
+  };
+  constexpr int STRIDE = WAVES * DS_KEYS;
+  const int kb0 = wave * DS_KEYS;
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+    if (kb0 + i * STRIDE < n) fetch(i, kb0 + i * STRIDE);
+
+  ds_floatx4 o[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) o[ct] = (ds_floatx4){0, 0, 0, 0};
+  float m = -INFINITY, l = 0.f;  // of head lq; l: this lane group's keys
+  const uint32_t k_at = ring + lq * (D * 2);
+  const int v_key = 4 * gr + (lq >> 2);  // row of the transposing read; 16 rows further the swizzle is the same
+  const uint32_t v_at = ring + Shape::K_BYTES + v_key * (CT * 32) + 8 * (lq & 3);
+  int buf = 0;
+  for (int kb = kb0; kb < n; kb += STRIDE) {
+    // the step's loads have landed, those of the NB - 2 behind it stay in flight (loads return in order)
+    if (kb + (NB - 2) * STRIDE < n)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * Shape::LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // (the place that is filled here was read in the step before: those reads' results have been used)
+    if (kb + (NB - 1) * STRIDE < n) fetch(buf == 0 ? NB - 1 : buf - 1, kb + (NB - 1) * STRIDE);
+    const uint32_t off = buf * Shape::STEP_BYTES;
+    dc_u32x4 kr[2][KS];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        kr[i][ks] = ds_read_k(k_at + off + i * 16 * (D * 2) + (((4 * ks + gr) ^ ds_swz_k<D>(lq)) << 4));
+    if constexpr (KS == 4)
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(kr[0][0]), "+v"(kr[0][1]), "+v"(kr[0][2]), "+v"(kr[0][3]), "+v"(kr[1][0]), "+v"(kr[1][1]), "+v"(kr[1][2]), "+v"(kr[1][3]));
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(kr[0][0]), "+v"(kr[0][1]), "+v"(kr[1][0]), "+v"(kr[1][1]));
+    if constexpr (!FULL) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        if (32 * ks + 8 * gr >= d) kr[0][ks] = kr[1][ks] = (dc_u32x4){0, 0, 0, 0};
+    }
+    ds_u32x2 vr[CT][2];  // on their way under the logits
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const uint32_t at = v_at + off + ((ct ^ ds_swz_v<CT>(v_key)) << 5);
+      vr[ct][0] = ds_read_v<0>(at);
+      vr[ct][1] = ds_read_v<16 * CT * 32>(at);
+    }
+    ds_floatx4 s[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      s[i] = (ds_floatx4){0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, kr[i][ks]), qb[ks], s[i], 0, 0, 0);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[i][j] = kb + 16 * i + 4 * gr + j < n ? s[i][j] * scale_log2 : -INFINITY;
+        mx = fmaxf(mx, s[i][j]);
+      }
+    const float m_new = fmaxf(m, ds_quad_max(mx));
+    const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 in the first step
+    float add = 0.f;
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(s[i][j] - m_new), p1 = __builtin_amdgcn_exp2f(s[i][j + 1] - m_new);
+        const uint32_t w = dc_pack2(p0, p1);
+        hi[2 * i + j / 2] = w;
+        lo[2 * i + j / 2] = dc_pack2(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xffff0000u));
+        add += p0 + p1;
+      }
+    l = l * alpha + add;
+    m = m_new;
+    const dc_bf16x8 ph = __builtin_bit_cast(dc_bf16x8, (dc_u32x4){hi[0], hi[1], hi[2], hi[3]});
+    const dc_bf16x8 pl = __builtin_bit_cast(dc_bf16x8, (dc_u32x4){lo[0], lo[1], lo[2], lo[3]});
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(vr[ct][0]), "+v"(vr[ct][1]));
+      const dc_u32x4 raw = __builtin_shufflevector(vr[ct][0], vr[ct][1], 0, 1, 2, 3);
+      o[ct] *= alpha;
+      o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, raw), ph, o[ct], 0, 0, 0);
+      o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, raw), pl, o[ct], 0, 0, 0);
+    }
+    buf = buf + 1 == NB ? 0 : buf + 1;
+  }
+  l = ds_quad_sum(l);
+  __syncthreads();  // the rings are free
+  auto o_s = reinterpret_cast<float(*)[DS_GMAX][CW + 4]>(ds_lds);
+  if (lq < g) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<ds_floatx4*>(&o_s[wave][lq][16 * ct + 4 * gr]) = o[ct];
+    if (gr == 0) {
+      m_s[wave][lq] = m;
+      l_s[wave][lq] = l;
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < g * (CW / 4); i += WAVES * SP_WAVE) {
+    const int h = i / (CW / 4), c = i % (CW / 4) * 4;
+    if (!FULL && slice * CW + c >= d) continue;
+    float top = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, m_s[w][h]);
+    ds_floatx4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(m_s[w][h] - top);  // (a wave without keys: 0)
+      sum += l_s[w][h] * f;
+      acc += *reinterpret_cast<const ds_floatx4*>(&o_s[w][h][c]) * f;
+    }
+    if (splits > 1) {  // (uniform) the merging kernel goes on
+      const int64_t at = (bh * splits + split) * g + h;
+      *reinterpret_cast<dc_floatx4*>(o_part + at * DC_D + c) = acc;
+      if (c == 0) ml_part[at] = make_float2(top, sum);
+      continue;
+    }
+    const float inv = 1.0f / sum;
+    *reinterpret_cast<uint2*>(out + (bh * g + h) * d + slice * CW + c) =
+        make_uint2(dc_pack2(acc[0] * inv, acc[1] * inv), dc_pack2(acc[2] * inv, acc[3] * inv));
+  }
+}
+
+template <int D, int CT, bool FULL>
+static int ds_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv, int32_t d, const DcStrides& st,
+                     float scale_log2, int splits, int keys_per_split, float* o_part, float2* ml_part, void* out, hipStream_t s) {
+  using Shape = DsShape<D, CT>;
+  static bool attr_set[64] = {false};  // per device, once (idempotent)
+  int dev = 0;
+  SP_HIP(hipGetDevice(&dev));
+  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "decode attention: device index %d", dev);
+  if (!attr_set[dev]) {
+    SP_HIP(hipFuncSetAttribute((const void*)sp_decode_ring_kernel<D, CT, FULL>, hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS_BYTES));
+    attr_set[dev] = true;
+  }
+  const int slices = D / 16 / CT;
+  auto launch = [&](dim3 grid, int64_t b0, int32_t count) {
+    hipLaunchKernelGGL((sp_decode_ring_kernel<D, CT, FULL>), grid, dim3(Shape::WAVES * SP_WAVE), Shape::LDS_BYTES, s, (const sp_bf16*)q + b0 * st.q_b,
+                       (const sp_bf16*)k + b0 * st.k_b, (const sp_bf16*)v + b0 * st.v_b, (int)n, hq / hkv, (int)hkv, (int)d, (int)count,
+                       (uint32_t)sp_ceil_div(65536, hkv), st, scale_log2, keys_per_split, o_part, ml_part, (sp_bf16*)out + b0 * hq * d);
+  };
+  if (slices > 1)  // (at most 256 workgroups)
+    launch(dim3(8, slices, (unsigned)sp_ceil_div((int64_t)batch * hkv, 8)), 0, batch);
+  else
+    for (int64_t b0 = 0; b0 < batch; b0 += DC_MAX_GRID_Z) {  // (a batch of more sequences than a grid's z axis is not split)
+      const int32_t count = (int32_t)(batch - b0 < DC_MAX_GRID_Z ? batch - b0 : DC_MAX_GRID_Z);
+      launch(dim3(hkv, splits, (unsigned)count), b0, count);
+    }
+  SP_LAUNCH_CHECK();
+  return SP_OK;
+}
+
 // ---- host -------------------------------------------------------------------------------------------------
 // Chunks per (sequence, kv head): about two workgroups per CU over the whole batch, which is what the kernel's LDS
 // lets a CU hold, and no chunk below one tile of keys.
-#define DC_MAX_GRID_Z 65535
 static_assert(DC_MAX_GRID_Z >= 512, "");  // (the number of chunks is 1 before a batch needs a second launch)
 static int dc_cut(int32_t batch, int64_t n, int32_t hkv) {
   const int64_t tiles = sp_ceil_div(n, DC_TILE);
@@ -327,16 +634,48 @@ static int dc_cut(int32_t batch, int64_t n, int32_t hkv) {
   return (int)want;
 }
 
-// Workgroups per (sequence, kv head).  A cache of up to two tiles is walked by one, chunk by chunk, which makes the result itself: a
-// launch less, and no scratch.  One launch against two, us a step of 32 layers with caches of their own, 32 query / 8 kv heads, in a
-// replayed graph (the GPU's time) and called one by one (the host's, of which the second launch is 3.3):
-//   200 keys            8.0 / 7.9 and 8.8 / 12.1;  16 sequences 8.9 / 9.9 and 8.8 / 12.2;  64 channels 6.6 / 7.0 and 9.1 / 13.4
-//   384 keys, not taken 10.8 / 8.1 and 10.8 / 12.3;  16 sequences 11.9 / 12.0 and 11.9 / 13.3;  64 channels 8.7 / 7.1 and 8.9 / 13.3
-// The third tile in series (2.7 us) costs the GPU more than the second launch does.  (One workgroup of sixteen waves with four tiles at a
-// time, called one by one: 500 keys 11.1, 1025 18.6.)
+// Splits per (sequence, kv head) at most, and what the workspace is sized for.  A cache of up to two tiles is one: no partials.
 #define DC_ONE_LAUNCH_TILES 2
 static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
   return n <= DC_ONE_LAUNCH_TILES * DC_TILE ? 1 : dc_cut(batch, n, hkv);
+}
+
+// How a call of the ring kernel is cut: slices of the channels in one launch, or splits of the keys and the merging launch -- the
+// cheaper by the times they were measured to take with caches that come from memory (replayed graphs over 600 MB of caches; 28 / 4 and
+// 32 / 8 heads of 128, 14 / 2 and 32 / 8 of 64 channels, 600 to 4001 keys, 1 to 16 sequences; within some 10 %).  ns:
+//   3600 a launch with its first and last step, 3400 the merging one;
+//   a key takes a workgroup 5.2 to 8.6 by the slice's width (64 channels 3.8 to 4.1) and a third of what it takes from memory beside the
+//   others, or, where that is more, what it takes from memory, at 5.85 TB/s.
+// A launch's host time, 3300, counts half: whether the host or the GPU bounds a step is the caller's.  us, one launch / two: 1025 keys
+// 9.1 / 8.5 (called one by one 9.5 / 12.9), 2048 14.3 / 8.7; 4 sequences of 1025 9.8 / 10.3, of 2048 16.0 / 12.4; 8 of 700 8.7 / 11.1, of
+// 4001 32.9 / 29.4; 16 of 2000 26.0 / 29.5.
+struct DsPlan {
+  int ct, splits;
+};
+static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
+  const int64_t bh = (int64_t)batch * hkv;
+  const int full = d / 16;  // channel tiles
+  auto cost = [&](int ct, int64_t heads /* kv heads' keys in flight */, int64_t wgs, int64_t keys) {
+    const int64_t alone = d == 64 ? (ct == 1 ? 3800 : 4100) : ct == 1 ? 5200 : ct == 2 ? 5600 : ct == 4 ? 6200 : 8600;  // (ps a key)
+    const int64_t memory = heads * 4 * d * 1000 / 5850;
+    const int64_t shared = alone + (memory < alone ? memory : alone) / 3;
+    return 3600 + sp_ceil_div(wgs, 256) * keys * (memory > shared ? memory : shared) / 1000;
+  };
+  DsPlan best = {full, 1};
+  int64_t least = INT64_MAX;
+  for (int ct = 1; ct <= full; ct *= 2) {
+    const int64_t wgs = bh * (full / ct);
+    if (ct < full && wgs > 256) continue;
+    const int64_t c = cost(ct, bh < 256 ? bh : 256, wgs, n);
+    if (c < least) least = c, best.ct = ct;
+  }
+  const int room = dc_splits(batch, n, hkv);  // (what the workspace is sized for; 1: there is none)
+  const int64_t splits = 256 / bh < room ? 256 / bh : room;
+  if (splits > 1) {
+    const int64_t keys = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE, wgs = bh * sp_ceil_div(n, keys);
+    if (cost(full, wgs, wgs, keys) + 3400 + 1650 < least) best = {full, (int)splits};
+  }
+  return best;
 }
 
 static size_t dc_partial_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv) {
@@ -379,6 +718,31 @@ static int dc_check(const char* who, const void* q, const void* k, const void* v
 static int dc_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv,
                      int32_t d, const DcStrides& st, float softmax_scale, void* out, void* partials, hipStream_t s) {
   const int g = hq / hkv;
+  // (8-byte stores; offsets inside 32 keys and the token count have 32 bits)
+  if (g <= DS_GMAX && n < (1 << 30) && (uintptr_t)out % 8 == 0 && st.k_n >= 0 && st.v_n >= 0 && st.k_n < (1 << 25) && st.v_n < (1 << 25)) {
+    const float scale_log2 = softmax_scale * 1.4426950408889634f;
+    const DsPlan plan = ds_plan(batch, n, hkv, d > 64 ? 128 : 64);
+    const int keys_per_split = (int)(sp_ceil_div(sp_ceil_div(n, plan.splits), DC_TILE) * DC_TILE);
+    const int splits = (int)sp_ceil_div(n, keys_per_split);  // (none without keys)
+    float* o_part = (float*)partials;
+    float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
+    auto go = [&](auto launch) { return launch(q, k, v, batch, n, hq, hkv, d, st, scale_log2, splits, keys_per_split, o_part, ml_part, out, s); };
+    auto by_slice = [&](auto whole) {
+      constexpr bool FULL = decltype(whole)::value;
+      if (d > 64)
+        return plan.ct == 8   ? go(ds_launch<128, 8, FULL>)
+               : plan.ct == 4 ? go(ds_launch<128, 4, FULL>)
+               : plan.ct == 2 ? go(ds_launch<128, 2, FULL>)
+                              : go(ds_launch<128, 1, FULL>);
+      return plan.ct == 4 ? go(ds_launch<64, 4, FULL>) : plan.ct == 2 ? go(ds_launch<64, 2, FULL>) : go(ds_launch<64, 1, FULL>);
+    };
+    const int rc = d == 64 || d == 128 ? by_slice(std::true_type{}) : by_slice(std::false_type{});
+    if (rc || splits == 1) return rc;
+    hipLaunchKernelGGL(sp_decode_combine_kernel, dim3((unsigned)((int64_t)batch * hq)), dim3(32 * DC_COMBINE_GROUPS), 0, s, o_part, ml_part, g, splits,
+                       (int)d, (sp_bf16*)out);
+    SP_LAUNCH_CHECK();
+    return SP_OK;
+  }
   const int splits = dc_splits(batch, n, hkv);
   const int64_t keys_per_split = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE;
   const int tiles_per_chunk = (int)sp_ceil_div(sp_ceil_div(n, dc_cut(1, n, hkv)), DC_TILE);
@@ -395,10 +759,12 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
   };
   auto by_width = [&](auto g8) {
     constexpr int G8 = decltype(g8)::value;
+    // (whole rows of up to 16 heads come here only where the ring kernel cannot take them)
+    constexpr bool WHOLE = G8 == 4;
     if (d > 64)
-      d == 128 ? launch(sp_decode_partial_kernel<128, G8, true>) : launch(sp_decode_partial_kernel<128, G8, false>);
+      d == 128 && WHOLE ? launch(sp_decode_partial_kernel<128, G8, WHOLE>) : launch(sp_decode_partial_kernel<128, G8, false>);
     else
-      d == 64 ? launch(sp_decode_partial_kernel<64, G8, true>) : launch(sp_decode_partial_kernel<64, G8, false>);
+      d == 64 && WHOLE ? launch(sp_decode_partial_kernel<64, G8, WHOLE>) : launch(sp_decode_partial_kernel<64, G8, false>);
   };
   if (g <= 8)
     by_width(std::integral_constant<int, 1>{});

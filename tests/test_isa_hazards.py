@@ -160,3 +160,12 @@ def test_nothing_touches_a_transposing_read_in_flight():
         count, found = touched_in_flight(body)
         assert count >= 16
         assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
+
+
+def test_nothing_touches_a_transposing_read_in_flight_in_the_decode_ring():
+    kernels = _kernels("sp_decode.hip", "sp_decode_ring_kernel")
+    assert len(kernels) == 14, "whole and padded rows x 64 channels in 1, 2, 4 tiles, 128 in 1, 2, 4, 8"
+    for name, body in kernels.items():
+        count, found = touched_in_flight(body)
+        assert count >= 2
+        assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
