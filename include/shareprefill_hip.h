@@ -264,15 +264,17 @@ int sp_block_sparse_attn_pivot_fwd_bf16(const void* q, const void* k, const void
                                   sp_stream_t stream);
 
 /* The same attention for short prompts, bs = 128, d = 64 or 128 (no padding): one kernel that reads v as it is, needs no
- * repack and no scheduler area, and writes the pivot heads' maps itself.  Correct for any n up to 65536;
+ * repack and no scheduler area, and writes the pivot heads' maps itself.  Correct for any n up to 131072;
  * sp_short_attn_max_tokens(d) is the length up to which it is the faster of the two on a selection's masks,
- * sp_short_attn_max_dense_tokens(d) where every block is kept.
+ * sp_short_attn_max_dense_tokens(d) where every block is kept, sp_short_attn_max_steady_tokens(d, pattern_threshold) on the masks of a
+ * selection at that coverage in a layer whose heads become no pivots.
  * avg_attn without decision: no head is a pivot, the maps are cleared (with decision only DENSE heads' maps are written).
  * workspace, with decision and avg_attn: sp_attn_pivot_scratch_bytes(n, 128) bytes (block sums) for every head that can be
  * DENSE, or sp_short_attn_workspace_bytes(n, hq) bytes for hq of them.  DENSE heads beyond those it has room for get NaN
  * for a map and update no pivot. */
 int64_t sp_short_attn_max_tokens(int32_t d);
 int64_t sp_short_attn_max_dense_tokens(int32_t d);
+int64_t sp_short_attn_max_steady_tokens(int32_t d, float pattern_threshold);
 size_t sp_short_attn_workspace_bytes(int64_t n, int32_t hq);
 int sp_short_attn_fwd_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv, int32_t d,
                            int64_t q_stride_n, int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h,

@@ -83,6 +83,7 @@ SIGNATURES = {
                                                    _P, _P, _P, _P, _P, _SZ, _U32, _ST, _P, _F, _P]),
     "sp_short_attn_max_tokens": (_I64, [_I32]),
     "sp_short_attn_max_dense_tokens": (_I64, [_I32]),
+    "sp_short_attn_max_steady_tokens": (_I64, [_I32, _F]),
     "sp_short_attn_workspace_bytes": (_SZ, [_I64, _I32]),
     "sp_short_attn_fwd_bf16": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P, _P,
                                       _P, _P, _P, _SZ, _P]),

@@ -99,6 +99,7 @@ class AttentionSharing:
         self.plans: List[LayerPlan] = []
         self._scratch: Dict[torch.device, Tuple[torch.Tensor, torch.Tensor]] = {}
         self._max_pivots: Dict[Tuple[int, int], int] = {}
+        self._opens_cluster: Dict[Tuple[int, int], bool] = {}
         self.reset_state()
 
     # ---- table ------------------------------------------------------------------------------------
@@ -223,6 +224,17 @@ class AttentionSharing:
                      for c in (self._pair_to_cluster.get((layer_idx, h)),) if c in self._slot})
             self._max_pivots[key] = n
         return n
+
+    def opens_cluster(self, layer_idx: int, hq: int) -> bool:
+        """Whether some shared cluster has its first heads in this layer: where pivots are elected as a rule.  (A cluster whose
+        heads of that layer are all query-aware elects its pivot in a later one.)"""
+        key = (layer_idx, hq)
+        opens = self._opens_cluster.get(key)
+        if opens is None:
+            here = {c for h in range(hq) for c in (self._pair_to_cluster.get((layer_idx, h)),) if c in self._slot}
+            before = {c for (layer, _), c in self._pair_to_cluster.items() if layer < layer_idx}
+            opens = self._opens_cluster[key] = not here <= before
+        return opens
 
     def _qa_scratch(self, hq: int, nb: int, device) -> torch.Tensor:
         """fp32 [Hq, nb, nb] scratch of the query-aware selection, owned by this object (one model, one stream of

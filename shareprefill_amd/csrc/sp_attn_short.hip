@@ -63,7 +63,7 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 #define AS_TILE 64      // keys per step
 #define AS_THREADS 256  // 4 waves x 32 queries
 #define AS_WAVES 4
-#define AS_MAX_NB 512     // blocks of a row: its mask is at most eight words, its maps fit the tiles' LDS
+#define AS_MAX_NB 1024    // blocks of a row: a lane holds a word of its mask, its maps fit the tiles' LDS
 #define AS_LDS_BYTES(D) (4 * AS_TILE * (D) * 2)
 #define AS_NO_MAX (-1.0e30f)         // "no key seen yet": finite, so exp2(S * scale - m) is +inf or 0, never NaN
 #define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
@@ -524,12 +524,27 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
 //   8 / 2 6656 148 / 156.
 // So up to 6656 tokens this kernel is never behind by more than 1 %, whatever the coverage; beyond, it is ahead at low coverage and
 // behind at 0.99.  (The line of dense masks stands a little low: 5632 is this kernel's too.)
+// (These lines hold for any layer; where none of its heads can be elected see sp_short_attn_max_steady_tokens.)
 // 64 channels, where the persistent kernel computes on zero-padded tiles (padding counted), 32 / 8 heads: 0.65 8192 148 / 254, 32768
 // 448 / 810, 49152 715 / 1244; 0.95 143 / 253, 583 / 907, 1268 / 1692; 0.99 147 / 261, 1177 / 1422, 2970 / 3100; every block kept 311 / 409,
 // 4920 / 5135, 10775 / 11010; 14 / 2 heads 0.95 32768 333 / 462, every block 2062 / 2198.  The line is where both were once even without
 // the padding; what lies beyond it is not measured but for these lengths, and each pivot's block sums take 16.8 MB there.
 extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
+}
+// The same where no pivot is elected, by the coverage the masks are made at (share of the softmax mass: what the density grows with).
+// A pivot's rows keep every block, which the persistent kernel's rows of two share out better: whole passes of an electing layer and a
+// steady one, us here / there, 32 / 8 heads of 128 channels 8192 tokens at 0.95 709 / 665, 9000 at 0.9 775 / 681; 64 channels 40000 at 0.95
+// 4462 / 4666, 100000 at 0.65 19754 / 17016.  Steady layers:
+//   128 channels, 32 / 8 and 28 / 4 heads: 0.65 8192 tokens 185 / 201, 173 / 197, 10007 239 / 257, 219 / 234, 12288 271 / 289, 248 / 263,
+//   16384 362 / 379, 324 / 334; 0.9 8192 201 / 222, 189 / 209, 10007 260 / 270, 238 / 246, 11000 313 / 316, 279 / 283, 12288 332 / 335,
+//   307 / 301; 0.95 8192 237 / 249, 222 / 232, 10007 307 / 310, 286 / 282 (not taken: masks of query-aware heads at 0.95 are
+//   denser, 1162 / 1140 of a decoder layer's half of 8192 tokens);
+//   64 channels, 32 / 8 and 14 / 2 heads: 0.65 36000 570 / 983, 299 / 489, 131072 2078 / 3397, 992 / 1543; 0.95 36000 782 / 1153, 437 / 598,
+//   90001 5319 / 5631, 2401 / 2755, 131072 12202 / 12458, 5986 / 6266; 0.99 65536 5742 / 5806, 2518 / 2798, 90001 11976 / 11675, 5534 / 5696.
+extern "C" int64_t sp_short_attn_max_steady_tokens(int32_t d, float pattern_threshold) {
+  if (d == 64) return pattern_threshold <= 0.951f ? AS_MAX_NB * AS_BS : pattern_threshold <= 0.991f ? 65536 : sp_short_attn_max_tokens(d);
+  return pattern_threshold <= 0.651f ? 16384 : pattern_threshold <= 0.901f ? 10240 : sp_short_attn_max_tokens(d);
 }
 extern "C" int64_t sp_short_attn_max_dense_tokens(int32_t d) {
   return d == 64 ? 32768 : 5120;

@@ -187,10 +187,19 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
     assert query_states.dtype == torch.bfloat16, "SharePrefill attention expects bfloat16 q/k/v"
     assert key_states.shape[2] == q_len, "prefill expects q_len == k_len (no cached prefix)"
     block_size = config.block_size
+    sharing = module.attention_sharing
+    nb = -(-q_len // block_size)
+    minb, maxb = budget_blocks(config.min_budget, config.max_budget, block_size)
+    dense = q_len < block_size or (nb <= minb and nb <= maxb and getattr(config, "dense_short_prompts", True))
+    # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
+    plan_here = not dense and getattr(sharing.plan_layer, "__func__", None) is _PLAN_LAYER
     # a short prompt's attention is one launch that reads v as it is (ops.short_attention) and takes 64 channels as they
     # are; longer ones repack v and run the persistent kernel on 128
     head_dim = 64 if model_dim in PADDED_HEAD_DIMS else model_dim
     short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
+    if not short and plan_here and block_size == 128:
+        short = _short_in_steady_layers(sharing, module.layer_idx, num_heads, q_len, head_dim, config.pattern_threshold,
+                                        key_states, value_states)
     if model_dim == KERNEL_HEAD_DIM and value_states.stride(2) * 128 >= 2 ** 31:
         short = False  # the short-prompt kernel's offsets inside a block of v have 32 bits, the repack's 64
     if model_dim in PADDED_HEAD_DIMS:
@@ -203,10 +212,7 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
                                                       (query_states, key_states, value_states))
 
     q, k, v = query_states[0], key_states[0], value_states[0]
-    nb = -(-q_len // block_size)
-    sharing = module.attention_sharing
-    minb, maxb = budget_blocks(config.min_budget, config.max_budget, block_size)
-    if q_len < block_size or (nb <= minb and nb <= maxb and getattr(config, "dense_short_prompts", True)):
+    if dense:
         # (a) Shorter than one block: a single diagonal block, nothing to select (the reference cannot run here).
         # (b) The prompt has no more blocks than the minimum budget, nor than the maximum.  Every head's budgets are
         # then raised to min_budget and cut to min(max_budget, nb) = nb (attention_sharing.py:173-176; with a maximum
@@ -239,9 +245,7 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
         max_pivots = min(possible, (16 << 30) // slab, _lib.SP_ATTN_MAX_PIVOTS)
         all_fit = max_pivots == possible
         ws = ops.attention_workspace(q_len, num_heads, key_states.shape[1], head_dim, block_size, q.device, max_pivots)
-    # A subclass or a wrapper that has its own plan_layer or update_pivotal_attns is called as the steps are by themselves.
     plan_args = {"scale_dim": model_dim}
-    plan_here = getattr(sharing.plan_layer, "__func__", None) is _PLAN_LAYER
     if plan_here:
         plan_args["avg_attn"] = avg_attn[0]  # (cleared on the way)
         if not short:
@@ -268,6 +272,18 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
     if not update_here:
         sharing.update_pivotal_attns(module.layer_idx, avg_attn, plan.decision, config.pattern_threshold)
     return _first_channels(out.unsqueeze(0), model_dim), avg_attn
+
+
+def _short_in_steady_layers(sharing, layer_idx: int, num_heads: int, q_len: int, head_dim: int, pattern_threshold: float,
+                            key_states: torch.Tensor, value_states: torch.Tensor) -> bool:
+    """Whether a layer past the length where the short-prompt kernel is the faster one in any layer still takes it: not where a
+    cluster's pivot is elected as a rule, nor where its block sums for the possible pivots would pass the 16 GiB that the
+    persistent kernel's are held to, or a block of k or v the kernel's 32-bit offsets."""
+    lib = _lib.load()
+    return (q_len <= lib.sp_short_attn_max_steady_tokens(head_dim, pattern_threshold)
+            and not sharing.opens_cluster(layer_idx, num_heads)
+            and sharing.max_pivots(layer_idx, num_heads) * lib.sp_attn_pivot_scratch_bytes(q_len, 128) <= 16 << 30
+            and max(key_states.stride(2), value_states.stride(2)) * 128 < 2 ** 31)
 
 
 def _first_channels(out: torch.Tensor, model_dim: int) -> torch.Tensor:

@@ -218,3 +218,55 @@ def test_dense_prompts_on_both_sides_of_the_line(gpu_device, tmp_path, d, past):
     want = ops.block_sparse_attention(*(torch.nn.functional.pad(t[0], (0, 128 - d)) for t in qkv), mask, 128, d ** -0.5,
                                       half_channels=d == 64)[..., :d]
     assert torch.equal(out[0], want) and not maps.any() and maps.shape == (1, 2, nb, nb)
+
+
+@pytest.mark.parametrize("hq,hkv,n", [(3, 1, 65537),  # more than eight mask words a row
+                                      (2, 1, 131072)])
+def test_long_prompts_of_64_channels_have_the_long_prompt_kernels_bits(gpu_device, hq, hkv, n):
+    from shareprefill_amd import ops
+
+    d, nb = 64, -(-n // 128)
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    q, k, v = (torch.randn(h, n, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h in (hq, hkv, hkv))
+    mask = np.tril(np.random.default_rng(n).random((hq, nb, nb)) < 4.0 / nb)
+    mask[:, np.arange(nb), np.arange(nb)] = True
+    bits = ops.bool_to_mask(torch.from_numpy(mask)).to(gpu_device)
+    wide = (torch.nn.functional.pad(t, (0, 128 - d)) for t in (q, k, v))
+    long = ops.block_sparse_attention(*wide, bits, 128, d ** -0.5, half_channels=True)[..., :d]
+    assert torch.equal(ops.short_attention(q, k, v, bits, d ** -0.5), long)
+
+
+@pytest.mark.parametrize("hq,hkv,n,d,pattern", [(8, 2, 6657, 128, 0.9), (8, 2, 10241, 128, 0.65), (4, 2, 32769, 64, 0.95),
+                                                (4, 2, 65537, 64, 0.99)])
+def test_steady_layers_take_the_short_prompt_kernel_further(gpu_device, tmp_path, monkeypatch, hq, hkv, n, d, pattern):
+    """Three layers, the first of which opens every cluster: the others are the short-prompt kernel's up to a line that depends on the
+    coverage; outputs, maps and state are those of the persistent kernel in every layer."""
+    import types
+
+    from shareprefill_amd import AttentionSharing, _lib, ops, shareprefill_attention_forward, shareprefill_attn, synthetic
+
+    lib = _lib.load()
+    further = lib.sp_short_attn_max_tokens(d) < n <= lib.sp_short_attn_max_steady_tokens(d, pattern)
+    assert further == (n != 65537)
+    path = synthetic.write_cluster_table(synthetic.random_cluster_table(hq, 2, 3, n), str(tmp_path / "table.json"))
+    cfg = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=pattern, similarity_threshold=0.5,
+                                fallback_threshold=1e9, queryaware_threshold=0.1)
+    qkv = [synthetic.planted_qkv(hq, hkv, n, d, 7 + layer, device=gpu_device, q_head_gain=1.0) for layer in range(3)]
+    calls = []
+    short = ops.short_attention
+    monkeypatch.setattr(ops, "short_attention", lambda *a, **kw: calls.append(len(results)) or short(*a, **kw))
+    passes = []
+    for steady in (True, False):
+        if not steady:
+            monkeypatch.setattr(shareprefill_attn, "_short_in_steady_layers", lambda *a: False)
+        sharing, results = AttentionSharing(path), []
+        assert [sharing.opens_cluster(layer, hq) for layer in range(3)] == [True, False, False]
+        for layer in range(3):
+            mod = types.SimpleNamespace(config=cfg, attention_sharing=sharing, layer_idx=layer, scaling=d ** -0.5)
+            results.append(shareprefill_attention_forward(mod, *qkv[layer], None, scaling=d ** -0.5))
+        passes.append((results, sharing._state))
+    assert calls == ([1, 2] if further else [])
+    (got, state), (want, state_want) = passes
+    for (out, maps), (out_want, maps_want) in zip(got, want):
+        assert torch.equal(out, out_want) and torch.equal(maps, maps_want)
+    assert torch.equal(state.info, state_want.info) and torch.equal(state.pattern, state_want.pattern)
