@@ -11,9 +11,9 @@
 //   probs   : recomputes the logits tile by tile; the column sums (vertical) and, through a permutation of keys and
 //             query rows, the anti-diagonal sums (slash) both start in registers, and only a 32 KiB digest of the
 //             128x128 probability tile goes through LDS.  A slash bin receives its upper part from the previous key
-//             tile; that part is carried through LDS, and each workgroup recomputes one leading tile so that no
-//             cross-workgroup accumulation (and no float atomic) is needed.
-// Every sum runs in a fixed order, so results are reproducible run to run.
+//             tile; that part is carried through LDS, and where a workgroup's tiles end it is added to the next one's first
+//             tile in memory, which the first kernel has cleared: two addends and zero, the same sum in either order.
+// Results are reproducible run to run: every other sum runs in a fixed order.
 #include "sp_block_probs.h"
 #include "sp_pool.h"
 
@@ -122,11 +122,17 @@ __device__ static __forceinline__ void lq_issue_k_direct(const sp_bf16* __restri
   }
 }
 
+// The tiles of the slash vector that two workgroups of the probabilities kernel add to: every tiles-th one but the first
+struct LqSeams {
+  float *slash_tok, *slash_blk;
+  int64_t nb, tiles;
+};
+
 template <int D>
 __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
     const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, int64_t n, int hkv, int group, int64_t sq_n,
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, int n_chunks, int tiles_per_wg,
-    float2* __restrict__ partial /* [hq][n_chunks][128] */, PoolArgs pool) {
+    float2* __restrict__ partial /* [hq][n_chunks][128] */, LqSeams seams, PoolArgs pool) {
   __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES(D)];
   const int pairs = lq_pairs(group);
   // The rows of the grid behind the scores' own pool K beside them (dispatched last, two units per workgroup): the vector
@@ -150,6 +156,12 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
   const int lq = lane & 31, hi = lane >> 5;
   const sp_bf16* qh = q + (int64_t)h * sq_h;
   const sp_bf16* kh = k + (int64_t)kvh * sk_h;
+  if (has_head)  // the seams are cleared, each by the head's four waves of one chunk
+    for (int64_t tile = (1 + chunk) * seams.tiles; tile * LQ_TILE < n; tile += (int64_t)n_chunks * seams.tiles) {
+      const int i = wave * SP_WAVE + lane;
+      if (i < LQ_TILE && tile * LQ_TILE + i < n) seams.slash_tok[(int64_t)h * n + tile * LQ_TILE + i] = 0.f;
+      if (i == 0 && seams.slash_blk != nullptr) seams.slash_blk[(int64_t)h * seams.nb + tile] = 0.f;
+    }
   bf16x8 qa[D / 16];  // the lane's query (row 32 wave + lq of the last block), channels 16 ks + 8 hi .. + 7
   lq_load_q<false, D / 16>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
   float m = LQ_NO_MAX, l = 0.f;
@@ -305,8 +317,11 @@ __device__ static __forceinline__ float lq_wave_sum(float v) {
 // as two aligned 16-byte LDS stores (offsets 0..3 to Dm[G], 4..6 to Dh[G], which is Dm shifted by one chunk), 32 KiB
 // for the whole 128 x 128 tile, and a thread collects four bins with 16-byte reads:
 // an eighth of the LDS traffic of a full probability tile, and no select between this tile's and the next tile's bins.
-// Bins 128..254 of a tile belong to the next tile's first 127 tokens: they are carried through LDS, and each
-// workgroup recomputes one leading tile so that no cross-workgroup accumulation (and no float atomic) is needed.
+// Bins 128..254 of a tile belong to the next tile's first 127 tokens: they are carried through LDS, and those of a workgroup's last
+// tile are added to the next one's first tile in memory, as that workgroup adds its own part: two addends onto a cleared place, the same
+// sum in either order.  With a leading tile of its own
+// for them instead -- a third of a workgroup's tiles at 3001 tokens -- layers take, us: 1500 tokens 74.7 (now 70.6), 3001 106.5 (103.0), 8192
+// 247.9 (244.0), 16384 356 (354); 64 channels 6177 119.0 (117.7).
 // LDS of the workgroup (one per CU, two waves per SIMD): two K tiles (the next one is fetched while the current one is
 // used), and per head the diagonal digest, the column partials, the carried bins and the block-sum parts.
 #define LQP_D_FLOATS (2 * 32 * LQ_TILE)  // Dm[32][128] | Dh[32][128]
@@ -314,7 +329,7 @@ struct LqpHeadLds {
   float D[LQP_D_FLOATS];
   float vpart[8][LQ_TILE];  // column sums per (wave, lane half)
   float carry[2][LQ_TILE];  // bins 128..255 of the previous tile, by tile parity
-  float bpart[2][2][4];     // [tile parity][slash, vertical][wave] block-sum parts
+  float bpart[2][2][4];     // [tile parity][slash, vertical][wave] block-sum parts; slash 2, 3: of the carried bins
   float zero16[4];
 };
 #define LQP_LDS_BYTES(D) (2 * LQ_KSW_BYTES(D) + LQ_WG_HEADS * sizeof(LqpHeadLds))
@@ -342,11 +357,10 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   const sp_bf16* kh = k + (int64_t)kvh * sk_h;
   const int64_t n_tiles = sp_ceil_div(n, LQ_TILE);
   const int64_t first = (int64_t)blockIdx.x * tiles_per_wg;
-  const int64_t t_begin = first > 0 ? first - 1 : 0;
   const int64_t t_end = first + tiles_per_wg < n_tiles ? first + tiles_per_wg : n_tiles;
   constexpr int SWZ = D == 128 ? 2 : 1;  // lines / 4 rows
   const LqKLane<D, SWZ> kl = lq_k_lane<D, SWZ>(sk_n, wave8, lane);
-  lq_issue_k_direct<D, SWZ>(kh, n, sk_n, t_begin * LQ_TILE, R2 + (t_begin & 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
+  lq_issue_k_direct<D, SWZ>(kh, n, sk_n, first * LQ_TILE, R2 + (first & 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
   bf16x8 qa[D / 16];
   lq_load_q<true, D / 16>(qh, n, sq_n, wave, lane, inv_sqrt_d, qa);
   float2* const fold = reinterpret_cast<float2*>(L.D);  // [128] (max, 1 / sum) per query row
@@ -395,15 +409,24 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
   }
   const float inv_rows = 1.0f / (float)bs;
   const bool write_blk = bs == LQ_ROWS;  // the block sums of smaller blocks come from sp_lastq_block_sums_kernel
+  auto block_sums = [&](int64_t tile) {
+    const float* bp = &L.bpart[tile & 1][0][0];
+    float* const at = slash_blk + (int64_t)h * nb + tile;
+    if (tile == first && first > 0)
+      unsafeAtomicAdd(at, bp[0] + bp[1]);
+    else
+      *at = bp[0] + bp[1];
+    vert_blk[(int64_t)h * nb + tile] = (bp[4] + bp[5]) + (bp[6] + bp[7]);
+  };
   float* Dm = L.D;
   float* Dh = Dm + 32 * LQ_TILE;
-  if (tid < LQ_TILE) L.carry[(t_begin & 1) ^ 1][tid] = 0.f;  // nothing is carried into the first tile
+  if (tid < LQ_TILE) L.carry[(first & 1) ^ 1][tid] = 0.f;  // (what the first tile is owed arrives in memory)
   if (tid < 4) L.zero16[tid] = 0.f;
   // B operand of key sub-tile nt, k-step ks: K row 4 lq + nt, logical 16-byte chunk 2 ks + hi (swizzled by row / 4)
   const int b_off = lq * 4 * D * 2;
   const int b_swz = lq & 15;
 
-  for (int64_t tile = t_begin; tile < t_end; ++tile) {
+  for (int64_t tile = first; tile < t_end; ++tile) {
     const int64_t kb = tile * LQ_TILE;
     const int par = (int)(tile & 1);
     const char* R = R2 + par * LQ_KSW_BYTES(D);
@@ -411,11 +434,8 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
     __syncthreads();  // ... and everyone's; the previous tile's K reads and digest reads are done
     if (tile + 1 < t_end)  // the next K tile, into the buffer the previous tile has left
       lq_issue_k_direct<D, SWZ>(kh, n, sk_n, kb + LQ_TILE, R2 + (par ^ 1) * LQ_KSW_BYTES(D), wave8, lane, kl);
-    if (tid == 0 && tile > first && has_head && write_blk) {  // the previous tile's block sums: its parts were complete one barrier ago
-      const float* bp = &L.bpart[par ^ 1][0][0];
-      slash_blk[(int64_t)h * nb + tile - 1] = bp[0] + bp[1];
-      vert_blk[(int64_t)h * nb + tile - 1] = (bp[4] + bp[5]) + (bp[6] + bp[7]);
-    }
+    if (tid == 0 && tile > first && has_head && write_blk)  // the previous tile's block sums: its parts were complete one barrier ago
+      block_sums(tile - 1);
     if (has_head) {
       // acc[nt][r] = S[row i' = 32 w + 8 (r / 4) + 4 hi + r % 4][key kb + 4 lq + nt]
       floatx16 acc[4];
@@ -487,10 +507,7 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
       *reinterpret_cast<float4*>(&L.vpart[2 * wave + hi][4 * lq]) = make_float4(vs[0], vs[1], vs[2], vs[3]);
     }
     __syncthreads();
-    // Of the leading tile only the carried bins are wanted: waves 2 and 3, and no columns (a workgroup has one such tile in three at
-    // 3001 tokens; layers, us: 110.4 -> 109.7, 6177 tokens of 64 channels 122.2 -> 121.4).
-    const bool emit = tile >= first;
-    if (has_head && (emit || wave >= 2)) {
+    if (has_head) {
       // slash: thread (pg, qd) gathers bins 4 pg .. 4 pg + 3 from the eight groups G = 8 qd .. 8 qd + 7 (Dm[G] holds
       // bins 4 G .. 4 G + 127, Dh[G] bins 4 G + 4 .. 4 G + 131), then the four lane quarters of the wave meet.
       // Every LDS read of the stage -- digest chunks, carried bins, column partials -- is issued before the first
@@ -531,16 +548,29 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
           for (int d = 0; d < 4; ++d) {
             float val = (crv[d] + sv[d]) * inv_rows;
             if (kb + p0 + d >= n) val = 0.f;
+            else if (tile == first && first > 0) unsafeAtomicAdd(tok + d, val);
             else tok[d] = val;
             tot += val;
           }
         }
         tot = lq_wave_sum(tot);
         if (ln == 0) L.bpart[par][0][wave] = tot;
-      } else if (ln < 16) {
-        *reinterpret_cast<float4*>(&L.carry[par][p0 - LQ_TILE]) = make_float4(sv[0], sv[1], sv[2], sv[3]);
+      } else if (tile + 1 < t_end || tile + 1 == n_tiles) {
+        if (ln < 16) *reinterpret_cast<float4*>(&L.carry[par][p0 - LQ_TILE]) = make_float4(sv[0], sv[1], sv[2], sv[3]);
+      } else {  // the next workgroup's first tile
+        float tot = 0.f;
+        if (ln < 16) {
+          float* tok = slash_tok + (int64_t)h * n + kb + p0;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const float val = kb + p0 + d < n ? sv[d] * inv_rows : 0.f;
+            if (kb + p0 + d < n) unsafeAtomicAdd(tok + d, val);
+            tot += val;
+          }
+        }
+        tot = lq_wave_sum(tot);
+        if (ln == 0) L.bpart[par][0][wave] = tot;
       }
-      if (!emit) continue;
       // vertical: lanes 0..31 of wave w fold the eight partials of columns 32 w .. 32 w + 31
       float val = 0.f;
       if (ln < 32) {
@@ -553,10 +583,10 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
     }
   }
   __syncthreads();
-  if (tid == 0 && t_end > first && has_head && write_blk) {  // the last tile's block sums
+  if (tid == 0 && t_end > first && has_head && write_blk) {  // the last tile's block sums, and the carried bins'
+    block_sums(t_end - 1);
     const float* bp = &L.bpart[(t_end - 1) & 1][0][0];
-    slash_blk[(int64_t)h * nb + t_end - 1] = bp[0] + bp[1];
-    vert_blk[(int64_t)h * nb + t_end - 1] = (bp[4] + bp[5]) + (bp[6] + bp[7]);
+    if (t_end < n_tiles) unsafeAtomicAdd(slash_blk + (int64_t)h * nb + t_end, bp[2] + bp[3]);
   }
 }
 
@@ -623,16 +653,15 @@ static inline int lq_tiles_per_wg(int64_t n, int32_t hq) {
   }
   return best;
 }
-// Output tiles per workgroup of the probabilities kernel.  A workgroup of T output tiles computes T + 1 (the leading
-// tile), and the launch runs in ceil(workgroups / 256) rounds, one workgroup per CU: take the T that minimises
-// rounds x (T + 1).
+// Tiles per workgroup of the probabilities kernel: the launch runs in ceil(workgroups / 256) rounds, one workgroup per CU, and a round
+// takes 4.3 us a tile and 6 besides.
 static inline int lq_probs_tiles_per_wg(int64_t nb, int32_t wg_rows) {
   const int64_t slots = 256;
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int t = 1; t <= 64; ++t) {
     const int64_t wgs = sp_ceil_div(nb, t) * wg_rows;
-    const int64_t cost = sp_ceil_div(wgs, slots) * (t + (sp_ceil_div(nb, t) > 1 ? 1 : 0));
+    const int64_t cost = sp_ceil_div(wgs, slots) * (10 * t + 14);
     if (cost < best_cost) best_cost = cost, best = t;
   }
   return best;
@@ -683,10 +712,12 @@ int sp_lastq_scores_run(const void* q, const void* k, int64_t n, int32_t hq, int
   if (kbar != nullptr) pool = pool_args(k, kbar, n, hkv, d, k_stride_n, k_stride_h, bs, SP_POOL_TAIL_TRUE_LENGTH, nullptr);
   const int64_t pool_rows = sp_ceil_div(sp_ceil_div(pool.units, 2), n_chunks);
   SP_REQUIRE(wg_rows + pool_rows <= 65535, SP_ERR_UNSUPPORTED, "sp_lastq_scores_bf16: grid too large");
+  const int tiles_probs = lq_probs_tiles_per_wg(nb_tiles, wg_rows);
+  const LqSeams seams = {slash_tok, bs == LQ_ROWS ? slash_blk : nullptr, nb, tiles_probs};
   auto launch_stats = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(n_chunks, wg_rows + pool_rows), dim3(LQ_WG_THREADS), 0, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,
                        group, q_stride_n, q_stride_h, k_stride_n, k_stride_h, inv_sqrt_d, flags, n_chunks, tiles_per_wg,
-                       partial, pool);
+                       partial, seams, pool);
   };
   d == 64 ? launch_stats(sp_lastq_stats_kernel<64>) : launch_stats(sp_lastq_stats_kernel<128>);
   SP_LAUNCH_CHECK();
@@ -707,7 +738,6 @@ int sp_lastq_scores_run(const void* q, const void* k, int64_t n, int32_t hq, int
                                (int)LQP_LDS_BYTES(128)));
     attr_set[dev] = true;
   }
-  const int tiles_probs = lq_probs_tiles_per_wg(nb_tiles, wg_rows);
   const int grid_x = (int)sp_ceil_div(nb_tiles, tiles_probs);
   auto launch_probs = [&](auto kernel, size_t lds) {
     hipLaunchKernelGGL(kernel, dim3(grid_x, wg_rows), dim3(LQ_WG_THREADS), lds, s, (const sp_bf16*)q, (const sp_bf16*)k, n, hkv,

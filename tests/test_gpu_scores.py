@@ -74,6 +74,33 @@ def test_lastq_scores_in_chunks_of_any_number_of_tiles(gpu_device, hq, hkv, n):
     assert torch.allclose(st, sref, rtol=2e-4, atol=1e-8)
 
 
+@pytest.mark.parametrize("bs", [128, 64])
+@pytest.mark.parametrize("hq,hkv,n", [(32, 8, 3001), (32, 8, 4097), (14, 2, 9999), (2, 1, 128)])
+def test_seams_between_workgroups_do_not_depend_on_what_stood_there(gpu_device, hq, hkv, n, bs):
+    """Two workgroups add to the first tile of all but the first of them: the same bits every time, over NaN as over zeros, and block
+    sums that are those of the tokens."""
+    from shareprefill_amd import _lib, ops
+
+    lib = _lib.load()
+    q, k = (t.to(gpu_device) for t in _inputs(hq, hkv, n, n))
+    nb = -(-n // bs)
+    ws = torch.empty(lib.sp_lastq_scores_workspace_bytes(n, hq, bs), dtype=torch.uint8, device=gpu_device)
+    runs = []
+    for fill in (0.0, float("nan"), 7.0):
+        outs = [torch.full((hq, m), fill, device=gpu_device) for m in (n, n, nb, nb)]
+        rc = lib.sp_lastq_scores_bf16(q.data_ptr(), k.data_ptr(), n, hq, hkv, 128, q.stride(1), q.stride(0), k.stride(1), k.stride(0), bs,
+                                      _lib.SP_FLAG_LOGITS_BF16, ws.data_ptr(), ws.numel(), *(t.data_ptr() for t in outs),
+                                      torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "sp_lastq_scores_bf16")
+        runs.append(outs)
+    for other in runs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(runs[0], other))
+    vt, st, vb, sb = (t.cpu() for t in runs[0])
+    assert torch.allclose(sb, O.block_sum(st, bs), rtol=1e-5, atol=1e-9)
+    assert torch.allclose(vb, O.block_sum(vt, bs), rtol=1e-5, atol=1e-9)
+    assert torch.allclose(st.sum(-1), torch.ones(hq), atol=1e-4)
+
+
 @pytest.mark.parametrize("bs", [64, 32, 16])
 @pytest.mark.parametrize("hq,hkv,n", [(4, 2, 1024), (6, 2, 1000), (7, 1, 389), (2, 1, 128), (4, 4, 2100), (4, 2, 100),
                                       (2, 2, 64), (3, 1, 127)])  # the last three: prompts shorter than 128 tokens
