@@ -308,6 +308,17 @@ int sp_decode_attn_bf16(const void* q, const void* k, const void* v, int64_t n, 
  * workspace: sp_decode_batch_workspace_bytes(batch, n, hq, hkv) bytes of device scratch (zero where every sequence is one
  * chunk: a null pointer will do), 8-byte aligned. */
 size_t sp_decode_batch_workspace_bytes(int32_t batch, int64_t n, int32_t hq, int32_t hkv);
+/* sp_decode_attn_batch_bf16's arguments in memory, for callers whose calls cost by the argument (a foreign-function interface). */
+typedef struct {
+  const void *q, *k, *v;
+  void *out, *workspace;
+  uint64_t workspace_bytes;
+  int64_t batch, n, hq, hkv, d;
+  int64_t q_stride_b, q_stride_h, k_stride_b, k_stride_n, k_stride_h, v_stride_b, v_stride_n, v_stride_h;
+  double softmax_scale;
+  sp_stream_t stream;
+} sp_decode_batch_args;
+int sp_decode_attn_batch_args_bf16(const sp_decode_batch_args* args);
 int sp_decode_attn_batch_bf16(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq,
                               int32_t hkv, int32_t d, int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_b,
                               int64_t k_stride_n, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_n,

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 # SHAREPREFILL_HIP_LIB overrides the in-tree library path (e.g. to try an experimental build)
 LIB_PATH = os.environ.get("SHAREPREFILL_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc",
@@ -95,6 +96,7 @@ SIGNATURES = {
     "sp_decode_batch_workspace_bytes": (_SZ, [_I32, _I64, _I32, _I32]),
     "sp_decode_attn_batch_bf16": (_I32, [_P, _P, _P, _I32, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _I64,
                                          _I64, _I64, _F, _P, _P, _SZ, _P]),
+    "sp_decode_attn_batch_args_bf16": (_I32, [C.c_char_p]),  # (DECODE_BATCH_ARGS.pack(...))
     "sp_decode_attn_static_bf16": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _F, _P, _P]),
     "sp_rope_inplace_bf16": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _I64, _I64, _I64, _I64, _I64, _P]),
     "sp_pivot_update": (_I32, [_ST, _P, _P, _P, _I32, _I32, _F, _P]),
@@ -103,6 +105,9 @@ SIGNATURES = {
     "sp_block_idx_to_mask": (_I32, [_P, _I64, _I64, _I32, _I32, _P, _P]),
     "sp_block_idx_row_pointers": (_I32, [_P, _I64, _I64, _I32, _I32, _P, _P]),
 }
+
+# sp_decode_batch_args
+DECODE_BATCH_ARGS = struct.Struct("@5PQ13qdP")
 
 _lib = None
 

@@ -401,7 +401,7 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
   constexpr int KC = D / 8, VC = CW / 8;                                          // chunks of a row
   constexpr int KI = Shape::K_BYTES / 1024, VI = Shape::V_BYTES / 1024;           // instructions of a step
   constexpr int KR = SP_WAVE / KC, VR = SP_WAVE / VC;                             // rows of an instruction
-  extern __shared__ __attribute__((aligned(1024))) char ds_lds[];
+  __shared__ __attribute__((aligned(1024))) char ds_lds[Shape::LDS_BYTES];
   __shared__ float m_s[WAVES][DS_GMAX], l_s[WAVES][DS_GMAX];
   const int slice = CW == D ? 0 : blockIdx.y, split = CW == D ? blockIdx.y : 0, splits = CW == D ? gridDim.y : 1;
   int kvh = blockIdx.x;
@@ -596,17 +596,9 @@ template <int D, int CT, bool FULL>
 static int ds_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv, int32_t d, const DcStrides& st,
                      float scale_log2, int splits, int keys_per_split, float* o_part, float2* ml_part, void* out, hipStream_t s) {
   using Shape = DsShape<D, CT>;
-  static bool attr_set[64] = {false};  // per device, once (idempotent)
-  int dev = 0;
-  SP_HIP(hipGetDevice(&dev));
-  SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "decode attention: device index %d", dev);
-  if (!attr_set[dev]) {
-    SP_HIP(hipFuncSetAttribute((const void*)sp_decode_ring_kernel<D, CT, FULL>, hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS_BYTES));
-    attr_set[dev] = true;
-  }
   const int slices = D / 16 / CT;
   auto launch = [&](dim3 grid, int64_t b0, int32_t count) {
-    hipLaunchKernelGGL((sp_decode_ring_kernel<D, CT, FULL>), grid, dim3(Shape::WAVES * SP_WAVE), Shape::LDS_BYTES, s, (const sp_bf16*)q + b0 * st.q_b,
+    hipLaunchKernelGGL((sp_decode_ring_kernel<D, CT, FULL>), grid, dim3(Shape::WAVES * SP_WAVE), 0, s, (const sp_bf16*)q + b0 * st.q_b,
                        (const sp_bf16*)k + b0 * st.k_b, (const sp_bf16*)v + b0 * st.v_b, (int)n, hq / hkv, (int)hkv, (int)d, (int)count,
                        (uint32_t)sp_ceil_div(65536, hkv), st, scale_log2, keys_per_split, o_part, ml_part, (sp_bf16*)out + b0 * hq * d);
   };
@@ -793,6 +785,15 @@ extern "C" int sp_decode_attn_batch_bf16(const void* q, const void* k, const voi
   SP_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace % 8) == 0,
              SP_ERR_WORKSPACE, "sp_decode_attn_batch_bf16: workspace too small or misaligned");
   return dc_launch(q, k, v, batch, n, hq, hkv, d, st, softmax_scale, out, workspace, (hipStream_t)stream);
+}
+
+extern "C" int sp_decode_attn_batch_args_bf16(const sp_decode_batch_args* a) {
+  SP_REQUIRE(a != nullptr, SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_batch_args_bf16: null pointer");
+  SP_REQUIRE(a->batch == (int32_t)a->batch && a->hq == (int32_t)a->hq && a->hkv == (int32_t)a->hkv && a->d == (int32_t)a->d,
+             SP_ERR_INVALID_ARGUMENT, "sp_decode_attn_batch_args_bf16: a size beyond 32 bits");
+  return sp_decode_attn_batch_bf16(a->q, a->k, a->v, (int32_t)a->batch, a->n, (int32_t)a->hq, (int32_t)a->hkv, (int32_t)a->d, a->q_stride_b,
+                                   a->q_stride_h, a->k_stride_b, a->k_stride_n, a->k_stride_h, a->v_stride_b, a->v_stride_n, a->v_stride_h,
+                                   (float)a->softmax_scale, a->out, a->workspace, (size_t)a->workspace_bytes, a->stream);
 }
 
 extern "C" int sp_decode_attn_bf16(const void* q, const void* k, const void* v, int64_t n, int32_t hq, int32_t hkv,

@@ -92,13 +92,17 @@ def pool(x: torch.Tensor, block_size: int, pool_type: str) -> torch.Tensor:
 
 
 _workspaces = {}
+_device_names = {}  # str(device) of the devices seen: a decode step takes longer to write the name than to look its scratch up
 
 
-def _workspace(tag: str, nbytes: int, device) -> torch.Tensor:
+def _workspace(tag: str, nbytes: int, device, stream: Optional[int] = None) -> torch.Tensor:
     """Grow-only scratch buffers keyed by purpose, device AND stream (reused across layers).  Work on one stream is
     ordered, so consecutive calls may share a buffer; two streams of one device (two models, two threads) get
     buffers of their own and cannot race on the scheduler tickets or the repacked V they hold."""
-    key = (tag, str(device), _stream_handle(device))
+    name = _device_names.get(device)
+    if name is None:
+        name = _device_names[device] = str(device)
+    key = (tag, name, _stream_handle(device) if stream is None else stream)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
@@ -490,14 +494,17 @@ def decode_attention_batch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, so
     if min(k.shape[0], v.shape[0]) < b or v.shape[1] < hkv or v.shape[2] < n or min(k.shape[3], v.shape[3]) < d:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} do not match q {tuple(q.shape)}")
     stream = _stream_handle(dev)
-    out = torch.empty((b, 1, hq, d), dtype=torch.bfloat16, device=dev)
+    out = q.new_empty((b, 1, hq, d))
     need = lib.sp_decode_batch_workspace_bytes(b, n, hq, hkv)
-    ws = _workspace("decode", need, dev) if need else out  # (nothing is kept: any address will do)
+    ws = _workspace("decode", need, dev, stream) if need else out  # (nothing is kept: any address will do)
     if b == 1:
         q_b = k_b = v_b = 0  # (the stride of an axis of one entry means nothing)
-    st = lib.sp_decode_attn_batch_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b, n, hq, hkv, d, q_b, q_h, k_b, k_n, k_h,
-                                       v_b, v_n, v_h, softmax_scale, out.data_ptr(), ws.data_ptr(), ws.numel() if need else 0, stream)
-    _lib.check(st, "sp_decode_attn_batch_bf16")
+    # one argument in memory instead of twenty-one: the step's host time is most of a short cache's
+    st = lib.sp_decode_attn_batch_args_bf16(_lib.DECODE_BATCH_ARGS.pack(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel() if need else 0, b, n, hq, hkv, d, q_b, q_h, k_b,
+        k_n, k_h, v_b, v_n, v_h, softmax_scale, stream))
+    if st:
+        _lib.check(st, "sp_decode_attn_batch_bf16")
     return out
 
 
