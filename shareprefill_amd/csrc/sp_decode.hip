@@ -528,14 +528,15 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
         mx = fmaxf(mx, s[i][j]);
       }
     const float m_new = fmaxf(m, ds_quad_max(mx));
-    const float alpha = __builtin_amdgcn_exp2f(m - m_new);  // 0 in the first step
+    const float base = m_new == -INFINITY ? 0.f : m_new;   // (no key so far has a finite logit: every weight is exp2(-inf) = 0)
+    const float alpha = __builtin_amdgcn_exp2f(m - base);  // 0 in the first step
     float add = 0.f;
     uint32_t hi[4], lo[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 4; j += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(s[i][j] - m_new), p1 = __builtin_amdgcn_exp2f(s[i][j + 1] - m_new);
+        const float p0 = __builtin_amdgcn_exp2f(s[i][j] - base), p1 = __builtin_amdgcn_exp2f(s[i][j + 1] - base);
         const uint32_t w = dc_pack2(p0, p1);
         hi[2 * i + j / 2] = w;
         lo[2 * i + j / 2] = dc_pack2(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xffff0000u));
@@ -576,7 +577,8 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
     ds_floatx4 acc = {0, 0, 0, 0};
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const float f = __builtin_amdgcn_exp2f(m_s[w][h] - top);  // (a wave without keys: 0)
+      // (a wave without keys, or without a finite logit: 0)
+      const float f = m_s[w][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_s[w][h] - top);
       sum += l_s[w][h] * f;
       acc += *reinterpret_cast<const ds_floatx4*>(&o_s[w][h][c]) * f;
     }

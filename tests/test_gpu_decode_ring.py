@@ -69,3 +69,20 @@ def test_results_on_odd_addresses_and_caches_of_one_row_a_token(gpu_device, n, d
     assert one.stride(2) == 0
     out = ops.decode_attention_batch(q, one, v, d ** -0.5)
     assert _error(out, _exact(q, one, v, d ** -0.5)) <= BOUND
+
+
+@pytest.mark.parametrize("b,n", [(1, 300), (1, 3000)])  # one launch; splits
+def test_keys_whose_logits_are_minus_infinity(gpu_device, b, n):
+    """Keys that no query can see, among them whole steps, whole waves' shares and a whole split: they weigh nothing."""
+    from shareprefill_amd import ops
+
+    hq, hkv, d = 8, 2, 128
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(b, hq, 1, d).abs(), mk(b, hkv, n, d), mk(b, hkv, n, d)
+    seen = torch.ones(n, dtype=torch.bool, device=gpu_device)
+    seen[:70] = seen[128:256] = seen[260:290:2] = False
+    k[:, :, ~seen] = k[:, :, ~seen].abs()
+    k[:, :, ~seen, 5] = float("-inf")
+    want = _exact(q, k[:, :, seen], v[:, :, seen], d ** -0.5)
+    assert _error(ops.decode_attention_batch(q, k, v, d ** -0.5), want) <= BOUND
