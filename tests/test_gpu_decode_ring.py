@@ -86,3 +86,27 @@ def test_keys_whose_logits_are_minus_infinity(gpu_device, b, n):
     k[:, :, ~seen, 5] = float("-inf")
     want = _exact(q, k[:, :, seen], v[:, :, seen], d ** -0.5)
     assert _error(ops.decode_attention_batch(q, k, v, d ** -0.5), want) <= BOUND
+
+
+@pytest.mark.parametrize("b,hq,hkv,n,d", [(1, 8, 2, 300, 128), (1, 8, 2, 3000, 128), (12, 32, 8, 193, 128), (33, 8, 8, 129, 128),
+                                          (1, 14, 2, 1025, 64), (1, 6, 2, 1025, 96)])  # slices of every width, splits
+def test_values_that_are_infinite(gpu_device, b, hq, hkv, n, d):
+    """A channel whose values hold one infinity is that infinity, and NaN where they hold both, as in 64 bits: the probabilities'
+    second part is zero for some keys and negative for others.  The other channels do not notice."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(b, hq, 1, d), mk(b, hkv, n, d), mk(b, hkv, n, d)
+    keys = torch.randperm(n - 1, generator=gen, device=gpu_device)[:d]  # (the last key also stands in for those behind the cache, weight 0)
+    channels = torch.arange(0, d, 2, device=gpu_device)  # one infinity in every other channel, the second sign in some
+    sign = 1.0 - 2.0 * (channels % 4 == 0)
+    v[:, :, keys[:d // 2], channels] = (sign * float("inf")).to(torch.bfloat16)
+    v[:, :, keys[d // 2:d // 2 + 3], channels[:3]] = (-sign[:3] * float("inf")).to(torch.bfloat16)
+    q[0, 0] = 0  # equal weights, all of them bf16 values: no second part
+    out, want = ops.decode_attention_batch(q, k, v, d ** -0.5), _exact(q, k, v, d ** -0.5)
+    assert torch.equal(out.isnan(), want.isnan()) and want[..., channels[:3]].isnan().all()
+    inf = want.isinf()
+    assert inf[..., channels[3:]].all() and torch.equal(out[inf].double(), want[inf])
+    rest = want.isfinite()
+    assert _error(out[rest], want[rest]) <= BOUND
