@@ -156,14 +156,15 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
     __syncthreads();
     float m_new = m_run, alpha = 1.f;
     if (head_ok) {
-      m_new = fmaxf(fmaxf(fmaxf(wmax[0][lh], wmax[1][lh]), fmaxf(wmax[2][lh], wmax[3][lh])), m_run);  // finite
-      alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first tile
+      m_new = fmaxf(fmaxf(fmaxf(wmax[0][lh], wmax[1][lh]), fmaxf(wmax[2][lh], wmax[3][lh])), m_run);
+      const float base = m_new == -INFINITY ? 0.f : m_new;  // (no key so far has a finite logit: every weight is exp2(-inf) = 0)
+      alpha = __builtin_amdgcn_exp2f(m_run - base);         // 0 on the first tile
       float ls = 0.f;
       sp_bf16* prow = Ps + lh * DC_PITCH + 32 * wave + 4 * hi;
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
-        const float p0 = __builtin_amdgcn_exp2f(acc[4 * r4 + 0] - m_new), p1 = __builtin_amdgcn_exp2f(acc[4 * r4 + 1] - m_new);
-        const float p2 = __builtin_amdgcn_exp2f(acc[4 * r4 + 2] - m_new), p3 = __builtin_amdgcn_exp2f(acc[4 * r4 + 3] - m_new);
+        const float p0 = __builtin_amdgcn_exp2f(acc[4 * r4 + 0] - base), p1 = __builtin_amdgcn_exp2f(acc[4 * r4 + 1] - base);
+        const float p2 = __builtin_amdgcn_exp2f(acc[4 * r4 + 2] - base), p3 = __builtin_amdgcn_exp2f(acc[4 * r4 + 3] - base);
         ls += (p0 + p1) + (p2 + p3);
         *reinterpret_cast<uint2*>(prow + 8 * r4) = make_uint2(dc_pack2(p0, p1), dc_pack2(p2, p3));
       }
@@ -212,8 +213,8 @@ __global__ __launch_bounds__(DC_THREADS, 2) void sp_decode_partial_kernel(
       tiles_left = tiles_per_chunk;
       if (folded || !last) {
         folded = true;
-        const float m = fmaxf(m_sum, m_run);
-        const float before = __builtin_amdgcn_exp2f(m_sum - m), here = __builtin_amdgcn_exp2f(m_run - m);
+        const float m = fmaxf(m_sum, m_run), base = m == -INFINITY ? 0.f : m;
+        const float before = __builtin_amdgcn_exp2f(m_sum - base), here = __builtin_amdgcn_exp2f(m_run - base);
         l_sum = l_sum * before + l_run * here;
         m_sum = m;
 #pragma unroll

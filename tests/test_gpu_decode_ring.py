@@ -110,3 +110,22 @@ def test_values_that_are_infinite(gpu_device, b, hq, hkv, n, d):
     assert inf[..., channels[3:]].all() and torch.equal(out[inf].double(), want[inf])
     rest = want.isfinite()
     assert _error(out[rest], want[rest]) <= BOUND
+
+
+@pytest.mark.parametrize("hq,hkv", [(40, 2), (17, 1), (32, 1)])  # the kernel of groups of 17 to 32 heads
+@pytest.mark.parametrize("b,n,d", [(1, 256, 128), (300, 512, 128), (1, 3000, 128), (1, 3000, 64)])  # two chunks and four of a workgroup; splits
+def test_keys_whose_logits_are_minus_infinity_in_large_groups(gpu_device, b, n, d, hq, hkv):
+    """The other kernel's case of test_keys_whose_logits_are_minus_infinity: whole tiles of 128 keys, which are chunks and splits of
+    their own, have no key that a query can see.  Probabilities are one bf16 value there (2^-8 more)."""
+    from shareprefill_amd import ops
+
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=gpu_device).to(torch.bfloat16)
+    q, k, v = mk(b, hq, 1, d).abs(), mk(b, hkv, n, d), mk(b, hkv, n, d)
+    seen = torch.ones(n, dtype=torch.bool, device=gpu_device)
+    seen[:128] = seen[256:384] = seen[140:170:2] = seen[2816:] = False
+    k[:, :, ~seen] = k[:, :, ~seen].abs()
+    k[:, :, ~seen, 5] = float("-inf")
+    out = ops.decode_attention_batch(q, k, v, d ** -0.5)
+    some = sorted({0, b // 2, b - 1})
+    assert _error(out[some], _exact(q[some], k[some][:, :, seen], v[some][:, :, seen], d ** -0.5)) <= BOUND + 2.0 ** -8
