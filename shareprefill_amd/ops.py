@@ -340,6 +340,16 @@ def attention_workspace(n: int, hq: int, hkv: int, d: int, block_size: int, devi
     return _workspace("attn_vt", need, device), need
 
 
+def attention_block_sums(n: int, hq: int, hkv: int, block_size: int, device, max_pivots: int) -> Optional[torch.Tensor]:
+    """The part of attention_workspace's buffer that holds the block sums of max_pivots heads (None: of none), for a
+    short_attention call at a length where other layers of the prompt take block_sparse_attention: the two run in order on a stream
+    and a slab is 256 MiB at 131072 tokens, so they are not held twice.  What block_sparse_attention keeps in front of it stays."""
+    if max_pivots == 0:
+        return None
+    buf, need = attention_workspace(n, hq, hkv, 128, block_size, device, max_pivots)
+    return buf[need - min(max_pivots, hq) * _lib.load().sp_attn_pivot_scratch_bytes(n, block_size):need]
+
+
 def repack_v(v: torch.Tensor, block_size: int, ws: torch.Tensor) -> None:
     """Key-major repack of v [Hkv, N, D] into the attention workspace (the step depends on v alone)."""
     lib = _lib.load()
@@ -401,13 +411,15 @@ def block_sparse_attention(q, k, v, mask, block_size, softmax_scale, decision=No
     return out
 
 
-def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, pivot=None, max_pivots=None) -> torch.Tensor:
+def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, pivot=None, max_pivots=None,
+                    block_sums=None) -> torch.Tensor:
     """block_sparse_attention for short prompts (block size 128, head_dim 64 or 128): q [Hq,N,D], k/v [Hkv,N,D] views,
     mask int64 [Hq,nb,nbw] -> out bf16 [N,Hq,D].  One launch, whatever decision says: v is read as it is and the maps of
     DENSE heads are written by the same kernel (avg_attn without decision is cleared).
     pivot = (state, head_cluster, pattern_threshold): pivot_update with decision and avg_attn is part of the launch.
     max_pivots: how many heads can be DENSE (an upper bound the host knows; default all of them): what is kept for their maps
-    is sized by it, and DENSE heads beyond it get NaN for a map."""
+    is sized by it, and DENSE heads beyond it get NaN for a map.
+    block_sums: memory for that (attention_block_sums) instead of a buffer of this call's own kind."""
     lib = _lib.load()
     _check_hnd(q, "q")
     _check_hnd(k, "k")
@@ -421,7 +433,11 @@ def short_attention(q, k, v, mask, softmax_scale, decision=None, avg_attn=None, 
     ws, ws_bytes = None, 0
     if decision is not None and avg_attn is not None:
         ws_bytes = (hq if max_pivots is None else min(max_pivots, hq)) * lib.sp_attn_pivot_scratch_bytes(n, 128)
-        ws = _workspace("attn_short", ws_bytes, dev) if ws_bytes else None
+        ws = block_sums
+        if ws is None:
+            ws = _workspace("attn_short", ws_bytes, dev) if ws_bytes else None
+        elif ws.numel() < ws_bytes:
+            raise ValueError(f"block_sums holds {ws.numel()} bytes, {ws_bytes} are needed")
     timer = kernel_timer
     if timer is not None:
         timer.start("attn")

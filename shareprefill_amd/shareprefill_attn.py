@@ -197,8 +197,9 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
     # are; longer ones repack v and run the persistent kernel on 128
     head_dim = 64 if model_dim in PADDED_HEAD_DIMS else model_dim
     short = block_size == 128 and q_len <= _lib.load().sp_short_attn_max_tokens(head_dim)
+    further = False  # short past the length up to which every layer is
     if not short and plan_here and block_size == 128:
-        short = _short_in_steady_layers(sharing, module.layer_idx, num_heads, q_len, head_dim, config.pattern_threshold,
+        short = further = _short_in_steady_layers(sharing, module.layer_idx, num_heads, q_len, head_dim, config.pattern_threshold,
                                         key_states, value_states)
     if model_dim == KERNEL_HEAD_DIM and value_states.stride(2) * 128 >= 2 ** 31:
         short = False  # the short-prompt kernel's offsets inside a block of v have 32 bits, the repack's 64
@@ -262,9 +263,11 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
         getattr(sharing.update_pivotal_attns, "__func__", None) is _UPDATE_PIVOTAL_ATTNS)
     pivot = sharing.pivot_slabs(module.layer_idx, num_heads, q.device, config.pattern_threshold) if update_here else None
     if short:
+        max_pivots = sharing.max_pivots(module.layer_idx, num_heads) if plan_here else None
+        # (the layers in front of one that goes further hold block sums for the persistent kernel)
+        sums = ops.attention_block_sums(q_len, num_heads, key_states.shape[1], block_size, q.device, max_pivots) if further else None
         out = ops.short_attention(q, k, v, plan.mask, softmax_scale, decision=plan.decision, avg_attn=avg_attn[0],
-                                  max_pivots=sharing.max_pivots(module.layer_idx, num_heads) if plan_here else None,
-                                  pivot=pivot)
+                                  max_pivots=max_pivots, pivot=pivot, block_sums=sums)
     else:
         out = ops.block_sparse_attention(q, k, v, plan.mask, block_size, softmax_scale, decision=plan.decision,
                                          avg_attn=avg_attn[0], max_pivots=max_pivots, workspace=ws,

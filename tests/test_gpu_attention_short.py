@@ -270,3 +270,47 @@ def test_steady_layers_take_the_short_prompt_kernel_further(gpu_device, tmp_path
     for (out, maps), (out_want, maps_want) in zip(got, want):
         assert torch.equal(out, out_want) and torch.equal(maps, maps_want)
     assert torch.equal(state.info, state_want.info) and torch.equal(state.pattern, state_want.pattern)
+
+
+@pytest.mark.parametrize("hq,hkv,n,d,pattern", [(8, 2, 6913, 128, 0.9), (2, 1, 65665, 64, 0.95), (2, 1, 131072, 64, 0.95)])
+def test_a_steady_layer_that_elects_after_all(gpu_device, tmp_path, monkeypatch, hq, hkv, n, d, pattern):
+    """A first layer whose heads are all query-aware elects no pivot, the second, which opens no cluster, does: in the short-prompt
+    kernel, up to its longest rows, with the persistent one's output.  A map's entries are differences of running sums of weights that
+    come to at most 1 each query, kept in fp32: 2^-20 from the persistent kernel's, which moves a block in or out of a pattern here and
+    there.  Both kernels keep block sums in one place, which is no larger than the persistent kernel's alone."""
+    import types
+
+    from shareprefill_amd import AttentionSharing, _lib, ops, shareprefill_attention_forward, shareprefill_attn, synthetic
+
+    lib = _lib.load()
+    assert lib.sp_short_attn_max_tokens(d) < n <= lib.sp_short_attn_max_steady_tokens(d, pattern)
+    path = synthetic.write_cluster_table(synthetic.random_cluster_table(hq, 2, 2, n), str(tmp_path / "table.json"))
+    qkv = [synthetic.planted_qkv(hq, hkv, n, d, 7 + layer, device=gpu_device, q_head_gain=1.0) for layer in range(2)]
+    calls = []
+    short = ops.short_attention
+    monkeypatch.setattr(ops, "short_attention", lambda *a, **kw: calls.append(len(results)) or short(*a, **kw))
+    passes, held = [], []
+    for steady in (True, False):
+        if not steady:
+            monkeypatch.setattr(shareprefill_attn, "_short_in_steady_layers", lambda *a: False)
+        sharing, results = AttentionSharing(path), []
+        torch.cuda.synchronize()
+        ops.release_workspaces()
+        for layer in range(2):
+            cfg = types.SimpleNamespace(block_size=128, min_budget=1024, max_budget=None, pattern_threshold=pattern, similarity_threshold=0.5,
+                                        fallback_threshold=1e9, queryaware_threshold=0.0 if layer else 2.0)
+            mod = types.SimpleNamespace(config=cfg, attention_sharing=sharing, layer_idx=layer, scaling=d ** -0.5)
+            out, maps = shareprefill_attention_forward(mod, *qkv[layer], None, scaling=d ** -0.5)
+            results.append((out, maps, sharing.plans[-1].decision))
+        passes.append((results, sharing._state))
+        held.append(sum(buf.numel() for key, buf in ops._workspaces.items() if key[0].startswith("attn_")))
+    assert calls == [1] and held[0] == held[1]
+    (got, state), (want, state_want) = passes
+    assert (got[0][2] == _lib.SP_DEC_QA).all() and (got[1][2] == _lib.SP_DEC_DENSE).any()
+    for (out, maps, decision), (out_want, maps_want, decision_want) in zip(got, want):
+        assert torch.equal(decision, decision_want) and torch.equal(out, out_want)
+        assert (maps - maps_want).abs().max().item() <= 2.0 ** -20
+    assert torch.equal(state.info, state_want.info) and (state.info[:, 1] != 0).any()
+    nb = -(-n // 128)
+    moved = ops.mask_to_bool(state.pattern, nb) != ops.mask_to_bool(state_want.pattern, nb)
+    assert moved.float().mean().item() <= 1e-4
