@@ -314,3 +314,8 @@ def test_a_steady_layer_that_elects_after_all(gpu_device, tmp_path, monkeypatch,
     nb = -(-n // 128)
     moved = ops.mask_to_bool(state.pattern, nb) != ops.mask_to_bool(state_want.pattern, nb)
     assert moved.float().mean().item() <= 1e-4
+
+
+@pytest.mark.parametrize("n", [65665, 131072])  # 514 and 1024 blocks
+def test_pivot_patterns_of_the_longest_rows(gpu_device, n):
+    test_pivot_patterns_in_the_attention_launch(gpu_device, 3, 1, n, 64)
