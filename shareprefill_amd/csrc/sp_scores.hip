@@ -16,11 +16,10 @@
 // Results are reproducible run to run: every other sum runs in a fixed order.
 #include "sp_block_probs.h"
 #include "sp_pool.h"
+#include "sp_scores_plan.h"
 
                              // D, the head dim, is 64 or 128: a template parameter of every kernel here
 #define LQ_THREADS 256       // 4 waves per head, wave w owns 32 query rows of the last block
-#define LQ_MIN_TILES 1       // key tiles per workgroup of the statistics kernel (lq_tiles_per_wg)
-#define LQ_MAX_TILES 32
 // lane's operand: scaled last-block queries, D / 16 k-steps x 8 bf16; MFMA row m = lane % 32 of wave w is query 32 w + m of
 // the last block, or query 127 - (32 w + m) with REVERSED
 template <bool REVERSED, int KS>
@@ -62,9 +61,7 @@ __device__ static __forceinline__ void lq_load_q(const sp_bf16* __restrict__ q, 
 // traffic of these fetches that bounds the kernels otherwise (one tile per (query head, key tile): 1 GiB per pass at
 // 128K tokens and 32 heads, about 5 TB/s when nothing else is done).  A group with an odd head count leaves the second
 // half of its last workgroup without a head: those waves fetch and synchronise, and compute nothing.
-#define LQ_WG_HEADS 2
 #define LQ_WG_THREADS (LQ_THREADS * LQ_WG_HEADS)
-static inline __host__ __device__ int lq_pairs(int group) { return (group + LQ_WG_HEADS - 1) / LQ_WG_HEADS; }
 
 // Four wave-instructions per wave fill the tile: instruction `it` of wave w (0..7) writes the 1 KiB segment 8 * it + w
 // (4 key rows); lane i writes chunk position i of the segment and fetches the global chunk that belongs there.
@@ -134,7 +131,7 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
     int64_t sq_h, int64_t sk_n, int64_t sk_h, float inv_sqrt_d, uint32_t flags, int n_chunks, int tiles_per_wg,
     float2* __restrict__ partial /* [hq][n_chunks][128] */, LqSeams seams, PoolArgs pool) {
   __shared__ __attribute__((aligned(1024))) char Ksw[LQ_KSW_BYTES(D)];
-  const int pairs = lq_pairs(group);
+  const int pairs = (group + LQ_WG_HEADS - 1) / LQ_WG_HEADS;
   // The rows of the grid behind the scores' own pool K beside them (dispatched last, two units per workgroup): the vector
   // ALU bounds the scores, so the keys' second way through memory fits beside them (131072 tokens: statistics 195 us alone, 196
   // with it, where a launch of its own takes 43; a launch with nothing to do takes 2 to 2.7).
@@ -252,7 +249,6 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 4) void sp_lastq_stats_kernel(
 // One workgroup per head: 8 groups of 128 threads; group j folds chunks j, j+8, ... of every row, then the eight
 // group results are merged in a fixed order.
 #define LQ_COMBINE_GROUPS 8
-#define LQ_FOLD_CHUNKS 32  // chunks up to which the probabilities kernel folds them in its prologue instead: 16 loads per lane
 __global__ __launch_bounds__(LQ_ROWS * LQ_COMBINE_GROUPS) void sp_lastq_combine_kernel(
     const float2* __restrict__ partial, int n_chunks, float2* __restrict__ rowstat /* [hq][128] */) {
   __shared__ float gm[LQ_COMBINE_GROUPS][LQ_ROWS], gl[LQ_COMBINE_GROUPS][LQ_ROWS];
@@ -343,7 +339,7 @@ __global__ __launch_bounds__(LQ_WG_THREADS, 2) void sp_lastq_probs_kernel(
     float* __restrict__ slash_blk, int64_t nb, int tiles_per_wg, int bs) {
   extern __shared__ __attribute__((aligned(1024))) char lqp_lds[];
   char* R2 = lqp_lds;  // [2][LQ_KSW_BYTES(D)]
-  const int pairs = lq_pairs(group);
+  const int pairs = (group + LQ_WG_HEADS - 1) / LQ_WG_HEADS;
   const int kvh = blockIdx.y / pairs;
   const int wave8 = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wave = wave8 & 3;
@@ -635,46 +631,10 @@ int sp_block_probs_mfma_launch(const void* qbar, const void* kbar, const int32_t
 }
 
 // ---- host -------------------------------------------------------------------------------------------------
-// Key tiles per workgroup of the statistics kernel: of all counts the one whose launch is the shortest, by the times it was measured
-// to take (0.01 us; 128 channels, 3001 to 131072 tokens, counts 1 to 32, each within 10 %): a tile 2.9 us in a workgroup that has its CU
-// to itself and 2.35 per tile of a CU with two, 6 and 9.5 us besides, and the launch that folds what the probabilities kernel does not
-// fold itself; a CU without a workgroup counts 0.03 us, by what layers take (6177 tokens of 64 channels: 208 workgroups of four tiles
-// 122.2 us, 400 of two 121.6).  Against counts that were powers of two and made some 512 workgroups, us for both: 4500 tokens
-// 17.8 / 15.5, 10007 of 28 heads 24.1 / 19.4, 16384 30.6 / 27.6, 20000 of 64 channels 34.9 / 24.0, 65001 90.7 / 85.0.
-static inline int lq_tiles_per_wg(int64_t n, int32_t hq) {
-  const int64_t tiles = sp_ceil_div(n, LQ_TILE), rows = (hq + LQ_WG_HEADS - 1) / LQ_WG_HEADS;
-  int best = 1;
-  int64_t best_cost = INT64_MAX;
-  for (int t = LQ_MIN_TILES; t <= LQ_MAX_TILES; ++t) {
-    const int64_t chunks = sp_ceil_div(tiles, t), per_cu = sp_ceil_div(chunks * rows, 256);
-    const int64_t cost = (per_cu == 1 ? 290 * t + 600 + 3 * (256 - chunks * rows) : 235 * t * per_cu + 950 + 130 * (sp_ceil_div(per_cu, 2) - 1)) +
-                         (chunks > LQ_FOLD_CHUNKS ? 450 : 0);
-    if (cost < best_cost) best_cost = cost, best = t;
-  }
-  return best;
-}
-// Tiles per workgroup of the probabilities kernel: the launch runs in ceil(workgroups / 256) rounds, one workgroup per CU, and a round
-// takes 4.3 us a tile and 6 besides.
-static inline int lq_probs_tiles_per_wg(int64_t nb, int32_t wg_rows) {
-  const int64_t slots = 256;
-  int best = 1;
-  int64_t best_cost = INT64_MAX;
-  for (int t = 1; t <= 64; ++t) {
-    const int64_t wgs = sp_ceil_div(nb, t) * wg_rows;
-    const int64_t cost = sp_ceil_div(wgs, slots) * (10 * t + 14);
-    if (cost < best_cost) best_cost = cost, best = t;
-  }
-  return best;
-}
-// chunk count of the launch (the workspace is sized for it)
-static inline int lq_chunks(int64_t n, int32_t hq) {
-  return (int)sp_ceil_div(sp_ceil_div(n, LQ_TILE), lq_tiles_per_wg(n, hq));
-}
-
 extern "C" size_t sp_lastq_scores_workspace_bytes(int64_t n, int32_t hq, int32_t bs) {
   (void)bs;
   if (n <= 0 || hq <= 0) return 0;
-  size_t partial = (size_t)hq * lq_chunks(n, hq) * LQ_ROWS * sizeof(float2);
+  size_t partial = (size_t)hq * lq_max_chunks(sp_ceil_div(n, LQ_TILE), hq) * LQ_ROWS * sizeof(float2);
   size_t rowstat = (size_t)hq * LQ_ROWS * sizeof(float2);
   return partial + rowstat;
 }
@@ -699,15 +659,15 @@ int sp_lastq_scores_run(const void* q, const void* k, int64_t n, int32_t hq, int
              SP_ERR_UNSUPPORTED, "sp_lastq_scores_bf16: q/k must be 16-byte aligned with strides multiple of 8");
   SP_REQUIRE(workspace_bytes >= sp_lastq_scores_workspace_bytes(n, hq, bs), SP_ERR_WORKSPACE,
              "sp_lastq_scores_bf16: workspace too small");
-  const int tiles_per_wg = lq_tiles_per_wg(n, hq);
-  const int n_chunks = (int)sp_ceil_div(sp_ceil_div(n, LQ_TILE), tiles_per_wg);
   const int64_t nb = sp_ceil_div(n, bs);          // blocks of the caller's size: the length of vert_blk / slash_blk
   const int64_t nb_tiles = sp_ceil_div(n, LQ_TILE);  // 128-token tiles the kernels walk
-  float2* partial = (float2*)workspace;
-  float2* rowstat = partial + (size_t)hq * lq_chunks(n, hq) * LQ_ROWS;
-  const float inv_sqrt_d = sp_inv_sqrt_dim(flags, d);
   const int group = hq / hkv;
-  const int wg_rows = hkv * lq_pairs(group);  // workgroups per key chunk: LQ_WG_HEADS heads of one kv group each
+  const int wg_rows = lq_wg_rows(hq, hkv);
+  const int tiles_per_wg = lq_tiles_per_wg(nb_tiles, wg_rows);
+  const int n_chunks = (int)sp_ceil_div(nb_tiles, tiles_per_wg);
+  float2* partial = (float2*)workspace;
+  float2* rowstat = partial + (size_t)hq * n_chunks * LQ_ROWS;
+  const float inv_sqrt_d = sp_inv_sqrt_dim(flags, d);
   PoolArgs pool = {};
   if (kbar != nullptr) pool = pool_args(k, kbar, n, hkv, d, k_stride_n, k_stride_h, bs, SP_POOL_TAIL_TRUE_LENGTH, nullptr);
   const int64_t pool_rows = sp_ceil_div(sp_ceil_div(pool.units, 2), n_chunks);

@@ -61,7 +61,8 @@ def test_lastq_scores_seeded_random_shapes(gpu_device):
         assert torch.allclose(sb, O.block_sum(st, 128), rtol=1e-5, atol=1e-9), tag
 
 
-@pytest.mark.parametrize("hq,hkv,n", [(28, 4, 10007), (32, 8, 4609), (14, 2, 20001), (7, 1, 33000)])
+@pytest.mark.parametrize("hq,hkv,n", [(28, 4, 10007), (32, 8, 4609), (14, 2, 20001), (7, 1, 33000),
+                                      (20, 4, 10007), (8, 8, 30001)])
 def test_lastq_scores_in_chunks_of_any_number_of_tiles(gpu_device, hq, hkv, n):
     """Lengths whose statistics are cut into chunks of 3 to 5 tiles, the last of them short, up to and beyond the number of chunks
     that the probabilities kernel folds itself."""
