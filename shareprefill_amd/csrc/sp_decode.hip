@@ -337,15 +337,34 @@ typedef float ds_floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t ds_u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void* ds_lds_ptr;
 
-// CT: channel tiles of 16 a slice has.  As many waves and steps of the ring as fit one workgroup's LDS.
-template <int D, int CT>
+// CT_: channel tiles of 16 a slice has.  As many waves and steps of the ring as fit the LDS that the workgroup may have.
+template <int D_, int CT_, int WAVES_, int KIB>
 struct DsShape {
+  static constexpr int D = D_, CT = CT_, WAVES = WAVES_;
   static constexpr int K_BYTES = DS_KEYS * D * 2, V_BYTES = DS_KEYS * CT * 32, STEP_BYTES = K_BYTES + V_BYTES;
-  static constexpr int WAVES = D == 64 || CT == 1 ? 8 : CT == 2 ? 7 : CT == 4 ? 6 : 4;
-  static constexpr int NB = 152 * 1024 / (WAVES * STEP_BYTES) < 4 ? 152 * 1024 / (WAVES * STEP_BYTES) : 4;
+  static constexpr int NB = KIB * 1024 / (WAVES * STEP_BYTES) < 4 ? KIB * 1024 / (WAVES * STEP_BYTES) : 4;
   static constexpr int LOADS = STEP_BYTES / 1024;  // of a step
   static constexpr int LDS_BYTES = WAVES * NB * STEP_BYTES;
   static_assert(NB >= 2 && LDS_BYTES >= WAVES * DS_GMAX * (16 * CT + 4) * 4, "");
+};
+// one to a CU
+template <int D, int CT>
+using DsWide = DsShape<D, CT, D == 64 || CT == 1 ? 8 : CT == 2 ? 7 : CT == 4 ? 6 : 4, 152>;
+// two to a CU, and four or more, each taking all channels of a (sequence, kv head): for more of those than CUs (ds_plan)
+template <int D>
+using DsPair = DsShape<D, D / 16, D == 64 ? 4 : 2, 72>;
+template <int D>
+using DsSolo = DsShape<D, D / 16, 1, D == 64 ? 20 : 40>;
+struct DsArgs {
+  const sp_bf16 *q, *k, *v;
+  int n_keys, g, hkv, d, batch;
+  uint32_t hkv_mul;  // i / hkv = (i * hkv_mul) >> 16
+  DcStrides st;
+  float scale_log2;
+  int keys_per_split;
+  float* o_part;
+  float2* ml_part;
+  sp_bf16* out;
 };
 
 __device__ static __forceinline__ float ds_quad_max(float v) {  // over the lanes l, l ^ 16, l ^ 32, l ^ 48 that share a head
@@ -405,11 +424,11 @@ __device__ static __forceinline__ int ds_swz_v(int row) {
 // places the slices of a kv head on one XCD: they read the same keys (4 caches of 2048 keys, 4 kv heads: 13.0 us across two XCDs)
 // FULL: d == D; a smaller head's rows read as zero-padded: its loads behind the row's end read the row's first chunk instead, K's are
 // dropped from the operands and V's channels there are not written
-template <int D, int CT, bool FULL>
-__global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_ring_kernel(
-    const sp_bf16* __restrict__ q, const sp_bf16* __restrict__ k, const sp_bf16* __restrict__ v, int n_keys, int g, int hkv,
-    int d, int batch, uint32_t hkv_mul /* i / hkv = (i * hkv_mul) >> 16 */, DcStrides st, float scale_log2, int keys_per_split, float* __restrict__ o_part, float2* __restrict__ ml_part, sp_bf16* __restrict__ out) {
-  using Shape = DsShape<D, CT>;
+template <class Shape, bool FULL>
+__device__ static __forceinline__ void ds_workgroup(const DsArgs& a) {
+  constexpr int D = Shape::D, CT = Shape::CT;
+  const DcStrides& st = a.st;
+  const int g = a.g, hkv = a.hkv, d = a.d;
   constexpr int KS = D / 32, CW = 16 * CT, WAVES = Shape::WAVES, NB = Shape::NB;  // channel steps of S, channels of the slice
   constexpr int KC = D / 8, VC = CW / 8;                                          // chunks of a row
   constexpr int KI = Shape::K_BYTES / 1024, VI = Shape::V_BYTES / 1024;           // instructions of a step
@@ -421,24 +440,24 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
   int64_t b = blockIdx.z;
   if constexpr (CW < D) {
     const uint32_t i = blockIdx.z * 8 + blockIdx.x;  // (sequence, kv head)
-    b = (i * hkv_mul) >> 16;
+    b = (i * a.hkv_mul) >> 16;
     kvh = i - (uint32_t)b * hkv;
-    if (b >= batch || (!FULL && slice * CW >= d)) return;  // (uniform)
+    if (b >= a.batch || (!FULL && slice * CW >= d)) return;  // (uniform)
   }
   const int64_t bh = b * hkv + kvh;
-  const int begin = split * keys_per_split, n = n_keys - begin < keys_per_split ? n_keys - begin : keys_per_split;
+  const int begin = split * a.keys_per_split, n = a.n_keys - begin < a.keys_per_split ? a.n_keys - begin : a.keys_per_split;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lq = lane & 15, gr = lane >> 4;  // head (or key row, channel) in a 16-wide tile, lane group
   dc_bf16x8 qb[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const bool real = lq < g && (FULL || 32 * ks + 8 * gr < d);
-    const dc_u32x4 raw = *reinterpret_cast<const dc_u32x4*>(q + b * st.q_b + (int64_t)(kvh * g + (lq < g ? lq : 0)) * st.q_h +
+    const dc_u32x4 raw = *reinterpret_cast<const dc_u32x4*>(a.q + b * st.q_b + (int64_t)(kvh * g + (lq < g ? lq : 0)) * st.q_h +
                                                            (FULL || real ? 32 * ks + 8 * gr : 0));
     qb[ks] = __builtin_bit_cast(dc_bf16x8, real ? raw : (dc_u32x4){0, 0, 0, 0});
   }
-  const char* const kh = (const char*)(k + b * st.k_b + kvh * st.k_h + begin * st.k_n);
-  const char* const vh = (const char*)(v + b * st.v_b + kvh * st.v_h + begin * st.v_n);
+  const char* const kh = (const char*)(a.k + b * st.k_b + kvh * st.k_h + begin * st.k_n);
+  const char* const vh = (const char*)(a.v + b * st.v_b + kvh * st.v_h + begin * st.v_n);
   const uint32_t k_row = (uint32_t)st.k_n * 2u, v_row = (uint32_t)st.v_n * 2u;  // bytes
   const uint32_t ring = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)ds_lds + wave * NB * Shape::STEP_BYTES;
 
@@ -537,7 +556,7 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        s[i][j] = kb + 16 * i + 4 * gr + j < n ? s[i][j] * scale_log2 : -INFINITY;
+        s[i][j] = kb + 16 * i + 4 * gr + j < n ? s[i][j] * a.scale_log2 : -INFINITY;
         mx = fmaxf(mx, s[i][j]);
       }
     const float m_new = fmaxf(m, ds_quad_max(mx));
@@ -599,25 +618,56 @@ __global__ __launch_bounds__((DsShape<D, CT>::WAVES * SP_WAVE)) void sp_decode_r
     }
     if (splits > 1) {  // (uniform) the merging kernel goes on
       const int64_t at = (bh * splits + split) * g + h;
-      *reinterpret_cast<dc_floatx4*>(o_part + at * DC_D + c) = acc;
-      if (c == 0) ml_part[at] = make_float2(top, sum);
+      *reinterpret_cast<dc_floatx4*>(a.o_part + at * DC_D + c) = acc;
+      if (c == 0) a.ml_part[at] = make_float2(top, sum);
       continue;
     }
     const float inv = 1.0f / sum;
-    *reinterpret_cast<uint2*>(out + (bh * g + h) * d + slice * CW + c) =
+    *reinterpret_cast<uint2*>(a.out + (bh * g + h) * d + slice * CW + c) =
         make_uint2(dc_pack2(acc[0] * inv, acc[1] * inv), dc_pack2(acc[2] * inv, acc[3] * inv));
   }
 }
+// (the arguments one by one: as one struct they came in one more round of scalar loads, 0.04 us of a step)
+#define DS_PARAMS                                                                                                                        \
+  const sp_bf16 *__restrict__ q, const sp_bf16 *__restrict__ k, const sp_bf16 *__restrict__ v, int n_keys, int g, int hkv, int d,        \
+      int batch, uint32_t hkv_mul, DcStrides st, float scale_log2, int keys_per_split, float *__restrict__ o_part,                       \
+      float2 *__restrict__ ml_part, sp_bf16 *__restrict__ out
+#define DS_ARGS {q, k, v, n_keys, g, hkv, d, batch, hkv_mul, st, scale_log2, keys_per_split, o_part, ml_part, out}
+template <int D, int CT, bool FULL>
+__global__ __launch_bounds__((DsWide<D, CT>::WAVES * SP_WAVE)) void sp_decode_ring_kernel(DS_PARAMS) {
+  ds_workgroup<DsWide<D, CT>, FULL>(DS_ARGS);
+}
+template <int D, bool FULL>
+__global__ __launch_bounds__((DsPair<D>::WAVES * SP_WAVE)) void sp_decode_ring_pair_kernel(DS_PARAMS) {
+  ds_workgroup<DsPair<D>, FULL>(DS_ARGS);
+}
+template <int D, bool FULL>
+__global__ __launch_bounds__((DsSolo<D>::WAVES * SP_WAVE)) void sp_decode_ring_solo_kernel(DS_PARAMS) {
+  ds_workgroup<DsSolo<D>, FULL>(DS_ARGS);
+}
+
+// How a call of the ring kernel is cut: slices of ct channel tiles (all of them: 16 ct = d) or splits of the keys
+enum DsFill { DS_WIDE, DS_PAIR, DS_SOLO };
+struct DsPlan {
+  int ct, splits;
+  DsFill fill;  // (other than DS_WIDE: all channels, no splits)
+};
 
 template <int D, int CT, bool FULL>
 static int ds_launch(const void* q, const void* k, const void* v, int32_t batch, int64_t n, int32_t hq, int32_t hkv, int32_t d, const DcStrides& st,
-                     float scale_log2, int splits, int keys_per_split, float* o_part, float2* ml_part, void* out, hipStream_t s) {
-  using Shape = DsShape<D, CT>;
+                     float scale_log2, const DsPlan& plan, int splits, int keys_per_split, float* o_part, float2* ml_part, void* out, hipStream_t s) {
   const int slices = D / 16 / CT;
   auto launch = [&](dim3 grid, int64_t b0, int32_t count) {
-    hipLaunchKernelGGL((sp_decode_ring_kernel<D, CT, FULL>), grid, dim3(Shape::WAVES * SP_WAVE), 0, s, (const sp_bf16*)q + b0 * st.q_b,
-                       (const sp_bf16*)k + b0 * st.k_b, (const sp_bf16*)v + b0 * st.v_b, (int)n, hq / hkv, (int)hkv, (int)d, (int)count,
-                       (uint32_t)sp_ceil_div(65536, hkv), st, scale_log2, keys_per_split, o_part, ml_part, (sp_bf16*)out + b0 * hq * d);
+    auto go = [&](auto kernel, int waves) {
+      hipLaunchKernelGGL(kernel, grid, dim3(waves * SP_WAVE), 0, s, (const sp_bf16*)q + b0 * st.q_b, (const sp_bf16*)k + b0 * st.k_b,
+                         (const sp_bf16*)v + b0 * st.v_b, (int)n, hq / hkv, (int)hkv, (int)d, (int)count, (uint32_t)sp_ceil_div(65536, hkv), st,
+                         scale_log2, keys_per_split, o_part, ml_part, (sp_bf16*)out + b0 * hq * d);
+    };
+    if constexpr (CT * 16 == D) {
+      if (plan.fill == DS_PAIR) return go(sp_decode_ring_pair_kernel<D, FULL>, DsPair<D>::WAVES);
+      if (plan.fill == DS_SOLO) return go(sp_decode_ring_solo_kernel<D, FULL>, DsSolo<D>::WAVES);
+    }
+    go(sp_decode_ring_kernel<D, CT, FULL>, DsWide<D, CT>::WAVES);
   };
   if (slices > 1)  // (at most 256 workgroups)
     launch(dim3(8, slices, (unsigned)sp_ceil_div((int64_t)batch * hkv, 8)), 0, batch);
@@ -655,12 +705,15 @@ static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
 //   3600 a launch with its first and last step, 3400 the merging one;
 //   a key takes a workgroup 5.2 to 8.6 by the slice's width (64 channels 3.8 to 4.1) and a third of what it takes from memory beside the
 //   others, or, where that is more, what it takes from memory, at 5.85 TB/s.
+// More (sequence, kv head) pairs than CUs are not cut.  Up to 512 of them two workgroups a CU take them in one round; beyond, short caches
+// go to four and more, whose ends pass under each other's loads, and long ones, which keep the memory busy either way, to one.  us, in the
+// wide shape / so, 32 / 8 heads: 264 pairs of 300 keys 16.7 / 13.0, of 4001 126 / 114; 640 of 100 13.8 / 10.9, of 300 26.7 / 22.4, of 2048 114
+// (as a pair 130, solo 118); 1536 of 500 71.7 (solo 74.2); 4096 of 100 63.7 / 43.7, without groups of 200 92.2 / 74.2; 64 channels 640 of
+// 100 10.3 / 7.3, 4096 of 300 73.3 / 58.1, 2048 of 700 68.7 / 63.8, 1536 of 2048 132 (solo 138).
 // A launch's host time, 3300, counts half: whether the host or the GPU bounds a step is the caller's.  us, one launch / two: 1025 keys
 // 9.1 / 8.5 (called one by one 9.5 / 12.9), 2048 14.3 / 8.7; 4 sequences of 1025 9.8 / 10.3, of 2048 16.0 / 12.4; 8 of 700 8.7 / 11.1, of
 // 4001 32.9 / 29.4; 16 of 2000 26.0 / 29.5.
-struct DsPlan {
-  int ct, splits;
-};
+#define DS_SOLO_KEYS 400  // of 128 channels
 static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
   const int64_t bh = (int64_t)batch * hkv;
   const int full = d / 16;  // channel tiles
@@ -670,7 +723,7 @@ static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
     const int64_t shared = alone + (memory < alone ? memory : alone) / 3;
     return 3600 + sp_ceil_div(wgs, 256) * keys * (memory > shared ? memory : shared) / 1000;
   };
-  DsPlan best = {full, 1};
+  DsPlan best = {full, 1, DS_WIDE};
   int64_t least = INT64_MAX;
   for (int ct = 1; ct <= full; ct *= 2) {
     const int64_t wgs = bh * (full / ct);
@@ -682,8 +735,9 @@ static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
   const int64_t splits = 256 / bh < room ? 256 / bh : room;
   if (splits > 1) {
     const int64_t keys = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE, wgs = bh * sp_ceil_div(n, keys);
-    if (cost(full, wgs, wgs, keys) + 3400 + 1650 < least) best = {full, (int)splits};
+    if (cost(full, wgs, wgs, keys) + 3400 + 1650 < least) best = {full, (int)splits, DS_WIDE};
   }
+  if (bh > 256) best.fill = bh <= 512 ? DS_PAIR : n * d <= DS_SOLO_KEYS * 128 ? DS_SOLO : DS_WIDE;
   return best;
 }
 
@@ -735,7 +789,7 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
     const int splits = (int)sp_ceil_div(n, keys_per_split);  // (none without keys)
     float* o_part = (float*)partials;
     float2* ml_part = (float2*)(o_part + (size_t)splits * batch * hq * DC_D);
-    auto go = [&](auto launch) { return launch(q, k, v, batch, n, hq, hkv, d, st, scale_log2, splits, keys_per_split, o_part, ml_part, out, s); };
+    auto go = [&](auto launch) { return launch(q, k, v, batch, n, hq, hkv, d, st, scale_log2, plan, splits, keys_per_split, o_part, ml_part, out, s); };
     auto by_slice = [&](auto whole) {
       constexpr bool FULL = decltype(whole)::value;
       if (d > 64)

@@ -89,7 +89,7 @@ def test_keys_whose_logits_are_minus_infinity(gpu_device, b, n):
 
 
 @pytest.mark.parametrize("b,hq,hkv,n,d", [(1, 8, 2, 300, 128), (1, 8, 2, 3000, 128), (12, 32, 8, 193, 128), (33, 8, 8, 129, 128),
-                                          (1, 14, 2, 1025, 64), (1, 6, 2, 1025, 96)])  # slices of every width, splits
+                                          (1, 14, 2, 1025, 64), (1, 6, 2, 1025, 96), (80, 16, 8, 100, 128)])  # slices of every width, splits
 def test_values_that_are_infinite(gpu_device, b, hq, hkv, n, d):
     """A channel whose values hold one infinity is that infinity, and NaN where they hold both, as in 64 bits: the probabilities'
     second part is zero for some keys and negative for others.  The other channels do not notice."""
@@ -129,3 +129,13 @@ def test_keys_whose_logits_are_minus_infinity_in_large_groups(gpu_device, b, n, 
     out = ops.decode_attention_batch(q, k, v, d ** -0.5)
     some = sorted({0, b // 2, b - 1})
     assert _error(out[some], _exact(q[some], k[some][:, :, seen], v[some][:, :, seen], d ** -0.5)) <= BOUND + 2.0 ** -8
+
+
+@pytest.mark.parametrize("b,hq,hkv,n,d", [
+    (33, 16, 8, 97, 128), (64, 16, 8, 501, 128), (300, 2, 1, 1, 128), (33, 24, 8, 300, 64), (512, 1, 1, 31, 64),  # two workgroups a CU
+    (65, 16, 8, 33, 128), (65, 8, 8, 400, 128), (200, 28, 4, 64, 128), (513, 1, 1, 1, 128), (65, 16, 8, 800, 64), (520, 7, 1, 65, 64),  # more
+    (65, 8, 8, 401, 128), (65, 8, 8, 801, 64),  # one
+    (40, 8, 8, 300, 96), (65, 16, 8, 257, 72), (40, 8, 8, 300, 40), (70, 16, 8, 129, 8)])
+def test_more_pairs_of_sequence_and_kv_head_than_cus(gpu_device, b, hq, hkv, n, d):
+    test_against_64_bits(gpu_device, b, hq, hkv, n, d, False)
+    test_against_64_bits(gpu_device, b, hq, hkv, n, d, True)
