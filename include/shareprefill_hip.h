@@ -267,7 +267,8 @@ int sp_block_sparse_attn_pivot_fwd_bf16(const void* q, const void* k, const void
  * repack and no scheduler area, and writes the pivot heads' maps itself.  Correct for any n up to 131072;
  * sp_short_attn_max_tokens(d) is the length up to which it is the faster of the two on a selection's masks,
  * sp_short_attn_max_dense_tokens(d) where every block is kept, sp_short_attn_max_steady_tokens(d, pattern_threshold) on the masks of a
- * selection at that coverage in a layer whose heads become no pivots.
+ * selection at that coverage in a layer whose heads become no pivots (128 channels: and with a minimum budget of at most a sixth of
+ * the tokens).
  * avg_attn without decision: no head is a pivot, the maps are cleared (with decision only DENSE heads' maps are written).
  * workspace, with decision and avg_attn: sp_attn_pivot_scratch_bytes(n, 128) bytes (block sums) for every head that can be
  * DENSE, or sp_short_attn_workspace_bytes(n, hq) bytes for hq of them.  DENSE heads beyond those it has room for get NaN

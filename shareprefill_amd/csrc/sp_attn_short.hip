@@ -536,23 +536,30 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
 // 64 channels, where the persistent kernel computes on zero-padded tiles (padding counted), 32 / 8 heads: 0.65 8192 148 / 254, 32768
 // 448 / 810, 49152 715 / 1244; 0.95 143 / 253, 583 / 907, 1268 / 1692; 0.99 147 / 261, 1177 / 1422, 2970 / 3100; every block kept 311 / 409,
 // 4920 / 5135, 10775 / 11010; 14 / 2 heads 0.95 32768 333 / 462, every block 2062 / 2198.  The line is where both were once even without
-// the padding; what lies beyond it is not measured but for these lengths, and each pivot's block sums take 16.8 MB there.
+// the padding; layers with pivots beyond it are slower here at low coverage (below), and each pivot's block sums take 16.8 MB there.
 extern "C" int64_t sp_short_attn_max_tokens(int32_t d) {
   return d == 64 ? 32768 : 6656;
 }
 // The same where no pivot is elected, by the coverage the masks are made at (share of the softmax mass: what the density grows with).
 // A pivot's rows keep every block, which the persistent kernel's rows of two share out better: whole passes of an electing layer and a
 // steady one, us here / there, 32 / 8 heads of 128 channels 8192 tokens at 0.95 709 / 665, 9000 at 0.9 775 / 681; 64 channels 40000 at 0.95
-// 4462 / 4666, 100000 at 0.65 19754 / 17016.  Steady layers:
-//   128 channels, 32 / 8 and 28 / 4 heads: 0.65 8192 tokens 185 / 201, 173 / 197, 10007 239 / 257, 219 / 234, 12288 271 / 289, 248 / 263,
-//   16384 362 / 379, 324 / 334; 0.9 8192 201 / 222, 189 / 209, 10007 260 / 270, 238 / 246, 11000 313 / 316, 279 / 283, 12288 332 / 335,
-//   307 / 301; 0.95 8192 237 / 249, 222 / 232, 10007 307 / 310, 286 / 282 (not taken: masks of query-aware heads at 0.95 are
-//   denser, 1162 / 1140 of a decoder layer's half of 8192 tokens);
-//   64 channels, 32 / 8 and 14 / 2 heads: 0.65 36000 570 / 983, 299 / 489, 131072 2078 / 3397, 992 / 1543; 0.95 36000 782 / 1153, 437 / 598,
-//   90001 5319 / 5631, 2401 / 2755, 131072 12202 / 12458, 5986 / 6266; 0.99 65536 5742 / 5806, 2518 / 2798, 90001 11976 / 11675, 5534 / 5696.
+// 4462 / 4666, 100000 at 0.65 19754 / 17016.
+// Query-aware heads keep far more blocks at the same coverage (0.86 of them at 0.9, 0.53 at 0.65 where vertical-slash heads keep 0.2 to
+// 0.3) and are known on the device alone, so a line lies where a layer of nothing else is even.  Steady layers, 128 channels, 32 / 8 and
+// 28 / 4 heads:
+//   query-aware     0.9 7424 474 / 484, 438 / 474, 7680 506 / 505, 457 / 496, 8192 562 / 552, 492 / 531, 10240 807 / 783, 719 / 701;
+//                   0.65 10241 593 / 603, 536 / 551, 11264 672 / 678, 602 / 616, 12288 759 / 749, 661 / 673, 16384 1201 / 1157, 1056 / 1031;
+//   vertical-slash  0.9 7000 181 / 198, 156 / 177, 10240 248 / 266, 229 / 248; 0.65 8192 200 / 209, 182 / 202, 16384 354 / 375, 321 / 330;
+//   at 0.95 8192 237 / 249, 222 / 232, but 1162 / 1140 of a decoder layer's half with query-aware heads there: not taken.
+// A minimum budget sets a floor of its own: of a quarter of 10241 tokens at 0.65 437 / 432, of half of 8192 426 / 414, of half of 16384 1518 /
+// 1401, of a sixth 344 / 353, 383 / 387 at 11264 (that much is asked of the caller).
+// 64 channels, 32 / 8 and 14 / 2 heads: vertical-slash 0.65 36000 546 / 961, 291 / 479, 131072 1965 / 3287, 941 / 1497; 0.95 36000 745 / 1113,
+// 402 / 576, 131072 11717 / 12320, 5784 / 5969; 0.99 65536 5500 / 5627, 2406 / 2780, 90001 11976 / 11675, 5534 / 5696; query-aware 0.65 131072
+// 33557 / 34114, 0.9 65536 15790 / 16352, 131072 60853 / 60756, 27383 / 27736, 0.95 131072 67357 / 67303, 30320 / 30424, 0.99 65536 18809 / 19347;
+// a minimum budget of half of 131072 54434 / 54978.
 extern "C" int64_t sp_short_attn_max_steady_tokens(int32_t d, float pattern_threshold) {
   if (d == 64) return pattern_threshold <= 0.951f ? AS_MAX_NB * AS_BS : pattern_threshold <= 0.991f ? 65536 : sp_short_attn_max_tokens(d);
-  return pattern_threshold <= 0.651f ? 16384 : pattern_threshold <= 0.901f ? 10240 : sp_short_attn_max_tokens(d);
+  return pattern_threshold <= 0.651f ? 11264 : pattern_threshold <= 0.901f ? 7680 : sp_short_attn_max_tokens(d);
 }
 extern "C" int64_t sp_short_attn_max_dense_tokens(int32_t d) {
   return d == 64 ? 32768 : 5120;

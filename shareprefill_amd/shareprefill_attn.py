@@ -200,7 +200,7 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
     further = False  # short past the length up to which every layer is
     if not short and plan_here and block_size == 128:
         short = further = _short_in_steady_layers(sharing, module.layer_idx, num_heads, q_len, head_dim, config.pattern_threshold,
-                                        key_states, value_states)
+                                                  minb, key_states, value_states)
     if model_dim == KERNEL_HEAD_DIM and value_states.stride(2) * 128 >= 2 ** 31:
         short = False  # the short-prompt kernel's offsets inside a block of v have 32 bits, the repack's 64
     if model_dim in PADDED_HEAD_DIMS:
@@ -278,12 +278,14 @@ def _prefill_layer(module, query_states: torch.Tensor, key_states: torch.Tensor,
 
 
 def _short_in_steady_layers(sharing, layer_idx: int, num_heads: int, q_len: int, head_dim: int, pattern_threshold: float,
-                            key_states: torch.Tensor, value_states: torch.Tensor) -> bool:
+                            min_blocks: int, key_states: torch.Tensor, value_states: torch.Tensor) -> bool:
     """Whether a layer past the length where the short-prompt kernel is the faster one in any layer still takes it: not where a
-    cluster's pivot is elected as a rule, nor where its block sums for the possible pivots would pass the 16 GiB that the
+    cluster's pivot is elected as a rule, nor with 128 channels where the minimum budget makes masks denser than the line of the coverage
+    allows for, nor where its block sums for the possible pivots would pass the 16 GiB that the
     persistent kernel's are held to, or a block of k or v the kernel's 32-bit offsets."""
     lib = _lib.load()
     return (q_len <= lib.sp_short_attn_max_steady_tokens(head_dim, pattern_threshold)
+            and (head_dim == 64 or 6 * min_blocks * 128 <= q_len)
             and not sharing.opens_cluster(layer_idx, num_heads)
             and sharing.max_pivots(layer_idx, num_heads) * lib.sp_attn_pivot_scratch_bytes(q_len, 128) <= 16 << 30
             and max(key_states.stride(2), value_states.stride(2)) * 128 < 2 ** 31)
