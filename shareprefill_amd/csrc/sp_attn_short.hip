@@ -69,7 +69,6 @@ typedef uint32_t as_u32x2 __attribute__((ext_vector_type(2)));
 #define AS_P_TOO_LARGE 0x40004000u   // bf16 pair: exponent >= 128 in either half
 
 typedef __attribute__((address_space(3))) void* as_lds_ptr;
-typedef const __attribute__((address_space(1))) void* as_gbl_ptr;
 
 // K and V tiles are [64 keys][D] bf16 in 16-byte chunks, the chunk index XOR-swizzled by the row so that each kind of operand read
 // is free of bank conflicts.  The LDS serves 256 bytes a cycle: 16 lanes of a K read (one chunk of 16 consecutive rows), so K's
@@ -184,8 +183,9 @@ __device__ __forceinline__ float as_groupmax(float v) {
 
 // Args = AsPivotArgs: with the pivots' patterns (an instance of its own: prompts that select nothing, whose launch is the
 // whole layer, run 1.5 % slower with that code in theirs).
-template <int D, typename Args>
-__global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
+// RAISE: the products go before the other workgroups' softmax and loads on the SIMD (as_raise).
+template <int D, typename Args, bool RAISE>
+__device__ __forceinline__ void as_row(const Args a) {
   constexpr int QT = 2;                             // 16-query tiles per wave
   constexpr int KS = D / 32, CT = D / 16;           // channel steps of S, channel tiles of O
   constexpr int WAVES = AS_WAVES, THREADS = AS_THREADS, WQ = 16 * QT;
@@ -346,11 +346,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
         };
         fetch_k(std::integral_constant<int, 0>{});
         fetch_k(std::integral_constant<int, 1>{});
-        // The products go before the other workgroup's softmax and loads on the SIMD (layers, us, without / with: 3001 tokens 103.2 / 100.9,
-        // 28 / 4 heads 98.5 / 95.0, 6600 at coverage 0.99 244.4 / 238.9, 64 channels 6177 117.5 / 115.5; where every workgroup is resident
-        // from the start the long rows wait for the short ones: 1500 71.0 / 71.9, 2048 74.3 / 75.2).  Around S alone it does nothing,
-        // around P . V alone half of that; behind a condition the branches cost what it gives.
-        __builtin_amdgcn_s_setprio(1);
+        if constexpr (RAISE) __builtin_amdgcn_s_setprio(1);
         as_static_for<0, 4>([&](auto kc) {
           constexpr int kt = decltype(kc)::value;
           as_wait_k<(kt < 3 ? KS : 0)>(kr[kt & 1]);
@@ -374,7 +370,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
             for (int j = 0; j < 4; ++j)
               if (half * AS_TILE + 16 * kt + 4 * g + j > q_off + 16 * qt) s[kt][qt][j] = -INFINITY;
       }
-      __builtin_amdgcn_s_setprio(0);
+      if constexpr (RAISE) __builtin_amdgcn_s_setprio(0);
       fetch_v(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
       uint32_t pk[QT][8];
       auto softmax = [&](int qt, int hh) {  // half hh: 32 keys
@@ -392,7 +388,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
         softmax(qt, 0);
         softmax(qt, 1);
       }
-      __builtin_amdgcn_s_setprio(1);
+      if constexpr (RAISE) __builtin_amdgcn_s_setprio(1);
       as_static_for<0, 2>([&](auto hc) {
         constexpr int hh = decltype(hc)::value;
         // The running max is lazy, as in the persistent kernel and in its steps of 32 keys, which gives its bits: it moves
@@ -448,7 +444,7 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
         });
       });
     }
-    __builtin_amdgcn_s_setprio(0);
+    if constexpr (RAISE) __builtin_amdgcn_s_setprio(0);
     if (pu != nullptr && half == 1) {  // pivot head: the block's softmax mass, log2 units
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
@@ -521,7 +517,26 @@ __global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
   }
 }
 
+template <int D, typename Args>
+__global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_kernel(Args a) {
+  as_row<D, Args, true>(a);
+}
+template <int D, typename Args>
+__global__ __launch_bounds__(AS_THREADS, 2) void sp_attn_short_level_kernel(Args a) {
+  as_row<D, Args, false>(a);
+}
+
 // ---- host ---------------------------------------------------------------------------------------------
+// Whether a wave raises its priority around S and P . V, by the rows of the launch.  Where rows wait for a place it lets a CU's workgroups
+// take turns with the matrix core (attention, us, without / with: every block kept, 32 / 8 heads of 128 3001 tokens 98.7 / 92.1, 40 / 8 2432
+// 82.9 / 76.3; 64 channels 4500 125 / 110, 14 / 2 9984 234 / 213; half of them, 28 / 4 of 128 4500 117 / 108).  Where every row is resident
+// from the start, or nearly, the long rows wait for the short ones: 28 / 4 3200 tokens (700 rows) 90.8 / 95.2, 32 / 8 2048 58.6 / 60.1; 64
+// channels 3001 62.5 / 65.6, 14 / 2 6656 (728 rows) 119 / 128, 16128 of 8 / 2 (1008) 304 / 320.  With 128 channels there are 512 places and 720 to
+// 760 rows are even, with 64 768 and 1008 to 1064: a third beyond is taken in by the rows that end first.  A row alone on its CU has nobody to go before; the instance with the
+// priority is 0.3 to 1 % ahead there.  (Around S alone it does nothing, around P . V alone half; behind a condition in the kernel the
+// branches cost what it gives.)
+static bool as_raise(int d, int64_t rows) { return rows <= 256 || rows > (d == 64 ? 1024 : 736); }
+
 // The lines between this kernel and the persistent one, where the latter's shared tiles outweigh its fixed costs.  Whole layers,
 // us here / there, in one call (two runs of one side within 0.5 %).  128 channels:
 //   masks of the selection, 32 query / 8 kv heads: coverage 0.65 6656 tokens 180 / 189, 8192 198 / 202, 10007 243 / 256; 0.95 201 / 210,
@@ -607,9 +622,11 @@ static int as_launch(const char* who, const void* q, const void* k, const void* 
   SP_HIP(hipGetDevice(&dev));
   SP_REQUIRE(dev >= 0 && dev < 64, SP_ERR_UNSUPPORTED, "%s: device index %d", who, dev);
   if (!attr_set[dev]) {
-    const void* kernels[4] = {
+    const void* kernels[8] = {
         (const void*)sp_attn_short_kernel<64, AsArgs>, (const void*)sp_attn_short_kernel<128, AsArgs>,
-        (const void*)sp_attn_short_kernel<64, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, AsPivotArgs>};
+        (const void*)sp_attn_short_kernel<64, AsPivotArgs>, (const void*)sp_attn_short_kernel<128, AsPivotArgs>,
+        (const void*)sp_attn_short_level_kernel<64, AsArgs>, (const void*)sp_attn_short_level_kernel<128, AsArgs>,
+        (const void*)sp_attn_short_level_kernel<64, AsPivotArgs>, (const void*)sp_attn_short_level_kernel<128, AsPivotArgs>};
     for (const void* f : kernels)
       SP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, AS_LDS_BYTES(128)));
     attr_set[dev] = true;
@@ -619,7 +636,10 @@ static int as_launch(const char* who, const void* q, const void* k, const void* 
   };
   auto pick = [&](const auto& args) {
     using Args = std::decay_t<decltype(args)>;
-    d == 64 ? launch(sp_attn_short_kernel<64, Args>, args) : launch(sp_attn_short_kernel<128, Args>, args);
+    if (as_raise(d, nb * hq))
+      d == 64 ? launch(sp_attn_short_kernel<64, Args>, args) : launch(sp_attn_short_kernel<128, Args>, args);
+    else
+      d == 64 ? launch(sp_attn_short_level_kernel<64, Args>, args) : launch(sp_attn_short_level_kernel<128, Args>, args);
   };
   if (pivot != nullptr) {
     AsPivotArgs with;

@@ -24,3 +24,14 @@ def test_nothing_touches_an_operand_read_in_flight():
         count, found = touched_in_flight(_inline_reads_as_transposing(body))
         assert count >= 8
         assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
+
+
+def test_nothing_touches_an_operand_read_in_flight_where_the_priority_stays_level():
+    kernels = _kernels("sp_attn_short.hip", "sp_attn_short_level_kernel")
+    assert len(kernels) == 4
+    for name, body in kernels.items():
+        assert not any("s_setprio" in l for l in body)
+        for lines, least in ((_inline_reads_as_transposing(body), 8), (body, 16)):
+            count, found = touched_in_flight(lines)
+            assert count >= least
+            assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
