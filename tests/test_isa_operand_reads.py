@@ -35,3 +35,15 @@ def test_nothing_touches_an_operand_read_in_flight_where_the_priority_stays_leve
             count, found = touched_in_flight(lines)
             assert count >= least
             assert not found, f"{name}: '{found[0][1]}' while '{found[0][0]}' is in flight"
+
+
+def test_the_first_tile_is_asked_for_before_the_mask_is_there():
+    """The mask's word is a row's first load, the first tile's the next ones: nothing in between may wait for memory."""
+    kernels = _kernels("sp_attn_short.hip", "sp_attn_short_(?:level_)?kernel")
+    assert len(kernels) == 8
+    for name, body in kernels.items():
+        loads = [i for i, l in enumerate(body) if l.strip().startswith(("global_load", "buffer_load", "flat_load"))]
+        first, tile = loads[0], next(i for i in loads if " lds" in body[i])
+        assert "global_load_dwordx2" in body[first] and loads.index(tile) == 1, name
+        waits = [l.strip() for l in body[first:tile] if "s_waitcnt" in l and "vmcnt" in l]
+        assert not waits, f"{name}: '{waits[0]}'"
