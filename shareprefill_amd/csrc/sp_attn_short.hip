@@ -225,12 +225,17 @@ __device__ __forceinline__ void as_row(const Args a) {
     as_issue<D, true>(v_blk, v_row, blk_rows, part, v_lane, at + TILE_BYTES, wave, lane);
   };
   // The row's mask, one word per lane; the kept blocks are walked bit by bit in scalar registers.  The first tile of block 0, which
-  // nearly every row keeps, is on its way before the mask is there (a row that does not fetches its own into the same place: loads
-  // land in order).
+  // nearly every row keeps, is asked for before the word is looked at (a row that does not keep it fetches its own into the same place:
+  // loads land in order); with 64 channels before the word is there: us, with its trimming in front / behind the tile, 300 tokens 10.4 /
+  // 10.2, 700 17.9 / 17.5, 1024 22.9 / 22.4.  With 128 the trimming is a branch in front of the tile, which waits for the word: without
+  // the wait nothing is won (the tile's loads take 600 cycles to issue), and the code of the other form runs 0.5 to 1 % slower, with the wait
+  // or without (700 23.3 / 23.5, 1024 31.1 / 31.3).
   const uint64_t* const mask_row = a.mask + ((int64_t)h * a.nb + r) * a.nbw;
   const int last_w = r >> 6;
   uint64_t lane_word = 0;
   if (lane <= last_w) lane_word = mask_row[lane];
+  if constexpr (D == 128)
+    if (lane == last_w && (r & 63) != 63) lane_word &= (2ull << (r & 63)) - 1ull;
   open_block(0);
   issue(0, 0);
   const int q_off = wave * WQ + lq;  // the first of the lane's queries; the others are 16 further each
@@ -244,9 +249,7 @@ __device__ __forceinline__ void as_row(const Args a) {
     for (int ks = 0; ks < KS; ++ks)
       qb[qt][ks] = __builtin_bit_cast(as_bf16x8, *reinterpret_cast<const uint4*>(src + 32 * ks));
   }
-  // (What needs the word stands behind the loads: a branch in front of them waited for it.  us: 64 channels 300 tokens 10.7 -> 10.5, 700
-  // 18.1 -> 17.7, 128 channels even.)
-  lane_word &= lane == last_w ? ~0ull >> (63 - (r & 63)) : ~0ull;
+  if constexpr (D == 64) lane_word &= lane == last_w ? ~0ull >> (63 - (r & 63)) : ~0ull;  // (no branch: one would wait in front of the loads)
   const uint32_t word_lo = (uint32_t)lane_word, word_hi = (uint32_t)(lane_word >> 32);
   auto word = [&](int w) {
     return (uint64_t)(uint32_t)__builtin_amdgcn_readlane(word_lo, w) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane(word_hi, w) << 32;
