@@ -120,16 +120,19 @@ def test_decode_batch_matches_oracle(gpu_device, b, hq, hkv, n, d):
         assert ((out[i, 0] - ref).abs().mean() / ref.abs().mean()).item() <= MEAN_REL
 
 
-@pytest.mark.parametrize("b", [1, 128, 600])  # the four tiles of a cache: a workgroup each, two to a workgroup, all in one
+# Groups of 17 to 32 heads: the four tiles of a cache are a workgroup each, two to a workgroup, all in one.  Smaller groups: splits, one
+# launch of a workgroup to a CU, more than CUs.
+@pytest.mark.parametrize("b", [1, 128, 600])
+@pytest.mark.parametrize("hq,hkv", [(40, 2), (4, 2)])
 @pytest.mark.parametrize("d", [64, 128])
-def test_decode_weights_that_bf16_holds_are_not_rounded(gpu_device, b, d):
+def test_decode_weights_that_bf16_holds_are_not_rounded(gpu_device, b, hq, hkv, d):
     """The probabilities of a chunk are rounded to bf16 relative to the chunk's largest, whatever the other sequences of
-    the batch: keys whose weights in their tile are bf16 values keep them, though the tiles' largest logits lie
-    fractions of an octave apart."""
+    the batch (groups of 17 heads and more; those of smaller groups are two bf16 values): keys whose weights in their tile are bf16
+    values keep them, though the tiles' largest logits lie fractions of an octave apart."""
     from shareprefill_amd import ops
     from tests.test_gpu_attention_precision import FP32, LN2, bf16_weights, half_ulp, logit_keys
 
-    n, hq, hkv = 512, 4, 2
+    n = 512
     logits = torch.full((n,), -60.0)
     for tile, top in enumerate((3.3, 2.55, 1.9, 2.87)):
         logits[128 * tile:128 * tile + 16] = top + torch.log2(bf16_weights(16, tile))

@@ -46,13 +46,13 @@ def test_against_64_bits(gpu_device, b, hq, hkv, n, d, token_major):
     assert torch.equal(out, ops.decode_attention_batch(q, k, v, d ** -0.5))
 
 
-@pytest.mark.parametrize("n,d", [(200, 128), (1025, 64)])
-def test_results_on_odd_addresses_and_caches_of_one_row_a_token(gpu_device, n, d):
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (24, 2)])  # that kernel's instances of up to 8 and 16 heads a group
+@pytest.mark.parametrize("n,d", [(200, 128), (1025, 64), (3000, 96)])
+def test_results_on_odd_addresses_and_caches_of_one_row_a_token(gpu_device, n, d, hq, hkv):
     """A result that no wide store may write, and keys that are one row for every token (a stride of zero): the former goes to the
     other kernel, whose probabilities are one bf16 value (2^-8 more)."""
     from shareprefill_amd import _lib, ops
 
-    hq, hkv = 8, 2
     gen = torch.Generator(device=gpu_device).manual_seed(n)
     mk = lambda *s: torch.randn(*s, generator=gen, device=gpu_device).to(torch.bfloat16)
     q, k, v = mk(1, hq, 1, d), mk(1, hkv, n, d), mk(1, hkv, n, d)

@@ -49,19 +49,22 @@ def test_no_scratch_where_none_is_asked_for(gpu_device, b, n):
 
 
 @pytest.mark.parametrize("d", [8, 64, 72, 128])
-def test_scratch_may_hold_anything(gpu_device, d):
+@pytest.mark.parametrize("hq,hkv", [(6, 2), (34, 2)])  # the ring kernel's splits, whose padded widths leave part of a partial; the other kernel's
+def test_scratch_may_hold_anything(gpu_device, hq, hkv, d):
     """The second kernel takes nothing from the scratch that the first has not written."""
     import torch
 
     from shareprefill_amd import _lib, ops
 
-    b, hq, hkv, n = 2, 6, 2, 700
+    b, n = 2, 4000
     gen = torch.Generator(device=gpu_device).manual_seed(d)
     q, k, v = (torch.randn(b, h, m, d, generator=gen, device=gpu_device).to(torch.bfloat16) for h, m in ((hq, 1), (hkv, n), (hkv, n)))
     need = _lib.load().sp_decode_batch_workspace_bytes(b, n, hq, hkv)
     assert need > 0
     outs = []
     for byte in (0, 0xFF):  # (zeros, NaN)
-        ops._workspace("decode", need, gpu_device).fill_(byte)
+        scratch = ops._workspace("decode", need, gpu_device)
+        scratch.fill_(byte)
         outs.append(ops.decode_attention_batch(q, k, v, d ** -0.5))
+        assert (scratch != byte).any(), "this call leaves no partials: it does not test what it is for"
     assert outs[0].isfinite().all() and torch.equal(outs[0], outs[1])
