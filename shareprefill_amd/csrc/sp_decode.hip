@@ -330,7 +330,8 @@ __global__ __launch_bounds__(32 * DC_COMBINE_GROUPS) void sp_decode_combine_kern
 // Bound: HBM at 5.85 TB/s of a batch (16 caches of 8000 tokens 100 -> 89 us), the waves' chain of steps otherwise.  K's rows straight from
 // memory into the operand registers (16 rows x 64 bytes an instruction) took 50 cycles an instruction, whole rows by way of LDS take
 // 16 (1025 keys 11.3 -> 6.9 us); a ring one step deeper changes nothing.  us, GPU time in replayed graphs: 200 keys 8.0 -> 3.5, 1025
-// 8.8 -> 6.9, 16 caches of 1025 22.7 -> 15.4, 131072 keys 97.9 -> 97.2; called one by one 200 keys 9.1 -> 8.6, 1025 13.0 -> 9.5.
+// 8.8 -> 6.9, 16 caches of 1025 22.7 -> 15.4, 131072 keys 97.9 -> 97.2; called one by one from Python, arguments in memory included, 200 keys
+// 10.1 -> 9.0, 1025 14.0 -> 9.2, 2048 14.2 -> 12.7.
 #define DS_GMAX 16
 #define DS_KEYS 32  // keys of a wave's step
 typedef float ds_floatx4 __attribute__((ext_vector_type(4)));
