@@ -351,11 +351,11 @@ struct DsShape {
 // one to a CU
 template <int D, int CT>
 using DsWide = DsShape<D, CT, D == 64 || CT == 1 ? 8 : CT == 2 ? 7 : CT == 4 ? 6 : 4, 152>;
-// two to a CU, and four or more, each taking all channels of a (sequence, kv head): for more of those than CUs (ds_plan)
+// two to a CU, and four, each taking all channels of a (sequence, kv head): for more of those than CUs (ds_plan)
 template <int D>
 using DsPair = DsShape<D, D / 16, D == 64 ? 4 : 2, 72>;
 template <int D>
-using DsSolo = DsShape<D, D / 16, 1, D == 64 ? 20 : 40>;
+using DsQuad = DsShape<D, D / 16, D == 64 ? 2 : 1, 40>;
 struct DsArgs {
   const sp_bf16 *q, *k, *v;
   int n_keys, g, hkv, d, batch;
@@ -643,12 +643,12 @@ __global__ __launch_bounds__((DsPair<D>::WAVES * SP_WAVE)) void sp_decode_ring_p
   ds_workgroup<DsPair<D>, FULL>(DS_ARGS);
 }
 template <int D, bool FULL>
-__global__ __launch_bounds__((DsSolo<D>::WAVES * SP_WAVE)) void sp_decode_ring_solo_kernel(DS_PARAMS) {
-  ds_workgroup<DsSolo<D>, FULL>(DS_ARGS);
+__global__ __launch_bounds__((DsQuad<D>::WAVES * SP_WAVE)) void sp_decode_ring_quad_kernel(DS_PARAMS) {
+  ds_workgroup<DsQuad<D>, FULL>(DS_ARGS);
 }
 
 // How a call of the ring kernel is cut: slices of ct channel tiles (all of them: 16 ct = d) or splits of the keys
-enum DsFill { DS_WIDE, DS_PAIR, DS_SOLO };
+enum DsFill { DS_WIDE, DS_PAIR, DS_QUAD };
 struct DsPlan {
   int ct, splits;
   DsFill fill;  // (other than DS_WIDE: all channels, no splits)
@@ -666,7 +666,7 @@ static int ds_launch(const void* q, const void* k, const void* v, int32_t batch,
     };
     if constexpr (CT * 16 == D) {
       if (plan.fill == DS_PAIR) return go(sp_decode_ring_pair_kernel<D, FULL>, DsPair<D>::WAVES);
-      if (plan.fill == DS_SOLO) return go(sp_decode_ring_solo_kernel<D, FULL>, DsSolo<D>::WAVES);
+      if (plan.fill == DS_QUAD) return go(sp_decode_ring_quad_kernel<D, FULL>, DsQuad<D>::WAVES);
     }
     go(sp_decode_ring_kernel<D, CT, FULL>, DsWide<D, CT>::WAVES);
   };
@@ -707,15 +707,16 @@ static int dc_splits(int32_t batch, int64_t n, int32_t hkv) {
 //   a key takes a workgroup 5.2 to 8.6 by the slice's width (64 channels 3.8 to 4.1) and a third of what it takes from memory beside the
 //   others, or, where that is more, what it takes from memory, at 5.85 TB/s.
 // More (sequence, kv head) pairs than CUs are not cut.  Up to 512 of them two workgroups a CU take them in one round; beyond, short caches
-// go to four and more, whose ends pass under each other's loads, and long ones, which keep the memory busy either way, to one.  us, in the
-// wide shape / so, 32 / 8 heads: 264 pairs of 300 keys 16.7 / 13.0, of 4001 126 / 114; 640 of 100 13.8 / 10.9, of 300 26.7 / 22.4, of 2048 114
-// (as a pair 130, solo 118); 1536 of 500 71.7 (solo 74.2); 4096 of 100 63.7 / 43.7, without groups of 200 92.2 / 74.2; 64 channels 640 of
-// 100 10.3 / 7.3, 4096 of 300 73.3 / 58.1, 2048 of 700 68.7 / 63.8, 1536 of 2048 132 (solo 138).
+// go four to a CU, whose ends pass under each other's loads, and long ones, which keep the memory busy either way, one.  us, one to a CU / so,
+// 32 / 8 heads: 264 pairs of 300 keys 16.7 / 13.0, of 4001 126 / 114; 640 of 100 13.8 / 10.9, of 300 26.7 / 22.4, of 2048 114 (two 130, four
+// 118); 1536 of 500 71.7 (four 74.2); 4096 of 100 63.7 / 43.7, without groups of 200 92.2 / 74.2; 96 channels 4096 of 500 149 / 138; 64 channels
+// 640 of 100 10.3 / 6.5, 4096 of 300 73.3 / 57.5, 2048 of 700 68.7 / 66.7, 1536 of 2048 132 (four 144; with one wave to a workgroup, which
+// nine fit of, 138, and 2 to 5 % behind the streaming kernel at 100 keys).
 // A launch's host time, 3300, counts half: whether the host or the GPU bounds a step is the caller's.  us, one launch / two: 1025 keys
 // 9.1 / 8.5 (called one by one 9.5 / 12.9), 2048 14.3 / 8.7; 4 sequences of 1025 9.8 / 10.3, of 2048 16.0 / 12.4; 8 of 700 8.7 / 11.1, of
 // 4001 32.9 / 29.4; 16 of 2000 26.0 / 29.5.
-#define DS_SOLO_KEYS 400  // of 128 channels
-static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
+#define DS_QUAD_KEYS 400  // of 128 channels: what is read counts, a padded head's rows are as long as they are
+static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d, int32_t real_d) {
   const int64_t bh = (int64_t)batch * hkv;
   const int full = d / 16;  // channel tiles
   auto cost = [&](int ct, int64_t heads /* kv heads' keys in flight */, int64_t wgs, int64_t keys) {
@@ -738,7 +739,7 @@ static DsPlan ds_plan(int32_t batch, int64_t n, int32_t hkv, int32_t d) {
     const int64_t keys = sp_ceil_div(sp_ceil_div(n, splits), DC_TILE) * DC_TILE, wgs = bh * sp_ceil_div(n, keys);
     if (cost(full, wgs, wgs, keys) + 3400 + 1650 < least) best = {full, (int)splits, DS_WIDE};
   }
-  if (bh > 256) best.fill = bh <= 512 ? DS_PAIR : n * d <= DS_SOLO_KEYS * 128 ? DS_SOLO : DS_WIDE;
+  if (bh > 256) best.fill = bh <= 512 ? DS_PAIR : n * (d == 64 ? 64 : real_d) <= DS_QUAD_KEYS * 128 ? DS_QUAD : DS_WIDE;
   return best;
 }
 
@@ -785,7 +786,7 @@ static int dc_launch(const void* q, const void* k, const void* v, int32_t batch,
   // (8-byte stores; offsets inside 32 keys and the token count have 32 bits)
   if (g <= DS_GMAX && n < (1 << 30) && (uintptr_t)out % 8 == 0 && st.k_n >= 0 && st.v_n >= 0 && st.k_n < (1 << 25) && st.v_n < (1 << 25)) {
     const float scale_log2 = softmax_scale * 1.4426950408889634f;
-    const DsPlan plan = ds_plan(batch, n, hkv, d > 64 ? 128 : 64);
+    const DsPlan plan = ds_plan(batch, n, hkv, d > 64 ? 128 : 64, d);
     const int keys_per_split = (int)(sp_ceil_div(sp_ceil_div(n, plan.splits), DC_TILE) * DC_TILE);
     const int splits = (int)sp_ceil_div(n, keys_per_split);  // (none without keys)
     float* o_part = (float*)partials;

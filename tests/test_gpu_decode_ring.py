@@ -133,8 +133,9 @@ def test_keys_whose_logits_are_minus_infinity_in_large_groups(gpu_device, b, n, 
 
 @pytest.mark.parametrize("b,hq,hkv,n,d", [
     (33, 16, 8, 97, 128), (64, 16, 8, 501, 128), (300, 2, 1, 1, 128), (33, 24, 8, 300, 64), (512, 1, 1, 31, 64),  # two workgroups a CU
-    (65, 16, 8, 33, 128), (65, 8, 8, 400, 128), (200, 28, 4, 64, 128), (513, 1, 1, 1, 128), (65, 16, 8, 800, 64), (520, 7, 1, 65, 64),  # more
-    (65, 8, 8, 401, 128), (65, 8, 8, 801, 64),  # one
+    (65, 16, 8, 33, 128), (65, 8, 8, 400, 128), (200, 28, 4, 64, 128), (513, 1, 1, 1, 128), (65, 16, 8, 800, 64), (520, 7, 1, 65, 64),  # four
+    (65, 8, 8, 533, 96), (65, 16, 8, 711, 72),  # four, rows as long as they are
+    (65, 8, 8, 401, 128), (65, 8, 8, 801, 64), (65, 8, 8, 534, 96),  # one
     (40, 8, 8, 300, 96), (65, 16, 8, 257, 72), (40, 8, 8, 300, 40), (70, 16, 8, 129, 8)])
 def test_more_pairs_of_sequence_and_kv_head_than_cus(gpu_device, b, hq, hkv, n, d):
     test_against_64_bits(gpu_device, b, hq, hkv, n, d, False)

@@ -172,8 +172,8 @@ def test_nothing_touches_a_transposing_read_in_flight_in_the_decode_ring():
 
 
 def test_nothing_touches_a_transposing_read_in_flight_in_the_decode_rings_of_many_pairs():
-    kernels = _kernels("sp_decode.hip", "sp_decode_ring_(?:pair|solo)_kernel")
-    assert len(kernels) == 8, "whole and padded rows x 64 and 128 channels x two workgroups a CU and more"
+    kernels = _kernels("sp_decode.hip", "sp_decode_ring_(?:pair|quad)_kernel")
+    assert len(kernels) == 8, "whole and padded rows x 64 and 128 channels x two workgroups a CU and four"
     for name, body in kernels.items():
         count, found = touched_in_flight(body)
         assert count >= 2
