@@ -101,7 +101,8 @@ __device__ __forceinline__ uint32_t as_pack2(float a, float b) {
 // 3001 105.0 -> 103.7, 6600 at coverage 0.99 255.4 -> 252.9; 64 channels 6177 tokens 120.4 -> 119.0, 20000 at 0.99 514 -> 499).  Of the
 // rest the loads' issue is 600; spread over the products, rings of three and four tiles, 16 queries a wave in twice the waves (the LDS's
 // reads double: 8 % slower), tiles of 32 keys with a third workgroup on the CU (15 %) and products between the probabilities' arithmetic
-// (a wave alone issues no faster) gain nothing.
+// (a wave alone issues no faster) gain nothing.  The two descriptors beside the walk spill 16 scalars of the 128-channel instance to
+// vector lanes (42 with the pivots' patterns), of which 6 and 8 are read back per block.
 template <int D, bool V>
 __device__ __forceinline__ uint32_t as_lane_off(int64_t stride_n, int wave, int lane) {
   constexpr int CHUNKS = D / 8, ROWS = 64 / CHUNKS;  // chunks per row, rows per wave-instruction
